@@ -1,0 +1,216 @@
+// GEMM with at most 128 rows (or columns) on one side and k contiguous in both operands: one decoding
+// step, or a short prefill, of a projection.
+#include "gemm_tiled.hpp"
+
+namespace miw {
+
+struct skinny_params {
+    const half_t *W, *S;  // wide operand (one row per entry of D's long dimension) and narrow one, k contiguous in both
+    const void *C;
+    void *D;
+    int wide, K;
+    long ldw, lds, sw, ss, sc, sd;  // row pitches and batch strides in elements
+    long cw, cn, dw, dn;            // element strides of C and D along the long and the short dimension
+    int use_c, c_f32, d_f32;
+    float alpha, beta;
+};
+
+constexpr int SKINNY_WAVES = 8;
+
+// What bounds this is the one read of the wide operand from HBM, so nothing goes through LDS on the
+// way in: a lane loads its fragments of v_mfma_f32_16x16x32_f16 (16 contiguous bytes of one row) straight
+// into registers, two buffers of UN chunks each, and the next buffer is requested before the
+// MFMAs of this one.  A workgroup owns 16 * WT entries of the long dimension and all 16 * MT of the short
+// one; its eight wavefronts take the 64-k chunks (128 bytes of a row) in turn, so that together they
+// walk each row in 1 KiB pieces, and add their partial sums in wavefront order through LDS: no second
+// kernel, no workspace, no dependence on timing.  The narrow operand is read again by every workgroup,
+// from the caches; WT = 2 halves those reads where enough workgroups are left.
+template <int MT, int WT>
+__global__ __launch_bounds__(64 * SKINNY_WAVES) void k_gemm_skinny(skinny_params p)
+{
+    constexpr int UN = MT + WT <= 2 ? 4 : MT + WT == 3 ? 3 : MT + WT <= 5 ? 2 : 1;  // two buffers stay below 256 VGPRs
+    __shared__ float4_t part[SKINNY_WAVES][MT][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const long w0 = (long)blockIdx.x * (16 * WT), bt = blockIdx.y;
+    const half_t *W = p.W + bt * p.sw + (w0 + r) * p.ldw + 8 * q;
+    const half_t *S = p.S + bt * p.ss + (long)r * p.lds + 8 * q;
+    const int chunks = p.K / 64, tail = p.K % 64;
+    const int own = (chunks - wave + SKINNY_WAVES - 1) / SKINNY_WAVES;  // chunks wave, wave + 8, ... (K >= 64: none below zero)
+    const int steps = (own + UN - 1) / UN;
+
+    float4_t acc[WT][MT];
+#pragma unroll
+    for (int t = 0; t < WT; t++)
+#pragma unroll
+        for (int m = 0; m < MT; m++) acc[t][m] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    half8_t w[2][UN][WT][2], s[2][UN][MT][2];
+    // A step past the wavefront's last chunk requests that chunk again (in bounds, from the cache) and
+    // compute() skips it.
+    auto request = [&](auto buf, int step) {
+        constexpr int b = decltype(buf)::value;
+#pragma unroll
+        for (int u = 0; u < UN; u++) {
+            const int n = step * UN + u < own ? step * UN + u : own - 1;
+            const long k0 = 64l * (wave + SKINNY_WAVES * n);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+#pragma unroll
+                for (int t = 0; t < WT; t++) w[b][u][t][h] = *(const half8_t *)(W + 16l * t * p.ldw + k0 + 32 * h);
+#pragma unroll
+                for (int m = 0; m < MT; m++) s[b][u][m][h] = *(const half8_t *)(S + 16l * m * p.lds + k0 + 32 * h);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // the requests go out before the MFMAs of the other buffer
+    };
+    auto compute = [&](auto buf, int step) {
+        constexpr int b = decltype(buf)::value;
+#pragma unroll
+        for (int u = 0; u < UN; u++) {
+            if (UN > 1 && step * UN + u >= own) break;
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int t = 0; t < WT; t++)
+#pragma unroll
+                    for (int m = 0; m < MT; m++)
+                        acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[b][u][t][h], s[b][u][m][h], acc[t][m], 0, 0, 0);
+        }
+    };
+    constexpr std::integral_constant<int, 0> b0{};
+    constexpr std::integral_constant<int, 1> b1{};
+    if (steps > 0) request(b0, 0);
+    for (int i = 0; i < steps; i += 2) {
+        if (i + 1 < steps) request(b1, i + 1);
+        compute(b0, i);
+        if (i + 1 >= steps) break;
+        if (i + 2 < steps) request(b0, i + 2);
+        compute(b1, i + 1);
+    }
+    // The 16, 32 or 48 k-values that 64 leaves, by the wavefront whose turn it is; what lies past K is zero in both operands.
+    if (tail && wave == chunks % SKINNY_WAVES) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const bool in = 32 * h + 8 * q < tail;
+            half8_t a[WT], b[MT];
+#pragma unroll
+            for (int t = 0; t < WT; t++) {
+                a[t] = half8_t{};
+                if (in) a[t] = *(const half8_t *)(W + 16l * t * p.ldw + 64l * chunks + 32 * h);
+            }
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+                b[m] = half8_t{};
+                if (in) b[m] = *(const half8_t *)(S + 16l * m * p.lds + 64l * chunks + 32 * h);
+            }
+#pragma unroll
+            for (int t = 0; t < WT; t++)
+#pragma unroll
+                for (int m = 0; m < MT; m++) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], b[m], acc[t][m], 0, 0, 0);
+        }
+    }
+    // Lane (q, r) of a tile holds entries 4q .. 4q + 3 of the long dimension, entry r of the short one.
+    for (int t = 0; t < WT; t++) {
+        if (t) __syncthreads();
+#pragma unroll
+        for (int m = 0; m < MT; m++) part[wave][m][lane] = WT == 1 || t == 0 ? acc[0][m] : acc[WT - 1][m];
+        __syncthreads();
+        if (wave >= MT) continue;  // (MT <= 8: one tile per wavefront)
+        float4_t v = part[0][wave][lane];
+#pragma unroll
+        for (int x = 1; x < SKINNY_WAVES; x++) {
+            const float4_t y = part[x][wave][lane];
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] += y[e];
+        }
+        const long i = w0 + 16 * t + 4 * q, j = 16 * wave + r;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            v[e] *= p.alpha;
+            if (p.use_c) {
+                const long at = bt * p.sc + (i + e) * p.cw + j * p.cn;
+                v[e] = __builtin_fmaf(p.beta, p.c_f32 ? ((const float *)p.C)[at] : (float)((const half_t *)p.C)[at], v[e]);
+            }
+        }
+        const long at = bt * p.sd + i * p.dw + j * p.dn;
+        if (p.d_f32) {
+            float *d = (float *)p.D + at;
+            if (p.dw == 1) *(float4_t *)d = v;
+            else for (int e = 0; e < 4; e++) d[e * p.dw] = v[e];
+        } else {
+            half_t *d = (half_t *)p.D + at;
+            if (p.dw == 1) *(half4_t *)d = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+            else for (int e = 0; e < 4; e++) d[e * p.dw] = (half_t)v[e];
+        }
+    }
+}
+
+// Entries of the long dimension per workgroup: 32 where that leaves two workgroups' worth per CU or the
+// reads of a large narrow operand from the caches outweigh the CUs left idle.
+static int skinny_width(const gemm_params &g)
+{
+    const long wide = g.M <= g.N ? g.N : g.M, narrow = g.M <= g.N ? g.M : g.N;
+    return wide % 32 == 0 && wide * g.batch >= 8192 && narrow >= 64 ? 2 : 1;
+}
+
+// Can k_gemm_skinny run this problem?  One extent of at most 128, k contiguous in both operands, at
+// least one chunk of K, and what its 16-byte loads and 8- or 16-byte stores assume of the alignment.
+bool skinny_fits(const gemm_params &g, int d_type, bool f16acc)
+{
+    const long wide = g.M <= g.N ? g.N : g.M, narrow = g.M <= g.N ? g.M : g.N;
+    if (f16acc || narrow > 128 || g.K < 64 || !g.a_row || g.b_row || g.K > (1l << 30) || wide > (1l << 30)) return false;
+    if (((uintptr_t)g.A & 15) || ((uintptr_t)g.B & 15) || g.lda % 8 || g.ldb % 8 || g.sa % 8 || g.sb % 8) return false;
+    const long dper = d_type == 0 ? 8 : 4;
+    return !((uintptr_t)g.D & 15) && g.ldd % dper == 0 && g.sd % dper == 0;
+}
+
+// Estimated duration in microseconds: launch and reduction, the operands at what HBM gives, and what a CU's
+// workgroups read through its L1.
+double skinny_estimate_us(const gemm_params &g, int c_type, int d_type, int cus)
+{
+    const long wide = g.M <= g.N ? g.N : g.M, narrow = g.M <= g.N ? g.M : g.N;
+    const int wt = skinny_width(g);
+    const double groups = (double)((wide + 16 * wt - 1) / (16 * wt)) * (double)g.batch;
+    const double rounds = __builtin_ceil(groups / cus);
+    const double mn = (double)wide * (double)narrow * (double)g.batch;
+    const double hbm = 2.0 * (double)(wide + narrow) * (double)g.K * (double)g.batch + mn * ((d_type ? 4 : 2) + (g.use_c ? (c_type ? 4 : 2) : 0));
+    const double l1 = rounds * 2.0 * (double)(16 * wt + narrow) * (double)g.K;
+    return 4.0 + (hbm / 5.0e6 > l1 / 0.08e6 ? hbm / 5.0e6 : l1 / 0.08e6);
+}
+
+hipError_t launch_gemm_skinny(const gemm_params &g, int c_type, int d_type, hipStream_t s)
+{
+    skinny_params p;
+    const bool nm = g.M <= g.N;  // the short dimension is M
+    p.W = nm ? g.B : g.A; p.S = nm ? g.A : g.B;
+    p.ldw = nm ? g.ldb : g.lda; p.lds = nm ? g.lda : g.ldb;
+    p.sw = nm ? g.sb : g.sa; p.ss = nm ? g.sa : g.sb;
+    p.wide = (int)(nm ? g.N : g.M); p.K = (int)g.K;
+    const bool d_wide = (g.d_row != 0) == nm, c_wide = (g.c_row != 0) == nm;  // contiguous along the long dimension
+    p.dw = d_wide ? 1 : g.ldd; p.dn = d_wide ? g.ldd : 1;
+    p.cw = c_wide ? 1 : g.ldc; p.cn = c_wide ? g.ldc : 1;
+    p.C = g.C; p.D = g.D; p.sc = g.sc; p.sd = g.sd;
+    p.use_c = g.use_c; p.c_f32 = c_type; p.d_f32 = d_type;
+    p.alpha = g.alpha; p.beta = g.beta;
+    const int mt = (int)((nm ? g.M : g.N) / 16), wt = skinny_width(g);
+    const dim3 grid((unsigned)(p.wide / (16 * wt)), (unsigned)g.batch), block(64 * SKINNY_WAVES);
+    auto go = [&]<int MT>(std::integral_constant<int, MT>) {
+        if (wt == 1) hipLaunchKernelGGL((k_gemm_skinny<MT, 1>), grid, block, 0, s, p);
+        else if constexpr (MT >= 4) hipLaunchKernelGGL((k_gemm_skinny<MT, 2>), grid, block, 0, s, p);
+    };
+    switch (mt) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 5: go(std::integral_constant<int, 5>{}); break;
+    case 6: go(std::integral_constant<int, 6>{}); break;
+    case 7: go(std::integral_constant<int, 7>{}); break;
+    case 8: go(std::integral_constant<int, 8>{}); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+}  // namespace miw

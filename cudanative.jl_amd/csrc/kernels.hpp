@@ -36,6 +36,10 @@ hipError_t launch_wmma_mac(int c_type, int d_type, const void *A, const void *B,
 hipError_t launch_gemm_fragops(const gemm_params &p, int c_type, int d_type, bool f16acc, hipStream_t s);
 // Wavefronts that share one 16x16 tile's K loop in the fragment-op kernel launch_gemm_fragops picks (1: none).
 int fragops_ksplit(const gemm_params &p, bool f16acc);
+// --- gemm_skinny.hip: what launch_gemm_fragops takes for a D with one extent of at most 128 and k contiguous in both operands
+bool skinny_fits(const gemm_params &p, int d_type, bool f16acc);
+double skinny_estimate_us(const gemm_params &p, int c_type, int d_type, int cus);
+hipError_t launch_gemm_skinny(const gemm_params &p, int c_type, int d_type, hipStream_t s);
 hipError_t launch_dummy_store(float *ptr, int threads, hipStream_t s);
 const void *frag_kernel_symbol(const char *name);
 int frag_kernel_count();
