@@ -287,8 +287,7 @@ const std::vector<int> &variant_order()
     return order;
 }
 
-// 1-based id of the LDS-tiled variant for this problem, 0 when none fits.
-int pick_tiled(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place, double *us_out = nullptr)
+int pick_variant(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place)
 {
     // Candidates in the order of variant_order(); a later candidate replaces an earlier one only when it is estimated 3 % faster.
     const std::vector<int> &order = variant_order();
@@ -300,21 +299,8 @@ int pick_tiled(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, i
         const double us = estimate_us(i, p, c_type, d_type);
         if (best < 0 || us < 0.97 * best_us) { best = i; best_us = us; }
     }
-    if (us_out) *us_out = best_us;
-    return best + 1;
-}
-
-int pick_variant(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place)
-{
-    double us = 0.0;
-    const int v = pick_tiled(p, c_type, d_type, f16acc, acc_chunk, in_place, &us);
-    if (v == 0) return miw::tiled_variant_count() + 1;  // fragment-op kernels
-    // 64 to 128 rows or columns with k contiguous in both operands: the kernel that reads the long operand
-    // once, straight into registers, where its estimate is below that of LDS tiles that leave most CUs idle.
-    if (std::max(p.M, p.N) >= 1024 && p.K >= 512 && miw::skinny_fits(p, d_type, f16acc) &&
-        miw::skinny_estimate_us(p, c_type, d_type, g_cu_count > 0 ? g_cu_count : 256) < 0.97 * us)
-        return miw::tiled_variant_count() + 1;
-    return v;
+    if (best >= 0) return best + 1;
+    return miw::tiled_variant_count() + 1;  // fragment-op kernel
 }
 
 // Resolve the variant (0 = pick) and check that it can run this problem; touches no device.
@@ -962,21 +948,22 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     if (p.batch != 1) return fail(MIW_ERR_UNSUPPORTED, "gemm_splitk: one problem per call (batch %lld asked)", (long long)p.batch);
     if (d->variant != 0) return fail(MIW_ERR_INVALID_VALUE, "gemm_splitk: the variant is chosen per slice; desc.variant must be 0");
     if (splits < 0 || splits > 256) return fail(MIW_ERR_INVALID_VALUE, "gemm_splitk: splits must be 0 (choose) or 1..256, got %d", splits);
+    const int nt = miw::tiled_variant_count();
     const bool in_place = c_shares_d(d, p);
     static char dummy alignas(16);
     // Variant and estimated duration of s slices (s = 1: the plain launch); false when no tiled kernel fits.
     auto try_splits = [&](int s, int *variant, double *us) {
         if (p.K % (64l * s)) return false;
         if (s == 1) {
-            const int v = pick_tiled(p, d->c_type, d->d_type, false, 0, in_place);
-            if (v == 0) return false;
+            const int v = pick_variant(p, d->c_type, d->d_type, false, 0, in_place);
+            if (v == nt + 1) return false;
             *variant = v;
             *us = estimate_us(v - 1, p, d->c_type, d->d_type);
             return true;
         }
         const miw::gemm_params q = splitk_slices(p, s, &dummy);
-        const int v = pick_tiled(q, MIW_F32, MIW_F32, false, 0, false);
-        if (v == 0) return false;
+        const int v = pick_variant(q, MIW_F32, MIW_F32, false, 0, false);
+        if (v == nt + 1) return false;
         *variant = v;
         // second kernel: launch, a quarter of a microsecond per slice (each thread adds its slices
         // in order), and the slices, C and D at the same pace as above

@@ -2,6 +2,7 @@
 (flatten/unflatten, fragment broadcasting, DevicePtr), argument validation of the
 C ABI, and that the shared library exports what include/miwmma.h declares."""
 import ctypes
+import itertools
 import os
 import re
 
@@ -252,6 +253,24 @@ def test_gemm_plan_covers_the_problem(miw):
     for k, tiled in ((48, False), (64, True), (80, True), (4112, True)):
         d = G.make_desc(512, 512, k)
         assert (G.plan(d)[0]["variant"] != frag) == tiled and len(G.plan(d)) == 1, k
+
+
+@pytest.mark.parametrize("a_row,b_row", [(False, False), (True, False), (False, True), (True, True)])
+def test_narrow_problems_that_a_tile_fits_run_on_tiles(miw, a_row, b_row):
+    """64 to 128 rows or columns: an LDS tile fits, and every launch of the plan is one, in every operand
+    layout, alone and as what a body of large tiles leaves of a ragged problem."""
+    G, W = miw.GEMM, miw.WMMA
+    frag = G.variants()[-1]["id"]
+    lay = lambda row: W.RowMajor if row else W.ColMajor  # noqa: E731
+    for long, k, narrow, kw in itertools.product((1024, 2064, 4096, 8192), (512, 1040, 2048, 8192), (64, 80, 96, 112, 128),
+                                                 (dict(use_c=False, d_type=np.float16), dict())):
+        for m, n in ((narrow, long), (long, narrow)):
+            for d_row in (False, True):
+                d = G.make_desc(m, n, k, a_layout=lay(a_row), b_layout=lay(b_row), c_layout=lay(d_row), d_layout=lay(d_row), **kw)
+                assert G.pick_variant(d) != frag and all(q["variant"] != frag for q in G.plan(d)), (m, n, k)
+    for m, n, k in ((2064, 2048, 2048), (4144, 4096, 4096), (2480, 3392, 3136), (3888, 2128, 4224), (2112, 4016, 2848)):
+        d = G.make_desc(m, n, k, a_layout=lay(a_row), b_layout=lay(b_row), d_layout=W.RowMajor, d_type=np.float16, use_c=False)
+        assert all(q["variant"] != frag for q in G.plan(d)), (m, n, k)
 
 
 def test_variant_table_and_selection(miw):
