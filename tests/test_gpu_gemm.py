@@ -679,6 +679,67 @@ def test_thin_problems_share_a_tile_between_wavefronts(gpu, orc, al, bl, cl, dl)
                               D2[live].view(np.uint16 if g.d_type == orc.F16 else np.uint32))
 
 
+def _check_block(orc, g, D, want, where):
+    """D's extent equals `want` bit for bit; the padding of its leading dimension still holds the prefill 7."""
+    gr = g.resolved()
+    other, inner = (g.M, g.N) if g.d_layout == orc.ROW else (g.N, g.M)
+    for bt in range(max(gr.batch, 1)):
+        got = D[bt * gr.stride_d: bt * gr.stride_d + gr.ldd * other].reshape(other, gr.ldd)
+        exp = want[bt * gr.stride_d: bt * gr.stride_d + gr.ldd * other].reshape(other, gr.ldd)
+        assert np.array_equal(got[:, :inner], exp[:, :inner]), where
+        assert np.all(got[:, inner:] == 7.0), where
+
+
+@pytest.mark.parametrize("tiles,wide_tiles", [(t, 1) for t in range(1, 9)] + [(t, 2) for t in range(4, 9)])
+def test_narrow_kernel_on_k_contiguous_operands(gpu, orc, tiles, wide_tiles):
+    """The kernel behind the fragment-op id for one extent of at most 128 and k contiguous in both operands:
+    every instance (tiles of 16 of the short extent, tiles of the long extent per workgroup), at chunk
+    counts around its eight wavefronts and their buffers (none for some wavefronts, parts of a buffer,
+    whole buffers, both), with every tail of K.  The short side is D's rows and D's columns in turn; C is
+    absent, Float16, Float32, laid out as D or transposed, or D itself; batches; padded leading dimensions.
+    Bit-exact on integers (every partial sum is exact, |sum| < 2^24), against float64 on random data."""
+    frag = _variants(gpu)[-1]["id"]
+    narrow = 16 * tiles
+    un = {2: 4, 3: 3, 4: 2, 5: 2}.get(tiles + wide_tiles, 1)      # chunks of 64 k-values per buffer
+    counts = (1, 2, 8, 9, 8 * un + 5, 16 * un, 16 * un + 11, 24 * un + 8) if wide_tiles == 1 else (1, 7, 8, 17, 26)
+    for n, chunks in enumerate(counts):
+        # more than 128 workgroups, and for two tiles per workgroup more than 256 of 16 columns
+        wide, batch = ((2064, 1), (272, 8), (688, 3))[n % 3] if wide_tiles == 1 else ((8192, 1), (416, 20), (2080, 4))[n % 3]
+        K = 64 * chunks + 16 * ((n + tiles) % 4)
+        M, N = (narrow, wide) if (n + tiles) % 2 else (wide, narrow)
+        dl, ct, dt = (n >> 1) & 1, (n + tiles) & 1, (n >> 1 ^ n) & 1
+        use_c = n % 4 != 3
+        # up to 64 k-values with C laid out as D belong to the short-K kernel
+        cl = 1 - dl if use_c and (K == 64 or n % 3 == 1) else dl
+        if K == 64 and not use_c:
+            K = 80
+        pad = 8 * (n % 2)
+        g = orc.GemmDesc(M=M, N=N, K=K, a_layout=orc.ROW, b_layout=orc.COL, c_layout=cl, d_layout=dl, c_type=ct, d_type=dt,
+                         use_c=int(use_c), batch=batch, alpha=(1.0, -2.0, 0.5)[n % 3], beta=(1.0, 0.5, -1.0)[n % 3],
+                         lda=K + pad, ldb=K + 2 * pad, ldc=(N if cl == orc.ROW else M) + pad // 2, ldd=(N if dl == orc.ROW else M) + pad)
+        where = (M, N, K, batch, cl, dl, ct, dt, use_c)
+        A, B, C = _inputs(orc, g, 1700 + 100 * tiles + n, ints=True)
+        D = _run(gpu, orc, g, A, B, C if use_c else None, variant=frag, prefill=7.0)
+        _check_block(orc, g, D, orc.gemm(g, A, B, C), where)
+    # C is D, and values that are not whole: against float64, and the same bits on a second run
+    wide, batch = (2064, 1) if wide_tiles == 1 else (2080, 4)
+    K = 16 * 33
+    for M, N in ((narrow, wide), (wide, narrow)):
+        g = orc.GemmDesc(M=M, N=N, K=K, a_layout=orc.ROW, b_layout=orc.COL, c_layout=orc.ROW, d_layout=orc.ROW, alpha=0.75, beta=-1.25, batch=batch)
+        A, B, C = _inputs(orc, g, 2600 + tiles)
+        dA, dB = gpu.DeviceArray(A), gpu.DeviceArray(B)
+        desc = gpu.GEMM.make_desc(M, N, K, a_layout=gpu.WMMA.RowMajor, c_layout=gpu.WMMA.RowMajor, d_layout=gpu.WMMA.RowMajor,
+                                  alpha=0.75, beta=-1.25, batch=batch, variant=frag)
+        outs = []
+        for _ in range(2):
+            dD = gpu.DeviceArray(C.copy())
+            gpu.GEMM.gemm(dA, dB, dD, dD, desc)
+            gpu.synchronize()
+            outs.append(dD.to_host())
+        assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+        assert orc.normalized_error(g, outs[0], orc.gemm_f64(g, A, B, C)) <= TIGHT_F32, (M, N, K)
+
+
 def test_tiled_with_padded_leading_dimensions_and_batch(gpu, orc):
     g = orc.GemmDesc(M=128, N=128, K=192, lda=136, ldb=200, ldc=132, ldd=144, batch=5, a_layout=orc.COL, b_layout=orc.COL)
     A, B, C = _inputs(orc, g, 41)
