@@ -353,17 +353,18 @@ struct gemm_part {
     long m0, n0, k0;  // where the part sits in the caller's problem
 };
 
-// The fragment-op kernels.  Up to 64 k-values with C laid out as D: the short-K kernel, which moves C
-// and D at copy speed.  Otherwise every wavefront walks K alone, 16 k-values per step, straight
-// from global memory.
+// The kernels behind the fragment-op id, in the order launch_gemm_fragops asks.  Up to 64 k-values with C
+// laid out as D: the short-K kernel, which moves C and D at copy speed.  One extent of at most 128 and k contiguous
+// in both operands: the narrow kernel, where it pays.  Few tiles and a long K: several wavefronts share a tile's K
+// loop.  Otherwise every wavefront walks K alone, 16 k-values per step, straight from global memory.
 double estimate_fragops_us(const miw::gemm_params &p, int c_type, int d_type)
 {
     const double mn = (double)p.M * (double)p.N * (double)p.batch;
     const double cd_bytes = mn * (double)(dtype_size(d_type) + (p.use_c ? dtype_size(c_type) : 0));
     const double flop = 2.0 * mn * (double)p.K;
     if (p.K <= 64 && (!p.use_c || p.c_row == p.d_row)) return std::max(6.5, 3.0 + std::max(cd_bytes / 5.5e6, flop / 75e6));
-    if (miw::skinny_fits(p, d_type, false)) return miw::skinny_estimate_us(p, c_type, d_type, g_cu_count > 0 ? g_cu_count : 256);
-    const int split = miw::fragops_ksplit(p, false);  // few tiles, long K: several wavefronts share a tile's K loop
+    if (miw::skinny_pays(p, d_type, false)) return miw::skinny_estimate_us(p, g_cu_count > 0 ? g_cu_count : 256);
+    const int split = miw::fragops_ksplit(p, false);
     const double walk = 0.45 * (double)(p.K / 16) / split + (split > 1 ? 2.0 : 0.0);
     return 5.0 + std::max(walk, std::max(flop / 45e6, cd_bytes / 2.0e6));
 }

@@ -578,11 +578,13 @@ static int ksplit_tiles(const gemm_params &p, int *thin_m)
 // Wavefronts per tile k_gemm_fragops_ksplit would use for this problem, or 1 for the
 // one-wavefront-per-tile kernel: few tiles (fewer than 32 wavefronts per CU of a 256-CU part even
 // with the split) and at least four k-steps per wavefront.
-int fragops_ksplit(const gemm_params &p, bool f16acc)
+int fragops_ksplit(const gemm_params &p, bool f16acc, int *tiles_together)
 {
-    if (f16acc) return 1;
     int thin_m;
-    const long groups = (p.M / 16) * (p.N / 16) / ksplit_tiles(p, &thin_m) * p.batch;  // workgroups
+    const int t = ksplit_tiles(p, &thin_m);
+    if (tiles_together) *tiles_together = t;
+    if (f16acc) return 1;
+    const long groups = (p.M / 16) * (p.N / 16) / t * p.batch;  // workgroups
     int s = 16;
     while (s > 1 && (groups * s > 8192 || p.K / (16l * s) < 4)) s >>= 1;
     return s >= 4 ? s : 1;
@@ -663,7 +665,7 @@ hipError_t launch_wmma_mac(int c_type, int d_type, const void *A, const void *B,
 hipError_t launch_gemm_fragops(const gemm_params &p, int c_type, int d_type, bool f16acc, hipStream_t s)
 {
     if (shortk_fits(p, c_type, d_type, f16acc)) return launch_gemm_shortk(p, c_type, d_type, s);
-    if (skinny_fits(p, d_type, f16acc)) return launch_gemm_skinny(p, c_type, d_type, s);
+    if (skinny_pays(p, d_type, f16acc)) return launch_gemm_skinny(p, c_type, d_type, s);
     if (const int split = fragops_ksplit(p, f16acc); split > 1) {
         int thin_m;
         const int T = ksplit_tiles(p, &thin_m);

@@ -24,7 +24,7 @@ constexpr int SKINNY_WAVES = 8;
 // one; its eight wavefronts take the 64-k chunks (128 bytes of a row) in turn, so that together they
 // walk each row in 1 KiB pieces, and add their partial sums in wavefront order through LDS: no second
 // kernel, no workspace, no dependence on timing.  The narrow operand is read again by every workgroup,
-// from the caches; WT = 2 halves those reads where enough workgroups are left.
+// from the caches; WT = 2 halves those reads.
 // Below K of about 2048 a wavefront has fewer chunks than a buffer, and what bounds it is the requests
 // that go through the CU's L1: each chunk is asked for once (16 x 4096 x 512: 3.5 us; 5.5 us when a buffer
 // that K does not fill asks for its last chunk again; 32 x 4096 x 2048: 8.8 and 11.2).  From there on the
@@ -154,12 +154,16 @@ __global__ __launch_bounds__(64 * SKINNY_WAVES) void k_gemm_skinny(skinny_params
     }
 }
 
-// Entries of the long dimension per workgroup: 32 where that leaves two workgroups' worth per CU or the
-// reads of a large narrow operand from the caches outweigh the CUs left idle.
+constexpr long SKINNY_CUS = 256;  // (one workgroup per CU: the registers of eight wavefronts)
+
+// Tiles of 16 of the long dimension that a workgroup takes: two, with 64 or more of the short one, where
+// one tile each would need a second round over the CUs.  The wavefronts' requests through the L1 are what
+// takes the time then, and two tiles share the narrow operand's (128 x 8192 x 2048: 23 us, 39 with one
+// tile); within one round it is the other way round (128 x 4096 x 2048: 22 and 20).
 static int skinny_width(const gemm_params &g)
 {
     const long wide = g.M <= g.N ? g.N : g.M, narrow = g.M <= g.N ? g.M : g.N;
-    return wide % 32 == 0 && wide * g.batch >= 8192 && narrow >= 64 ? 2 : 1;
+    return wide % 32 == 0 && narrow >= 64 && wide / 16 * g.batch > SKINNY_CUS ? 2 : 1;
 }
 
 // Can k_gemm_skinny run this problem?  One extent of at most 128, k contiguous in both operands, at
@@ -173,18 +177,50 @@ bool skinny_fits(const gemm_params &g, int d_type, bool f16acc)
     return !((uintptr_t)g.D & 15) && g.ldd % dper == 0 && g.sd % dper == 0;
 }
 
-// Estimated duration in microseconds: launch and reduction, the operands at what HBM gives, and what a CU's
-// workgroups read through its L1.
-double skinny_estimate_us(const gemm_params &g, int c_type, int d_type, int cus)
+// Rounds of workgroups over `cus` CUs.
+static long skinny_rounds(const gemm_params &g, long cus)
 {
-    const long wide = g.M <= g.N ? g.N : g.M, narrow = g.M <= g.N ? g.M : g.N;
-    const int wt = skinny_width(g);
-    const double groups = (double)((wide + 16 * wt - 1) / (16 * wt)) * (double)g.batch;
-    const double rounds = __builtin_ceil(groups / cus);
-    const double mn = (double)wide * (double)narrow * (double)g.batch;
-    const double hbm = 2.0 * (double)(wide + narrow) * (double)g.K * (double)g.batch + mn * ((d_type ? 4 : 2) + (g.use_c ? (c_type ? 4 : 2) : 0));
-    const double l1 = rounds * 2.0 * (double)(16 * wt + narrow) * (double)g.K;
-    return 4.0 + (hbm / 5.0e6 > l1 / 0.08e6 ? hbm / 5.0e6 : l1 / 0.08e6);
+    const long wide = g.M <= g.N ? g.N : g.M;
+    return (wide / (16 * skinny_width(g)) * g.batch + cus - 1) / cus;
+}
+
+// Does k_gemm_skinny run this problem faster than the fragment-op kernels (k_gemm_fragops
+// on one wavefront per tile, or k_gemm_fragops_ksplit on 4 to 16)?  Measured over 16 to 128 x 64 to 131072 x
+// 80 to 8192 and batches up to 256 (profiles/gemm_narrow_k_contiguous_sweep.md): where the rule says yes the
+// time is 0.16 to 1.06 of the other kernel's (median 0.77), and where it says no it would be 0.86 or more.
+//   K < 256: the others give a tile to one wavefront, and its chain of steps takes longer than a round of
+//     workgroups here (16 x 4096 x 128: 2.8 us against 4.7).  With more than two rounds the six of eight
+//     wavefronts that have no chunk cost more than the chain (16 x 32768 x 128: 10.7 against 7.5), unless
+//     three tiles or more share the wide operand.
+//   K >= 256, one wavefront per tile there (more than 2048 workgroups): only 16 rows with a short K are faster there
+//     (16 x 65536 x 256: 1.2 times; at K = 512 this kernel takes 0.89, at 1024 0.72).
+//   K >= 256, K split there: the tile reads per CU, the bound of both, decide.  Without tiles of the short
+//     dimension in one workgroup the other kernel spreads few tiles over more CUs (48 x 512 x 4096: 16.6 against
+//     10.0).  Within one round of workgroups this kernel is ahead (16 x 4096 x 512: 3.5 against 3.9; 32 x 4096 x
+//     4096: 14.3 against 17.1); each further round shows its start and its reduction, which a K per round of 1024,
+//     384 or 256 for one, two or three tiles of the short dimension makes up for (16 x 16384: 0.97 at K = 4096,
+//     1.03 at 2048; 32 x 16384: 0.93 at 1536, 1.0 at 1024; 48 x 16384: 0.98 at 1024).
+bool skinny_pays(const gemm_params &g, int d_type, bool f16acc)
+{
+    if (!skinny_fits(g, d_type, f16acc)) return false;
+    const long wide = g.M <= g.N ? g.N : g.M, mt = (g.M <= g.N ? g.M : g.N) / 16;
+    const long rounds = skinny_rounds(g, SKINNY_CUS);
+    if (g.K < 256) return rounds <= 2 || (mt >= 3 && g.K >= 128);
+    int together;
+    if (fragops_ksplit(g, f16acc, &together) == 1) return mt >= 2 || g.K >= 512;
+    if (together == 1 && rounds * (mt + skinny_width(g)) > 2 * ((mt * (wide / 16) * g.batch + SKINNY_CUS - 1) / SKINNY_CUS)) return false;
+    return rounds == 1 || mt >= 4 || g.K >= (mt == 1 ? 1024 : mt == 2 ? 384 : 256) * rounds;
+}
+
+// Estimated duration in microseconds, for the planner: launch, start and reduction of each round of
+// workgroups, and the larger of a CU's requests through its L1 (0.96 ns per tile row of 16 and k-value) and the
+// operands at 3.7 TB/s.  Fitted to the launches of the same sweep that skinny_pays takes: within 20 % on nine of ten.
+double skinny_estimate_us(const gemm_params &g, int cus)
+{
+    const long rounds = skinny_rounds(g, cus), narrow = g.M <= g.N ? g.M : g.N;
+    const double l1 = 0.96e-3 * (double)rounds * (double)(narrow / 16 + skinny_width(g)) * (double)g.K;
+    const double hbm = 2.0 * (double)(g.M + g.N) * (double)g.K * (double)g.batch / 3.7e6;
+    return 3.0 + 1.1 * (double)rounds + (l1 > hbm ? l1 : hbm);
 }
 
 hipError_t launch_gemm_skinny(const gemm_params &g, int c_type, int d_type, hipStream_t s)

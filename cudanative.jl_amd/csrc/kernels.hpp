@@ -34,11 +34,14 @@ hipError_t launch_wmma_mac(int c_type, int d_type, const void *A, const void *B,
                            long ldb, long ldc, long ldd, int a_row, int b_row, int c_row, int d_row, int use_c,
                            int shared, float alpha, float beta, hipStream_t s);
 hipError_t launch_gemm_fragops(const gemm_params &p, int c_type, int d_type, bool f16acc, hipStream_t s);
-// Wavefronts that share one 16x16 tile's K loop in the fragment-op kernel launch_gemm_fragops picks (1: none).
-int fragops_ksplit(const gemm_params &p, bool f16acc);
-// --- gemm_skinny.hip: what launch_gemm_fragops takes for a D with one extent of at most 128 and k contiguous in both operands
+// Wavefronts that would share one 16x16 tile's K loop in k_gemm_fragops_ksplit (1: k_gemm_fragops runs instead);
+// *tiles_together (may be null) = tiles a workgroup of it takes together.
+int fragops_ksplit(const gemm_params &p, bool f16acc, int *tiles_together = nullptr);
+// --- gemm_skinny.hip: D with one extent of at most 128 and k contiguous in both operands.  Can the kernel run
+// the problem; is it the one launch_gemm_fragops takes; its estimated duration.
 bool skinny_fits(const gemm_params &p, int d_type, bool f16acc);
-double skinny_estimate_us(const gemm_params &p, int c_type, int d_type, int cus);
+bool skinny_pays(const gemm_params &p, int d_type, bool f16acc);
+double skinny_estimate_us(const gemm_params &p, int cus);
 hipError_t launch_gemm_skinny(const gemm_params &p, int c_type, int d_type, hipStream_t s);
 hipError_t launch_dummy_store(float *ptr, int threads, hipStream_t s);
 const void *frag_kernel_symbol(const char *name);

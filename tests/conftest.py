@@ -1,3 +1,4 @@
+import ctypes
 import importlib.util
 import os
 import sys
@@ -65,3 +66,31 @@ def orc():
     from oracle import oracle
     oracle.lib()
     return oracle
+
+
+class _GemmParams(ctypes.Structure):
+    """gemm_params of csrc/kernels.hpp, which the library's own dispatch rules take."""
+    _fields_ = ([(x, ctypes.c_void_p) for x in "ABCD"] +
+                [(x, ctypes.c_long) for x in ("M", "N", "K", "lda", "ldb", "ldc", "ldd", "sa", "sb", "sc", "sd", "batch")] +
+                [(x, ctypes.c_int) for x in ("a_row", "b_row", "c_row", "d_row", "use_c")] +
+                [("alpha", ctypes.c_float), ("beta", ctypes.c_float)])
+
+
+@pytest.fixture(scope="session")
+def narrow_kernel(miw):
+    """narrow_kernel(rule, M, N, K, ...): what the library's own rule `rule` says of the kernel for D with one
+    extent of at most 128 ("fits": it can run the problem; "pays": launch_gemm_fragops takes it)."""
+    lib = ctypes.CDLL(miw._lib.LIB_PATH)
+
+    def ask(rule, M, N, K, batch=1, a_row=1, b_row=0, c_row=1, d_row=1, use_c=0, d_type=0, f16acc=False, lda=0, ldb=0, ldd=0, offset=0):
+        f = getattr(lib, "_ZN3miw11skinny_%sERKNS_11gemm_paramsEib" % rule)
+        f.restype, f.argtypes = ctypes.c_bool, [ctypes.POINTER(_GemmParams), ctypes.c_int, ctypes.c_bool]
+        lda, ldb = lda or (K if a_row else M), ldb or (N if b_row else K)
+        ldc, ldd = N if c_row else M, ldd or (N if d_row else M)
+        base = 1 << 32
+        p = _GemmParams(base + offset, base + (1 << 40), base + (2 << 40), base + (3 << 40), M, N, K, lda, ldb, ldc, ldd,
+                        lda * (M if a_row else K), ldb * (K if b_row else N), ldc * (M if c_row else N), ldd * (M if d_row else N),
+                        batch, a_row, b_row, c_row, d_row, use_c, 1.0, 1.0)
+        return f(ctypes.byref(p), d_type, f16acc)
+
+    return ask

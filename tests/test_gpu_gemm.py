@@ -691,7 +691,7 @@ def _check_block(orc, g, D, want, where):
 
 
 @pytest.mark.parametrize("tiles,wide_tiles", [(t, 1) for t in range(1, 9)] + [(t, 2) for t in range(4, 9)])
-def test_narrow_kernel_on_k_contiguous_operands(gpu, orc, tiles, wide_tiles):
+def test_narrow_kernel_on_k_contiguous_operands(gpu, orc, narrow_kernel, tiles, wide_tiles):
     """The kernel behind the fragment-op id for one extent of at most 128 and k contiguous in both operands:
     every instance (tiles of 16 of the short extent, tiles of the long extent per workgroup), at chunk
     counts around its eight wavefronts and their buffers (none for some wavefronts, parts of a buffer,
@@ -718,6 +718,7 @@ def test_narrow_kernel_on_k_contiguous_operands(gpu, orc, tiles, wide_tiles):
                          use_c=int(use_c), batch=batch, alpha=(1.0, -2.0, 0.5)[n % 3], beta=(1.0, 0.5, -1.0)[n % 3],
                          lda=K + pad, ldb=K + 2 * pad, ldc=(N if cl == orc.ROW else M) + pad // 2, ldd=(N if dl == orc.ROW else M) + pad)
         where = (M, N, K, batch, cl, dl, ct, dt, use_c)
+        assert narrow_kernel("pays", M, N, K, batch=batch, c_row=cl == orc.ROW, d_row=dl == orc.ROW), where
         A, B, C = _inputs(orc, g, 1700 + 100 * tiles + n, ints=True)
         D = _run(gpu, orc, g, A, B, C if use_c else None, variant=frag, prefill=7.0)
         _check_block(orc, g, D, orc.gemm(g, A, B, C), where)
@@ -725,6 +726,7 @@ def test_narrow_kernel_on_k_contiguous_operands(gpu, orc, tiles, wide_tiles):
     wide, batch = (2064, 1) if wide_tiles == 1 else (2080, 4)
     K = 16 * 33
     for M, N in ((narrow, wide), (wide, narrow)):
+        assert narrow_kernel("pays", M, N, K, batch=batch)
         g = orc.GemmDesc(M=M, N=N, K=K, a_layout=orc.ROW, b_layout=orc.COL, c_layout=orc.ROW, d_layout=orc.ROW, alpha=0.75, beta=-1.25, batch=batch)
         A, B, C = _inputs(orc, g, 2600 + tiles)
         dA, dB = gpu.DeviceArray(A), gpu.DeviceArray(B)

@@ -273,6 +273,29 @@ def test_narrow_problems_that_a_tile_fits_run_on_tiles(miw, a_row, b_row):
         assert all(q["variant"] != frag for q in G.plan(d)), (m, n, k)
 
 
+def test_narrow_kernel_runs_where_it_was_measured_ahead(narrow_kernel):
+    """Which problems behind the fragment-op id the kernel for k-contiguous narrow ones takes, on both sides of every line
+    of its rule.  The refused ones were up to 2.6 times slower there than on the kernels that take them now."""
+    for yes, M, N, K, batch in (
+            # fewer than 256 k-values: two rounds of workgroups, or any number with three tiles together and 128 k-values
+            (True, 16, 4096, 80, 1), (True, 16, 8192, 240, 1), (False, 16, 8208, 240, 1), (False, 16, 65536, 80, 1), (False, 16, 4096, 80, 8),
+            (False, 32, 512, 80, 64), (True, 48, 65536, 128, 1), (False, 48, 65536, 112, 1),
+            # one wavefront per tile on the other side
+            (True, 48, 65536, 256, 1), (False, 16, 65536, 496, 1), (True, 16, 65536, 512, 1), (True, 32, 128, 512, 256),
+            # K split on the other side, few tiles: the tile reads per CU
+            (False, 32, 32, 4096, 1), (False, 48, 48, 4096, 1), (False, 48, 512, 4096, 1), (False, 48, 112, 2048, 1), (True, 16, 16, 1024, 1),
+            (True, 48, 1024, 4096, 1), (False, 128, 1024, 4096, 1), (True, 128, 3072, 4096, 1), (False, 32, 64, 1024, 16), (True, 32, 256, 1024, 16),
+            # rounds of workgroups
+            (True, 16, 4096, 512, 1), (False, 16, 8192, 2032, 1), (True, 16, 8192, 2048, 1), (False, 16, 16384, 4080, 1), (True, 16, 16384, 4096, 1),
+            (False, 32, 8192, 752, 1), (True, 32, 8192, 768, 1), (False, 48, 8192, 496, 1), (True, 48, 8192, 512, 1), (True, 64, 16384, 256, 1)):
+        for m, n in ((M, N), (N, M)):
+            assert narrow_kernel("pays", m, n, K, batch=batch) == yes, (m, n, K, batch)
+    # what it cannot run it does not take
+    for no in (dict(a_row=0), dict(b_row=1), dict(f16acc=True), dict(lda=4097), dict(ldb=4100), dict(ldd=4100), dict(offset=8)):
+        assert not narrow_kernel("pays", 16, 4096, 4096, **no), no
+    assert not narrow_kernel("pays", 144, 4096, 4096) and not narrow_kernel("pays", 16, 4096, 48)
+
+
 def test_variant_table_and_selection(miw):
     G = miw.GEMM
     vs = G.variants()
