@@ -391,7 +391,8 @@ def main():
         roof = {"bound": "mfma", "achieved": flops / (kernel_ms * 1e-3) / 1e12, "peak": PEAK_F16_DENSE_TFLOPS,
                 "unit": "TFLOP/s"}
     roof["frac"] = roof["achieved"] / roof["peak"]
-    family = ("k_gemm_fragops" if vinfo["fragment_ops"] else
+    family = ("k_gemm_skinny" if vinfo["name"] == "narrow_k_contiguous" else
+              "k_gemm_fragops" if vinfo["fragment_ops"] else
               "k_gemm_w128" if vinfo["wave128"] else
               "k_gemm_tiled" if not vinfo["pingpong"] else
               "k_gemm_pp" if vinfo["block"][:2] == (256, 256) else "k_gemm_pp64")

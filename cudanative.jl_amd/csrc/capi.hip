@@ -287,7 +287,13 @@ const std::vector<int> &variant_order()
     return order;
 }
 
-int pick_variant(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place)
+// Ids behind the tiled variants: the kernel for one extent of at most 128 with k contiguous in both operands,
+// and the fragment-op kernels.  Both take every problem (a problem the first cannot run goes to the others).
+int narrow_id() { return miw::tiled_variant_count() + 1; }
+int fragops_id() { return miw::tiled_variant_count() + 2; }
+
+// 1-based id of the LDS-tiled variant for this problem and its estimated duration, 0 when none fits.
+int pick_tiled(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place, double *us_out = nullptr)
 {
     // Candidates in the order of variant_order(); a later candidate replaces an earlier one only when it is estimated 3 % faster.
     const std::vector<int> &order = variant_order();
@@ -299,18 +305,25 @@ int pick_variant(const miw::gemm_params &p, int c_type, int d_type, bool f16acc,
         const double us = estimate_us(i, p, c_type, d_type);
         if (best < 0 || us < 0.97 * best_us) { best = i; best_us = us; }
     }
-    if (best >= 0) return best + 1;
-    return miw::tiled_variant_count() + 1;  // fragment-op kernel
+    if (us_out) *us_out = best_us;
+    return best + 1;
+}
+
+int pick_variant(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place)
+{
+    if (const int v = pick_tiled(p, c_type, d_type, f16acc, acc_chunk, in_place))
+        return miw::skinny_beats_tiles(p, d_type, f16acc) ? narrow_id() : v;
+    // Thinner than every tile: the fragment-op kernels, which hand the problem on where that pays.
+    return std::min(p.M, p.N) >= 64 && miw::skinny_pays(p, d_type, f16acc) ? narrow_id() : fragops_id();
 }
 
 // Resolve the variant (0 = pick) and check that it can run this problem; touches no device.
 int check_gemm(const miw_gemm_desc *d, const miw::gemm_params &p, bool f16acc, bool in_place, int *variant_out)
 {
-    const int nt = miw::tiled_variant_count();
     int variant = d->variant;
-    if (variant < 0 || variant > nt + 1) return fail(MIW_ERR_INVALID_VALUE, "gemm: unknown variant %d", variant);
+    if (variant < 0 || variant > fragops_id()) return fail(MIW_ERR_INVALID_VALUE, "gemm: unknown variant %d", variant);
     if (variant == 0) variant = pick_variant(p, d->c_type, d->d_type, f16acc, d->acc_chunk, in_place);
-    if (variant == nt + 1) {
+    if (variant >= narrow_id()) {
         if (f16acc && d->acc_chunk != 0 && d->acc_chunk != 16)
             return fail(MIW_ERR_UNSUPPORTED, "gemm: the fragment-op kernel rounds every 16 k-values (acc_chunk %d asked)",
                         d->acc_chunk);
@@ -331,7 +344,8 @@ int check_gemm(const miw_gemm_desc *d, const miw::gemm_params &p, bool f16acc, b
 
 int launch_gemm(int variant, const miw::gemm_params &p, int c_type, int d_type, bool f16acc, hipStream_t s)
 {
-    if (variant == miw::tiled_variant_count() + 1) HIP_TRY(miw::launch_gemm_fragops(p, c_type, d_type, f16acc, s));
+    if (variant == narrow_id() && miw::skinny_fits(p, d_type, f16acc)) HIP_TRY(miw::launch_gemm_skinny(p, c_type, d_type, s));
+    else if (variant >= narrow_id()) HIP_TRY(miw::launch_gemm_fragops(p, c_type, d_type, f16acc, s));
     else HIP_TRY(miw::launch_gemm_tiled(variant - 1, p, c_type, d_type, f16acc, s));
     return 0;
 }
@@ -347,14 +361,14 @@ int launch_gemm(int variant, const miw::gemm_params &p, int c_type, int d_type, 
 //     seventeen rows of large tiles, i.e. two rounds over the CUs).
 // A cut is made only where the estimate says it pays.
 struct gemm_part {
-    int variant;  // 1-based; tiled_variant_count() + 1: the fragment-op kernel
+    int variant;  // 1-based
     int c_type;
     miw::gemm_params p;
     long m0, n0, k0;  // where the part sits in the caller's problem
 };
 
 // The kernels behind the fragment-op id, in the order launch_gemm_fragops asks.  Up to 64 k-values with C
-// laid out as D: the short-K kernel, which moves C and D at copy speed.  One extent of at most 128 and k contiguous
+// laid out as D: the short-K kernel, which moves C and D at copy speed.  Less than 64 rows or columns and k contiguous
 // in both operands: the narrow kernel, where it pays.  Few tiles and a long K: several wavefronts share a tile's K
 // loop.  Otherwise every wavefront walks K alone, 16 k-values per step, straight from global memory.
 double estimate_fragops_us(const miw::gemm_params &p, int c_type, int d_type)
@@ -363,7 +377,7 @@ double estimate_fragops_us(const miw::gemm_params &p, int c_type, int d_type)
     const double cd_bytes = mn * (double)(dtype_size(d_type) + (p.use_c ? dtype_size(c_type) : 0));
     const double flop = 2.0 * mn * (double)p.K;
     if (p.K <= 64 && (!p.use_c || p.c_row == p.d_row)) return std::max(6.5, 3.0 + std::max(cd_bytes / 5.5e6, flop / 75e6));
-    if (miw::skinny_pays(p, d_type, false)) return miw::skinny_estimate_us(p, g_cu_count > 0 ? g_cu_count : 256);
+    if (miw::fragops_run_skinny(p, d_type, false)) return miw::skinny_estimate_us(p, g_cu_count > 0 ? g_cu_count : 256);
     const int split = miw::fragops_ksplit(p, false);
     const double walk = 0.45 * (double)(p.K / 16) / split + (split > 1 ? 2.0 : 0.0);
     return 5.0 + std::max(walk, std::max(flop / 45e6, cd_bytes / 2.0e6));
@@ -384,13 +398,17 @@ miw::gemm_params sub_block(const miw::gemm_params &p, int c_type, int d_type, lo
 struct gemm_planner {
     int d_type;
     bool in_place;  // C and D share memory
-    int nt = miw::tiled_variant_count();
 
     double single(const miw::gemm_params &p, int c_type, long m0, long n0, long k0, std::vector<gemm_part> *out) const
     {
         const int v = pick_variant(p, c_type, d_type, false, 0, in_place);
         if (out) out->push_back(gemm_part{v, c_type, p, m0, n0, k0});
-        return v == nt + 1 ? estimate_fragops_us(p, c_type, d_type) : estimate_us(v - 1, p, c_type, d_type);
+        if (v == fragops_id()) return estimate_fragops_us(p, c_type, d_type);
+        if (v != narrow_id()) return estimate_us(v - 1, p, c_type, d_type);
+        // (the tiles' paces are those of operands that start on whole cache lines; the cuts are weighed as if these did)
+        double us = 0.0;
+        const double narrow_us = miw::skinny_estimate_us(p, g_cu_count > 0 ? g_cu_count : 256);
+        return pick_tiled(p, c_type, d_type, false, 0, in_place, &us) ? std::min(us, narrow_us) : narrow_us;
     }
 
     // Appends the parts of p to *out (when given) and returns the estimated duration.
@@ -465,7 +483,7 @@ int plan_gemm(const miw_gemm_desc *d, const miw::gemm_params &p, bool f16acc, bo
         gemm_planner pl{d->d_type, in_place};
         pl.plan(p, d->c_type, 0, 0, 0, 0, parts);
         for (const gemm_part &part : *parts)
-            if (part.variant == pl.nt + 1 && (part.p.M / 16) * (part.p.N / 16) / 4 >= (1l << 31))
+            if (part.variant >= narrow_id() && (part.p.M / 16) * (part.p.N / 16) / 4 >= (1l << 31))
                 return fail(MIW_ERR_UNSUPPORTED, "gemm: %lld x %lld tiles of 16 x 16 do not fit the launch grid",
                             (long long)(part.p.M / 16), (long long)(part.p.N / 16));
     }
@@ -776,15 +794,22 @@ int miw_wmma_mac(const miw_mac_desc *d, const void *A, const void *B, const void
 
 // ------------------------------------------------------------------ GEMM ---
 
-int miw_gemm_variant_count(void) { return miw::tiled_variant_count() + 1; }
+int miw_gemm_variant_count(void) { return fragops_id(); }
 
 int miw_gemm_variant_info_get(int variant, miw_gemm_variant_info *out)
 {
     if (!out) return fail(MIW_ERR_NULL_POINTER, "gemm_variant_info: null output");
-    const int nt = miw::tiled_variant_count();
-    if (variant < 1 || variant > nt + 1) return fail(MIW_ERR_INVALID_VALUE, "gemm_variant_info: unknown variant %d", variant);
+    if (variant < 1 || variant > fragops_id()) return fail(MIW_ERR_INVALID_VALUE, "gemm_variant_info: unknown variant %d", variant);
     memset(out, 0, sizeof(*out));
-    if (variant == nt + 1) {
+    if (variant == narrow_id()) {
+        snprintf(out->name, sizeof(out->name), "narrow_k_contiguous");
+        out->block_m = 16; out->block_n = 16; out->block_k = 64;
+        out->waves_m = 1; out->waves_n = 1;  // (its eight wavefronts share K)
+        out->stages = 0; out->lds_bytes = 0; out->fragment_ops = 1;
+        out->f16_accumulate = 1;
+        return 0;
+    }
+    if (variant == fragops_id()) {
         snprintf(out->name, sizeof(out->name), "fragment_ops");
         out->block_m = 16; out->block_n = 16; out->block_k = 16;
         out->waves_m = 1; out->waves_n = 1; out->stages = 1; out->lds_bytes = 0; out->fragment_ops = 1;
@@ -803,13 +828,12 @@ int miw_gemm_variant_info_get(int variant, miw_gemm_variant_info *out)
 int miw_gemm_variant_supports(const miw_gemm_desc *desc, int variant, int *supported)
 {
     if (!supported) return fail(MIW_ERR_NULL_POINTER, "gemm_variant_supports: null output");
-    const int nt = miw::tiled_variant_count();
-    if (variant < 1 || variant > nt + 1) return fail(MIW_ERR_INVALID_VALUE, "gemm_variant_supports: unknown variant %d", variant);
+    if (variant < 1 || variant > fragops_id()) return fail(MIW_ERR_INVALID_VALUE, "gemm_variant_supports: unknown variant %d", variant);
     miw::gemm_params p;
     bool f16acc;
-    static char dummy alignas(16);
+    static char dummy alignas(128);
     if (int rc = resolve_gemm(desc, &dummy, &dummy, &dummy, &dummy, &p, &f16acc)) return rc;
-    if (variant == nt + 1) *supported = !(f16acc && desc->acc_chunk != 0 && desc->acc_chunk != 16);
+    if (variant >= narrow_id()) *supported = !(f16acc && desc->acc_chunk != 0 && desc->acc_chunk != 16);
     else *supported = tiled_fits(variant - 1, p, desc->c_type, desc->d_type, f16acc, desc->acc_chunk, false) ? 1 : 0;
     return 0;
 }
@@ -820,7 +844,7 @@ int miw_gemm_pick_variant(const miw_gemm_desc *desc, int *variant)
     miw::gemm_params p;
     bool f16acc;
     // Alignment of real pointers cannot be known here: assume aligned operands.
-    static char dummy alignas(16);
+    static char dummy alignas(128);
     if (int rc = resolve_gemm(desc, &dummy, &dummy, &dummy, &dummy, &p, &f16acc)) return rc;
     *variant = pick_variant(p, desc->c_type, desc->d_type, f16acc, desc->acc_chunk, false);
     return 0;
@@ -854,7 +878,7 @@ int miw_gemm_acc_chunk(const miw_gemm_desc *desc, int *acc_chunk)
     int v = 0;
     if (int rc = miw_gemm_pick_variant(desc, &v)) return rc;
     if (desc->variant != 0) v = desc->variant;
-    *acc_chunk = v == miw::tiled_variant_count() + 1 ? 16 : miw::tiled_f16acc_chunk();
+    *acc_chunk = v >= narrow_id() ? 16 : miw::tiled_f16acc_chunk();
     return 0;
 }
 
@@ -867,7 +891,7 @@ int miw_gemm_resolve(const miw_gemm_desc *desc, const void *A, const void *B, co
     if (int rc = plan_gemm(desc, p, f16acc, c_shares_d(desc, p), &parts)) return rc;
     const int v = parts.empty() ? 0 : parts[0].variant;
     if (variant) *variant = v;
-    if (acc_chunk) *acc_chunk = !f16acc ? 0 : v == miw::tiled_variant_count() + 1 ? 16 : miw::tiled_f16acc_chunk();
+    if (acc_chunk) *acc_chunk = !f16acc ? 0 : v >= narrow_id() ? 16 : miw::tiled_f16acc_chunk();
     return 0;
 }
 
@@ -949,22 +973,19 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     if (p.batch != 1) return fail(MIW_ERR_UNSUPPORTED, "gemm_splitk: one problem per call (batch %lld asked)", (long long)p.batch);
     if (d->variant != 0) return fail(MIW_ERR_INVALID_VALUE, "gemm_splitk: the variant is chosen per slice; desc.variant must be 0");
     if (splits < 0 || splits > 256) return fail(MIW_ERR_INVALID_VALUE, "gemm_splitk: splits must be 0 (choose) or 1..256, got %d", splits);
-    const int nt = miw::tiled_variant_count();
     const bool in_place = c_shares_d(d, p);
-    static char dummy alignas(16);
+    static char dummy alignas(128);
     // Variant and estimated duration of s slices (s = 1: the plain launch); false when no tiled kernel fits.
     auto try_splits = [&](int s, int *variant, double *us) {
         if (p.K % (64l * s)) return false;
         if (s == 1) {
-            const int v = pick_variant(p, d->c_type, d->d_type, false, 0, in_place);
-            if (v == nt + 1) return false;
-            *variant = v;
-            *us = estimate_us(v - 1, p, d->c_type, d->d_type);
+            if (!pick_tiled(p, d->c_type, d->d_type, false, 0, in_place, us)) return false;
+            *variant = pick_variant(p, d->c_type, d->d_type, false, 0, in_place);
             return true;
         }
         const miw::gemm_params q = splitk_slices(p, s, &dummy);
-        const int v = pick_variant(q, MIW_F32, MIW_F32, false, 0, false);
-        if (v == nt + 1) return false;
+        const int v = pick_tiled(q, MIW_F32, MIW_F32, false, 0, false);
+        if (v == 0) return false;
         *variant = v;
         // second kernel: launch, a quarter of a microsecond per slice (each thread adds its slices
         // in order), and the slices, C and D at the same pace as above
@@ -1005,10 +1026,9 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
 int run_splitk(const miw_gemm_desc *d, splitk_plan &plan, void *ws, hipStream_t s)
 {
     if (plan.splits == 1) {
-        if (!tiled_fits(plan.variant - 1, plan.full, d->c_type, d->d_type, false, 0, c_shares_d(d, plan.full)))
+        if (plan.variant != narrow_id() && !tiled_fits(plan.variant - 1, plan.full, d->c_type, d->d_type, false, 0, c_shares_d(d, plan.full)))
             return fail(MIW_ERR_MISALIGNED, "gemm_splitk: operands must be 16-byte aligned");
-        HIP_TRY(miw::launch_gemm_tiled(plan.variant - 1, plan.full, d->c_type, d->d_type, false, s));
-        return 0;
+        return launch_gemm(plan.variant, plan.full, d->c_type, d->d_type, false, s);
     }
     plan.slice.D = ws;
     // the slices are checked against the real operand pointers (plan_splitk assumed aligned ones)

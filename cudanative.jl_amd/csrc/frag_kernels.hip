@@ -665,7 +665,7 @@ hipError_t launch_wmma_mac(int c_type, int d_type, const void *A, const void *B,
 hipError_t launch_gemm_fragops(const gemm_params &p, int c_type, int d_type, bool f16acc, hipStream_t s)
 {
     if (shortk_fits(p, c_type, d_type, f16acc)) return launch_gemm_shortk(p, c_type, d_type, s);
-    if (skinny_pays(p, d_type, f16acc)) return launch_gemm_skinny(p, c_type, d_type, s);
+    if (fragops_run_skinny(p, d_type, f16acc)) return launch_gemm_skinny(p, c_type, d_type, s);
     if (const int split = fragops_ksplit(p, f16acc); split > 1) {
         int thin_m;
         const int T = ksplit_tiles(p, &thin_m);

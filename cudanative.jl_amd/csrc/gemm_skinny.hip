@@ -212,6 +212,29 @@ bool skinny_pays(const gemm_params &g, int d_type, bool f16acc)
     return rounds == 1 || mt >= 4 || g.K >= (mt == 1 ? 1024 : mt == 2 ? 384 : 256) * rounds;
 }
 
+// Does k_gemm_skinny run this problem faster than the LDS tile it would get?  Where the rows of both operands start on
+// whole cache lines, never (64 to 128 x 256 to 16384 x 256 to 4096: 0.99 to 2.3 times the tile's time; a tile of 64 x 64
+// reads 64 rows of each operand once, a workgroup here 16 of one and all of the other).  Pitches that 64 elements, 128
+// bytes, do not divide slow the tiles' direct-to-LDS loads down (64 x 4096: 17.7 us at K = 3072, 26.2 at 3088) and
+// leave these alone (17.6 and 17.0); with one operand on whole lines the two are level.  The tile rows of 16 that a CU
+// reads here then decide (profiles/gemm_narrow_k_contiguous_sweep.md): up to 6, i.e. 64 and 80 in one round of
+// workgroups, 0.60 to 1.04 of the tile's time; 7 and 8, i.e. 96 and 112, only where rows also straddle 64-byte halves and
+// K makes up for the start (96 x 4096 x 528: 0.98; 112 x 4096 x 1040: 0.93; 112 x 2064: 1.02 at K = 1040, 0.91 at 3088).
+// Rows that all start at the same place inside a line cost the tiles less: 0.7 to 0.95 at 64, 0.83 to 1.13 at 80.
+bool skinny_beats_tiles(const gemm_params &g, int d_type, bool f16acc)
+{
+    const long wide = g.M <= g.N ? g.N : g.M, narrow = g.M <= g.N ? g.M : g.N;
+    if (narrow < 64 || g.K < 256 || !skinny_fits(g, d_type, f16acc)) return false;
+    // 0: rows start on cache lines, 1: at one place inside a line, 2: at several, 3: also inside 64-byte halves
+    auto straddles = [](const half_t *x, long ld) { return ld % 32 ? 3 : ld % 64 ? 2 : (uintptr_t)x & 127 ? 1 : 0; };
+    const int a = straddles(g.A, g.lda), b = straddles(g.B, g.ldb), worst = a < b ? a : b;
+    const long rows = skinny_rounds(g, SKINNY_CUS) * (narrow / 16 + skinny_width(g));
+    if (worst < 2) return worst == 1 && rows <= 5;
+    if (rows <= 6) return true;
+    if (worst != 3) return false;
+    return rows == 7 ? g.K >= 512 : rows == 8 && g.K >= 1024 && wide * g.batch >= (g.K >= 3072 ? 1024 : 4096);
+}
+
 // Estimated duration in microseconds, for the planner: launch, start and reduction of each round of
 // workgroups, and the larger of a CU's requests through its L1 (0.96 ns per tile row of 16 and k-value) and the
 // operands at 3.7 TB/s.  Fitted to the launches of the same sweep that skinny_pays takes: within 20 % on nine of ten.

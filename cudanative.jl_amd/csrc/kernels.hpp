@@ -38,11 +38,18 @@ hipError_t launch_gemm_fragops(const gemm_params &p, int c_type, int d_type, boo
 // *tiles_together (may be null) = tiles a workgroup of it takes together.
 int fragops_ksplit(const gemm_params &p, bool f16acc, int *tiles_together = nullptr);
 // --- gemm_skinny.hip: D with one extent of at most 128 and k contiguous in both operands.  Can the kernel run
-// the problem; is it the one launch_gemm_fragops takes; its estimated duration.
+// the problem; is it faster there than the fragment-op kernels, than the LDS tiles; its estimated duration.
 bool skinny_fits(const gemm_params &p, int d_type, bool f16acc);
 bool skinny_pays(const gemm_params &p, int d_type, bool f16acc);
+bool skinny_beats_tiles(const gemm_params &p, int d_type, bool f16acc);
 double skinny_estimate_us(const gemm_params &p, int cus);
 hipError_t launch_gemm_skinny(const gemm_params &p, int c_type, int d_type, hipStream_t s);
+// Does launch_gemm_fragops hand the problem to k_gemm_skinny?  Only below the smallest tile: from there on the
+// two have ids of their own.
+inline bool fragops_run_skinny(const gemm_params &p, int d_type, bool f16acc)
+{
+    return (p.M < 64 || p.N < 64) && skinny_pays(p, d_type, f16acc);
+}
 hipError_t launch_dummy_store(float *ptr, int threads, hipStream_t s);
 const void *frag_kernel_symbol(const char *name);
 int frag_kernel_count();

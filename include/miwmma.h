@@ -188,8 +188,8 @@ typedef struct miw_gemm_desc {
 
 /* D = alpha*A*B + beta*C, the chain of mma calls the reference describes
    (docs/src/device/wmma.md:51-52) carried over the whole K extent.  M, N, K
-   must be multiples of 16; the LDS-tiled variants need multiples of their tile
-   (otherwise the fragment-op variant is used). */
+   must be multiples of 16; what no LDS-tiled variant can run (miw_gemm_plan says what they
+   need) runs on one of the last two variants. */
 int miw_gemm(const miw_gemm_desc *desc, const void *A, const void *B, const void *C, void *D, void *stream);
 
 /* Enumerate kernel variants (variant ids are 1..count). */
@@ -200,7 +200,12 @@ typedef struct miw_gemm_variant_info {
     int waves_m, waves_n;
     int stages;
     int lds_bytes;
-    int fragment_ops;   /* 1: built from load_a/load_b/mma on global memory, no LDS */
+    int fragment_ops;   /* 1: operands go from global memory to registers, not through LDS tiles; runs every
+                           problem.  "fragment_ops": one wavefront per 16x16 tile built from load_a/load_b/mma, or
+                           the kernel that serves the problem faster (K of at most 64; few tiles and a long K; less
+                           than 64 rows or columns with k contiguous in both operands).  "narrow_k_contiguous":
+                           at most 128 rows or columns, k contiguous in both operands, 16-byte aligned; what it
+                           cannot run goes to fragment_ops' kernels */
     int f16_accumulate; /* 1: has a Float16-accumulate form (accumulators fit in ordinary VGPRs) */
     int pingpong;       /* 1: the two wavefronts of a SIMD alternate between matrix-core and memory phases;
                            2: one wavefront per SIMD with a 128x128 sub-tile issues its memory instructions

@@ -79,16 +79,18 @@ class _GemmParams(ctypes.Structure):
 @pytest.fixture(scope="session")
 def narrow_kernel(miw):
     """narrow_kernel(rule, M, N, K, ...): what the library's own rule `rule` says of the kernel for D with one
-    extent of at most 128 ("fits": it can run the problem; "pays": launch_gemm_fragops takes it)."""
+    extent of at most 128 ("fits": it can run the problem; "pays": it is faster there than the fragment-op kernels;
+    "beats_tiles": than the LDS tiles)."""
     lib = ctypes.CDLL(miw._lib.LIB_PATH)
 
-    def ask(rule, M, N, K, batch=1, a_row=1, b_row=0, c_row=1, d_row=1, use_c=0, d_type=0, f16acc=False, lda=0, ldb=0, ldd=0, offset=0):
-        f = getattr(lib, "_ZN3miw11skinny_%sERKNS_11gemm_paramsEib" % rule)
+    def ask(rule, M, N, K, batch=1, a_row=1, b_row=0, c_row=1, d_row=1, use_c=0, d_type=0, f16acc=False, lda=0, ldb=0, ldd=0, offset=0, offset_b=0):
+        name = "skinny_" + rule
+        f = getattr(lib, "_ZN3miw%d%sERKNS_11gemm_paramsEib" % (len(name), name))
         f.restype, f.argtypes = ctypes.c_bool, [ctypes.POINTER(_GemmParams), ctypes.c_int, ctypes.c_bool]
         lda, ldb = lda or (K if a_row else M), ldb or (N if b_row else K)
         ldc, ldd = N if c_row else M, ldd or (N if d_row else M)
         base = 1 << 32
-        p = _GemmParams(base + offset, base + (1 << 40), base + (2 << 40), base + (3 << 40), M, N, K, lda, ldb, ldc, ldd,
+        p = _GemmParams(base + offset, base + (1 << 40) + offset_b, base + (2 << 40), base + (3 << 40), M, N, K, lda, ldb, ldc, ldd,
                         lda * (M if a_row else K), ldb * (K if b_row else N), ldc * (M if c_row else N), ldd * (M if d_row else N),
                         batch, a_row, b_row, c_row, d_row, use_c, 1.0, 1.0)
         return f(ctypes.byref(p), d_type, f16acc)

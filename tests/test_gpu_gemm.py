@@ -692,13 +692,13 @@ def _check_block(orc, g, D, want, where):
 
 @pytest.mark.parametrize("tiles,wide_tiles", [(t, 1) for t in range(1, 9)] + [(t, 2) for t in range(4, 9)])
 def test_narrow_kernel_on_k_contiguous_operands(gpu, orc, narrow_kernel, tiles, wide_tiles):
-    """The kernel behind the fragment-op id for one extent of at most 128 and k contiguous in both operands:
+    """The kernel for one extent of at most 128 and k contiguous in both operands, forced by its id:
     every instance (tiles of 16 of the short extent, tiles of the long extent per workgroup), at chunk
     counts around its eight wavefronts and their buffers (none for some wavefronts, parts of a buffer,
     whole buffers, both), with every tail of K.  The short side is D's rows and D's columns in turn; C is
     absent, Float16, Float32, laid out as D or transposed, or D itself; batches; padded leading dimensions.
     Bit-exact on integers (every partial sum is exact, |sum| < 2^24), against float64 on random data."""
-    frag = _variants(gpu)[-1]["id"]
+    vid = _vid(gpu, "narrow_k_contiguous")
     narrow = 16 * tiles
     un = {2: 4, 3: 3, 4: 2, 5: 2}.get(tiles + wide_tiles, 1)      # chunks of 64 k-values per buffer
     counts = (1, 2, 8, 9, 8 * un + 5, 16 * un, 16 * un + 11, 24 * un + 8) if wide_tiles == 1 else (1, 7, 8, 17, 26)
@@ -709,29 +709,25 @@ def test_narrow_kernel_on_k_contiguous_operands(gpu, orc, narrow_kernel, tiles, 
         M, N = (narrow, wide) if (n + tiles) % 2 else (wide, narrow)
         dl, ct, dt = (n >> 1) & 1, (n + tiles) & 1, (n >> 1 ^ n) & 1
         use_c = n % 4 != 3
-        # up to 64 k-values with C laid out as D belong to the short-K kernel
-        cl = 1 - dl if use_c and (K == 64 or n % 3 == 1) else dl
-        if K == 64 and not use_c:
-            K = 80
+        cl = 1 - dl if use_c and n % 3 == 1 else dl
         pad = 8 * (n % 2)
         g = orc.GemmDesc(M=M, N=N, K=K, a_layout=orc.ROW, b_layout=orc.COL, c_layout=cl, d_layout=dl, c_type=ct, d_type=dt,
                          use_c=int(use_c), batch=batch, alpha=(1.0, -2.0, 0.5)[n % 3], beta=(1.0, 0.5, -1.0)[n % 3],
                          lda=K + pad, ldb=K + 2 * pad, ldc=(N if cl == orc.ROW else M) + pad // 2, ldd=(N if dl == orc.ROW else M) + pad)
         where = (M, N, K, batch, cl, dl, ct, dt, use_c)
-        assert narrow_kernel("pays", M, N, K, batch=batch, c_row=cl == orc.ROW, d_row=dl == orc.ROW), where
+        assert narrow_kernel("fits", M, N, K, batch=batch, c_row=cl == orc.ROW, d_row=dl == orc.ROW), where
         A, B, C = _inputs(orc, g, 1700 + 100 * tiles + n, ints=True)
-        D = _run(gpu, orc, g, A, B, C if use_c else None, variant=frag, prefill=7.0)
+        D = _run(gpu, orc, g, A, B, C if use_c else None, variant=vid, prefill=7.0)
         _check_block(orc, g, D, orc.gemm(g, A, B, C), where)
     # C is D, and values that are not whole: against float64, and the same bits on a second run
     wide, batch = (2064, 1) if wide_tiles == 1 else (2080, 4)
     K = 16 * 33
     for M, N in ((narrow, wide), (wide, narrow)):
-        assert narrow_kernel("pays", M, N, K, batch=batch)
         g = orc.GemmDesc(M=M, N=N, K=K, a_layout=orc.ROW, b_layout=orc.COL, c_layout=orc.ROW, d_layout=orc.ROW, alpha=0.75, beta=-1.25, batch=batch)
         A, B, C = _inputs(orc, g, 2600 + tiles)
         dA, dB = gpu.DeviceArray(A), gpu.DeviceArray(B)
         desc = gpu.GEMM.make_desc(M, N, K, a_layout=gpu.WMMA.RowMajor, c_layout=gpu.WMMA.RowMajor, d_layout=gpu.WMMA.RowMajor,
-                                  alpha=0.75, beta=-1.25, batch=batch, variant=frag)
+                                  alpha=0.75, beta=-1.25, batch=batch, variant=vid)
         outs = []
         for _ in range(2):
             dD = gpu.DeviceArray(C.copy())
@@ -740,6 +736,30 @@ def test_narrow_kernel_on_k_contiguous_operands(gpu, orc, narrow_kernel, tiles, 
             outs.append(dD.to_host())
         assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
         assert orc.normalized_error(g, outs[0], orc.gemm_f64(g, A, B, C)) <= TIGHT_F32, (M, N, K)
+
+
+@pytest.mark.parametrize("cl,dl", [(1, 1), (0, 1), (1, 0), (0, 0)])
+def test_narrow_problems_through_every_route(gpu, orc, narrow_kernel, cl, dl):
+    """k contiguous in both operands, narrow: what miw_gemm picks, the narrow kernel's id and the fragment-op id
+    (several wavefronts per tile, one wavefront per tile, the narrow kernel below 64) agree with the oracle bit for
+    bit on integers.  Pitches that 8 elements do not divide keep the narrow kernel out of all three."""
+    frag, vid = _variants(gpu)[-1]["id"], _vid(gpu, "narrow_k_contiguous")
+    tiles = {v["id"] for v in _variants(gpu) if not v["fragment_ops"]}
+    for n, (M, N, K, pad, auto, kw) in enumerate([
+            (16, 1040, 1040, 0, {frag}, {}), (1040, 48, 528, 8, {frag}, dict(alpha=0.5)), (32, 512, 80, 0, {frag}, dict(batch=3)),
+            (48, 64, 1024, 0, {frag}, dict(d_type=orc.F16)), (32, 272, 1024, 2, {frag}, {}), (1040, 48, 1024, 4, {frag}, dict(beta=-1.0)),
+            (64, 1040, 1040, 0, {vid}, {}), (1040, 80, 528, 0, {vid}, dict(use_c=0)), (96, 2064, 1040, 0, {vid}, dict(c_type=orc.F16, d_type=orc.F16)),
+            (64, 1040, 1040, 2, {frag}, {}), (64, 1024, 1024, 0, tiles, {}), (112, 1040, 1040, 0, tiles, dict(batch=2)),
+            (1024, 80, 1024, 0, tiles, {}), (80, 272, 2064, 2, {frag}, {})]):
+        g = orc.GemmDesc(M=M, N=N, K=K, a_layout=orc.ROW, b_layout=orc.COL, c_layout=cl, d_layout=dl, lda=K + pad, ldb=K + pad,
+                         ldd=(N if dl == orc.ROW else M) + 8, **kw)
+        plan = {q["variant"] for q in _plan(gpu, orc, g)}
+        assert plan <= auto, (M, N, K, pad, plan)
+        assert narrow_kernel("fits", M, N, K, lda=K + pad, ldb=K + pad, batch=max(g.batch, 1)) == (pad % 8 == 0)
+        A, B, C = _inputs(orc, g, 2700 + n, ints=True)
+        want = orc.gemm(g, A, B, C)
+        for variant in (0, vid, frag):
+            _check_block(orc, g, _run(gpu, orc, g, A, B, C if g.use_c else None, variant=variant, prefill=7.0), want, (M, N, K, pad, variant))
 
 
 def test_tiled_with_padded_leading_dimensions_and_batch(gpu, orc):

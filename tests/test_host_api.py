@@ -256,21 +256,55 @@ def test_gemm_plan_covers_the_problem(miw):
 
 
 @pytest.mark.parametrize("a_row,b_row", [(False, False), (True, False), (False, True), (True, True)])
-def test_narrow_problems_that_a_tile_fits_run_on_tiles(miw, a_row, b_row):
-    """64 to 128 rows or columns: an LDS tile fits, and every launch of the plan is one, in every operand
-    layout, alone and as what a body of large tiles leaves of a ragged problem."""
+def test_narrow_problems_that_a_tile_fits_are_not_fragment_op_problems(miw, a_row, b_row):
+    """64 to 128 rows or columns: an LDS tile fits, and no launch of the plan is the fragment-op variant, in any operand
+    layout, alone and as what a body of large tiles leaves of a ragged problem.  Every launch is a tile unless k is
+    contiguous in both operands and their pitches are no whole number of cache lines."""
     G, W = miw.GEMM, miw.WMMA
-    frag = G.variants()[-1]["id"]
+    vs = G.variants()
+    frag, narrow_id = vs[-1]["id"], vs[-2]["id"]
+    assert vs[-2]["name"] == "narrow_k_contiguous"
     lay = lambda row: W.RowMajor if row else W.ColMajor  # noqa: E731
     for long, k, narrow, kw in itertools.product((1024, 2064, 4096, 8192), (512, 1040, 2048, 8192), (64, 80, 96, 112, 128),
                                                  (dict(use_c=False, d_type=np.float16), dict())):
+        allowed = {frag, narrow_id} if k % 64 == 0 or not (a_row and not b_row) else {frag}      # ids that are not allowed
         for m, n in ((narrow, long), (long, narrow)):
             for d_row in (False, True):
                 d = G.make_desc(m, n, k, a_layout=lay(a_row), b_layout=lay(b_row), c_layout=lay(d_row), d_layout=lay(d_row), **kw)
-                assert G.pick_variant(d) != frag and all(q["variant"] != frag for q in G.plan(d)), (m, n, k)
+                assert G.pick_variant(d) not in allowed and all(q["variant"] not in allowed for q in G.plan(d)), (m, n, k)
     for m, n, k in ((2064, 2048, 2048), (4144, 4096, 4096), (2480, 3392, 3136), (3888, 2128, 4224), (2112, 4016, 2848)):
         d = G.make_desc(m, n, k, a_layout=lay(a_row), b_layout=lay(b_row), d_layout=W.RowMajor, d_type=np.float16, use_c=False)
         assert all(q["variant"] != frag for q in G.plan(d)), (m, n, k)
+
+
+def test_narrow_kernel_against_the_tiles(miw, narrow_kernel):
+    """Both sides of every line of the rule that takes the narrow kernel in place of an LDS tile, and that
+    miw_gemm_pick_variant, the plan, the split-K call of one slice and a forced id agree with it."""
+    G, W = miw.GEMM, miw.WMMA
+    vs = G.variants()
+    narrow_id = vs[-2]["id"]
+    for yes, m, n, k, kw in (
+            (True, 64, 4096, 3088, {}), (False, 64, 4096, 3072, {}), (True, 64, 4096, 3104, {}), (False, 64, 4096, 240, {}), (True, 64, 64, 272, {}),
+            (False, 64, 4096, 3072, dict(lda=3088)), (False, 64, 4096, 3072, dict(ldb=3088)), (True, 64, 4096, 3072, dict(lda=3088, ldb=3080)),
+            (True, 80, 4096, 3104, {}), (False, 80, 4112, 3104, {}), (True, 64, 8192, 3104, {}), (False, 64, 8224, 3104, {}),
+            (True, 96, 4096, 528, {}), (False, 96, 4096, 496, {}), (False, 96, 4096, 1056, {}), (True, 112, 1024, 3088, {}),
+            (False, 112, 1008, 3088, {}), (False, 112, 1024, 2992, {}), (True, 112, 4096, 1040, {}), (False, 112, 4096, 1008, {}), (False, 128, 4096, 3088, {}), (True, 64, 1024, 528, dict(batch=8)), (False, 64, 64, 272, dict(batch=256))):
+        for mm, nn in ((m, n), (n, m)):
+            if mm != m:
+                kw = dict(kw, lda=kw.get("ldb", 0), ldb=kw.get("lda", 0))
+            assert narrow_kernel("beats_tiles", mm, nn, k, **kw) == yes, (mm, nn, k, kw)
+            d = G.make_desc(mm, nn, k, a_layout=W.RowMajor, b_layout=W.ColMajor, c_layout=W.RowMajor, d_layout=W.RowMajor, d_type=np.float16, use_c=False, **kw)
+            assert (G.pick_variant(d) == narrow_id) == yes and (G.plan(d)[0]["variant"] == narrow_id) == yes, (mm, nn, k, kw)
+            assert G.variant_supports(d, narrow_id)
+    # pitches of whole lines, rows that start inside one
+    for yes, m, kw in ((True, 64, dict(offset=32, offset_b=16)), (False, 64, dict(offset=32)), (False, 64, dict(offset_b=64)), (False, 80, dict(offset=32, offset_b=32))):
+        assert narrow_kernel("beats_tiles", m, 4096, 2048, **kw) == yes, (m, kw)
+    assert not narrow_kernel("beats_tiles", 48, 4096, 3088)           # thinner than every tile: no tile to beat
+    # what no tile takes (80 rows with C in D's place) but the narrow kernel does
+    d = G.make_desc(80, 4096, 4096, a_layout=W.RowMajor, b_layout=W.ColMajor)
+    assert [q["variant"] for q in G.plan(d, in_place=True)] == [narrow_id]
+    # a pitch of whole lines and a split-K call: as before; and one slice with other pitches is still one launch
+    assert G.splitk_workspace(G.make_desc(64, 4096, 512, a_layout=W.RowMajor, lda=528, ldb=528)) == (1, 0)
 
 
 def test_narrow_kernel_runs_where_it_was_measured_ahead(narrow_kernel):
