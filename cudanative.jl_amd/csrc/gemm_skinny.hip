@@ -167,12 +167,14 @@ static int skinny_width(const gemm_params &g)
 }
 
 // Can k_gemm_skinny run this problem?  One extent of at most 128, k contiguous in both operands, at
-// least one chunk of K, and what its 16-byte loads and 8- or 16-byte stores assume of the alignment.
+// least one chunk of K, what its 16-byte loads and 8- or 16-byte stores assume of the alignment, and fewer than 2^32
+// threads along x (the long extent of a problem that is thin enough to fit in memory can exceed that).
 bool skinny_fits(const gemm_params &g, int d_type, bool f16acc)
 {
     const long wide = g.M <= g.N ? g.N : g.M, narrow = g.M <= g.N ? g.M : g.N;
     if (f16acc || narrow > 128 || g.K < 64 || !g.a_row || g.b_row || g.K > (1l << 30) || wide > (1l << 30)) return false;
     if (((uintptr_t)g.A & 15) || ((uintptr_t)g.B & 15) || g.lda % 8 || g.ldb % 8 || g.sa % 8 || g.sb % 8) return false;
+    if (wide / (16 * skinny_width(g)) * (64 * SKINNY_WAVES) >= 1l << 32) return false;
     const long dper = d_type == 0 ? 8 : 4;
     return !((uintptr_t)g.D & 15) && g.ldd % dper == 0 && g.sd % dper == 0;
 }

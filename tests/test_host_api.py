@@ -459,6 +459,23 @@ def test_tile_counts_that_overflow_the_grid_are_refused(miw):
     assert not G.variant_supports(d, small) and G.variant_supports(d, large)
 
 
+def test_narrow_kernel_leaves_grids_it_cannot_launch_to_the_others(miw, narrow_kernel):
+    """2^32 threads along x: 2^23 workgroups of 512.  A thin problem of that many rows fits in memory (134217728 x 16 x 80:
+    21 GB of A) and runs on the kernel with one wavefront per tile, an eighth of the threads."""
+    edge = 1 << 27
+    for m, n in ((edge, 16), (16, edge)):
+        assert not narrow_kernel("fits", m, n, 80) and not narrow_kernel("pays", m, n, 512)
+    assert narrow_kernel("fits", edge - 16, 16, 80) and narrow_kernel("pays", edge - 16, 16, 512)
+    assert narrow_kernel("fits", edge, 64, 80) and not narrow_kernel("fits", 2 * edge, 64, 80)      # two tiles per workgroup
+    assert narrow_kernel("fits", edge - 16, 64, 80) and not narrow_kernel("fits", edge + 16, 64, 80)
+    # the planner and a forced id still take it: the fragment-op kernels run it
+    G, W = miw.GEMM, miw.WMMA
+    vs = G.variants()
+    for variant in (0, vs[-2]["id"], vs[-1]["id"]):
+        d = G.make_desc(edge, 16, 80, a_layout=W.RowMajor, variant=variant)
+        assert [q["variant"] for q in G.plan(d)] == [variant or vs[-1]["id"]]
+
+
 def test_module_entries_check_their_arguments_without_a_device(miw):
     L = miw._lib
     lib = L.load()
