@@ -66,6 +66,23 @@ def test_auto_picked_4096_kernels_have_no_spills(miw):
             assert r["spills"] == 0 and r["scratch"] == 0, k
 
 
+def test_narrow_kernel_codegen_and_resources(miw):
+    """Every instance of the narrow kernel (1 to 8 tiles of the short extent, two of the long one from 4 on) holds its two
+    buffers in registers: no scratch, two wavefronts per SIMD, operands by 16-byte global loads that go to
+    registers; what LDS holds is eight wavefronts' partial sums of one tile row."""
+    isa = miw.reflection.code_gcn("k_gemm_skinny<")
+    assert len(isa) == 13
+    res = miw.reflection.kernel_resources()
+    for tiles, wide in [(t, 1) for t in range(1, 9)] + [(t, 2) for t in range(4, 9)]:
+        name = "k_gemm_skinny<%d, %d>" % (tiles, wide)
+        (r,) = [v for k, v in res.items() if name in k]
+        assert r["spills"] == 0 and r["scratch"] == 0 and r["vgpr"] + r["agpr"] <= 256 and r["max_threads"] == 512, name
+        (text,) = [v for k, v in isa.items() if name in k]
+        ops = _ops(text)
+        assert ops["v_mfma_f32_16x16x32_f16"] >= 2 * tiles * wide and ops["global_load_dwordx4"] >= 2 * (tiles + wide), name
+        assert not any(o.startswith(("scratch_", "flat_", "global_load_lds", "v_accvgpr")) for o in ops), name
+
+
 def test_tiled_kernels_keep_spills_out_of_the_steady_state(miw):
     """The rolled K loop (the two pipeline steps up to the backward branch) never touches scratch
     memory; the unrolled trips that fold C in may hold a few spills in one operand layout."""
