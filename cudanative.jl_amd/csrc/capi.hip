@@ -843,7 +843,7 @@ int miw_gemm_pick_variant(const miw_gemm_desc *desc, int *variant)
     if (!variant) return fail(MIW_ERR_NULL_POINTER, "gemm_pick_variant: null output");
     miw::gemm_params p;
     bool f16acc;
-    // Alignment of real pointers cannot be known here: assume aligned operands.
+    // Alignment of real pointers cannot be known here: assume operands on whole cache lines.
     static char dummy alignas(128);
     if (int rc = resolve_gemm(desc, &dummy, &dummy, &dummy, &dummy, &p, &f16acc)) return rc;
     *variant = pick_variant(p, desc->c_type, desc->d_type, f16acc, desc->acc_chunk, false);
@@ -855,7 +855,7 @@ int miw_gemm_plan(const miw_gemm_desc *desc, int in_place, miw_gemm_part *out, i
     if (!count || (capacity > 0 && !out)) return fail(MIW_ERR_NULL_POINTER, "gemm_plan: null output");
     miw::gemm_params p;
     bool f16acc;
-    // Alignment of real pointers cannot be known here: assume 16-byte aligned operands far apart.
+    // Alignment of real pointers cannot be known here: assume operands on whole cache lines, far apart.
     char *const base = (char *)(uintptr_t)0x100000000ull;
     if (int rc = resolve_gemm(desc, base, base + (1ull << 40), base + (2ull << 40), base + (in_place ? 2ull << 40 : 3ull << 40), &p, &f16acc))
         return rc;
@@ -1046,7 +1046,7 @@ extern "C" {
 int miw_gemm_splitk_workspace(const miw_gemm_desc *desc, int splits, int *splits_out, size_t *bytes)
 {
     if (!bytes) return fail(MIW_ERR_NULL_POINTER, "gemm_splitk_workspace: null output");
-    // Alignment of real pointers cannot be known here: assume 16-byte aligned operands far apart.
+    // Alignment of real pointers cannot be known here: assume operands on whole cache lines, far apart.
     char *const base = (char *)(uintptr_t)0x100000000ull;
     splitk_plan plan;
     if (int rc = plan_splitk(desc, base, base + (1ull << 40), base + (2ull << 40), base + (3ull << 40), splits, &plan)) return rc;

@@ -186,10 +186,10 @@ static long skinny_rounds(const gemm_params &g, long cus)
     return (wide / (16 * skinny_width(g)) * g.batch + cus - 1) / cus;
 }
 
-// Does k_gemm_skinny run this problem faster than the fragment-op kernels (k_gemm_fragops
-// on one wavefront per tile, or k_gemm_fragops_ksplit on 4 to 16)?  Measured over 16 to 128 x 64 to 131072 x
-// 80 to 8192 and batches up to 256 (profiles/gemm_narrow_k_contiguous_sweep.md): where the rule says yes the
-// time is 0.16 to 1.06 of the other kernel's (median 0.77), and where it says no it would be 0.86 or more.
+// Does k_gemm_skinny run this problem faster than the fragment-op kernels (k_gemm_fragops on one wavefront per
+// tile, or k_gemm_fragops_ksplit on 4 to 16)?  Measured over 16 to 128 x 64 to 131072 x 80 to 8192 and batches up
+// to 256: where the rule says yes the time is 0.16 to 1.06 of the other kernel's (median 0.77), and where it says
+// no it would be 0.86 or more.
 //   K < 256: the others give a tile to one wavefront, and its chain of steps takes longer than a round of
 //     workgroups here (16 x 4096 x 128: 2.8 us against 4.7).  With more than two rounds the six of eight
 //     wavefronts that have no chunk cost more than the chain (16 x 32768 x 128: 10.7 against 7.5), unless
@@ -219,9 +219,8 @@ bool skinny_pays(const gemm_params &g, int d_type, bool f16acc)
 // reads 64 rows of each operand once, a workgroup here 16 of one and all of the other).  Pitches that 64 elements, 128
 // bytes, do not divide slow the tiles' direct-to-LDS loads down (64 x 4096: 17.7 us at K = 3072, 26.2 at 3088) and
 // leave these alone (17.6 and 17.0); with one operand on whole lines the two are level.  The tile rows of 16 that a CU
-// reads here then decide (profiles/gemm_narrow_k_contiguous_sweep.md): up to 6, i.e. 64 and 80 in one round of
-// workgroups, 0.60 to 1.04 of the tile's time; 7 and 8, i.e. 96 and 112, only where rows also straddle 64-byte halves and
-// K makes up for the start (96 x 4096 x 528: 0.98; 112 x 4096 x 1040: 0.93; 112 x 2064: 1.02 at K = 1040, 0.91 at 3088).
+// reads here then decide: up to 6, i.e. 64 and 80 in one round of workgroups, 0.60 to 1.04 of the tile's time; 7 and 8,
+// i.e. 96 and 112, only where rows also straddle 64-byte halves and K makes up for the start (96 x 4096 x 528: 0.98; 112 x 4096 x 1040: 0.93; 112 x 2064: 1.02 at K = 1040, 0.91 at 3088).
 // Rows that all start at the same place inside a line cost the tiles less: 0.7 to 0.95 at 64, 0.83 to 1.13 at 80.
 bool skinny_beats_tiles(const gemm_params &g, int d_type, bool f16acc)
 {

@@ -205,7 +205,8 @@ typedef struct miw_gemm_variant_info {
                            the kernel that serves the problem faster (K of at most 64; few tiles and a long K; less
                            than 64 rows or columns with k contiguous in both operands).  "narrow_k_contiguous":
                            at most 128 rows or columns, k contiguous in both operands, 16-byte aligned; what it
-                           cannot run goes to fragment_ops' kernels */
+                           cannot run goes to fragment_ops' kernels.  stages and lds_bytes are the operand ring's:
+                           0 here, although partial sums of wavefronts that share K go through up to 64 KiB of LDS */
     int f16_accumulate; /* 1: has a Float16-accumulate form (accumulators fit in ordinary VGPRs) */
     int pingpong;       /* 1: the two wavefronts of a SIMD alternate between matrix-core and memory phases;
                            2: one wavefront per SIMD with a 128x128 sub-tile issues its memory instructions
@@ -215,7 +216,7 @@ typedef struct miw_gemm_variant_info {
 int miw_gemm_variant_info_get(int variant, miw_gemm_variant_info *out);
 /* *supported = 1 when `variant` (1..count) can run this descriptor (M and N of at least one tile,
    K of at least 64, leading dimensions, accumulate type; pointers are assumed
-   16-byte aligned and C and D apart), else 0. */
+   128-byte aligned and C and D apart), else 0. */
 int miw_gemm_variant_supports(const miw_gemm_desc *desc, int variant, int *supported);
 /* Variant of a single launch of this descriptor (what miw_gemm runs unless miw_gemm_plan
    cuts the problem up): the one with the shortest estimated duration
@@ -246,7 +247,7 @@ typedef struct miw_gemm_part {
 } miw_gemm_part;
 int miw_gemm_plan(const miw_gemm_desc *desc, int in_place, miw_gemm_part *parts, int capacity, int *count);
 /* acc_chunk miw_gemm would use for this descriptor (fp16 accumulate only).  Like
-   miw_gemm_pick_variant it sees no pointers and assumes 16-byte aligned operands with C and D
+   miw_gemm_pick_variant it sees no pointers and assumes 128-byte aligned operands with C and D
    apart; operands that are not (or a C that is D, with M or N no whole number of tiles) can send
    miw_gemm to another kernel with another acc_chunk: miw_gemm_resolve answers for the real ones. */
 int miw_gemm_acc_chunk(const miw_gemm_desc *desc, int *acc_chunk);
