@@ -176,6 +176,7 @@ bool tiled_fits(int i, const miw::gemm_params &p, int c_type, int d_type, bool f
 }
 
 int g_cu_count = 0;
+int cu_count() { return g_cu_count > 0 ? g_cu_count : 256; }
 
 // Kernels of code objects the caller loaded (miw_module_load): handle -> module it belongs to.
 // miw_launch and the attribute queries tell them from the library's own kernels by this table.
@@ -247,7 +248,7 @@ int splitk_scratch(void **out);  // address of the current device's static split
 double estimate_us(int i, const miw::gemm_params &p, int c_type, int d_type)
 {
     const miw::tiled_variant &v = miw::tiled_variant_at(i);
-    const int cus = g_cu_count > 0 ? g_cu_count : 256;
+    const int cus = cu_count();
     const long I = p.d_row ? p.N : p.M, J = p.d_row ? p.M : p.N;
     const long tiles = ((I + v.bm - 1) / v.bm) * ((J + v.bn - 1) / v.bn) * p.batch;  // edge tiles overlap their neighbours
     const long per_cu = (tiles + cus - 1) / cus;
@@ -265,7 +266,7 @@ double estimate_us(int i, const miw::gemm_params &p, int c_type, int d_type)
 bool wave128_pays(int i, const miw::gemm_params &p)
 {
     const miw::tiled_variant &v = miw::tiled_variant_at(i);
-    const int cus = g_cu_count > 0 ? g_cu_count : 256;
+    const int cus = cu_count();
     const long I = p.d_row ? p.N : p.M, J = p.d_row ? p.M : p.N;
     const long tiles = ((I + v.bm - 1) / v.bm) * ((J + v.bn - 1) / v.bn) * p.batch;
     return !p.use_c && tiles <= cus;
@@ -346,7 +347,7 @@ int launch_gemm(int variant, const miw::gemm_params &p, int c_type, int d_type, 
 {
     if (variant == narrow_id() && miw::skinny_fits(p, d_type, f16acc)) HIP_TRY(miw::launch_gemm_skinny(p, c_type, d_type, s));
     else if (variant >= narrow_id()) HIP_TRY(miw::launch_gemm_fragops(p, c_type, d_type, f16acc, s));
-    else HIP_TRY(miw::launch_gemm_tiled(variant - 1, p, c_type, d_type, f16acc, s));
+    else HIP_TRY(miw::launch_gemm_tiled(variant - 1, p, c_type, d_type, f16acc, cu_count(), s));
     return 0;
 }
 
@@ -377,7 +378,7 @@ double estimate_fragops_us(const miw::gemm_params &p, int c_type, int d_type)
     const double cd_bytes = mn * (double)(dtype_size(d_type) + (p.use_c ? dtype_size(c_type) : 0));
     const double flop = 2.0 * mn * (double)p.K;
     if (p.K <= 64 && (!p.use_c || p.c_row == p.d_row)) return std::max(6.5, 3.0 + std::max(cd_bytes / 5.5e6, flop / 75e6));
-    if (miw::fragops_run_skinny(p, d_type, false)) return miw::skinny_estimate_us(p, g_cu_count > 0 ? g_cu_count : 256);
+    if (miw::fragops_run_skinny(p, d_type, false)) return miw::skinny_estimate_us(p, cu_count());
     const int split = miw::fragops_ksplit(p, false);
     const double walk = 0.45 * (double)(p.K / 16) / split + (split > 1 ? 2.0 : 0.0);
     return 5.0 + std::max(walk, std::max(flop / 45e6, cd_bytes / 2.0e6));
@@ -407,7 +408,7 @@ struct gemm_planner {
         if (v != narrow_id()) return estimate_us(v - 1, p, c_type, d_type);
         // (the tiles' paces are those of operands that start on whole cache lines; the cuts are weighed as if these did)
         double us = 0.0;
-        const double narrow_us = miw::skinny_estimate_us(p, g_cu_count > 0 ? g_cu_count : 256);
+        const double narrow_us = miw::skinny_estimate_us(p, cu_count());
         return pick_tiled(p, c_type, d_type, false, 0, in_place, &us) ? std::min(us, narrow_us) : narrow_us;
     }
 
@@ -1034,7 +1035,7 @@ int run_splitk(const miw_gemm_desc *d, splitk_plan &plan, void *ws, hipStream_t 
     // the slices are checked against the real operand pointers (plan_splitk assumed aligned ones)
     if (!tiled_fits(plan.variant - 1, plan.slice, MIW_F32, MIW_F32, false, 0, false))
         return fail(MIW_ERR_MISALIGNED, "gemm_splitk: operands and workspace must be 16-byte aligned");
-    HIP_TRY(miw::launch_gemm_tiled(plan.variant - 1, plan.slice, MIW_F32, MIW_F32, false, s));
+    HIP_TRY(miw::launch_gemm_tiled(plan.variant - 1, plan.slice, MIW_F32, MIW_F32, false, cu_count(), s));
     HIP_TRY(miw::launch_splitk_reduce(plan.full, d->c_type, d->d_type, plan.splits, (const float *)ws, s));
     return 0;
 }

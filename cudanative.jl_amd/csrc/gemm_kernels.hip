@@ -47,17 +47,18 @@ const void *tiled_kernel_128x128_w2x4_s4(bool xk, bool yk, int c_type, int d_typ
 const void *tiled_kernel_128x128_w2x2_s4(bool xk, bool yk, int c_type, int d_type, bool f16acc);
 const void *tiled_kernel_128x128_w2x2(bool xk, bool yk, int c_type, int d_type, bool f16acc);
 const void *tiled_kernel_64x64_w2x2(bool xk, bool yk, int c_type, int d_type, bool f16acc);
-const void *pp_kernel(int bm, int bn, bool xk, bool yk, int c_type, int d_type);
+const void *pp_kernel(int bm, int bn, bool xk, bool yk, int c_type, int d_type, bool fold);
+bool pp_folds(const tiled_params &p, int c_type);
 int pp_lds(int bm, int bn, bool xk, bool yk);
 const void *w128_kernel(bool xk, bool yk, int c_type, int d_type);
 const void *pp64_kernel(int bm, int bn, bool xk, bool yk, int c_type, int d_type, bool f16acc);
 
 
 // Tile shape in canonical (I, J) terms: bm applies to I, bn to J.
-static const void *pick_kernel(int i, bool xk, bool yk, int c_type, int d_type, bool f16acc)
+static const void *pick_kernel(int i, bool xk, bool yk, int c_type, int d_type, bool f16acc, bool fold = false)
 {
     const tiled_variant &v = g_variants[i];
-    if (v.kind == KIND_PINGPONG32) return f16acc ? nullptr : pp_kernel(v.bm, v.bn, xk, yk, c_type, d_type);
+    if (v.kind == KIND_PINGPONG32) return f16acc ? nullptr : pp_kernel(v.bm, v.bn, xk, yk, c_type, d_type, fold);
     if (v.kind == KIND_PINGPONG64) return pp64_kernel(v.bm, v.bn, xk, yk, c_type, d_type, f16acc);
     if (v.kind == KIND_WAVE128) return f16acc ? nullptr : w128_kernel(xk, yk, c_type, d_type);
     const int waves = v.wm * v.wn;
@@ -96,7 +97,7 @@ bool tiled_supports_layout(int i, const gemm_params &g)
     if (g_variants[i].kind != KIND_PINGPONG32) return true;
     bool xk, yk;
     canonical_layout(g, &xk, &yk);
-    return pp_kernel(g_variants[i].bm, g_variants[i].bn, xk, yk, 1, 1) != nullptr;  // (every layout has a ring that fits in LDS at 256 x 256)
+    return pp_kernel(g_variants[i].bm, g_variants[i].bn, xk, yk, 1, 1, false) != nullptr;  // (every layout has a ring that fits in LDS at 256 x 256)
 }
 
 // hipFuncAttributeMaxDynamicSharedMemorySize is a property of the kernel, not of the launch: set once.
@@ -112,7 +113,7 @@ static hipError_t allow_dynamic_lds(const void *fn, int bytes)
     return e;
 }
 
-hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type, bool f16acc, hipStream_t s)
+hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type, bool f16acc, int cus, hipStream_t s)
 {
     const tiled_variant &v = g_variants[i];
     tiled_params p;
@@ -136,6 +137,7 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
     }
     p.C = g.C; p.D = g.D;
     p.K = (int)g.K;
+    p.work = 0;
     p.ldc = g.ldc; p.ldd = g.ldd; p.sc = g.sc; p.sd = g.sd;
     p.use_c = g.use_c;
     p.alpha = g.alpha; p.beta = g.beta;
@@ -151,7 +153,8 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
     p.ts = nullptr;
     if (const char *e = getenv("MIW_TS")) p.ts = (long long *)strtoull(e, nullptr, 16);
 #endif
-    const void *fn = pick_kernel(i, xk, yk, c_type, d_type, f16acc);
+    const bool fold = v.kind == KIND_PINGPONG32 && pp_folds(p, c_type);
+    const void *fn = pick_kernel(i, xk, yk, c_type, d_type, f16acc, fold);
     if (!fn) return hipErrorInvalidValue;
     // (the 64-k ping-pong kernels stage a Float16 C tile beside the ring where both fit)
     const int c_stage = v.kind == KIND_PINGPONG64 && f16acc && v.lds_bytes + v.bm * v.bn * 2 <= 160 * 1024 ? v.bm * v.bn * 2 : 0;
@@ -163,6 +166,13 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
     void *args[] = {&p};
     // the tile count fits: tiled_grid_fits() is part of the caller's check
     dim3 grid((unsigned)(p.tiles_i * p.tiles_j), (unsigned)g.batch);
+    const long tiles = (long)p.tiles_i * p.tiles_j * g.batch;
+    // More tiles than CUs: one workgroup per CU, which walks every cus-th (its LDS admits one per CU in any case).
+    // Below four slots of K there is too little of it to request across two tiles, and the launch is bound by C and D.
+    if (v.kind == KIND_PINGPONG32 && tiles > cus && tiles < (1l << 30) && p.K > 3 * KGRAN) {
+        p.work = (int)tiles;
+        grid = dim3((unsigned)cus, 1);
+    }
     return hipLaunchKernel(fn, grid, dim3((unsigned)(v.wm * v.wn * 64)), args, (size_t)lds_bytes, s);
 }
 

@@ -57,8 +57,13 @@ namespace miw {
 #define MIW_PP_MIDDLE(pr)
 #endif
 
+// The lambdas of a kernel are called from many places: left to itself the compiler makes functions of them, and what
+// they capture goes to memory.
+#define MIW_INLINE __attribute__((always_inline))
+
 constexpr int PP_KMAJOR_SLOTS = 3;
 constexpr int PP_IMAJOR_ENTRIES = 4;
+constexpr int PP_FOLD_STEPS = 32;  // k-steps of 32 over which k_gemm_pp_fold adds C: one MFMA tile of the wavefront's 8 x 4 each
 
 // Slots of a K-major Y: two when X is K-major as well (see above), else three.
 constexpr int pp_y_slots(bool xk) { return xk ? 2 : PP_KMAJOR_SLOTS; }
@@ -140,9 +145,18 @@ struct pp_operand {
     }
 };
 
-template <int BI, int BJ, int WI, int WJ, bool XK, bool YK, class CT, class DT>
-__global__ __launch_bounds__(WI *WJ * 64) __attribute__((amdgpu_waves_per_eu(2)))
-void k_gemm_pp(tiled_params p)
+// Where the tiles outnumber the CUs a workgroup walks several (tiled_params::work), and the ring runs on from one
+// tile into the next: behind the last unit of a tile the first ones of the next are requested, so that they land
+// under the epilogue.  One workgroup per tile pays for a start of 2 to 3 us and for the dispatch, which hands
+// workgroups to the shader engines in turn and waits for the slowest, 1 to 5 us, in every round; what is left is the
+// store of D, whose acknowledgements the loads of the next tile's third k-step wait for (vmcnt counts in order).
+// 8192x8192x1024, alpha = -1, operands from HBM: 188 us with one tile per workgroup, 159 like this with C folded
+// from sixteen slots of K on (it was eighteen); without C 143 and 127; 6144^3 425 and 414; 8192^3 level (784, 779),
+// which is bound by energy.
+// FOLD: a Float32 C is added in the K loop; otherwise C, if any, in the epilogue.  They are kernels of their own: in
+// one kernel the accumulators of both forms meet in the last pair, and that spills.
+template <int BI, int BJ, int WI, int WJ, bool XK, bool YK, class CT, class DT, bool FOLD>
+__device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params &p)
 {
     constexpr int NT = WI * WJ * 64;
     static_assert(NT == 512, "two wavefronts per SIMD");
@@ -170,50 +184,51 @@ void k_gemm_pp(tiled_params p)
     const int wi = wave % WI, wj = wave / WI;
     const bool late_group = wave >= 4;
 
-    // Workgroup -> tile, as in k_gemm_tiled.
-    int tile_id;
-    {
-        const int total = p.tiles_i * p.tiles_j;
-        const int pid = blockIdx.x;
+    // Workgroup -> tile, as in k_gemm_tiled; the last tile of a row or column is shifted back so that it
+    // ends at the edge (see tiled_params).
+    // What only the start of a tile needs is read from the arguments again there: held through the K loop it
+    // would take more scalar registers than there are.
+    auto arguments = [] MIW_INLINE {
+        auto a = (const __attribute__((address_space(4))) tiled_params *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(a));
+        return a;
+    };
+    // (the divisions run on the VALU: their outcome goes back to scalar registers)
+    auto locate = [](auto a, int tile, int &bt, int &i0, int &j0) MIW_INLINE {
+        const int total = a->tiles_i * a->tiles_j;
+        if (a->work > total) bt = __builtin_amdgcn_readfirstlane(tile / total);
+        const int pid = a->work > total ? tile - bt * total : tile;
         const int per = total >> 3, rem = total & 7;
         const int xcd = pid & 7, loc = pid >> 3;
-        tile_id = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
-    }
-    int ti0, tj0;
-    {
-        const int gsz = p.group_i * p.tiles_j;
+        const int tile_id = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
+        const int gsz = a->group_i * a->tiles_j;
         const int gid = tile_id / gsz;
-        const int first = gid * p.group_i;
-        const int gi = min(p.tiles_i - first, p.group_i);
+        const int first = gid * a->group_i;
+        const int gi = min(a->tiles_i - first, a->group_i);
         const int in = tile_id - gid * gsz;
-        ti0 = first + in % gi;
-        tj0 = in / gi;
-    }
-    const long bt = blockIdx.y;
-    // the last tile of a row or column is shifted back so that it ends at the edge (see tiled_params)
-    const int i0 = min(ti0 * BI, p.I - BI), j0 = min(tj0 * BJ, p.J - BJ);
-
-    const half_t *X = p.X + bt * p.sx + (XK ? (long)i0 * p.ldx : (long)i0);
-    const half_t *Y = p.Y + bt * p.sy + (YK ? (long)j0 * p.ldy : (long)j0);
+        i0 = __builtin_amdgcn_readfirstlane(min((first + in % gi) * BI, a->I - BI));
+        j0 = __builtin_amdgcn_readfirstlane(min(in / gi * BJ, a->J - BJ));
+    };
+    auto x_origin = [](auto a, int bt, int i0) MIW_INLINE { return a->X + (long)bt * a->sx + (XK ? (long)i0 * a->ldx : (long)i0); };
+    auto y_origin = [](auto a, int bt, int j0) MIW_INLINE { return a->Y + (long)bt * a->sy + (YK ? (long)j0 * a->ldy : (long)j0); };
+    int tile = blockIdx.x, bt = blockIdx.y, i0, j0;
+    locate(arguments(), tile, bt, i0, j0);
+    const half_t *X = x_origin(arguments(), bt, i0);
+    const half_t *Y = y_origin(arguments(), bt, j0);
     const unsigned xoff = xop::lane_offset(tid, (int)p.ldx);
     const unsigned yoff = yop::lane_offset(tid, (int)p.ldy);
 
     xop xr;
     yop yr;
-    xr.init(wi * WTI, lane);
-    yr.init(wj * WTJ, lane);
+    // (the wavefront's place in the tile is added to the unit's address, a scalar: two operands of one kind
+    // then share their lane offsets)
+    static_assert(WTI % 64 == 0 && WTJ % 64 == 0, "wave tile");
+    xr.init(0, lane);
+    yr.init(0, lane);
+    const unsigned xwave = wi * WTI * (XK ? 128 : 64), ywave = wj * WTJ * (YK ? 128 : 64);
 
     const int q = lane >> 4, r = lane & 15;
-    const int row = i0 + wi * WTI + 4 * q;  // + 16*ti
-    const int col = j0 + wj * WTJ + r;      // + 16*tj
-    const CT *C = (const CT *)p.C + bt * p.sc;
-    DT *D = (DT *)p.D + bt * p.sd;
-
     float4_t acc[TI][TJ];
-#pragma unroll
-    for (int a = 0; a < TI; a++)
-#pragma unroll
-        for (int b = 0; b < TJ; b++) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
 
     const int NP = (p.K + KGRAN - 1) / KGRAN;  // pairs of k-steps
     const int NS = 2 * NP;                     // k-steps
@@ -227,7 +242,6 @@ void k_gemm_pp(tiled_params p)
     // slot of the current pair and `prev` the slot of the pair before it, which is the one being
     // refilled (with pair pr + 2).
     unsigned xpair = 0, xprev = 2 * xop::UNIT_BYTES, ypair = 0, yprev = (yop::UNITS - 1) * yop::UNIT_BYTES;
-    int xnext = 0, ynext = 0;  // next unit to request (step index for I-major, pair index for K-major)
     // Lane offsets of the loads of one unit: K-major loads differ by whole rows (a per-load lane
     // offset keeps one uniform base address), I-major loads by 256 bytes (the instruction's offset field).
     unsigned xvo[XK ? xop::NL : 1], yvo[YK ? yop::NL : 1];
@@ -236,33 +250,58 @@ void k_gemm_pp(tiled_params p)
 #pragma unroll
     for (int i = 0; i < (YK ? yop::NL : 1); i++) yvo[i] = yoff + 2u * (unsigned)yop::load_delta(i, p.ldy);
     // Load I of the unit at ring offset `unit` (bytes from the operand's region).
-    auto x_load = [&]<int I>(unsigned unit, std::integral_constant<int, I>) {
+    auto x_load = [&]<int I>(unsigned unit, std::integral_constant<int, I>) MIW_INLINE {
         if constexpr (XK) lds_dma16_at<I * NT * 16, 0>(X, xvo[I], wave_dst + unit);
         else lds_dma16_at<I * NT * 16, I * 256>(X, xvo[0], wave_dst + unit);
     };
-    auto y_load = [&]<int I>(unsigned unit, std::integral_constant<int, I>) {
+    auto y_load = [&]<int I>(unsigned unit, std::integral_constant<int, I>) MIW_INLINE {
         if constexpr (YK) lds_dma16_at<XB + I * NT * 16, 0>(Y, yvo[I], wave_dst + unit);
         else lds_dma16_at<XB + I * NT * 16, I * 256>(Y, yvo[0], wave_dst + unit);
     };
-    // Past the end of K the last unit is requested again, into a unit nobody reads any more.
     // Elements from one unit to the next; the first unit of the last pair (pair NP - 1, or entry NS - 2)
     // lies tail_skip k-values short of where it would follow on (a step back for an entry of 32 when 48
-    // repeat).  Both steps are kept as 64-bit values: computed per request, the multiplication by the
+    // repeat).  The steps are kept as 64-bit values: computed per request, the multiplication by the
     // leading dimension is a chain of scalar instructions at the end of every memory cluster, which is
     // the longer of the two clusters.
     constexpr int XUK = XK ? KGRAN : BKS, YUK = YK ? KGRAN : BKS;
-    const long xunit = XK ? (long)XUK : (long)XUK * p.ldx, xtail = XK ? (long)(XUK - tail_skip) : (long)(XUK - tail_skip) * p.ldx;
-    const long yunit = YK ? (long)YUK : (long)YUK * p.ldy, ytail = YK ? (long)(YUK - tail_skip) : (long)(YUK - tail_skip) * p.ldy;
-    auto x_advance = [&]() {
-        xnext++;
-        X += xnext == (XK ? NP - 1 : NS - 2) ? xtail : xnext < (XK ? NP : NS) ? xunit : 0;
+    long xunit = XK ? (long)XUK : (long)XUK * p.ldx, xtail = XK ? (long)(XUK - tail_skip) : (long)(XUK - tail_skip) * p.ldx;
+    long yunit = YK ? (long)YUK : (long)YUK * p.ldy, ytail = YK ? (long)(YUK - tail_skip) : (long)(YUK - tail_skip) * p.ldy;
+    // The requests run on past the end of K: unit XN of a tile is unit 0 of the workgroup's next tile,
+    // xjump elements from the last unit.  A workgroup without a next tile requests its last unit again (no
+    // step), into a unit nobody reads any more.
+    const int XN = XK ? NP : NS, YN = YK ? NP : NS;
+    int xnext = 0, ynext = 0;                                // unit to request next (step index for I-major, pair index for K-major)
+    long xjump = 0, yjump = 0;
+    bool has_next = false;
+    auto one_of = [](int next, int last, int end, long unit, long tail, long jump) MIW_INLINE {
+        return next == last ? tail : next == end ? jump : unit;
     };
-    auto y_advance = [&]() {
-        ynext++;
-        Y += ynext == (YK ? NP - 1 : NS - 2) ? ytail : ynext < (YK ? NP : NS) ? yunit : 0;
+    // ANY: the step may lead to the last pair or beyond; otherwise it is the plain one and xnext is not kept.
+    auto x_advance = [&]<bool ANY>(std::bool_constant<ANY>) MIW_INLINE {
+        if constexpr (ANY) {
+            xnext++;
+            X += one_of(xnext, XK ? NP - 1 : NS - 2, XN, xunit, xtail, xjump);
+            if (xnext >= XN && !has_next) xunit = 0;
+        } else {
+            X += xunit;
+        }
+    };
+    auto y_advance = [&]<bool ANY>(std::bool_constant<ANY>) MIW_INLINE {
+        if constexpr (ANY) {
+            ynext++;
+            Y += one_of(ynext, YK ? NP - 1 : NS - 2, YN, yunit, ytail, yjump);
+            if (ynext >= YN && !has_next) yunit = 0;
+        } else {
+            Y += yunit;
+        }
+    };
+    // Units requested when a tile's pair pr begins (both kinds of operand are ahead by that much).
+    auto next_units = [&](int pr) MIW_INLINE {
+        xnext = XK ? 2 + pr : 3 + 2 * pr;
+        ynext = KK ? 1 + pr : YK ? 2 + pr : 3 + 2 * pr;
     };
     // Request number N (0 .. ND-1) of the memory cluster of k-step 2 pr + H: the X loads, then the Y loads.
-    auto cluster_request = [&]<int H, int N>(std::integral_constant<int, H>, std::integral_constant<int, N>) {
+    auto cluster_request = [&]<int H, int N>(std::integral_constant<int, H>, std::integral_constant<int, N>) MIW_INLINE {
         if constexpr (KK) {
             // first cluster of a pair: all of Y's pair after next, into the slot of the pair before
             // (read to the end one barrier ago); second cluster: all of X's, likewise
@@ -277,11 +316,11 @@ void k_gemm_pp(tiled_params p)
             else y_load(H == 0 ? (ypair ^ (2u * yop::UNIT_BYTES)) + yop::UNIT_BYTES : ypair, std::integral_constant<int, M>{});
         }
     };
-    auto cluster_advance = [&]<int H>(std::integral_constant<int, H>) {
-        if constexpr (!XK || H == 1) x_advance();
-        if constexpr (!YK || H == (KK ? 0 : 1)) y_advance();
+    auto cluster_advance = [&]<int H, bool ANY>(std::integral_constant<int, H>, std::bool_constant<ANY> any) MIW_INLINE {
+        if constexpr (!XK || H == 1) x_advance(any);
+        if constexpr (!YK || H == (KK ? 0 : 1)) y_advance(any);
     };
-    auto pair_advance = [&]() {
+    auto pair_advance = [&]() MIW_INLINE {
         if constexpr (XK) {
             xprev = xpair;
             xpair = xpair + xop::UNIT_BYTES == xop::BYTES ? 0 : xpair + xop::UNIT_BYTES;
@@ -302,17 +341,17 @@ void k_gemm_pp(tiled_params p)
     // 0 have landed; the rest arrives under the first clusters.  The loop's own wait covers it: at the
     // end of memory cluster t it leaves 2 ND loads in flight, and the units of step 2 are at least ND
     // loads, so after cluster 0 the units of step 1 have landed and after cluster 1 those of step 2.
-    auto prologue_unit = [&]<int U>(std::integral_constant<int, U>, bool is_x) {
+    auto prologue_unit = [&]<int U>(std::integral_constant<int, U>, bool is_x) MIW_INLINE {
         if (is_x) {
             [&]<int... I>(std::integer_sequence<int, I...>) {
                 (x_load((unsigned)(U * xop::UNIT_BYTES), std::integral_constant<int, I>{}), ...);
             }(std::make_integer_sequence<int, xop::NL>{});
-            x_advance();
+            x_advance(std::true_type{});
         } else {
             [&]<int... I>(std::integer_sequence<int, I...>) {
                 (y_load((unsigned)(U * yop::UNIT_BYTES), std::integral_constant<int, I>{}), ...);
             }(std::make_integer_sequence<int, yop::NL>{});
-            y_advance();
+            y_advance(std::true_type{});
         }
     };
     constexpr std::integral_constant<int, 0> unit0{};
@@ -343,7 +382,7 @@ void k_gemm_pp(tiled_params p)
     // Fragment unit U of a step (the TI x-fragments, then the TJ y-fragments), preceded by the
     // requests that go out before it: request N before unit N * NFRAG / ND.
     auto cluster_unit = [&]<int H, int U>(MIW_LDS const char *xu, MIW_LDS const char *yu, std::integral_constant<int, H> h,
-                                          std::integral_constant<int, U>) {
+                                          std::integral_constant<int, U>) MIW_INLINE {
         [&]<int... N>(std::integer_sequence<int, N...>) {
             (([&] {
                  // (Y's loads of a two-K-major kernel have the least time to land: they go out first)
@@ -362,20 +401,20 @@ void k_gemm_pp(tiled_params p)
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto memory_cluster = [&]<int H>(std::integral_constant<int, H> h) {
-        MIW_LDS const char *xu = lds + xpair + (XK ? 0 : H * xop::UNIT_BYTES);
-        MIW_LDS const char *yu = lds + XB + ypair + (YK ? 0 : H * yop::UNIT_BYTES);
+    auto memory_cluster = [&]<int H, bool ANY>(std::integral_constant<int, H> h, std::bool_constant<ANY> any) MIW_INLINE {
+        MIW_LDS const char *xu = lds + xwave + xpair + (XK ? 0 : H * xop::UNIT_BYTES);
+        MIW_LDS const char *yu = lds + XB + ywave + ypair + (YK ? 0 : H * yop::UNIT_BYTES);
         [&]<int... U>(std::integer_sequence<int, U...>) {
             (cluster_unit(xu, yu, h, std::integral_constant<int, U>{}), ...);
         }(std::make_integer_sequence<int, NFRAG>{});
         // The ring state and the operand pointers move on here, behind the last fragment read and under its
         // latency.  (Measured: the same scalar instructions between the first MFMAs of the compute cluster
         // hold the matrix core up for 65 cycles per cluster; between the fragment reads, for 19.)
-        cluster_advance(h);
+        cluster_advance(h, any);
         if constexpr (H == 1) pair_advance();
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto compute_cluster = [&]() {
+    auto compute_cluster = [&]() MIW_INLINE {
         __builtin_amdgcn_sched_barrier(0);
         // serpentine order: every MFMA changes exactly one of its two operand fragments
 #pragma unroll
@@ -388,175 +427,251 @@ void k_gemm_pp(tiled_params p)
             }
     };
 
-    // Folding C.  With alpha == 1 the C operand is added into the accumulators during the last
-    // NFOLD k-steps, CPT MFMA tiles per memory cluster, so that the memory system delivers C
-    // while the matrix cores run and the epilogue only stores.  The tiles of fold step S are
-    // requested at the end of the memory cluster with ordinary loads into registers (the lane
-    // fetches the 16 bytes it owns); they are the youngest loads of their cluster, so the wait at
-    // the end of the cluster two steps later covers them, and that cluster adds them in: C has
-    // two clusters of both wavefront groups to arrive.  Three register stages rotate.  Tiles go in
-    // the order of their addresses: 16 rows (64 bytes, the instruction's offset field) further
-    // down a column block, then the next 16 columns.  The accumulators are registers, so the
-    // folding steps are unrolled.
-    constexpr int CPT = 1;
+    // Folding C.  The C operand is added into the accumulators during the last NFOLD k-steps, one MFMA tile per
+    // step, so that the memory system delivers C while the matrix cores run and the epilogue only stores.  The
+    // tile of fold step S is requested at the start of the step with an ordinary load into registers (the lane
+    // fetches the 16 bytes it owns); the wait at the end of the memory cluster two steps later covers it, and that
+    // cluster adds it in: C has two clusters of both wavefront groups to arrive, and what it takes longer stalls the
+    // loop, since loads return in order.  (Requested behind the cluster's own loads, or two tiles every other step,
+    // 8192x8192x1024 takes 3 % longer.)  Three register stages rotate.  Tiles go in the order of their addresses: 16
+    // rows (64 bytes, the instruction's offset field) further down a column block, then the next 16 columns.  The
+    // accumulators are registers, so the folding steps are unrolled.
     constexpr int NTILE = TI * TJ;
-    constexpr int NFOLD = NTILE / CPT;
-    constexpr bool CAN_FOLD = __is_same(CT, float) && TI % CPT == 0 && NFOLD % 2 == 0;
-    bool fold_c = false;
+    constexpr int NFOLD = NTILE;
+    static_assert(!FOLD || (__is_same(CT, float) && NFOLD == PP_FOLD_STEPS && NFOLD % 2 == 0), "fold steps");
+    float4_t cst[3];
+    const char *cnext = nullptr;
+    const float fold_beta = p.alpha * p.beta;  // the epilogue multiplies the sums by alpha
     // (the lane offset into the tile of C is kept in 32 bits)
-    if constexpr (CAN_FOLD) fold_c = p.use_c && !p.c_trans && p.alpha == 1.0f && NS >= NFOLD + 2 && p.ldc < (1l << 22);
-    float4_t cst[3][CPT];
-    const char *cnext = (const char *)(C + (long)j0 * p.ldc + i0);
     const unsigned coff = 4u * (unsigned)((wj * WTJ + r) * (int)p.ldc + wi * WTI + 4 * q);
-    auto fold_request = [&]<int S>(std::integral_constant<int, S>) {
-        [&]<int... U>(std::integer_sequence<int, U...>) {
-            (([&] {
-                 constexpr int a = (S * CPT + U) % TI;
-                 asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(cst[S % 3][U]) : "v"(coff), "s"(cnext), "n"(64 * a) : "memory");
-                 if constexpr (a == TI - 1) cnext += 64 * p.ldc;
-             }()),
-             ...);
-        }(std::make_integer_sequence<int, CPT>{});
+    auto fold_request = [&]<int S>(std::integral_constant<int, S>) MIW_INLINE {
+        constexpr int a = S % TI;
+        asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(cst[S % 3]) : "v"(coff), "s"(cnext), "n"(64 * a) : "memory");
+        if constexpr (a == TI - 1) cnext += 64 * p.ldc;
     };
-    auto fold_add = [&]<int S>(std::integral_constant<int, S>) {
+    auto fold_add = [&]<int S>(std::integral_constant<int, S>) MIW_INLINE {
+        constexpr int a = S % TI, b = S / TI;
 #pragma unroll
-        for (int u = 0; u < CPT; u++) {
-            const int a = (S * CPT + u) % TI, b = (S * CPT + u) / TI;
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[a][b][e] = __builtin_fmaf(p.beta, cst[S % 3][u][e], acc[a][b][e]);
-        }
+        for (int e = 0; e < 4; e++) acc[a][b][e] = __builtin_fmaf(fold_beta, cst[S % 3][e], acc[a][b][e]);
     };
-    // One k-step: memory cluster, barrier, compute cluster, barrier.  FS >= 0: fold step FS.
     // Zeroes the repeated k-values in the fragments of step H of the shifted last pair.
-    auto mask_tail = [&]<int H>(std::integral_constant<int, H>) {
-        const unsigned keep = tail_keep<H>(tail_skip);
+    auto mask_tail = [&]<int H>(std::integral_constant<int, H>) MIW_INLINE {
+        int skip = tail_skip;
+        asm volatile("" : "+s"(skip));  // (the mask is made here, not kept through the tiles)
+        const unsigned keep = tail_keep<H>(skip);
 #pragma unroll
         for (int a = 0; a < TI; a++) tail_apply(fx[a], keep);
 #pragma unroll
         for (int b = 0; b < TJ; b++) tail_apply(fy[b], keep);
     };
-    // FS >= 0: fold step FS (always folds).  FS == -1: a step that does not fold.  FS == -2: a step of
-    // the last pair: its fragments are masked, and it is fold step NFOLD - 2 + H when the launch folds C,
-    // which is decided here at run time, so that the last pair is one piece of code for both cases (two
-    // alternative pieces that each update all accumulators cost spills where they join).
-    auto fold_wait = [&]<int H, int FS>(std::integral_constant<int, H>, std::integral_constant<int, FS>) {
-        // fold step FS issues ND + CPT loads; steps before the first fold step issue ND
-        constexpr int YOUNGER = (KK && H == 1 ? ND : 2 * ND) + (FS >= 1 ? 2 : 1) * CPT;
+    // One k-step: memory cluster, barrier, compute cluster, barrier.  FS: fold step, or -1; ANY: see x_advance; LAST:
+    // a step of the last pair.  slack: a step of the first pair of a workgroup's second or later tile.  The NSTORE
+    // stores of the tile before are then younger than the loads that the wait is for and may stay in flight.
+    constexpr std::integral_constant<int, -1> no_fold{};
+    constexpr int NSTORE = TI * TJ;
+    auto wait_vm = [&]<int N>(std::integral_constant<int, N>) MIW_INLINE {
+        static_assert(N < 64, "vmcnt");
         asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt((YOUNGER & 15) | (7 << 4) | (0 << 8) | ((YOUNGER >> 4) << 14));
+        __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (0 << 8) | ((N >> 4) << 14));
         asm volatile("" ::: "memory");
     };
-    auto step = [&]<int H, int FS>(std::integral_constant<int, H> h, std::integral_constant<int, FS>) {
-        memory_cluster(h);
+    auto step_wait = [&]<int H, int FS>(std::integral_constant<int, H>, std::integral_constant<int, FS>, bool slack) MIW_INLINE {
+        // What may stay in flight: the cluster's own loads and, unless they have to land too, those of the cluster
+        // before; a fold step issues a load of C ahead of the cluster's.
+        constexpr bool BOTH = !(KK && H == 1);
+        constexpr int YOUNGER = (BOTH ? 2 : 1) * ND + (FS >= 0 ? (BOTH && FS >= 1 ? 2 : 1) : 0);
+        // (the second cluster of two K-major operands waits for loads that were issued behind the stores)
+        if (slack && BOTH) wait_vm(std::integral_constant<int, YOUNGER + NSTORE>{});
+        else wait_vm(std::integral_constant<int, YOUNGER>{});
+    };
+    auto barrier = [&]() {
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    auto step = [&]<int H, int FS, bool ANY, bool LAST>(std::integral_constant<int, H> h, std::integral_constant<int, FS> fs,
+                                                        std::bool_constant<ANY> any, std::bool_constant<LAST>, bool slack) MIW_INLINE {
         if constexpr (FS >= 0) {
-            fold_request(std::integral_constant<int, FS>{});
+            fold_request(fs);
             __builtin_amdgcn_sched_barrier(0);
-            fold_wait(h, std::integral_constant<int, FS>{});
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (FS >= 2) fold_add(std::integral_constant<int, FS - 2>{});
-            __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-        } else if constexpr (FS == -2 && CAN_FOLD) {
-            constexpr int LFS = NFOLD - 2 + H;
-            if (fold_c) {
-                fold_request(std::integral_constant<int, LFS>{});
-                fold_wait(h, std::integral_constant<int, LFS>{});
-                fold_add(std::integral_constant<int, LFS - 2>{});
-                __builtin_amdgcn_s_barrier();
-                asm volatile("" ::: "memory");
-            } else {
-                wait_loads_and_barrier<(KK && H == 1 ? ND : 2 * ND)>();
-            }
-        } else {
-            wait_loads_and_barrier<(KK && H == 1 ? ND : 2 * ND)>();
         }
-        if constexpr (FS == -2) mask_tail(h);
+        memory_cluster(h, any);
+        step_wait(h, fs, slack);
+        if constexpr (FS >= 2) {
+            __builtin_amdgcn_sched_barrier(0);
+            fold_add(std::integral_constant<int, FS - 2>{});
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        barrier();
+        if constexpr (LAST) mask_tail(h);
         compute_cluster();
         __builtin_amdgcn_s_barrier();
     };
-    constexpr std::integral_constant<int, -1> no_fold{};
-    constexpr std::integral_constant<int, -2> last_pair{};
+    constexpr std::true_type last_pair{};
+    constexpr std::false_type inner{};
+    constexpr std::integral_constant<int, 0> first_half{};
+    constexpr std::integral_constant<int, 1> second_half{};
+    constexpr std::true_type any{};     // the cluster's requests may reach the last pair
+    constexpr std::false_type plain{};
+
+    for (bool later = false;; later = true) {  // tiles of this workgroup
+    // Does another tile follow (then NP >= 4, see tiled_params::work), and how do the operands get there?
+    auto first_args = arguments();
+    has_next = tile + (int)gridDim.x < first_args->work;
+    if (has_next) {
+        int bt_next = bt, i0_next, j0_next;
+        locate(first_args, tile + (int)gridDim.x, bt_next, i0_next, j0_next);
+        xjump = x_origin(first_args, bt_next, i0_next) - x_origin(first_args, bt, i0) - ((XN - 2) * xunit + xtail);
+        yjump = y_origin(first_args, bt_next, j0_next) - y_origin(first_args, bt, j0) - ((YN - 2) * yunit + ytail);
+    } else {
+        xjump = yjump = 0;
+    }
+    if constexpr (FOLD) cnext = (const char *)((const CT *)first_args->C + (long)bt * first_args->sc + (long)j0 * first_args->ldc + i0);
+    float zero = 0.f;
+    asm volatile("" : "+s"(zero));  // (otherwise a zero vector is kept in registers through the tiles)
+#pragma unroll
+    for (int a = 0; a < TI; a++)
+#pragma unroll
+        for (int b = 0; b < TJ; b++) acc[a][b] = float4_t{zero, zero, zero, zero};
 
     MIW_PP_STAMP(1)
     if (late_group) __builtin_amdgcn_s_barrier();
-    // the loop runs the pairs that neither fold nor are the last one
-    const int NPM = fold_c ? NP - NFOLD / 2 : NP - 1;
-    for (int pr = 0; pr < NPM; pr++) {
+    // the pairs before NPM neither fold nor are the last one; those from NP - 4 on may request the last
+    // pair or the next tile
+    const int NPM = FOLD ? NP - NFOLD / 2 : NP - 1;
+    next_units(0);
+    if (NPM > 0) {
+        step(first_half, no_fold, any, inner, later);
+        step(second_half, no_fold, any, inner, later);
+    }
+    int pr = 1;
+    for (; pr < min(NPM, NP - 4); pr++) {
 #ifdef MIW_PP_TS
         if (pr == NPM / 2) MIW_PP_STAMP(2)
         if (pr == NPM / 2 + 1) MIW_PP_STAMP(3)
 #endif
-        step(std::integral_constant<int, 0>{}, no_fold);
-        step(std::integral_constant<int, 1>{}, no_fold);
+        step(first_half, no_fold, plain, inner, false);
+        step(second_half, no_fold, plain, inner, false);
+    }
+    next_units(pr);
+    for (; pr < NPM; pr++) {
+        step(first_half, no_fold, any, inner, false);
+        step(second_half, no_fold, any, inner, false);
     }
     MIW_PP_STAMP(9)
-    if constexpr (CAN_FOLD) {
-        if (fold_c) {
-            [&]<int... G>(std::integer_sequence<int, G...>) {
-                ((step(std::integral_constant<int, 0>{}, std::integral_constant<int, 2 * G>{}),
-                  step(std::integral_constant<int, 1>{}, std::integral_constant<int, 2 * G + 1>{})),
-                 ...);
-            }(std::make_integer_sequence<int, NFOLD / 2 - 1>{});
-        }
+    if constexpr (FOLD) {
+        constexpr int GANY = NFOLD / 2 - 4;  // first pair of the last four
+        [&]<int... G>(std::integer_sequence<int, G...>) {
+            (([&] {
+                 if constexpr (G == GANY) next_units(NP - 4);
+                 constexpr std::bool_constant<(G >= GANY)> a{};
+                 const bool slack = G == 0 && later && NPM == 0;
+                 step(first_half, std::integral_constant<int, 2 * G>{}, a, inner, slack);
+                 step(second_half, std::integral_constant<int, 2 * G + 1>{}, a, inner, slack);
+             }()),
+             ...);
+        }(std::make_integer_sequence<int, NFOLD / 2 - 1>{});
     }
-    step(std::integral_constant<int, 0>{}, last_pair);
-    step(std::integral_constant<int, 1>{}, last_pair);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may outlive the workgroup's LDS
-    if constexpr (CAN_FOLD) {
-        if (fold_c) {
-            fold_add(std::integral_constant<int, NFOLD - 2>{});
-            fold_add(std::integral_constant<int, NFOLD - 1>{});
-        }
+    step(first_half, std::integral_constant<int, FOLD ? NFOLD - 2 : -1>{}, any, last_pair, false);
+    step(second_half, std::integral_constant<int, FOLD ? NFOLD - 1 : -1>{}, any, last_pair, false);
+    if (FOLD || !has_next) wait_vm(std::integral_constant<int, 0>{});  // the last tiles of C; no load may outlive the workgroup's LDS
+    if constexpr (FOLD) {
+        fold_add(std::integral_constant<int, NFOLD - 2>{});
+        fold_add(std::integral_constant<int, NFOLD - 1>{});
     }
     if (!late_group) __builtin_amdgcn_s_barrier();
     MIW_PP_STAMP(4)
 
-    // Epilogue: each lane owns 4 consecutive i of one column j per MFMA tile.
-    auto read_c = [&](int a, int b, bool trans) -> float4_t {
-        float4_t c;
-        const int ii = row + 16 * a, jj = col + 16 * b;
-        if (trans) {
-#pragma unroll
-            for (int v = 0; v < 4; v++) c[v] = (float)C[(long)(ii + v) * p.ldc + jj];
-        } else if constexpr (__is_same(CT, float)) {
-            c = *(const float4_t *)(C + (long)jj * p.ldc + ii);
-        } else {
-            half4_t h = *(const half4_t *)(C + (long)jj * p.ldc + ii);
-            c = float4_t{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
-        }
-        return c;
-    };
+    // Epilogue: each lane owns 4 consecutive i of one column j per MFMA tile.  Pairs of tiles are exchanged between
+    // neighbouring lanes before C is added, so that C is read as D is stored, in pieces of whole lines.
     static_assert(TI % 2 == 0, "the epilogue stores pairs of tiles");
-    auto epilogue = [&](bool with_c, bool trans) {
-        auto value = [&](int a, int b) {
-            float4_t v = acc[a][b];
-#pragma unroll
-            for (int e = 0; e < 4; e++) v[e] *= p.alpha;
-            if (with_c) {
-                float4_t c = read_c(a, b, trans);
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = __builtin_fmaf(p.beta, c[e], v[e]);
-            }
-            return v;
-        };
+    auto args = arguments();
+    const long ldd = args->ldd, ldc = args->ldc;
+    int lane = tid & 63;
+    asm volatile("" : "+v"(lane));  // (what is made of it is made here, not kept through the K loop)
+    const bool odd = lane & 1;
+    const float alpha = args->alpha, beta = args->beta;
+    DT *D = (DT *)args->D + (long)bt * args->sd + (long)(j0 + wj * WTJ) * ldd + (i0 + wi * WTI) + pair_place(lane, ldd);
+    auto store = [](DT *to, float4_t v) MIW_INLINE {
+        if constexpr (__is_same(DT, float)) __builtin_nontemporal_store(v, (float4_t *)to);
+        else *(half4_t *)to = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+    };
+    // C_AT 0: no C, 1: laid out as D, 2: the other way round
+    auto epilogue = [&]<int C_AT, bool STREAM>(std::integral_constant<int, C_AT>, std::bool_constant<STREAM>) MIW_INLINE {
+        const CT *C = nullptr;
+        if constexpr (C_AT == 1) C = (const CT *)args->C + (long)bt * args->sc + (long)(j0 + wj * WTJ) * ldc + (i0 + wi * WTI) + pair_place(lane, ldc);
+        // (columns r - odd and the next, rows 16 odd + 4 q ..)
+        if constexpr (C_AT == 2) C = (const CT *)args->C + (long)bt * args->sc + (long)(i0 + wi * WTI + 16 * odd + 4 * (lane >> 4)) * ldc + (j0 + wj * WTJ + (lane & 14));
 #pragma unroll
         for (int b = 0; b < TJ; b++)
 #pragma unroll
-            for (int a = 0; a < TI; a += 2)
-                store_tile_pair<DT>(D, p.ldd, i0 + wi * WTI + 16 * a, j0 + wj * WTJ + 16 * b, lane, value(a, b), value(a + 1, b));
+            for (int a = 0; a < TI; a += 2) {
+                float4_t v[2] = {acc[a][b], acc[a + 1][b]};
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[t][e] *= alpha;
+                if constexpr (C_AT == 0) {
+                    store_pair_at<STREAM>(D + 16 * b * ldd + 16 * a, ldd, odd, v[0], v[1]);
+                } else {
+                    pair_exchange(odd, v[0], v[1]);
+#pragma unroll
+                    for (int t = 0; t < 2; t++) {
+                        float4_t c;
+                        if constexpr (C_AT == 2) {
+#pragma unroll
+                            for (int e = 0; e < 4; e++) c[e] = (float)C[(16 * a + e) * ldc + 16 * b + t];
+                        } else if constexpr (__is_same(CT, float)) {
+                            c = *(const float4_t *)(C + (16 * b + t) * ldc + 16 * a);
+                        } else {
+                            const half4_t h = *(const half4_t *)(C + (16 * b + t) * ldc + 16 * a);
+                            c = float4_t{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
+                        }
+#pragma unroll
+                        for (int e = 0; e < 4; e++) v[t][e] = __builtin_fmaf(beta, c[e], v[t][e]);
+                    }
+                    store(D + 16 * b * ldd + 16 * a, v[0]);
+                    store(D + (16 * b + 1) * ldd + 16 * a, v[1]);
+                }
+            }
     };
-    if (!p.use_c || fold_c) epilogue(false, false);
-    else if (p.c_trans) epilogue(true, true);
-    else epilogue(true, false);
+    // A Float32 D is written past the L2 where C or the operands of more tiles come through it at the same time
+    // (4096x4096x512 with C from HBM: 34 us, 42 through the L2; 8192x8192x1024 without C 126 and 134), and through it
+    // where nothing follows in the launch (4096x4096x512 without C: 26 us, 28 past it).
+    if (FOLD) epilogue(std::integral_constant<int, 0>{}, std::true_type{});
+    else if (args->use_c && args->c_trans) epilogue(std::integral_constant<int, 2>{}, std::true_type{});
+    else if (args->use_c) epilogue(std::integral_constant<int, 1>{}, std::true_type{});
+    else if (args->work) epilogue(std::integral_constant<int, 0>{}, std::true_type{});
+    else epilogue(std::integral_constant<int, 0>{}, std::false_type{});
 #ifdef MIW_PP_TS
     MIW_PP_STAMP(5)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     MIW_PP_STAMP(6)
     ts[7] = wall_clock64();
     if (p.ts && lane == 0)
-        for (int i = 0; i < 10; i++) p.ts[((long)(blockIdx.y * gridDim.x + blockIdx.x) * 8 + wave) * 10 + i] = ts[i];
+        for (int i = 0; i < 10; i++) p.ts[((long)(tile + (long)blockIdx.y * gridDim.x) * 8 + wave) * 10 + i] = ts[i];
+    ts[0] = clock64();
+    ts[8] = wall_clock64();
 #endif
+    if (!has_next) break;
+    tile += (int)gridDim.x;
+    locate(arguments(), tile, bt, i0, j0);
+    }
+}
+
+// C, if any, is read in the epilogue.
+template <int BI, int BJ, int WI, int WJ, bool XK, bool YK, class CT, class DT>
+__global__ __launch_bounds__(WI *WJ * 64) __attribute__((amdgpu_waves_per_eu(2)))
+void k_gemm_pp(tiled_params p)
+{
+    gemm_pp<BI, BJ, WI, WJ, XK, YK, CT, DT, false>(p);
+}
+
+// A Float32 C is folded into the K loop.
+template <int BI, int BJ, int WI, int WJ, bool XK, bool YK, class DT>
+__global__ __launch_bounds__(WI *WJ * 64) __attribute__((amdgpu_waves_per_eu(2)))
+void k_gemm_pp_fold(tiled_params p)
+{
+    gemm_pp<BI, BJ, WI, WJ, XK, YK, float, DT, true>(p);
 }
 
 // ---------------------------------------------------------------------------

@@ -84,6 +84,9 @@ struct tiled_params {
     // overlap from the same operands in the same order and store equal values.  The host allows
     // this only when C and D do not share memory.
     int tiles_i, tiles_j, group_i;
+    // Workgroups that walk several tiles (k_gemm_pp): number of tiles over the whole batch; a workgroup takes tile
+    // blockIdx.x, then every gridDim.x-th.  0: one tile per workgroup.  Needs K of four slots or more.
+    int work;
 #ifdef MIW_PP_TS
     long long *ts;  // measurement builds: 10 counters per wavefront (see k_gemm_pp64), or null
 #endif
@@ -267,24 +270,34 @@ __device__ inline unsigned quad_swap(unsigned v)
 {
     return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1 /* quad_perm:[1,0,3,2] */, 0xf, 0xf, true);
 }
-template <class DT>
-__device__ inline void store_tile_pair(DT *D, long ldd, int row, int col0, int lane, float4_t v0, float4_t v1)
+// pair_exchange makes the two columns' pieces of the accumulators, store_pair_at writes them; `even` points to
+// this lane's place in the even column, see pair_place.
+__device__ inline void pair_exchange(bool odd, float4_t &v0, float4_t &v1)
 {
-    const int r = lane & 15, q = lane >> 4;
-    const bool odd = r & 1;
-    // both instructions: this lane writes rows row + 16 * odd + 4 q .. + 3; column col0 + r - odd, then the next
-    DT *dst = D + (long)(col0 + r - (odd ? 1 : 0)) * ldd + (row + (odd ? 16 : 0) + 4 * q);
-    if constexpr (__is_same(DT, float)) {
-        const uint4_t p = __builtin_bit_cast(uint4_t, v0), t = __builtin_bit_cast(uint4_t, v1);
-        uint4_t s0, s1;
+    const uint4_t p = __builtin_bit_cast(uint4_t, v0), t = __builtin_bit_cast(uint4_t, v1);
+    uint4_t s0, s1;
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const unsigned ps = quad_swap(p[e]), ts = quad_swap(t[e]);
-            s0[e] = odd ? ts : p[e];   // even column: own upper tile | the even neighbour's lower tile
-            s1[e] = odd ? t[e] : ps;   // odd column: the odd neighbour's upper tile | own lower tile
+    for (int e = 0; e < 4; e++) {
+        const unsigned ps = quad_swap(p[e]), ts = quad_swap(t[e]);
+        s0[e] = odd ? ts : p[e];   // even column: own upper tile | the even neighbour's lower tile
+        s1[e] = odd ? t[e] : ps;   // odd column: the odd neighbour's upper tile | own lower tile
+    }
+    v0 = __builtin_bit_cast(float4_t, s0);
+    v1 = __builtin_bit_cast(float4_t, s1);
+}
+// STREAM: write past the L2 (Float32 only: half lines, as Float16 pairs write them, are better gathered there).
+template <bool STREAM = false, class DT>
+__device__ inline void store_pair_at(DT *even, long ldd, bool odd, float4_t v0, float4_t v1)
+{
+    if constexpr (__is_same(DT, float)) {
+        pair_exchange(odd, v0, v1);
+        if constexpr (STREAM) {
+            __builtin_nontemporal_store(v0, (float4_t *)even);
+            __builtin_nontemporal_store(v1, (float4_t *)(even + ldd));
+        } else {
+            *(float4_t *)even = v0;
+            *(float4_t *)(even + ldd) = v1;
         }
-        *(uint4_t *)dst = s0;
-        *(uint4_t *)(dst + ldd) = s1;
     } else {
         const half4_t h0 = {(half_t)v0[0], (half_t)v0[1], (half_t)v0[2], (half_t)v0[3]};
         const half4_t h1 = {(half_t)v1[0], (half_t)v1[1], (half_t)v1[2], (half_t)v1[3]};
@@ -296,9 +309,21 @@ __device__ inline void store_tile_pair(DT *D, long ldd, int row, int col0, int l
             s0[e] = odd ? ts : p[e];
             s1[e] = odd ? t[e] : ps;
         }
-        *(uint2_t *)dst = s0;
-        *(uint2_t *)(dst + ldd) = s1;
+        *(uint2_t *)even = s0;
+        *(uint2_t *)(even + ldd) = s1;
     }
+}
+// Elements from the first value of a pair of tiles to where this lane writes in the even columns: rows
+// 16 * odd + 4 q .. + 3 of column r - odd.
+__device__ inline long pair_place(int lane, long ldd)
+{
+    const int r = lane & 15, q = lane >> 4, odd = r & 1;
+    return (long)(r - odd) * ldd + 16 * odd + 4 * q;
+}
+template <class DT>
+__device__ inline void store_tile_pair(DT *D, long ldd, int row, int col0, int lane, float4_t v0, float4_t v1)
+{
+    store_pair_at(D + (long)col0 * ldd + row + pair_place(lane, ldd), ldd, lane & 1, v0, v1);
 }
 
 // Ordinal of the direct-to-LDS load issued after MFMA m of a step of nmfma

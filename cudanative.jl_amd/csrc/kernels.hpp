@@ -84,7 +84,7 @@ bool tiled_supports_f16acc(int i);
 // one tile (whole tiles when C and D share memory), K of at least 64, 16-byte alignment of
 // pointers and leading dimensions, and for fp16 accumulation c_type == d_type == Float16 and,
 // outside the 64-k ping-pong kernels, alpha == 1.
-hipError_t launch_gemm_tiled(int i, const gemm_params &p, int c_type, int d_type, bool f16acc, hipStream_t s);
+hipError_t launch_gemm_tiled(int i, const gemm_params &p, int c_type, int d_type, bool f16acc, int cus, hipStream_t s);
 // Does variant i have a kernel for this combination of operand layouts?
 bool tiled_supports_layout(int i, const gemm_params &p);
 // Does the problem's tile count fit the launch grid of variant i?

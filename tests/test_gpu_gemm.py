@@ -178,6 +178,26 @@ def test_c_folded_into_the_loop_exact_on_integers(gpu, orc, al, bl, dl, K):
         assert np.array_equal(D, orc.gemm(g, A, B, C)), (v["name"], al, bl, dl, K)
 
 
+@pytest.mark.parametrize("al,bl", itertools.product((0, 1), repeat=2))
+@pytest.mark.parametrize("K", [256, 272, 960, 976, 1024, 1040])
+def test_workgroups_that_walk_several_tiles(gpu, orc, al, bl, K):
+    """More 256x256 tiles than CUs: a workgroup's operand requests run on from one tile into the next.  Four slots
+    of K (the shortest that do), ragged last slots, fifteen (C added behind the loop) and sixteen (added from the
+    first step on); tiles of several batch members and shifted edge tiles; every form of C; bit-exact on integers."""
+    v = _vid(gpu, "tile256x256_pingpong")
+    rng = np.random.default_rng(K + 2 * al + bl)
+    forms = [dict(c_type=orc.F32, alpha=-1.0, beta=2.0), dict(c_type=orc.F32, use_c=0), dict(c_type=orc.F16, alpha=1.0),
+             dict(c_type=orc.F32, alpha=0.5, beta=0.5), dict(c_type=orc.F32, other_layout=True)]
+    for i in rng.permutation(len(forms))[:2]:
+        form = dict(forms[i])
+        dl = int(rng.integers(0, 2))
+        cl = 1 - dl if form.pop("other_layout", False) else dl
+        g = orc.GemmDesc(M=272 if dl else 256, N=256 if dl else 272, K=K, a_layout=al, b_layout=bl, c_layout=cl, d_layout=dl, batch=131, **form)
+        A, B, C = _inputs(orc, g, K + int(i), ints=True)
+        D = _run(gpu, orc, g, A, B, C if g.use_c else None, variant=v)
+        assert np.array_equal(D, orc.gemm(g, A, B, C)), (al, bl, cl, dl, K, form)
+
+
 def test_c_folded_into_the_loop_matches_the_epilogue_path(gpu, orc):
     """Random inputs, padded leading dimensions, batches: the folded C (alpha == 1, C laid out as D)
     agrees with float64 as tightly as the kernels that add C after the loop (alpha != 1, the
