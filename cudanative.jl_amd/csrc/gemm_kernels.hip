@@ -3,6 +3,7 @@
 // gemm_tile_*.hip translation units (one per tile family, so that they build in parallel).
 #include "gemm_tiled.hpp"
 
+#include <algorithm>
 #include <cstdlib>
 #include <mutex>
 #include <unordered_map>
@@ -52,6 +53,7 @@ bool pp_folds(const tiled_params &p, int c_type);
 int pp_lds(int bm, int bn, bool xk, bool yk);
 const void *w128_kernel(bool xk, bool yk, int c_type, int d_type);
 const void *pp64_kernel(int bm, int bn, bool xk, bool yk, int c_type, int d_type, bool f16acc);
+
 
 
 // Tile shape in canonical (I, J) terms: bm applies to I, bn to J.
@@ -113,26 +115,52 @@ static hipError_t allow_dynamic_lds(const void *fn, int bytes)
     return e;
 }
 
-hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type, bool f16acc, int cus, hipStream_t s)
+// Multiplier and shift for quotient() of gemm_tiled.hpp.
+static unsigned multiplier(long d, unsigned *shift)
 {
-    const tiled_variant &v = g_variants[i];
+    *shift = 0;
+    while ((1l << *shift) < d) ++*shift;
+    return (unsigned)(((1l << (31 + *shift)) + d - 1) / d);
+}
+
+// How the launch's workgroups find their tiles (see tile_at in gemm_tiled.hpp); walk: workgroups that take several.
+static void set_raster(tiled_params *p, long batch, bool walk)
+{
+    const long tiles = (long)p->tiles_i * p->tiles_j, all = tiles * batch;
+    const bool span = batch > 1 && (tiles > 1 || walk) && all < (1l << 30);
+    p->span = span ? (int)tiles : 0;
+    p->total = (int)(span ? all : tiles);
+    // Rows of tiles per raster group: about the square root of one XCD's share.
+    const long per_xcd = span ? std::min(tiles, (all + 7) / 8) : (tiles + 7) / 8;
+    long rows = 1;
+    while ((rows * 2) * (rows * 2) <= per_xcd) rows *= 2;
+    rows = std::min(rows, (long)p->tiles_i);
+    p->group_i = (int)rows;
+    const long group = rows * p->tiles_j, last = p->tiles_i % rows;
+    unsigned member_s = 0, group_s, rows_s, last_s = 0;
+    p->span_m = span ? multiplier(tiles, &member_s) : 0;
+    p->group_m = multiplier(group, &group_s);
+    p->rows_m = multiplier(rows, &rows_s);
+    p->last_m = last ? multiplier(last, &last_s) : 0;
+    p->shifts = member_s | group_s << 8 | rows_s << 16 | last_s << 24;
+}
+
+// The problem in canonical form (see gemm_tiled.hpp) on bi x bj tiles; *xk, *yk: k contiguous in X, in Y.
+static tiled_params canonical(const gemm_params &g, int bi, int bj, bool *xk, bool *yk)
+{
     tiled_params p;
-    bool xk, yk;
+    canonical_layout(g, xk, yk);
     if (!g.d_row) {
         // P = D (M x N, M contiguous): X = A, Y = B
         p.X = g.A; p.Y = g.B;
         p.I = (int)g.M; p.J = (int)g.N;
         p.ldx = g.lda; p.ldy = g.ldb; p.sx = g.sa; p.sy = g.sb;
-        xk = g.a_row != 0;   // A row-major: k contiguous
-        yk = g.b_row == 0;   // B column-major: k contiguous
         p.c_trans = g.c_row != 0;
     } else {
         // P = D^T (N x M, N contiguous): X = B^T, Y = A^T
         p.X = g.B; p.Y = g.A;
         p.I = (int)g.N; p.J = (int)g.M;
         p.ldx = g.ldb; p.ldy = g.lda; p.sx = g.sb; p.sy = g.sa;
-        xk = g.b_row == 0;
-        yk = g.a_row != 0;
         p.c_trans = g.c_row == 0;
     }
     p.C = g.C; p.D = g.D;
@@ -141,12 +169,20 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
     p.ldc = g.ldc; p.ldd = g.ldd; p.sc = g.sc; p.sd = g.sd;
     p.use_c = g.use_c;
     p.alpha = g.alpha; p.beta = g.beta;
-    p.tiles_i = (p.I + v.bm - 1) / v.bm;
-    p.tiles_j = (p.J + v.bn - 1) / v.bn;
-    // Rows of tiles per raster group: about the square root of one XCD's share.
-    int per_xcd = (p.tiles_i * p.tiles_j + 7) / 8, gi = 1;
-    while ((gi * 2) * (gi * 2) <= per_xcd) gi *= 2;
-    p.group_i = gi < p.tiles_i ? gi : p.tiles_i;
+    p.tiles_i = (p.I + bi - 1) / bi;
+    p.tiles_j = (p.J + bj - 1) / bj;
+    set_raster(&p, g.batch, false);
+#ifdef MIW_PP_TS
+    p.ts = nullptr;
+#endif
+    return p;
+}
+
+hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type, bool f16acc, int cus, hipStream_t s)
+{
+    const tiled_variant &v = g_variants[i];
+    bool xk, yk;
+    tiled_params p = canonical(g, v.bm, v.bn, &xk, &yk);
 
 #ifdef MIW_PP_TS
     // measurement builds: device address of the timestamp buffer, in hexadecimal
@@ -171,6 +207,7 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
     // Below four slots of K there is too little of it to request across two tiles, and the launch is bound by C and D.
     if (v.kind == KIND_PINGPONG32 && tiles > cus && tiles < (1l << 30) && p.K > 3 * KGRAN) {
         p.work = (int)tiles;
+        set_raster(&p, g.batch, true);
         grid = dim3((unsigned)cus, 1);
     }
     return hipLaunchKernel(fn, grid, dim3((unsigned)(v.wm * v.wn * 64)), args, (size_t)lds_bytes, s);
@@ -191,12 +228,28 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const float *ws, int spli
     if (idx >= quads * J) return;
     const long j = idx / quads, i = (idx - j * quads) * 4;
     const float *src = ws + j * I + i;
+    // (four slices at a time are on the way; one at a time each addition waits for the memory's latency)
+    const long slice = I * J;
     float4_t sum = *(const float4_t *)src;
-    for (int s = 1; s < splits; s++) {
-        const float4_t v = *(const float4_t *)(src + (long)s * I * J);
+    int s = 1;
+    for (; s + 4 <= splits; s += 4) {
+        float4_t v[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) sum[e] += v[e];
+        for (int u = 0; u < 4; u++) v[u] = *(const float4_t *)(src + (s + u) * slice);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) sum[e] += v[u][e];
     }
+    float4_t v[3];
+#pragma unroll
+    for (int u = 0; u < 3; u++)
+        if (s + u < splits) v[u] = *(const float4_t *)(src + (s + u) * slice);
+#pragma unroll
+    for (int u = 0; u < 3; u++)
+        if (s + u < splits)
+#pragma unroll
+            for (int e = 0; e < 4; e++) sum[e] += v[u][e];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         float v = alpha * sum[e];

@@ -57,10 +57,6 @@ namespace miw {
 #define MIW_PP_MIDDLE(pr)
 #endif
 
-// The lambdas of a kernel are called from many places: left to itself the compiler makes functions of them, and what
-// they capture goes to memory.
-#define MIW_INLINE __attribute__((always_inline))
-
 constexpr int PP_KMAJOR_SLOTS = 3;
 constexpr int PP_IMAJOR_ENTRIES = 4;
 constexpr int PP_FOLD_STEPS = 32;  // k-steps of 32 over which k_gemm_pp_fold adds C: one MFMA tile of the wavefront's 8 x 4 each
@@ -184,8 +180,6 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
     const int wi = wave % WI, wj = wave / WI;
     const bool late_group = wave >= 4;
 
-    // Workgroup -> tile, as in k_gemm_tiled; the last tile of a row or column is shifted back so that it
-    // ends at the edge (see tiled_params).
     // What only the start of a tile needs is read from the arguments again there: held through the K loop it
     // would take more scalar registers than there are.
     auto arguments = [] MIW_INLINE {
@@ -193,28 +187,13 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
         asm volatile("" : "+s"(a));
         return a;
     };
-    // (the divisions run on the VALU: their outcome goes back to scalar registers)
-    auto locate = [](auto a, int tile, int &bt, int &i0, int &j0) MIW_INLINE {
-        const int total = a->tiles_i * a->tiles_j;
-        if (a->work > total) bt = __builtin_amdgcn_readfirstlane(tile / total);
-        const int pid = a->work > total ? tile - bt * total : tile;
-        const int per = total >> 3, rem = total & 7;
-        const int xcd = pid & 7, loc = pid >> 3;
-        const int tile_id = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
-        const int gsz = a->group_i * a->tiles_j;
-        const int gid = tile_id / gsz;
-        const int first = gid * a->group_i;
-        const int gi = min(a->tiles_i - first, a->group_i);
-        const int in = tile_id - gid * gsz;
-        i0 = __builtin_amdgcn_readfirstlane(min((first + in % gi) * BI, a->I - BI));
-        j0 = __builtin_amdgcn_readfirstlane(min(in / gi * BJ, a->J - BJ));
-    };
     auto x_origin = [](auto a, int bt, int i0) MIW_INLINE { return a->X + (long)bt * a->sx + (XK ? (long)i0 * a->ldx : (long)i0); };
     auto y_origin = [](auto a, int bt, int j0) MIW_INLINE { return a->Y + (long)bt * a->sy + (YK ? (long)j0 * a->ldy : (long)j0); };
-    int tile = blockIdx.x, bt = blockIdx.y, i0, j0;
-    locate(arguments(), tile, bt, i0, j0);
-    const half_t *X = x_origin(arguments(), bt, i0);
-    const half_t *Y = y_origin(arguments(), bt, j0);
+    fetch_arguments(p);  // (what is read again later is then in the scalar cache)
+    int tile = blockIdx.x + blockIdx.y * (unsigned)p.span;
+    tile_place at = tile_at(*arguments(), tile, blockIdx.y, BI, BJ);
+    const half_t *X = x_origin(arguments(), at.bt, at.i0);
+    const half_t *Y = y_origin(arguments(), at.bt, at.j0);
     const unsigned xoff = xop::lane_offset(tid, (int)p.ldx);
     const unsigned yoff = yop::lane_offset(tid, (int)p.ldy);
 
@@ -518,14 +497,15 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
     auto first_args = arguments();
     has_next = tile + (int)gridDim.x < first_args->work;
     if (has_next) {
-        int bt_next = bt, i0_next, j0_next;
-        locate(first_args, tile + (int)gridDim.x, bt_next, i0_next, j0_next);
-        xjump = x_origin(first_args, bt_next, i0_next) - x_origin(first_args, bt, i0) - ((XN - 2) * xunit + xtail);
-        yjump = y_origin(first_args, bt_next, j0_next) - y_origin(first_args, bt, j0) - ((YN - 2) * yunit + ytail);
+        const tile_place next = tile_at(*first_args, tile + (int)gridDim.x, 0, BI, BJ);
+        xjump = x_origin(first_args, next.bt, next.i0) - x_origin(first_args, at.bt, at.i0) - ((XN - 2) * xunit + xtail);
+        yjump = y_origin(first_args, next.bt, next.j0) - y_origin(first_args, at.bt, at.j0) - ((YN - 2) * yunit + ytail);
     } else {
         xjump = yjump = 0;
     }
-    if constexpr (FOLD) cnext = (const char *)((const CT *)first_args->C + (long)bt * first_args->sc + (long)j0 * first_args->ldc + i0);
+    const int i0 = at.i0, j0 = at.j0;
+    const long bt = at.bt;
+    if constexpr (FOLD) cnext = (const char *)((const CT *)first_args->C + bt * first_args->sc + (long)j0 * first_args->ldc + i0);
     float zero = 0.f;
     asm volatile("" : "+s"(zero));  // (otherwise a zero vector is kept in registers through the tiles)
 #pragma unroll
@@ -590,7 +570,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
     asm volatile("" : "+v"(lane));  // (what is made of it is made here, not kept through the K loop)
     const bool odd = lane & 1;
     const float alpha = args->alpha, beta = args->beta;
-    DT *D = (DT *)args->D + (long)bt * args->sd + (long)(j0 + wj * WTJ) * ldd + (i0 + wi * WTI) + pair_place(lane, ldd);
+    DT *D = (DT *)args->D + bt * args->sd + (long)(j0 + wj * WTJ) * ldd + (i0 + wi * WTI) + pair_place(lane, ldd);
     auto store = [](DT *to, float4_t v) MIW_INLINE {
         if constexpr (__is_same(DT, float)) __builtin_nontemporal_store(v, (float4_t *)to);
         else *(half4_t *)to = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
@@ -598,9 +578,9 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
     // C_AT 0: no C, 1: laid out as D, 2: the other way round
     auto epilogue = [&]<int C_AT, bool STREAM>(std::integral_constant<int, C_AT>, std::bool_constant<STREAM>) MIW_INLINE {
         const CT *C = nullptr;
-        if constexpr (C_AT == 1) C = (const CT *)args->C + (long)bt * args->sc + (long)(j0 + wj * WTJ) * ldc + (i0 + wi * WTI) + pair_place(lane, ldc);
+        if constexpr (C_AT == 1) C = (const CT *)args->C + bt * args->sc + (long)(j0 + wj * WTJ) * ldc + (i0 + wi * WTI) + pair_place(lane, ldc);
         // (columns r - odd and the next, rows 16 odd + 4 q ..)
-        if constexpr (C_AT == 2) C = (const CT *)args->C + (long)bt * args->sc + (long)(i0 + wi * WTI + 16 * odd + 4 * (lane >> 4)) * ldc + (j0 + wj * WTJ + (lane & 14));
+        if constexpr (C_AT == 2) C = (const CT *)args->C + bt * args->sc + (long)(i0 + wi * WTI + 16 * odd + 4 * (lane >> 4)) * ldc + (j0 + wj * WTJ + (lane & 14));
 #pragma unroll
         for (int b = 0; b < TJ; b++)
 #pragma unroll
@@ -654,7 +634,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
 #endif
     if (!has_next) break;
     tile += (int)gridDim.x;
-    locate(arguments(), tile, bt, i0, j0);
+    at = tile_at(*arguments(), tile, 0, BI, BJ);
     }
 }
 
@@ -729,28 +709,10 @@ void k_gemm_pp64(tiled_params p)
     const int wi = wave % WI, wj = wave / WI;
     const bool late_group = wave >= 4;
 
-    // Workgroup -> tile, as in k_gemm_tiled.
-    int tile_id;
-    {
-        const int total = p.tiles_i * p.tiles_j;
-        const int pid = blockIdx.x;
-        const int per = total >> 3, rem = total & 7;
-        const int xcd = pid & 7, loc = pid >> 3;
-        tile_id = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
-    }
-    int ti0, tj0;
-    {
-        const int gsz = p.group_i * p.tiles_j;
-        const int gid = tile_id / gsz;
-        const int first = gid * p.group_i;
-        const int gi = min(p.tiles_i - first, p.group_i);
-        const int in = tile_id - gid * gsz;
-        ti0 = first + in % gi;
-        tj0 = in / gi;
-    }
-    const long bt = blockIdx.y;
-    // the last tile of a row or column is shifted back so that it ends at the edge (see tiled_params)
-    const int i0 = min(ti0 * BI, p.I - BI), j0 = min(tj0 * BJ, p.J - BJ);
+    fetch_arguments(p);
+    const tile_place at = workgroup_tile(p, BI, BJ);
+    const int i0 = at.i0, j0 = at.j0;
+    const long bt = at.bt;
 
     const half_t *X = p.X + bt * p.sx + (XK ? (long)i0 * p.ldx : (long)i0);
     const half_t *Y = p.Y + bt * p.sy + (YK ? (long)j0 * p.ldy : (long)j0);

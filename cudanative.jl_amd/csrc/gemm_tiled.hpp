@@ -52,6 +52,9 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int uint2_t __attribute__((ext_vector_type(2)));
 typedef unsigned int uint4_t __attribute__((ext_vector_type(4)));
 
+// The lambdas of a kernel are called from many places: left to itself the compiler makes functions of them, and what
+// they capture goes to memory.
+#define MIW_INLINE __attribute__((always_inline))
 #define MIW_LDS __attribute__((address_space(3)))
 #define MIW_GLOBAL __attribute__((address_space(1)))
 
@@ -66,24 +69,30 @@ constexpr int BKS = 32;    // k-values per pipeline step (one MFMA k-step)
 constexpr int KGRAN = 64;  // k-values per LDS slot and K granularity of the kernel
 
 struct tiled_params {
+    // What a workgroup needs before its first load comes first, in 96 bytes: the arguments are fetched from memory a
+    // cache line at a time.
     const half_t *X;
     const half_t *Y;
-    const void *C;
-    void *D;
-    // K: any multiple of 16 from 64 up.  The kernels walk K in slots of 64; when 64 does not divide K
-    // the last slot is shifted back to end at K, and the k-values it repeats from the slot before
-    // (the first 64 * ceil(K / 64) - K of it) are zeroed in the fragments of both operands.
-    int I, J, K;
-    long ldx, ldy, ldc, ldd;
-    long sx, sy, sc, sd;
-    int c_trans;  // C is stored with J contiguous (its layout differs from D's)
-    int use_c;
-    float alpha, beta;
     // tiles_i = ceil(I / BI), tiles_j = ceil(J / BJ).  Where the tile does not divide an extent the
     // last tile starts at I - BI (J - BJ) and overlaps its neighbour: both workgroups compute the
     // overlap from the same operands in the same order and store equal values.  The host allows
     // this only when C and D do not share memory.
     int tiles_i, tiles_j, group_i;
+    // What workgroup_tile divides by, as multipliers (see quotient); shifts: one byte for each.
+    int span;                                  // tiles of a batch member where the XCDs' runs go over the whole batch, else 0
+    int total;                                 // tiles the runs go over
+    unsigned span_m, group_m, rows_m, last_m, shifts;  // of span, group_i * tiles_j, group_i, rows of the last group
+    // K: any multiple of 16 from 64 up.  The kernels walk K in slots of 64; when 64 does not divide K
+    // the last slot is shifted back to end at K, and the k-values it repeats from the slot before
+    // (the first 64 * ceil(K / 64) - K of it) are zeroed in the fragments of both operands.
+    int I, J, K;
+    long ldx, ldy, sx, sy;
+    const void *C;
+    void *D;
+    long ldc, ldd, sc, sd;
+    int c_trans;  // C is stored with J contiguous (its layout differs from D's)
+    int use_c;
+    float alpha, beta;
     // Workgroups that walk several tiles (k_gemm_pp): number of tiles over the whole batch; a workgroup takes tile
     // blockIdx.x, then every gridDim.x-th.  0: one tile per workgroup.  Needs K of four slots or more.
     int work;
@@ -146,6 +155,50 @@ __device__ inline void lds_dma16_at(const void *base, unsigned voff, unsigned ld
 }
 
 __device__ inline int i_major_swizzle(int k) { return ((k >> 1) & 1) | (((k >> 3) & 1) << 1); }
+
+// n / d for 0 <= n < 2^31: with s = ceil(log2 d) and m = ceil(2^(31 + s) / d), which is below 2^32, m is at most
+// 2^(31 + s) / d + 1, and the excess of n * m over n / d * 2^(31 + s) stays below 2^(31 + s) / d.
+__device__ inline int quotient(int n, unsigned m, unsigned s) { return (int)(__umulhi(2u * (unsigned)n, m) >> s); }
+
+// Workgroup -> tile.  Consecutive workgroup ids (x first, then y) go round-robin over the 8 XCDs; each XCD gets a
+// contiguous run of tile ids, so that workgroups that share X row-panels and Y column-panels share one L2, and the
+// tile grid is walked in groups of group_i tile-rows.  With span the run is one of the tiles of all batch members in
+// turn: an XCD that takes an eighth of every member reads an eighth of the panels of each, in place of one member's
+// (512x512x16384 in sixteen slices of K: 26.4 us with a run per slice, 19.1 with one over all of them; 128 problems of
+// 192x208x144 18.8 and 13.1).  The divisions are multiplications by what the host prepared: on the VALU they were a fifth
+// of the 143 instructions in front of the first load.
+// The last tile of a row or column is shifted back so that it ends at the edge (see tiled_params).
+struct tile_place {
+    int bt, i0, j0;
+};
+template <class PARAMS>
+__device__ inline tile_place tile_at(const PARAMS &p, int id, int batch_member, int bi, int bj)
+{
+    const int per = p.total >> 3, rem = p.total & 7;
+    const int xcd = id & 7, loc = id >> 3;
+    id = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
+    const int gsz = p.group_i * p.tiles_j;
+    const int member = quotient(id, p.span_m, p.shifts & 31);
+    id -= member * p.span;
+    const int gid = quotient(id, p.group_m, (p.shifts >> 8) & 31), first = gid * p.group_i, in = id - gid * gsz;
+    const bool whole = p.tiles_i - first >= p.group_i;
+    const int column = quotient(in, whole ? p.rows_m : p.last_m, ((whole ? p.shifts >> 16 : p.shifts >> 24)) & 31);
+    const int row = first + in - column * (whole ? p.group_i : p.tiles_i - first);
+    return {p.span ? member : batch_member, min(row * bi, p.I - bi), min(column * bj, p.J - bj)};
+}
+__device__ inline tile_place workgroup_tile(const tiled_params &p, int bi, int bj)
+{
+    return tile_at(p, (int)(blockIdx.x + blockIdx.y * (unsigned)p.span), (int)blockIdx.y, bi, bj);
+}
+
+// All arguments into scalar registers at the start of the kernel.  Left to itself the compiler puts the loads of some off
+// to where they are first used, behind the K loop or right in front of the first operand load, where each waits for
+// memory (0.15 us of a launch).
+__device__ inline void fetch_arguments(const tiled_params &p)
+{
+    asm volatile("" ::"s"(p.X), "s"(p.Y), "s"(p.I), "s"(p.J), "s"(p.K), "s"(p.ldx), "s"(p.ldy), "s"(p.sx), "s"(p.sy), "s"(p.C), "s"(p.D),
+                 "s"(p.ldc), "s"(p.ldd), "s"(p.sc), "s"(p.sd), "s"(p.c_trans), "s"(p.use_c), "s"(p.alpha), "s"(p.beta));
+}
 
 // ------------------------------------------------------------ slot loader --
 // Fetches one slot (R rows/columns x 64 k-values) with NT threads.  Thread t
@@ -323,7 +376,9 @@ __device__ inline long pair_place(int lane, long ldd)
 template <class DT>
 __device__ inline void store_tile_pair(DT *D, long ldd, int row, int col0, int lane, float4_t v0, float4_t v1)
 {
-    store_pair_at(D + (long)col0 * ldd + row + pair_place(lane, ldd), ldd, lane & 1, v0, v1);
+    const int r = lane & 15, q = lane >> 4;
+    const bool odd = r & 1;
+    store_pair_at(D + (long)(col0 + r - (odd ? 1 : 0)) * ldd + (row + (odd ? 16 : 0) + 4 * q), ldd, odd, v0, v1);
 }
 
 // Ordinal of the direct-to-LDS load issued after MFMA m of a step of nmfma
@@ -396,31 +451,10 @@ void k_gemm_tiled(tiled_params p)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wi = wave % WI, wj = wave / WI;
 
-    // Workgroup -> tile.  Consecutive workgroup ids go round-robin over the 8
-    // XCDs; give each XCD a contiguous run of tile ids so that workgroups that
-    // share X row-panels and Y column-panels share one L2, then walk the tile
-    // grid in groups of group_i tile-rows.
-    int tile_id;
-    {
-        const int total = p.tiles_i * p.tiles_j;
-        const int pid = blockIdx.x;
-        const int per = total >> 3, rem = total & 7;
-        const int xcd = pid & 7, loc = pid >> 3;
-        tile_id = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
-    }
-    int ti0, tj0;
-    {
-        const int gsz = p.group_i * p.tiles_j;
-        const int gid = tile_id / gsz;
-        const int first = gid * p.group_i;
-        const int gi = min(p.tiles_i - first, p.group_i);
-        const int in = tile_id - gid * gsz;
-        ti0 = first + in % gi;
-        tj0 = in / gi;
-    }
-    const long bt = blockIdx.y;
-    // the last tile of a row or column is shifted back so that it ends at the edge (see tiled_params)
-    const int i0 = min(ti0 * BI, p.I - BI), j0 = min(tj0 * BJ, p.J - BJ);
+    fetch_arguments(p);
+    const tile_place at = workgroup_tile(p, BI, BJ);
+    const int i0 = at.i0, j0 = at.j0;
+    const long bt = at.bt;
 
     const half_t *X = p.X + bt * p.sx + (XK ? (long)i0 * p.ldx : (long)i0);
     const half_t *Y = p.Y + bt * p.sy + (YK ? (long)j0 * p.ldy : (long)j0);

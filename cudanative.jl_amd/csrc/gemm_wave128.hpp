@@ -109,27 +109,10 @@ void k_gemm_w128(tiled_params p)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wi = wave % WI, wj = wave / WI;
 
-    // Workgroup -> tile, as in k_gemm_tiled.
-    int tile_id;
-    {
-        const int total = p.tiles_i * p.tiles_j;
-        const int pid = blockIdx.x;
-        const int per = total >> 3, rem = total & 7;
-        const int xcd = pid & 7, loc = pid >> 3;
-        tile_id = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
-    }
-    int ti0, tj0;
-    {
-        const int gsz = p.group_i * p.tiles_j;
-        const int gid = tile_id / gsz;
-        const int first = gid * p.group_i;
-        const int gi = min(p.tiles_i - first, p.group_i);
-        const int in = tile_id - gid * gsz;
-        ti0 = first + in % gi;
-        tj0 = in / gi;
-    }
-    const long bt = blockIdx.y;
-    const int i0 = min(ti0 * BI, p.I - BI), j0 = min(tj0 * BJ, p.J - BJ);
+    fetch_arguments(p);
+    const tile_place at = workgroup_tile(p, BI, BJ);
+    const int i0 = at.i0, j0 = at.j0;
+    const long bt = at.bt;
 
     const half_t *X = p.X + bt * p.sx + (XK ? (long)i0 * p.ldx : (long)i0);
     const half_t *Y = p.Y + bt * p.sy + (YK ? (long)j0 * p.ldy : (long)j0);

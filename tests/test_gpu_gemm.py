@@ -782,6 +782,14 @@ def test_narrow_problems_through_every_route(gpu, orc, narrow_kernel, cl, dl):
             _check_block(orc, g, _run(gpu, orc, g, A, B, C if g.use_c else None, variant=variant, prefill=7.0), want, (M, N, K, pad, variant))
 
 
+def test_tiles_of_a_batch_in_one_run(gpu, orc):
+    """Several tiles per batch member: the XCDs' runs go over the whole batch; counts that 8 does not divide, partial raster groups."""
+    for v, (M, N, batch) in itertools.product(("tile64x64_w2x2", "tile128x128_w2x2", "tile128x128_pingpong"), ((192, 320, 5), (400, 208, 3), (144, 1040, 2))):
+        g = orc.GemmDesc(M=M, N=N, K=80, batch=batch)
+        A, B, C = _inputs(orc, g, M + batch, ints=True)
+        assert np.array_equal(_run(gpu, orc, g, A, B, C, variant=_vid(gpu, v)), orc.gemm(g, A, B, C)), (v, M, N, batch)
+
+
 def test_tiled_with_padded_leading_dimensions_and_batch(gpu, orc):
     g = orc.GemmDesc(M=128, N=128, K=192, lda=136, ldb=200, ldc=132, ldd=144, batch=5, a_layout=orc.COL, b_layout=orc.COL)
     A, B, C = _inputs(orc, g, 41)
