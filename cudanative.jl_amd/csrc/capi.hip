@@ -292,6 +292,12 @@ const std::vector<int> &variant_order()
 // and the fragment-op kernels.  Both take every problem (a problem the first cannot run goes to the others).
 int narrow_id() { return miw::tiled_variant_count() + 1; }
 int fragops_id() { return miw::tiled_variant_count() + 2; }
+// The smallest tile's.
+int small_id()
+{
+    static const int id = variant_order().back() + 1;
+    return id;
+}
 
 // 1-based id of the LDS-tiled variant for this problem and its estimated duration, 0 when none fits.
 int pick_tiled(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place, double *us_out = nullptr)
@@ -310,12 +316,25 @@ int pick_tiled(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, i
     return best + 1;
 }
 
-int pick_variant(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place)
+// *kw: the tile of k_gemm_kwave where that runs in the picked variant's place.  It has no id of its own: tile64x64_w2x2
+// stands for it, below 64 rows or columns fragment_ops, and narrow_k_contiguous where that was picked.
+int pick_variant(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place, miw::kwave_tile *kw_out = nullptr)
 {
-    if (const int v = pick_tiled(p, c_type, d_type, f16acc, acc_chunk, in_place))
-        return miw::skinny_beats_tiles(p, d_type, f16acc) ? narrow_id() : v;
-    // Thinner than every tile: the fragment-op kernels, which hand the problem on where that pays.
-    return std::min(p.M, p.N) >= 64 && miw::skinny_pays(p, d_type, f16acc) ? narrow_id() : fragops_id();
+    // (a batch keeps the bits that each of its members has under the picked id)
+    miw::kwave_tile kw = f16acc || p.batch > 1 ? miw::kwave_tile{0, 0} : miw::kwave_pays(p, c_type, d_type, in_place, cu_count());
+    int v = pick_tiled(p, c_type, d_type, f16acc, acc_chunk, in_place);
+    if (v) {
+        if (miw::skinny_beats_tiles(p, d_type, f16acc)) v = narrow_id();
+        else if (kw.bi) v = small_id();
+    } else if (std::min(p.M, p.N) < 64) {
+        // Thinner than every tile: the fragment-op kernels, which hand the problem on where that pays.
+        v = fragops_id();
+    } else {
+        v = miw::skinny_pays(p, d_type, f16acc) ? narrow_id() : fragops_id();
+        kw = {0, 0};
+    }
+    if (kw_out) *kw_out = kw;
+    return v;
 }
 
 // Resolve the variant (0 = pick) and check that it can run this problem; touches no device.
@@ -343,8 +362,13 @@ int check_gemm(const miw_gemm_desc *d, const miw::gemm_params &p, bool f16acc, b
     return 0;
 }
 
-int launch_gemm(int variant, const miw::gemm_params &p, int c_type, int d_type, bool f16acc, hipStream_t s)
+// kw: the tile of k_gemm_kwave, which runs in the variant's place unless that is forced (0: it does not).
+int launch_gemm(int variant, miw::kwave_tile kw, const miw::gemm_params &p, int c_type, int d_type, bool f16acc, hipStream_t s)
 {
+    if (kw.bi) {
+        HIP_TRY(miw::launch_gemm_kwave(kw, p, c_type, d_type, s));
+        return 0;
+    }
     if (variant == narrow_id() && miw::skinny_fits(p, d_type, f16acc)) HIP_TRY(miw::launch_gemm_skinny(p, c_type, d_type, s));
     else if (variant >= narrow_id()) HIP_TRY(miw::launch_gemm_fragops(p, c_type, d_type, f16acc, s));
     else HIP_TRY(miw::launch_gemm_tiled(variant - 1, p, c_type, d_type, f16acc, cu_count(), s));
@@ -366,6 +390,7 @@ struct gemm_part {
     int c_type;
     miw::gemm_params p;
     long m0, n0, k0;  // where the part sits in the caller's problem
+    miw::kwave_tile kw;
 };
 
 // The kernels behind the fragment-op id, in the order launch_gemm_fragops asks.  Up to 64 k-values with C
@@ -402,8 +427,10 @@ struct gemm_planner {
 
     double single(const miw::gemm_params &p, int c_type, long m0, long n0, long k0, std::vector<gemm_part> *out) const
     {
-        const int v = pick_variant(p, c_type, d_type, false, 0, in_place);
-        if (out) out->push_back(gemm_part{v, c_type, p, m0, n0, k0});
+        miw::kwave_tile kw;
+        const int v = pick_variant(p, c_type, d_type, false, 0, in_place, &kw);
+        if (out) out->push_back(gemm_part{v, c_type, p, m0, n0, k0, kw});
+        if (kw.bi) return miw::kwave_estimate_us(p, c_type, d_type, kw);
         if (v == fragops_id()) return estimate_fragops_us(p, c_type, d_type);
         if (v != narrow_id()) return estimate_us(v - 1, p, c_type, d_type);
         // (the tiles' paces are those of operands that start on whole cache lines; the cuts are weighed as if these did)
@@ -433,7 +460,7 @@ struct gemm_planner {
                     if (!tiled_fits(i, body, c_type, d_type, false, 0, in_place)) continue;
                     if (v.kind == miw::KIND_WAVE128 && !wave128_pays(i, body)) continue;
                     std::vector<gemm_part> cand;
-                    cand.push_back(gemm_part{i + 1, c_type, body, m0, n0, k0});
+                    cand.push_back(gemm_part{i + 1, c_type, body, m0, n0, k0, {0, 0}});
                     double us = estimate_us(i, body, c_type, d_type);
                     if (us >= best_us) continue;
                     const long sm = in_place || p.M < 64 ? mb : std::min(mb, p.M - 64);
@@ -479,7 +506,7 @@ int plan_gemm(const miw_gemm_desc *d, const miw::gemm_params &p, bool f16acc, bo
     if (d->variant != 0 || f16acc) {
         int variant = 0;
         if (int rc = check_gemm(d, p, f16acc, in_place, &variant)) return rc;
-        parts->push_back(gemm_part{variant, d->c_type, p, 0, 0, 0});
+        parts->push_back(gemm_part{variant, d->c_type, p, 0, 0, 0, {0, 0}});
     } else {
         gemm_planner pl{d->d_type, in_place};
         pl.plan(p, d->c_type, 0, 0, 0, 0, parts);
@@ -507,7 +534,7 @@ bool c_shares_d(const miw_gemm_desc *d, const miw::gemm_params &p)
 int launch_parts(const miw_gemm_desc *d, const std::vector<gemm_part> &parts, bool f16acc, hipStream_t s)
 {
     for (const gemm_part &part : parts)
-        if (int rc = launch_gemm(part.variant, part.p, part.c_type, d->d_type, f16acc, s)) return rc;
+        if (int rc = launch_gemm(part.variant, part.kw, part.p, part.c_type, d->d_type, f16acc, s)) return rc;
     return 0;
 }
 
@@ -944,6 +971,7 @@ struct splitk_plan {
     miw::gemm_params slice;  // first pass: `splits` independent products of K / splits k-values each
     int variant;             // tiled variant of the first pass (1-based)
     int splits;
+    miw::kwave_tile kw;      // what runs in its place, see pick_variant
     size_t bytes;            // workspace the first pass fills
 };
 
@@ -977,25 +1005,32 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     const bool in_place = c_shares_d(d, p);
     static char dummy alignas(128);
     // Variant and estimated duration of s slices (s = 1: the plain launch); false when no tiled kernel fits.
-    auto try_splits = [&](int s, int *variant, double *us) {
+    auto try_splits = [&](int s, int *variant, miw::kwave_tile *kw, double *us) {
         if (p.K % (64l * s)) return false;
         if (s == 1) {
             if (!pick_tiled(p, d->c_type, d->d_type, false, 0, in_place, us)) return false;
-            *variant = pick_variant(p, d->c_type, d->d_type, false, 0, in_place);
+            *variant = pick_variant(p, d->c_type, d->d_type, false, 0, in_place, kw);
+            // (only where C in D's place runs the same: the workspace's size is asked for without the pointers)
+            if (kw->bi && p.M % 64 == 0 && p.N % 64 == 0) *us = miw::kwave_estimate_us(p, d->c_type, d->d_type, *kw);
             return true;
         }
         const miw::gemm_params q = splitk_slices(p, s, &dummy);
-        const int v = pick_tiled(q, MIW_F32, MIW_F32, false, 0, false);
+        const int v = pick_tiled(q, MIW_F32, MIW_F32, false, 0, false, us);
         if (v == 0) return false;
         *variant = v;
-        // second kernel: launch, a quarter of a microsecond per slice (each thread adds its slices
-        // in order), and the slices, C and D at the same pace as above
+        *kw = miw::kwave_pays(q, MIW_F32, MIW_F32, false, cu_count());
+        const double kw_us = kw->bi ? miw::kwave_estimate_us(q, MIW_F32, MIW_F32, *kw) : 0.0;
+        if (kw->bi && kw_us < *us) *us = kw_us;
+        else *kw = {0, 0};
+        // second kernel: launch, the additions (each thread's slices in order), and the slices, C and D at
+        // the same pace as above
         const double mn = (double)p.M * (double)p.N;
-        *us = estimate_us(v - 1, q, MIW_F32, MIW_F32) + 6.0 + 0.25 * s +
+        *us += 2.5 + 0.03 * s +
               mn * (4.0 * s + (double)dtype_size(d->d_type) + (p.use_c ? (double)dtype_size(d->c_type) : 0.0)) / 5.5e6;
         return true;
     };
     int variant = 0;
+    miw::kwave_tile kw = {0, 0};
     double us = 0.0;
     if (splits == 0) {
         // The slice count with the shortest estimated duration, among 1 (no second pass) and the
@@ -1003,12 +1038,13 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
         double best_us = 0.0;
         for (int s = 1; s <= 64 && (s == 1 || p.K / s >= 128); s++) {
             int v;
+            miw::kwave_tile t;
             // a caller with a bounded workspace is offered only the counts that fit in it
             if (s > 1 && (size_t)s * (size_t)p.M * (size_t)p.N * sizeof(float) > workspace_cap) break;
-            if (!try_splits(s, &v, &us)) continue;
-            if (splits == 0 || us < 0.97 * best_us) { splits = s; variant = v; best_us = us; }
+            if (!try_splits(s, &v, &t, &us)) continue;
+            if (splits == 0 || us < 0.97 * best_us) { splits = s; variant = v; kw = t; best_us = us; }
         }
-    } else if (!try_splits(splits, &variant, &us)) {
+    } else if (!try_splits(splits, &variant, &kw, &us)) {
         splits = 0;
     }
     if (splits == 0)
@@ -1018,6 +1054,7 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     out->full = p;
     out->splits = splits;
     out->variant = variant;
+    out->kw = kw;
     // one slice is the plain launch: no workspace, no second kernel
     out->bytes = splits == 1 ? 0 : (size_t)splits * (size_t)p.M * (size_t)p.N * sizeof(float);
     out->slice = splitk_slices(p, splits, nullptr);
@@ -1027,15 +1064,15 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
 int run_splitk(const miw_gemm_desc *d, splitk_plan &plan, void *ws, hipStream_t s)
 {
     if (plan.splits == 1) {
-        if (plan.variant != narrow_id() && !tiled_fits(plan.variant - 1, plan.full, d->c_type, d->d_type, false, 0, c_shares_d(d, plan.full)))
+        if (plan.variant < narrow_id() && !tiled_fits(plan.variant - 1, plan.full, d->c_type, d->d_type, false, 0, c_shares_d(d, plan.full)))
             return fail(MIW_ERR_MISALIGNED, "gemm_splitk: operands must be 16-byte aligned");
-        return launch_gemm(plan.variant, plan.full, d->c_type, d->d_type, false, s);
+        return launch_gemm(plan.variant, plan.kw, plan.full, d->c_type, d->d_type, false, s);
     }
     plan.slice.D = ws;
     // the slices are checked against the real operand pointers (plan_splitk assumed aligned ones)
     if (!tiled_fits(plan.variant - 1, plan.slice, MIW_F32, MIW_F32, false, 0, false))
         return fail(MIW_ERR_MISALIGNED, "gemm_splitk: operands and workspace must be 16-byte aligned");
-    HIP_TRY(miw::launch_gemm_tiled(plan.variant - 1, plan.slice, MIW_F32, MIW_F32, false, cu_count(), s));
+    if (int rc = launch_gemm(plan.variant, plan.kw, plan.slice, MIW_F32, MIW_F32, false, s)) return rc;
     HIP_TRY(miw::launch_splitk_reduce(plan.full, d->c_type, d->d_type, plan.splits, (const float *)ws, s));
     return 0;
 }

@@ -53,7 +53,8 @@ bool pp_folds(const tiled_params &p, int c_type);
 int pp_lds(int bm, int bn, bool xk, bool yk);
 const void *w128_kernel(bool xk, bool yk, int c_type, int d_type);
 const void *pp64_kernel(int bm, int bn, bool xk, bool yk, int c_type, int d_type, bool f16acc);
-
+const void *kwave_kernel(int bi, int bj, bool xk, bool yk, int *lds_bytes);
+hipError_t launch_kwave(const void *fn, const tiled_params &t, int c_type, int d_type, dim3 grid, int lds_bytes, hipStream_t s);
 
 
 // Tile shape in canonical (I, J) terms: bm applies to I, bn to J.
@@ -176,6 +177,18 @@ static tiled_params canonical(const gemm_params &g, int bi, int bj, bool *xk, bo
     p.ts = nullptr;
 #endif
     return p;
+}
+
+hipError_t launch_gemm_kwave(kwave_tile t, const gemm_params &g, int c_type, int d_type, hipStream_t s)
+{
+    bool xk, yk;
+    const tiled_params p = canonical(g, t.bi, t.bj, &xk, &yk);
+    int lds_bytes;
+    const void *fn = kwave_kernel(t.bi, t.bj, xk, yk, &lds_bytes);
+    if (!fn || p.I < t.bi || p.J < t.bj || p.K < KGRAN) return hipErrorInvalidValue;
+    hipError_t e = allow_dynamic_lds(fn, lds_bytes);
+    if (e != hipSuccess) return e;
+    return launch_kwave(fn, p, c_type, d_type, dim3((unsigned)(p.tiles_i * p.tiles_j), (unsigned)g.batch), lds_bytes, s);
 }
 
 hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type, bool f16acc, int cus, hipStream_t s)

@@ -50,6 +50,14 @@ inline bool fragops_run_skinny(const gemm_params &p, int d_type, bool f16acc)
 {
     return (p.M < 64 || p.N < 64) && skinny_pays(p, d_type, f16acc);
 }
+// --- gemm_kwave.hip: tiles of at most 64 x 32 in one round over the CUs, K shared by a workgroup's wavefronts.
+struct kwave_tile {
+    int bi, bj;  // along D's contiguous dimension and the other; 0: the kernel does not run the problem, or not faster
+};
+// The tile with which the kernel is the fastest one for the problem.  in_place: C and D share memory.
+kwave_tile kwave_pays(const gemm_params &p, int c_type, int d_type, bool in_place, int cus);
+double kwave_estimate_us(const gemm_params &p, int c_type, int d_type, kwave_tile t);
+hipError_t launch_gemm_kwave(kwave_tile t, const gemm_params &p, int c_type, int d_type, hipStream_t s);
 hipError_t launch_dummy_store(float *ptr, int threads, hipStream_t s);
 const void *frag_kernel_symbol(const char *name);
 int frag_kernel_count();

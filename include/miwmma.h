@@ -221,7 +221,12 @@ int miw_gemm_variant_supports(const miw_gemm_desc *desc, int variant, int *suppo
 /* Variant of a single launch of this descriptor (what miw_gemm runs unless miw_gemm_plan
    cuts the problem up): the one with the shortest estimated duration
    (rounds of workgroups over the CUs, C and D traffic, and the K loop at each kernel's measured
-   pace per 64 k-values) among those that can run it. */
+   pace per 64 k-values) among those that can run it.  With batch 1, Float32 accumulation and
+   desc.variant 0, a problem that tiles of at most 64 x 32 cover in one round over the CUs may run
+   on a kernel without an id, whose wavefronts share K: tile64x64_w2x2's stands for it, where the
+   pitches are no whole cache lines narrow_k_contiguous', and fragment_ops' below 64 rows or
+   columns.  An id asked for in desc.variant runs its own kernel, which differs from that one by
+   the order of the Float32 additions. */
 int miw_gemm_pick_variant(const miw_gemm_desc *desc, int *variant);
 /* The launches miw_gemm makes for this descriptor (no counterpart in the reference, whose GEMM
    would be the caller's own kernel over docs/src/device/wmma.md:51-52).  The LDS-tiled kernels take any M and N of

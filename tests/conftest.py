@@ -96,3 +96,28 @@ def narrow_kernel(miw):
         return f(ctypes.byref(p), d_type, f16acc)
 
     return ask
+
+
+class _KwaveTile(ctypes.Structure):
+    _fields_ = [("bi", ctypes.c_int), ("bj", ctypes.c_int)]
+
+
+@pytest.fixture()
+def shared_k_tile(miw):
+    """shared_k_tile(M, N, K, ...): the tile (along D's contiguous dimension, along the other) with which the library's
+    own rule takes the kernel whose wavefronts share K, or None."""
+    lib = ctypes.CDLL(miw._lib.LIB_PATH)
+    f = lib._ZN3miw10kwave_paysERKNS_11gemm_paramsEiibi
+    f.restype, f.argtypes = _KwaveTile, [ctypes.POINTER(_GemmParams), ctypes.c_int, ctypes.c_int, ctypes.c_bool, ctypes.c_int]
+
+    def ask(M, N, K, batch=1, a_row=1, b_row=0, c_row=1, d_row=1, use_c=0, c_type=1, d_type=0, in_place=False, lda=0, ldb=0, ldd=0, offset=0, cus=256):
+        lda, ldb = lda or (K if a_row else M), ldb or (N if b_row else K)
+        ldc, ldd = N if c_row else M, ldd or (N if d_row else M)
+        base = 1 << 32
+        p = _GemmParams(base + offset, base + (1 << 40), base + (2 << 40), base + (3 << 40), M, N, K, lda, ldb, ldc, ldd,
+                        lda * (M if a_row else K), ldb * (K if b_row else N), ldc * (M if c_row else N), ldd * (M if d_row else N),
+                        batch, a_row, b_row, c_row, d_row, use_c, 1.0, 1.0)
+        t = f(ctypes.byref(p), c_type, d_type, in_place, cus)
+        return (t.bi, t.bj) if t.bi else None
+
+    return ask

@@ -782,6 +782,30 @@ def test_narrow_problems_through_every_route(gpu, orc, narrow_kernel, cl, dl):
             _check_block(orc, g, _run(gpu, orc, g, A, B, C if g.use_c else None, variant=variant, prefill=7.0), want, (M, N, K, pad, variant))
 
 
+@pytest.mark.parametrize("tile,al,bl,M,N,Ks", [
+    ((32, 16), 0, 1, 144, 176, (128, 144, 336, 1104, 2064)), ((16, 32), 0, 1, 16, 48, (1024, 1600)), ((32, 32), 0, 1, 512, 304, (128, 400)),
+    ((64, 32), 0, 1, 1008, 512, (512, 528)), ((32, 32), 1, 1, 80, 112, (128, 144, 336, 1104)), ((32, 32), 0, 0, 80, 112, (128, 144, 336, 1104)),
+    ((32, 32), 1, 0, 80, 112, (128, 144, 336, 1104)), ((64, 32), 1, 1, 1008, 512, (768, 784)), ((32, 64), 0, 0, 512, 1008, (768, 784)),
+    ((64, 32), 1, 0, 1008, 512, (768, 784, 1360))])
+@pytest.mark.parametrize("dl", (0, 1))
+def test_kernel_whose_wavefronts_share_k(gpu, orc, shared_k_tile, tile, al, bl, M, N, Ks, dl):
+    """Every tile and operand layout, shifted edge tiles, whole and ragged K around the wavefronts' turns and rings, every
+    form of C; exact on integers.  (al, bl, M, N as for a column-major D; a row-major D swaps the operands' roles.)"""
+    if not dl:
+        M, N, al, bl = N, M, 1 - bl, 1 - al
+    forms = [dict(c_type=orc.F32, beta=-2.0), dict(c_type=orc.F16, d_type=orc.F32, alpha=0.5), dict(use_c=0), dict(c_type=orc.F32, other=True)]
+    for i, K in enumerate(Ks):
+        form = dict(forms[(i + tile[0] + al) % 4])
+        cl = 1 - dl if form.pop("other", False) else dl
+        g = orc.GemmDesc(M=M, N=N, K=K, a_layout=al, b_layout=bl, c_layout=cl, d_layout=dl, **form)
+        got = shared_k_tile(M, N, K, a_row=int(al == orc.ROW), b_row=int(bl == orc.ROW), c_row=int(cl == orc.ROW), d_row=int(dl == orc.ROW),
+                            use_c=g.use_c, c_type=int(g.c_type == orc.F32), d_type=1)
+        assert got == tile, (got, M, N, K, al, bl, dl)
+        A, B, C = _inputs(orc, g, 900 + K, ints=True)
+        D = _run(gpu, orc, g, A, B, C if g.use_c else None)
+        assert np.array_equal(D, orc.gemm(g, A, B, C)), (tile, al, bl, dl, K, form)
+
+
 def test_tiles_of_a_batch_in_one_run(gpu, orc):
     """Several tiles per batch member: the XCDs' runs go over the whole batch; counts that 8 does not divide, partial raster groups."""
     for v, (M, N, batch) in itertools.product(("tile64x64_w2x2", "tile128x128_w2x2", "tile128x128_pingpong"), ((192, 320, 5), (400, 208, 3), (144, 1040, 2))):

@@ -330,6 +330,36 @@ def test_narrow_kernel_runs_where_it_was_measured_ahead(narrow_kernel):
     assert not narrow_kernel("pays", 144, 4096, 4096) and not narrow_kernel("pays", 16, 4096, 48)
 
 
+def test_shared_k_kernel_runs_where_it_was_measured_ahead(miw, shared_k_tile):
+    """Both sides of every line of the rule that takes the kernel with small tiles in one round over the CUs."""
+    for want, M, N, K, kw in (
+            # k contiguous in both operands: the smallest tile whose count the CUs hold; K of two slots
+            ((32, 16), 64, 64, 128, {}), (None, 64, 64, 112, {}), ((32, 16), 512, 256, 128, {}), ((32, 32), 512, 272, 128, {}),
+            ((32, 32), 512, 512, 128, {}), ((64, 32), 512, 528, 512, {}), (None, 512, 528, 496, {}), ((64, 32), 512, 1024, 512, {}), (None, 528, 1024, 512, {}),
+            # one operand or none: no 16-wide tiles, the 64-wide ones from K = 768 on
+            ((32, 32), 64, 64, 128, dict(a_row=0)), ((32, 32), 64, 64, 128, dict(a_row=0, b_row=1)), ((32, 64), 512, 1024, 768, dict(a_row=0)),
+            (None, 512, 1024, 752, dict(a_row=0)), ((64, 32), 512, 1024, 768, dict(b_row=1)), ((64, 32), 512, 1024, 768, dict(a_row=0, b_row=1)),
+            # thinner than every other tile
+            ((32, 16), 16, 4096, 1024, {}), (None, 16, 4096, 1008, {}), ((32, 16), 16, 4112, 128, {}), (None, 16, 8208, 4096, {}),
+            ((32, 16), 32, 4096, 512, {}), (None, 32, 4096, 496, {}), ((32, 32), 48, 4096, 512, {}), (None, 16, 4096, 2064, {}), (None, 48, 4096, 4160, dict(lda=4168)),
+            (None, 16, 4096, 4096, dict(a_row=0)), ((32, 32), 32, 2048, 512, dict(b_row=1)), (None, 32, 2032, 512, dict(b_row=1)), ((32, 32), 32, 2032, 1024, dict(b_row=1)),
+            # rows off whole cache lines, where the narrow kernel beats the 64x64 tile
+            ((32, 32), 64, 4096, 784, {}), (None, 64, 4096, 752, {}), (None, 64, 8192, 784, {}),
+            # C in D's place: whole tiles
+            ((32, 16), 80, 96, 128, dict(in_place=True)), (None, 80, 80, 128, dict(in_place=True, a_row=0)), ((32, 16), 80, 80, 128, {}),
+            # alignment
+            (None, 64, 64, 128, dict(offset=8)), (None, 64, 64, 128, dict(lda=132)), (None, 64, 64, 128, dict(ldd=68)), ((32, 16), 64, 64, 128, dict(ldd=68, d_type=1)),
+            # slices of K, and fewer CUs
+            ((32, 32), 128, 128, 1024, dict(a_row=0, b_row=1, batch=16)), (None, 128, 128, 1024, dict(a_row=0, b_row=1, batch=33)), ((32, 32), 512, 256, 128, dict(cus=128))):
+        assert shared_k_tile(M, N, K, **kw) == want, (M, N, K, kw)
+    # it has no id: the smallest tile's stands for it, the fragment-op one below 64 rows or columns, and a batch never takes it
+    G, W = miw.GEMM, miw.WMMA
+    rc = dict(a_layout=W.RowMajor, b_layout=W.ColMajor, d_layout=W.RowMajor, d_type=np.float16, use_c=False)
+    by = {v["name"]: v["id"] for v in G.variants()}
+    assert G.pick_variant(G.make_desc(128, 4096, 4096, **rc)) == by["tile64x64_w2x2"]
+    assert G.pick_variant(G.make_desc(48, 4096, 4096, **rc)) == by["fragment_ops"]
+
+
 def test_variant_table_and_selection(miw):
     G = miw.GEMM
     vs = G.variants()

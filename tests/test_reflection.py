@@ -66,6 +66,19 @@ def test_auto_picked_4096_kernels_have_no_spills(miw):
             assert r["spills"] == 0 and r["scratch"] == 0, k
 
 
+def test_shared_k_kernels_stay_in_registers(miw):
+    """No scratch in any instance; the rings are counted in vmcnt, so nothing but the C ahead of them and the loads to LDS
+    may read global memory before the last wait."""
+    res = {k: v for k, v in miw.reflection.kernel_resources().items() if "k_gemm_kwave<" in k}
+    assert len(res) == 10
+    for k, r in res.items():
+        assert r["spills"] == 0 and r["scratch"] == 0 and r["max_threads"] == 256, k
+    for k, text in miw.reflection.code_gcn("k_gemm_kwave<").items():
+        ops = _ops(text)
+        assert ops["v_mfma_f32_16x16x32_f16"] > 0 and ops["global_load_lds_dwordx4"] > 0, k
+        assert not any(o.startswith(("scratch_", "flat_", "v_accvgpr")) for o in ops), k
+
+
 def test_narrow_kernel_codegen_and_resources(miw):
     """Every instance of the narrow kernel (1 to 8 tiles of the short extent, two of the long one from 4 on) holds its two
     buffers in registers: no scratch, two wavefronts per SIMD, operands by 16-byte global loads that go to
