@@ -191,13 +191,21 @@ __device__ inline tile_place workgroup_tile(const tiled_params &p, int bi, int b
     return tile_at(p, (int)(blockIdx.x + blockIdx.y * (unsigned)p.span), (int)blockIdx.y, bi, bj);
 }
 
-// All arguments into scalar registers at the start of the kernel.  Left to itself the compiler puts the loads of some off
-// to where they are first used, behind the K loop or right in front of the first operand load, where each waits for
-// memory (0.15 us of a launch).
+// Arguments into scalar registers, at the start of the kernel or behind the first requests.  Left to itself the compiler
+// puts the loads of some off to where they are first used, behind the K loop or right in front of the first operand load,
+// where each waits for memory (0.15 us of a launch); waiting at the start for C's and D's too costs 0.05.
+__device__ inline void fetch_operand_arguments(const tiled_params &p)
+{
+    asm volatile("" ::"s"(p.X), "s"(p.Y), "s"(p.I), "s"(p.J), "s"(p.K), "s"(p.ldx), "s"(p.ldy), "s"(p.sx), "s"(p.sy));
+}
+__device__ inline void fetch_result_arguments(const tiled_params &p)
+{
+    asm volatile("" ::"s"(p.C), "s"(p.D), "s"(p.ldc), "s"(p.ldd), "s"(p.sc), "s"(p.sd), "s"(p.c_trans), "s"(p.use_c), "s"(p.alpha), "s"(p.beta));
+}
 __device__ inline void fetch_arguments(const tiled_params &p)
 {
-    asm volatile("" ::"s"(p.X), "s"(p.Y), "s"(p.I), "s"(p.J), "s"(p.K), "s"(p.ldx), "s"(p.ldy), "s"(p.sx), "s"(p.sy), "s"(p.C), "s"(p.D),
-                 "s"(p.ldc), "s"(p.ldd), "s"(p.sc), "s"(p.sd), "s"(p.c_trans), "s"(p.use_c), "s"(p.alpha), "s"(p.beta));
+    fetch_operand_arguments(p);
+    fetch_result_arguments(p);
 }
 
 // ------------------------------------------------------------ slot loader --
@@ -451,7 +459,7 @@ void k_gemm_tiled(tiled_params p)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wi = wave % WI, wj = wave / WI;
 
-    fetch_arguments(p);
+    fetch_operand_arguments(p);
     const tile_place at = workgroup_tile(p, BI, BJ);
     const int i0 = at.i0, j0 = at.j0;
     const long bt = at.bt;
@@ -628,6 +636,7 @@ void k_gemm_tiled(tiled_params p)
     // Prologue: every slot requested, pair 0 published and its first fragments fetched.
 #pragma unroll
     for (int s = 0; s < NSLOT; s++) request_pair();
+    fetch_result_arguments(p);
     wait_loads_and_barrier<(NSLOT - 1) * LPAIR>();
     [&]<int... U>(std::integer_sequence<int, U...>) {
         (fetch_unit(f0, lds, std::integral_constant<int, U>{}, first_half), ...);
