@@ -10,6 +10,7 @@ returns an array with the same shape and values.
 """
 import ctypes
 import gc
+import math
 
 import numpy as np
 
@@ -90,8 +91,11 @@ class DeviceArray:
             src = np.asarray(src)
             dtype, dims = src.dtype, src.shape
         self.dtype = np.dtype(dtype)
-        self.dims = tuple(int(d) for d in dims)
-        self.nbytes = int(np.prod(self.dims, dtype=np.int64)) * self.dtype.itemsize
+        self.dims = tuple(map(int, dims))
+        count = math.prod(self.dims)
+        if not 0 <= count < 1 << 63:
+            count = int(np.prod(self.dims, dtype=np.int64))  # refuses or wraps, as an Int does
+        self.nbytes = count * self.dtype.itemsize
         p = ctypes.c_void_p()
         rc = lib.miw_malloc(ctypes.byref(p), self.nbytes)
         if rc != 0:

@@ -247,20 +247,27 @@ def _new_image(T, FS):
 
 # ------------------------------------------------------------ load ----------
 
+# What a valid load's types resolve to: (matrix, element type, layout) -> codes, elements per lane, type parameters.
+_LOADS = {(mat, ty, L): (_USE_CODE[_USE[mat]], _dtype_code(ty), _layout_code(L), _NUM_ELEMS[(mat, nm)], _USE[mat],
+                         Unspecified if mat == "c" else L)
+          for mat in "abc" for ty, nm in _TYPE_STR.items() for L in _LAYOUT_STR if (mat, nm) in _NUM_ELEMS}
+
+
 def _load(mat, addr, stride, layout, config):
     if not isinstance(addr, DevicePtr):
         raise TypeError(f"load_{mat}: addr must be a DevicePtr")
+    T = addr.eltype
     get_hl_as_info(addr.addrspace)
     get_hl_layout(layout)
-    get_hl_shape(config.M, config.N, config.K)
-    num_els, _ = get_hl_frag_info(mat, addr.eltype)
-    U = _USE[mat]
-    L_ret = Unspecified if mat == "c" else layout
-    T = addr.eltype
+    M, N, K = config.M, config.N, config.K
+    get_hl_shape(M, N, K)
+    found = _LOADS.get((mat, np.dtype(T), layout))
+    if found is None:
+        get_hl_frag_info(mat, T)  # raises
+    use, ty, order, num_els, U, L_ret = found
     img = _new_image(T, num_els)
-    _lib.check(_lib.load().miw_frag_load(_USE_CODE[U], _dtype_code(T), _layout_code(layout), addr.addrspace,
-                                         config.M, config.N, config.K, addr.addr, int(stride), img.ptr, _stream()))
-    return Fragment(config.M, config.N, config.K, num_els, T, L_ret, U, image=img)
+    _lib.check(_lib.load().miw_frag_load(use, ty, order, addr.addrspace, M, N, K, addr.addr, int(stride), img.ptr, _stream()))
+    return Fragment(M, N, K, num_els, T, L_ret, U, image=img)
 
 
 def load_a(addr, stride, layout, config):
@@ -292,31 +299,38 @@ def fill_c(value, config):
 
 # ------------------------------------------------------------ mma -----------
 
+# What a valid multiply's types resolve to: element types of a, b, c and d, layouts of a and b -> codes, elements per lane of d.
+_MMAS = {(np.float16, np.float16, c.type, d.type, al, bl): (_layout_code(al), _layout_code(bl), _dtype_code(c), _dtype_code(d), _NUM_ELEMS[("d", nm)])
+         for c in _TYPE_STR for d, nm in _TYPE_STR.items() for al in _LAYOUT_STR for bl in _LAYOUT_STR}
+
+
 def mma(a, b, c, config):
     """D = A*B + C (wmma.jl:558-583).  Dispatch rules of the reference's signature:
     a is a MatrixA, b a MatrixB, c an Accumulator with layout Unspecified, all of
     config's shape."""
+    M, N, K = config.M, config.N, config.K
     for f, use, nm in ((a, MatrixA, "a"), (b, MatrixB, "b"), (c, Accumulator, "c")):
         if not isinstance(f, Fragment) or f.U is not use:
             raise TypeError(f"mma: argument {nm} must be a Fragment with use {use.__name__}")
-        if (f.M, f.N, f.K) != (config.M, config.N, config.K):
+        if f.M != M or f.N != N or f.K != K:
             raise TypeError("mma: fragments and Config differ in shape")
-        if not f.on_device:
+        if f._image is None:
             raise TypeError("mma: fragments must come from load_*/fill_c/mma")
     if c.L is not Unspecified:
         raise TypeError("mma: the accumulator's layout must be Unspecified")
-    get_hl_frag_info("a", a.T)
-    get_hl_frag_info("b", b.T)
-    get_hl_frag_info("c", c.T)
-    d_num, _ = get_hl_frag_info("d", config.d_type)
-    get_hl_layout(a.L)
-    get_hl_layout(b.L)
-    get_hl_shape(config.M, config.N, config.K)
+    found = _MMAS.get((a.T, b.T, c.T, config.d_type, a.L, b.L))
+    if found is None:  # one of these raises
+        get_hl_frag_info("a", a.T)
+        get_hl_frag_info("b", b.T)
+        get_hl_frag_info("c", c.T)
+        get_hl_frag_info("d", config.d_type)
+        get_hl_layout(a.L)
+        get_hl_layout(b.L)
+    get_hl_shape(M, N, K)
+    a_order, b_order, c_ty, d_ty, d_num = found
     img = _new_image(config.d_type, d_num)
-    _lib.check(_lib.load().miw_frag_mma(_layout_code(a.L), _layout_code(b.L), _dtype_code(c.T),
-                                        _dtype_code(config.d_type), a._image.ptr, b._image.ptr, c._image.ptr,
-                                        img.ptr, _stream()))
-    return Fragment(config.M, config.N, config.K, d_num, config.d_type, Unspecified, Accumulator, image=img)
+    _lib.check(_lib.load().miw_frag_mma(a_order, b_order, c_ty, d_ty, a._image.ptr, b._image.ptr, c._image.ptr, img.ptr, _stream()))
+    return Fragment(M, N, K, d_num, config.d_type, Unspecified, Accumulator, image=img)
 
 
 # ------------------------------------------------------------ store_d -------
@@ -328,9 +342,9 @@ def store_d(addr, d, stride, layout, config):
         raise TypeError("store_d: (DevicePtr, Fragment, stride, layout, config)")
     if d.U is not Accumulator or d.L is not Unspecified:
         raise TypeError("store_d: d must be an Accumulator fragment with layout Unspecified")
-    if not (np.dtype(addr.eltype) == np.dtype(d.T) == np.dtype(config.d_type)):
+    if not (d.T is config.d_type and addr.eltype == d.T) and not (np.dtype(addr.eltype) == np.dtype(d.T) == np.dtype(config.d_type)):
         raise TypeError("store_d: eltype(addr), eltype(d) and Config d_type must agree")
-    if (d.M, d.N, d.K) != (config.M, config.N, config.K):
+    if d.M != config.M or d.N != config.N or d.K != config.K:
         raise TypeError("store_d: fragment and Config differ in shape")
     get_hl_as_info(addr.addrspace)
     get_hl_layout(layout)

@@ -360,6 +360,26 @@ def test_shared_k_kernel_runs_where_it_was_measured_ahead(miw, shared_k_tile):
     assert G.pick_variant(G.make_desc(48, 4096, 4096, **rc)) == by["fragment_ops"]
 
 
+def test_fragment_signature_tables_agree_with_the_checks(miw):
+    """Every pair of types and layouts is in load's and mma's tables exactly where the checks let it pass."""
+    W, L = miw.WMMA, miw._lib
+    layouts = (W.RowMajor, W.ColMajor)
+    for mat, ty, lay in itertools.product("abc", (np.float16, np.float32, np.float64, np.int16, ">f2"), layouts + (W.Unspecified,)):
+        found = W._LOADS.get((mat, np.dtype(ty), lay))
+        try:
+            n, name = W.get_hl_frag_info(mat, ty)
+            W.get_hl_layout(lay)
+        except W.WMMAError:
+            assert found is None
+            continue
+        use = {"a": W.MatrixA, "b": W.MatrixB, "c": W.Accumulator}[mat]
+        assert found == (W._USE_CODE[use], L.F16 if name == "f16" else L.F32, L.ROW_MAJOR if lay is W.RowMajor else L.COL_MAJOR, n, use,
+                         W.Unspecified if mat == "c" else lay)
+    f16, f32 = np.float16, np.float32
+    assert len(W._MMAS) == 16 and all(W._MMAS[f16, f16, c, d, a, b] == (W._layout_code(a), W._layout_code(b), W._dtype_code(c), W._dtype_code(d), 4)
+                                      for c in (f16, f32) for d in (f16, f32) for a in layouts for b in layouts)
+
+
 def test_variant_table_and_selection(miw):
     G = miw.GEMM
     vs = G.variants()
