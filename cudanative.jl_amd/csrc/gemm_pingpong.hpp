@@ -709,7 +709,9 @@ void k_gemm_pp64(tiled_params p)
     const int wi = wave % WI, wj = wave / WI;
     const bool late_group = wave >= 4;
 
-    fetch_operand_arguments(p);
+    // (with Float16 accumulation C is requested ahead of the operands: one wait for all arguments)
+    if constexpr (F16ACC) fetch_arguments(p);
+    else fetch_operand_arguments(p);
     const tile_place at = workgroup_tile(p, BI, BJ);
     const int i0 = at.i0, j0 = at.j0;
     const long bt = at.bt;
@@ -856,7 +858,7 @@ void k_gemm_pp64(tiled_params p)
         (std::make_integer_sequence<int, LPAIR>{});
         end_request();
     }
-    fetch_result_arguments(p);
+    if constexpr (!F16ACC) fetch_result_arguments(p);
     // The loop starts when pair 0 (and the C operand, requested before it) has landed: the wait at the
     // end of memory cluster p leaves NSLOT - 2 pairs in flight, so pair p + 1 has landed by then, the
     // first time as every other.
