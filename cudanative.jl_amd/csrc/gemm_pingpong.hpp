@@ -191,9 +191,9 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
     auto y_origin = [](auto a, int bt, int j0) MIW_INLINE { return a->Y + (long)bt * a->sy + (YK ? (long)j0 * a->ldy : (long)j0); };
     fetch_arguments(p);  // (what is read again later is then in the scalar cache)
     int tile = blockIdx.x + blockIdx.y * (unsigned)p.span;
-    tile_place at = tile_at(*arguments(), tile, blockIdx.y, BI, BJ);
-    const half_t *X = x_origin(arguments(), at.bt, at.i0);
-    const half_t *Y = y_origin(arguments(), at.bt, at.j0);
+    tile_place at = tile_at(p, tile, blockIdx.y, BI, BJ);  // (the first tile's: already in registers)
+    const half_t *X = x_origin(&p, at.bt, at.i0);
+    const half_t *Y = y_origin(&p, at.bt, at.j0);
     const unsigned xoff = xop::lane_offset(tid, (int)p.ldx);
     const unsigned yoff = yop::lane_offset(tid, (int)p.ldy);
 
