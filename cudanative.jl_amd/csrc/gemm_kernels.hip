@@ -119,8 +119,7 @@ static hipError_t allow_dynamic_lds(const void *fn, int bytes)
 // Multiplier and shift for quotient() of gemm_tiled.hpp.
 static unsigned multiplier(long d, unsigned *shift)
 {
-    *shift = 0;
-    while ((1l << *shift) < d) ++*shift;
+    *shift = d > 1 ? 64u - (unsigned)__builtin_clzl((unsigned long)(d - 1)) : 0u;
     return (unsigned)(((1l << (31 + *shift)) + d - 1) / d);
 }
 
