@@ -146,9 +146,8 @@ struct pp_operand {
 // under the epilogue.  One workgroup per tile pays for a start of 2 to 3 us and for the dispatch, which hands
 // workgroups to the shader engines in turn and waits for the slowest, 1 to 5 us, in every round; what is left is the
 // store of D, whose acknowledgements the loads of the next tile's third k-step wait for (vmcnt counts in order).
-// 8192x8192x1024, alpha = -1, operands from HBM: 188 us with one tile per workgroup, 159 like this with C folded
-// from sixteen slots of K on (it was eighteen); without C 143 and 127; 6144^3 425 and 414; 8192^3 level (784, 779),
-// which is bound by energy.
+// 8192x8192x1024, alpha = -1, operands from HBM: 188 us with one tile per workgroup, 180 like this; without C 143
+// and 127; 6144^3 425 and 414; 8192^3 level (784, 779), which is bound by energy.
 // FOLD: a Float32 C is added in the K loop; otherwise C, if any, in the epilogue.  They are kernels of their own: in
 // one kernel the accumulators of both forms meet in the last pair, and that spills.
 template <int BI, int BJ, int WI, int WJ, bool XK, bool YK, class CT, class DT, bool FOLD>
@@ -412,15 +411,14 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
     // fetches the 16 bytes it owns); the wait at the end of the memory cluster two steps later covers it, and that
     // cluster adds it in: C has two clusters of both wavefront groups to arrive, and what it takes longer stalls the
     // loop, since loads return in order.  (Requested behind the cluster's own loads, or two tiles every other step,
-    // 8192x8192x1024 takes 3 % longer.)  Three register stages rotate.  Tiles go in the order of their addresses: 16
-    // rows (64 bytes, the instruction's offset field) further down a column block, then the next 16 columns.  The
-    // accumulators are registers, so the folding steps are unrolled.
+    // 8192x8192x1024 with C folded takes 3 % longer.)  Three register stages rotate.  Tiles go in the order of their
+    // addresses: 16 rows (64 bytes, the instruction's offset field) further down a column block, then the next 16
+    // columns.  The accumulators are registers, so the folding steps are unrolled.
     constexpr int NTILE = TI * TJ;
     constexpr int NFOLD = NTILE;
     static_assert(!FOLD || (__is_same(CT, float) && NFOLD == PP_FOLD_STEPS && NFOLD % 2 == 0), "fold steps");
     float4_t cst[3];
     const char *cnext = nullptr;
-    const float fold_beta = p.alpha * p.beta;  // the epilogue multiplies the sums by alpha
     // (the lane offset into the tile of C is kept in 32 bits)
     const unsigned coff = 4u * (unsigned)((wj * WTJ + r) * (int)p.ldc + wi * WTI + 4 * q);
     auto fold_request = [&]<int S>(std::integral_constant<int, S>) MIW_INLINE {
@@ -431,7 +429,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
     auto fold_add = [&]<int S>(std::integral_constant<int, S>) MIW_INLINE {
         constexpr int a = S % TI, b = S / TI;
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[a][b][e] = __builtin_fmaf(fold_beta, cst[S % 3][e], acc[a][b][e]);
+        for (int e = 0; e < 4; e++) acc[a][b][e] = __builtin_fmaf(p.beta, cst[S % 3][e], acc[a][b][e]);
     };
     // Zeroes the repeated k-values in the fragments of step H of the shifted last pair.
     auto mask_tail = [&]<int H>(std::integral_constant<int, H>) MIW_INLINE {

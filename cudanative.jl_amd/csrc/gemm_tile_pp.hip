@@ -34,13 +34,14 @@ const void *pp_kernel(int bm, int bn, bool xk, bool yk, int c_type, int d_type, 
     if (bm == 256 && bn == 256) return pp_layout<256, 256, 2, 4>(xk, yk, c_type, d_type, fold);
     return nullptr;
 }
-// Does k_gemm_pp_fold run the problem?  C Float32, laid out as D, lane offsets into its tile within 32 bits; enough
-// k-steps for one tile of C each; and alpha of 1 or -1, with which adding alpha * beta * C to the sums and
-// multiplying them by alpha afterwards rounds nothing.
+// Does k_gemm_pp_fold run the problem?  C Float32, laid out as D, lane offsets into its tile within 32 bits; more k-steps
+// than tiles of C, one of which each of the last ones adds; and alpha of 1.  Every MFMA behind C's addition rounds at C's
+// magnitude: with |C| of a hundred times |A B| that is three to five times the error of adding it once, behind the loop.
+// So alpha = -1 and sixteen slots of K do not take it, although they would gain: 8192x8192x1024, alpha = -1, takes 180 us, 159 with C folded.
 bool pp_folds(const tiled_params &p, int c_type)
 {
-    return p.use_c && c_type == 1 && !p.c_trans && (p.alpha == 1.0f || p.alpha == -1.0f) && p.ldc < (1l << 22) &&
-           (p.K + KGRAN - 1) / KGRAN * 2 >= PP_FOLD_STEPS;
+    return p.use_c && c_type == 1 && !p.c_trans && p.alpha == 1.0f && p.ldc < (1l << 22) &&
+           (p.K + KGRAN - 1) / KGRAN * 2 > PP_FOLD_STEPS;
 }
 int pp_lds(int bm, int bn, bool xk, bool yk) { return pp_lds_bytes(bm, bn, xk, yk); }
 

@@ -198,6 +198,30 @@ def test_workgroups_that_walk_several_tiles(gpu, orc, al, bl, K):
         assert np.array_equal(D, orc.gemm(g, A, B, C)), (al, bl, cl, dl, K, form)
 
 
+@pytest.mark.parametrize("alpha,K", [(-1.0, 976), (-1.0, 1024), (-1.0, 1168), (1.0, 976), (1.0, 1024)])
+@pytest.mark.parametrize("al,bl", itertools.product((0, 1), repeat=2))
+def test_c_is_added_once_behind_the_loop(gpu, orc, alpha, K, al, bl):
+    """alpha other than 1, or K of no more than sixteen slots on a 256-wide tile: D is the launch without C plus C in one
+    rounding, however much larger than the product C is, and exact cancellation gives the sign of zero that this has."""
+    for v in _variants(gpu):
+        if v["fragment_ops"] or (alpha == 1.0 and max(v["block"][:2]) < 256):     # (the 128x128 ping-pong tile folds from 592 on)
+            continue
+        big = max(v["block"][:2])
+        for dl in (0, 1):
+            g = orc.GemmDesc(M=big, N=big + 16, K=K, a_layout=al, b_layout=bl, c_layout=dl, d_layout=dl, alpha=alpha)
+            A, B, C = _inputs(orc, g, 1700 + K + v["id"])
+            A2, C2 = (A.reshape(big, K) if al == orc.ROW else A.reshape(K, big).T), C.reshape((big, big + 16) if dl == orc.ROW else (big + 16, big))
+            C *= 1000.0
+            A2[:16] = 0.0
+            (C2 if dl == orc.ROW else C2.T)[:16] = np.array([0.0, -0.0], dtype=F32)[np.arange(big + 16) % 2]
+            g0 = orc.GemmDesc(M=big, N=big + 16, K=K, a_layout=al, b_layout=bl, c_layout=dl, d_layout=dl, use_c=0)
+            S = _run(gpu, orc, g0, A, B, None, variant=v["id"])
+            if S is None:
+                continue
+            D = _run(gpu, orc, g, A, B, C, variant=v["id"])
+            assert np.array_equal(D.view(np.uint32), (F32(alpha) * S + C).view(np.uint32)), (v["name"], al, bl, dl, K, alpha)
+
+
 def test_c_folded_into_the_loop_matches_the_epilogue_path(gpu, orc):
     """Random inputs, padded leading dimensions, batches: the folded C (alpha == 1, C laid out as D)
     agrees with float64 as tightly as the kernels that add C after the loop (alpha != 1, the
