@@ -992,8 +992,9 @@ miw::gemm_params splitk_slices(const miw::gemm_params &p, int splits, void *ws)
     return q;
 }
 
+// cap: slice counts with a larger workspace are not chosen.  room: the workspace there is.
 int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void *C, void *D, int splits, splitk_plan *out,
-                size_t workspace_cap = SIZE_MAX)
+                size_t cap = SIZE_MAX, size_t room = SIZE_MAX)
 {
     bool f16acc;
     miw::gemm_params p;
@@ -1002,19 +1003,19 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     if (p.batch != 1) return fail(MIW_ERR_UNSUPPORTED, "gemm_splitk: one problem per call (batch %lld asked)", (long long)p.batch);
     if (d->variant != 0) return fail(MIW_ERR_INVALID_VALUE, "gemm_splitk: the variant is chosen per slice; desc.variant must be 0");
     if (splits < 0 || splits > 256) return fail(MIW_ERR_INVALID_VALUE, "gemm_splitk: splits must be 0 (choose) or 1..256, got %d", splits);
-    const bool in_place = c_shares_d(d, p);
+    const bool shares = c_shares_d(d, p);
     static char dummy alignas(128);
     // Variant and estimated duration of s slices (s = 1: the plain launch); false when no tiled kernel fits.
-    auto try_splits = [&](int s, int *variant, miw::kwave_tile *kw, double *us) {
-        if (p.K % (64l * s)) return false;
+    auto try_splits = [&](const miw::gemm_params &o, bool in_place, int s, int *variant, miw::kwave_tile *kw, double *us) {
+        if (o.K % (64l * s)) return false;
         if (s == 1) {
-            if (!pick_tiled(p, d->c_type, d->d_type, false, 0, in_place, us)) return false;
-            *variant = pick_variant(p, d->c_type, d->d_type, false, 0, in_place, kw);
-            // (only where C in D's place runs the same: the workspace's size is asked for without the pointers)
-            if (kw->bi && p.M % 64 == 0 && p.N % 64 == 0) *us = miw::kwave_estimate_us(p, d->c_type, d->d_type, *kw);
+            if (!pick_tiled(o, d->c_type, d->d_type, false, 0, in_place, us)) return false;
+            *variant = pick_variant(o, d->c_type, d->d_type, false, 0, in_place, kw);
+            // (ragged extents are priced as a tile's launch, which is what C in D's place may get)
+            if (kw->bi && o.M % 64 == 0 && o.N % 64 == 0) *us = miw::kwave_estimate_us(o, d->c_type, d->d_type, *kw);
             return true;
         }
-        const miw::gemm_params q = splitk_slices(p, s, &dummy);
+        const miw::gemm_params q = splitk_slices(o, s, &dummy);
         const int v = pick_tiled(q, MIW_F32, MIW_F32, false, 0, false, us);
         if (v == 0) return false;
         *variant = v;
@@ -1024,40 +1025,63 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
         else *kw = {0, 0};
         // second kernel: launch, the additions (each thread's slices in order), and the slices, C and D at
         // the same pace as above
-        const double mn = (double)p.M * (double)p.N;
+        const double mn = (double)o.M * (double)o.N;
         *us += 2.5 + 0.03 * s +
-              mn * (4.0 * s + (double)dtype_size(d->d_type) + (p.use_c ? (double)dtype_size(d->c_type) : 0.0)) / 5.5e6;
+              mn * (4.0 * s + (double)dtype_size(d->d_type) + (o.use_c ? (double)dtype_size(d->c_type) : 0.0)) / 5.5e6;
         return true;
     };
+    // one slice is the plain launch: no workspace, no second kernel
+    auto bytes = [&](int s) { return s == 1 ? 0 : (size_t)s * (size_t)p.M * (size_t)p.N * sizeof(float); };
     int variant = 0;
     miw::kwave_tile kw = {0, 0};
     double us = 0.0;
-    if (splits == 0) {
-        // The slice count with the shortest estimated duration, among 1 (no second pass) and the
-        // counts up to 64 that leave every slice two LDS slots' worth of K or more.
+    // The slice count with the shortest estimated duration, among 1 (no second pass) and the counts up to 64 that leave
+    // every slice two LDS slots' worth of K or more; 0 when none fits.
+    auto choose = [&](const miw::gemm_params &o, bool in_place) {
+        int best = 0, v;
         double best_us = 0.0;
-        for (int s = 1; s <= 64 && (s == 1 || p.K / s >= 128); s++) {
-            int v;
-            miw::kwave_tile t;
-            // a caller with a bounded workspace is offered only the counts that fit in it
-            if (s > 1 && (size_t)s * (size_t)p.M * (size_t)p.N * sizeof(float) > workspace_cap) break;
-            if (!try_splits(s, &v, &t, &us)) continue;
-            if (splits == 0 || us < 0.97 * best_us) { splits = s; variant = v; kw = t; best_us = us; }
+        miw::kwave_tile t;
+        for (int s = 1; s <= 64 && (s == 1 || o.K / s >= 128); s++) {
+            if (bytes(s) > cap) break;
+            if (!try_splits(o, in_place, s, &v, &t, &us)) continue;
+            if (best == 0 || us < 0.97 * best_us) { best = s; best_us = us; }
         }
-    } else if (!try_splits(splits, &variant, &kw, &us)) {
-        splits = 0;
+        return best;
+    };
+    // The count is chosen from what the query for the workspace knows: operands on whole cache lines, C and D apart.
+    // The real operands then decide what runs each slice.
+    miw::gemm_params lines = p;
+    lines.A = lines.B = (const _Float16 *)&dummy;
+    lines.C = p.use_c ? &dummy : nullptr;
+    lines.D = &dummy;
+    int count = splits ? splits : choose(lines, false);
+    const bool runs = count && try_splits(p, shares, count, &variant, &kw, &us);
+    if (!runs || bytes(count) > room) {
+        // Addresses off 16 bytes, C in D's place with extents that no tile divides, or a workspace of another size than
+        // the query's: what the real operands alone would choose.
+        const int other = splits ? 0 : choose(p, shares);
+        if (other && bytes(other) <= room) {
+            count = other;
+            try_splits(p, shares, count, &variant, &kw, &us);
+        } else if (count == 1 && !runs && shares && p.K % 64 == 0 && pick_tiled(p, d->c_type, d->d_type, false, 0, false) &&
+                   (p.M / 16) * (p.N / 16) / 4 < (1l << 31)) {
+            // (only C in D's place keeps the tiles from it: the plain launch on a kernel that has none)
+            variant = pick_variant(p, d->c_type, d->d_type, false, 0, shares, &kw);
+        } else if (!runs) {
+            count = other;
+            if (count) try_splits(p, shares, count, &variant, &kw, &us);
+        }
     }
-    if (splits == 0)
+    if (count == 0)
         return fail(MIW_ERR_UNSUPPORTED,
                     "gemm_splitk: needs K divisible by 64 * splits, M and N of at least one LDS tile (64), "
                     "16-byte aligned operands and leading dimensions");
     out->full = p;
-    out->splits = splits;
+    out->splits = count;
     out->variant = variant;
     out->kw = kw;
-    // one slice is the plain launch: no workspace, no second kernel
-    out->bytes = splits == 1 ? 0 : (size_t)splits * (size_t)p.M * (size_t)p.N * sizeof(float);
-    out->slice = splitk_slices(p, splits, nullptr);
+    out->bytes = bytes(count);
+    out->slice = splitk_slices(p, count, nullptr);
     return 0;
 }
 
@@ -1097,7 +1121,7 @@ int miw_gemm_splitk(const miw_gemm_desc *desc, const void *A, const void *B, con
                     void *workspace, size_t workspace_bytes, void *stream)
 {
     splitk_plan plan;
-    if (int rc = plan_splitk(desc, A, B, C, D, splits, &plan)) return rc;
+    if (int rc = plan_splitk(desc, A, B, C, D, splits, &plan, SIZE_MAX, workspace ? workspace_bytes : 0)) return rc;
     if (!workspace && plan.bytes) return fail(MIW_ERR_NULL_POINTER, "gemm_splitk: null workspace");
     if (workspace_bytes < plan.bytes)
         return fail(MIW_ERR_INVALID_VALUE, "gemm_splitk: workspace of %zu bytes, %d slices need %zu", workspace_bytes,

@@ -273,7 +273,9 @@ int miw_gemm_resolve(const miw_gemm_desc *desc, const void *A, const void *B, co
    the slice count with the shortest estimated duration (both kernels and the workspace traffic
    counted).  One slice, asked for or chosen, is the plain launch of miw_gemm: no workspace
    (0 bytes, `workspace` may be null) and no second kernel.  miw_gemm_splitk_workspace reports
-   the slice count and the bytes miw_gemm_splitk will ask for. */
+   the slice count and the bytes miw_gemm_splitk will ask for, whatever the operands' addresses (16-byte
+   aligned) and also with C in D's place (where no tile divides the extents and the workspace has room for
+   more slices, more are taken: one slice runs without LDS tiles there). */
 int miw_gemm_splitk_workspace(const miw_gemm_desc *desc, int splits, int *splits_out, size_t *bytes);
 int miw_gemm_splitk(const miw_gemm_desc *desc, const void *A, const void *B, const void *C, void *D, int splits,
                     void *workspace, size_t workspace_bytes, void *stream);

@@ -1,5 +1,6 @@
 """GPU parity tests of the tiled GEMM D = alpha*A*B + beta*C, through the C ABI,
 against the CPU oracle (exact fp64 reference and the fp16-accumulate model)."""
+import ctypes
 import itertools
 import os
 
@@ -1119,6 +1120,23 @@ def test_splitk_random_types_scalars_and_padding(gpu, orc):
     A, B, _ = _inputs(orc, g, 660)
     D = _run_splitk(gpu, orc, g, A, B, None)
     assert orc.normalized_error(g, D, orc.gemm_f64(g, A, B, None)) <= TIGHT_F32
+
+
+def test_splitk_in_place_on_extents_that_no_tile_divides(gpu, orc):
+    """One slice by the query, and no tile for it when C is D: the plain launch; with room for slices, slices."""
+    G = gpu.GEMM
+    g = orc.GemmDesc(M=496, N=672, K=256)
+    A, B, C = _inputs(orc, g, 45, ints=True)
+    desc = G.make_desc(496, 672, 256)
+    assert G.splitk_workspace(desc) == (1, 0)
+    dA, dB, ws = gpu.DeviceArray(A), gpu.DeviceArray(B), gpu.DeviceArray.undef(F32, 4 * 496 * 672)
+    want = orc.gemm(g, A, B, C)
+    for launch in (lambda d: G.gemm_splitk(dA, dB, d, d, desc), lambda d: G.gemm_splitk_static(dA, dB, d, d, desc),
+                   lambda d: gpu._lib.check(gpu._lib.load().miw_gemm_splitk(ctypes.byref(desc), dA.ptr, dB.ptr, d.ptr, d.ptr, 0, ws.ptr, ws.nbytes, None))):
+        dD = gpu.DeviceArray(C)
+        launch(dD)
+        gpu.synchronize()
+        assert np.array_equal(dD.to_host(), want)
 
 
 def test_splitk_slice_choice_and_errors(gpu, orc):

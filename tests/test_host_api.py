@@ -478,6 +478,36 @@ def test_device_entries_need_init(miw):
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stderr
 
 
+def test_splitk_takes_the_workspace_its_query_reports(miw):
+    """The slice count does not hang on what the query cannot see, where operands sit inside a cache line or C in D's place:
+    a call with exactly the bytes reported gets past every check (a process without miw_init: no launch).  One slice of a
+    problem that no tile divides, C in D's place, is the plain launch."""
+    import subprocess, sys
+    code = ("import sys, ctypes, random; sys.path.insert(0, %r); from tests.conftest import load_package; m = load_package();\n"
+            "L, G, W = m._lib, m.GEMM, m.WMMA; lib = L.load(); rng = random.Random(7); base = 1 << 32\n"
+            "p = lambda i, off=0: ctypes.c_void_p(base + (i << 40) + off)\n"
+            "side = lambda: rng.choice((W.RowMajor, W.ColMajor))\n"
+            "def check(M, N, K, offsets, in_place, **kw):\n"
+            "    d = G.make_desc(M, N, K, **kw); n, nbytes = G.splitk_workspace(d)\n"
+            "    a, b, c = (p(i, o) for i, o in enumerate(offsets)); D = c if in_place else p(3, 16 * rng.randrange(8))\n"
+            "    for splits in (0, n):\n"
+            "        rc = lib.miw_gemm_splitk(ctypes.byref(d), a, b, c, D, splits, p(4, 16 * rng.randrange(8)) if nbytes else None, nbytes, None)\n"
+            "        assert rc == L.ERR_NOT_INITIALIZED, (M, N, K, offsets, in_place, kw, n, nbytes, lib.miw_last_error())\n"
+            "    assert lib.miw_gemm_splitk_static(ctypes.byref(d), a, b, c, D, 0, None) == L.ERR_NOT_INITIALIZED\n"
+            "rc = dict(a_layout=W.RowMajor, use_c=False)\n"
+            "for M, N, K in ((64, 80, 1024), (64, 96, 2048), (64, 64, 3840), (64, 80, 896), (160, 64, 2048)):\n"
+            "    check(M, N, K, (16, 48, 0), False, **rc)\n"
+            "check(496, 672, 256, (0, 0, 0), True)\n"
+            "for _ in range(6000):\n"
+            "    M, N = (16 * rng.randint(4, 64) if rng.random() < 0.5 else 16 * rng.randint(4, 8) for _ in 'MN')\n"
+            "    lay = side(); in_place = rng.random() < 0.3\n"
+            "    check(M, N, 64 * rng.randint(2, 64), [16 * rng.randrange(8) for _ in range(3)], in_place, a_layout=side(), b_layout=side(),\n"
+            "          c_layout=lay, d_layout=lay, use_c=in_place or rng.random() < 0.5)\n"
+            "print('ok')\n") % ROOT
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0 and out.stdout.strip() == "ok", out.stderr
+
+
 def test_tiled_gemm_kernels_are_not_launchable_by_name(miw):
     """The LDS-tiled kernels take a private argument block, a fixed workgroup and dynamic LDS: they can be
     looked up (attribute queries) but miw_launch refuses them and points to miw_gemm."""
