@@ -178,7 +178,7 @@ def shape_sweep(mode):
             desc = G.make_desc(M, N, K, a_layout=la, **kind)
             plan = G.plan(desc)
             r = {"us": round(timed(desc, bufs, 0.25), 1),
-                 "launches": ["%s %dx%dx%d" % (names[q["variant"]], q["m"], q["n"], q["k"]) for q in plan]}
+                 "launches": ["%s %dx%dx%d" % (names[q["kernel"]], q["m"], q["n"], q["k"]) for q in plan]}
             best = None
             for v in () if f16out else G.variants():
                 d2 = G.make_desc(M, N, K, a_layout=la, variant=v["id"])
@@ -391,7 +391,8 @@ def main():
         roof = {"bound": "mfma", "achieved": flops / (kernel_ms * 1e-3) / 1e12, "peak": PEAK_F16_DENSE_TFLOPS,
                 "unit": "TFLOP/s"}
     roof["frac"] = roof["achieved"] / roof["peak"]
-    family = ("k_gemm_skinny" if vinfo["name"] == "narrow_k_contiguous" else
+    family = ("k_gemm_kwave" if vinfo["name"] == "shared_k" else
+              "k_gemm_skinny" if vinfo["name"] == "narrow_k_contiguous" else
               "k_gemm_fragops" if vinfo["fragment_ops"] else
               "k_gemm_w128" if vinfo["wave128"] else
               "k_gemm_tiled" if not vinfo["pingpong"] else

@@ -76,7 +76,7 @@ class GemmDesc(ctypes.Structure):
 
 
 class GemmPart(ctypes.Structure):
-    _fields_ = [("variant", ctypes.c_int), ("reserved", ctypes.c_int),
+    _fields_ = [("variant", ctypes.c_int), ("kernel", ctypes.c_int),
                 ("m0", ctypes.c_int64), ("n0", ctypes.c_int64), ("k0", ctypes.c_int64),
                 ("m", ctypes.c_int64), ("n", ctypes.c_int64), ("k", ctypes.c_int64)]
 

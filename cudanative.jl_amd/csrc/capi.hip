@@ -288,10 +288,13 @@ const std::vector<int> &variant_order()
     return order;
 }
 
-// Ids behind the tiled variants: the kernel for one extent of at most 128 with k contiguous in both operands,
-// and the fragment-op kernels.  Both take every problem (a problem the first cannot run goes to the others).
-int narrow_id() { return miw::tiled_variant_count() + 1; }
-int fragops_id() { return miw::tiled_variant_count() + 2; }
+// Ids behind the tiled variants: small tiles whose wavefronts share K, the kernel for one extent of at most 128 with k
+// contiguous in both operands, and the fragment-op kernels.  All three take every problem (what the first two cannot run
+// goes to the last).
+bool untiled(int variant) { return variant > miw::tiled_variant_count(); }
+int shared_k_id() { return miw::tiled_variant_count() + 1; }
+int narrow_id() { return miw::tiled_variant_count() + 2; }
+int fragops_id() { return miw::tiled_variant_count() + 3; }
 // The smallest tile's.
 int small_id()
 {
@@ -316,8 +319,8 @@ int pick_tiled(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, i
     return best + 1;
 }
 
-// *kw: the tile of k_gemm_kwave where that runs in the picked variant's place.  It has no id of its own: tile64x64_w2x2
-// stands for it, below 64 rows or columns fragment_ops, and narrow_k_contiguous where that was picked.
+// *kw: the tile of k_gemm_kwave where that runs in the picked variant's place, which is the smallest tile's, below 64 rows
+// or columns fragment_ops', or narrow_k_contiguous'.  The launch's own id is then shared_k_id().
 int pick_variant(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place, miw::kwave_tile *kw_out = nullptr)
 {
     // (a batch keeps the bits that each of its members has under the picked id)
@@ -343,7 +346,7 @@ int check_gemm(const miw_gemm_desc *d, const miw::gemm_params &p, bool f16acc, b
     int variant = d->variant;
     if (variant < 0 || variant > fragops_id()) return fail(MIW_ERR_INVALID_VALUE, "gemm: unknown variant %d", variant);
     if (variant == 0) variant = pick_variant(p, d->c_type, d->d_type, f16acc, d->acc_chunk, in_place);
-    if (variant >= narrow_id()) {
+    if (untiled(variant)) {
         if (f16acc && d->acc_chunk != 0 && d->acc_chunk != 16)
             return fail(MIW_ERR_UNSUPPORTED, "gemm: the fragment-op kernel rounds every 16 k-values (acc_chunk %d asked)",
                         d->acc_chunk);
@@ -362,7 +365,7 @@ int check_gemm(const miw_gemm_desc *d, const miw::gemm_params &p, bool f16acc, b
     return 0;
 }
 
-// kw: the tile of k_gemm_kwave, which runs in the variant's place unless that is forced (0: it does not).
+// kw: the tile of k_gemm_kwave, which runs in the variant's place (0: it does not).
 int launch_gemm(int variant, miw::kwave_tile kw, const miw::gemm_params &p, int c_type, int d_type, bool f16acc, hipStream_t s)
 {
     if (kw.bi) {
@@ -370,7 +373,7 @@ int launch_gemm(int variant, miw::kwave_tile kw, const miw::gemm_params &p, int 
         return 0;
     }
     if (variant == narrow_id() && miw::skinny_fits(p, d_type, f16acc)) HIP_TRY(miw::launch_gemm_skinny(p, c_type, d_type, s));
-    else if (variant >= narrow_id()) HIP_TRY(miw::launch_gemm_fragops(p, c_type, d_type, f16acc, s));
+    else if (untiled(variant)) HIP_TRY(miw::launch_gemm_fragops(p, c_type, d_type, f16acc, s));
     else HIP_TRY(miw::launch_gemm_tiled(variant - 1, p, c_type, d_type, f16acc, cu_count(), s));
     return 0;
 }
@@ -391,6 +394,7 @@ struct gemm_part {
     miw::gemm_params p;
     long m0, n0, k0;  // where the part sits in the caller's problem
     miw::kwave_tile kw;
+    int id() const { return kw.bi ? shared_k_id() : variant; }  // of the kernel that runs
 };
 
 // The kernels behind the fragment-op id, in the order launch_gemm_fragops asks.  Up to 64 k-values with C
@@ -506,12 +510,13 @@ int plan_gemm(const miw_gemm_desc *d, const miw::gemm_params &p, bool f16acc, bo
     if (d->variant != 0 || f16acc) {
         int variant = 0;
         if (int rc = check_gemm(d, p, f16acc, in_place, &variant)) return rc;
-        parts->push_back(gemm_part{variant, d->c_type, p, 0, 0, 0, {0, 0}});
+        const bool shared = variant == shared_k_id() && !f16acc;
+        parts->push_back(gemm_part{variant, d->c_type, p, 0, 0, 0, shared ? miw::kwave_fits(p, d->c_type, d->d_type, in_place, cu_count()) : miw::kwave_tile{0, 0}});
     } else {
         gemm_planner pl{d->d_type, in_place};
         pl.plan(p, d->c_type, 0, 0, 0, 0, parts);
         for (const gemm_part &part : *parts)
-            if (part.variant >= narrow_id() && (part.p.M / 16) * (part.p.N / 16) / 4 >= (1l << 31))
+            if (untiled(part.variant) && (part.p.M / 16) * (part.p.N / 16) / 4 >= (1l << 31))
                 return fail(MIW_ERR_UNSUPPORTED, "gemm: %lld x %lld tiles of 16 x 16 do not fit the launch grid",
                             (long long)(part.p.M / 16), (long long)(part.p.N / 16));
     }
@@ -829,6 +834,15 @@ int miw_gemm_variant_info_get(int variant, miw_gemm_variant_info *out)
     if (!out) return fail(MIW_ERR_NULL_POINTER, "gemm_variant_info: null output");
     if (variant < 1 || variant > fragops_id()) return fail(MIW_ERR_INVALID_VALUE, "gemm_variant_info: unknown variant %d", variant);
     memset(out, 0, sizeof(*out));
+    if (variant == shared_k_id()) {
+        snprintf(out->name, sizeof(out->name), "shared_k");
+        out->block_m = 32; out->block_n = 32; out->block_k = 64;
+        out->waves_m = 1; out->waves_n = 1;  // (its four wavefronts share K)
+        out->stages = 20; out->lds_bytes = 20 * (32 + 32) * 64 * 2;  // (five slots of each wavefront's)
+        out->fragment_ops = 1;
+        out->f16_accumulate = 1;
+        return 0;
+    }
     if (variant == narrow_id()) {
         snprintf(out->name, sizeof(out->name), "narrow_k_contiguous");
         out->block_m = 16; out->block_n = 16; out->block_k = 64;
@@ -861,7 +875,7 @@ int miw_gemm_variant_supports(const miw_gemm_desc *desc, int variant, int *suppo
     bool f16acc;
     static char dummy alignas(128);
     if (int rc = resolve_gemm(desc, &dummy, &dummy, &dummy, &dummy, &p, &f16acc)) return rc;
-    if (variant >= narrow_id()) *supported = !(f16acc && desc->acc_chunk != 0 && desc->acc_chunk != 16);
+    if (untiled(variant)) *supported = !(f16acc && desc->acc_chunk != 0 && desc->acc_chunk != 16);
     else *supported = tiled_fits(variant - 1, p, desc->c_type, desc->d_type, f16acc, desc->acc_chunk, false) ? 1 : 0;
     return 0;
 }
@@ -893,7 +907,7 @@ int miw_gemm_plan(const miw_gemm_desc *desc, int in_place, miw_gemm_part *out, i
     for (int i = 0; i < (int)parts.size() && i < capacity; i++) {
         const gemm_part &g = parts[(size_t)i];
         out[i].variant = g.variant;
-        out[i].reserved = 0;
+        out[i].kernel = g.id();
         out[i].m0 = g.m0; out[i].n0 = g.n0; out[i].k0 = g.k0;
         out[i].m = g.p.M; out[i].n = g.p.N; out[i].k = g.p.K;
     }
@@ -906,7 +920,7 @@ int miw_gemm_acc_chunk(const miw_gemm_desc *desc, int *acc_chunk)
     int v = 0;
     if (int rc = miw_gemm_pick_variant(desc, &v)) return rc;
     if (desc->variant != 0) v = desc->variant;
-    *acc_chunk = v >= narrow_id() ? 16 : miw::tiled_f16acc_chunk();
+    *acc_chunk = untiled(v) ? 16 : miw::tiled_f16acc_chunk();
     return 0;
 }
 
@@ -917,9 +931,9 @@ int miw_gemm_resolve(const miw_gemm_desc *desc, const void *A, const void *B, co
     if (int rc = resolve_gemm(desc, A, B, C, const_cast<void *>(D), &p, &f16acc)) return rc;
     std::vector<gemm_part> parts;
     if (int rc = plan_gemm(desc, p, f16acc, c_shares_d(desc, p), &parts)) return rc;
-    const int v = parts.empty() ? 0 : parts[0].variant;
+    const int v = parts.empty() ? 0 : parts[0].id();
     if (variant) *variant = v;
-    if (acc_chunk) *acc_chunk = !f16acc ? 0 : v >= narrow_id() ? 16 : miw::tiled_f16acc_chunk();
+    if (acc_chunk) *acc_chunk = !f16acc ? 0 : untiled(v) ? 16 : miw::tiled_f16acc_chunk();
     return 0;
 }
 
@@ -1088,7 +1102,7 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
 int run_splitk(const miw_gemm_desc *d, splitk_plan &plan, void *ws, hipStream_t s)
 {
     if (plan.splits == 1) {
-        if (plan.variant < narrow_id() && !tiled_fits(plan.variant - 1, plan.full, d->c_type, d->d_type, false, 0, c_shares_d(d, plan.full)))
+        if (!untiled(plan.variant) && !tiled_fits(plan.variant - 1, plan.full, d->c_type, d->d_type, false, 0, c_shares_d(d, plan.full)))
             return fail(MIW_ERR_MISALIGNED, "gemm_splitk: operands must be 16-byte aligned");
         return launch_gemm(plan.variant, plan.kw, plan.full, d->c_type, d->d_type, false, s);
     }

@@ -332,6 +332,50 @@ const void *kwave_kernel(int bi, int bj, bool xk, bool yk, int *lds_bytes)
 
 static bool multiple16(const void *x) { return ((uintptr_t)x & 15) == 0; }
 
+constexpr kwave_tile kwave_tiles[] = {{32, 16}, {16, 32}, {32, 32}, {64, 32}, {32, 64}};
+
+// Operands' layouts in canonical form.
+static void layouts(const gemm_params &g, bool *xk, bool *yk)
+{
+    *xk = g.d_row ? g.b_row == 0 : g.a_row != 0;
+    *yk = g.d_row ? g.a_row != 0 : g.b_row == 0;
+}
+
+// What the 16-byte loads and the 8- and 16-byte stores assume, and 32-bit offsets inside a slot.
+static bool kwave_runs(const gemm_params &g, int c_type, int d_type)
+{
+    const long cper = c_type == 0 ? 8 : 4, dper = d_type == 0 ? 8 : 4;
+    if (g.K < 2 * KGRAN || g.K > (1l << 30) || g.M > (1l << 30) || g.N > (1l << 30)) return false;
+    if (!multiple16(g.A) || !multiple16(g.B) || !multiple16(g.D) || g.lda % 8 || g.ldb % 8 || g.sa % 8 || g.sb % 8) return false;
+    if (g.ldd % dper || g.sd % dper || (g.use_c && (!multiple16(g.C) || g.ldc % cper || g.sc % cper))) return false;
+    return g.lda * 256 < (1l << 31) && g.ldb * 256 < (1l << 31);
+}
+
+// Workgroups on a tile, 0 where the kernel does not run the problem on it.
+static long kwave_groups(const gemm_params &g, kwave_tile t, bool in_place)
+{
+    const long I = g.d_row ? g.N : g.M, J = g.d_row ? g.M : g.N;
+    bool xk, yk;
+    layouts(g, &xk, &yk);
+    int lds;
+    if (I < t.bi || J < t.bj || !kwave_kernel(t.bi, t.bj, xk, yk, &lds)) return 0;
+    if (in_place && (I % t.bi || J % t.bj)) return 0;  // (edge tiles overlap their neighbours)
+    return (I + t.bi - 1) / t.bi * ((J + t.bj - 1) / t.bj) * g.batch;
+}
+
+kwave_tile kwave_fits(const gemm_params &g, int c_type, int d_type, bool in_place, int cus)
+{
+    kwave_tile best = {0, 0};
+    if (!kwave_runs(g, c_type, d_type)) return best;
+    for (const kwave_tile t : kwave_tiles) {
+        const long groups = kwave_groups(g, t, in_place);
+        if (groups == 0 || groups / g.batch * 64 * KWAVES >= (1l << 32)) continue;
+        best = t;
+        if (groups <= cus) break;
+    }
+    return best;
+}
+
 // The smallest of the kernel's tiles that covers D in one round over the CUs: the fewer bytes a CU has to fetch the
 // shorter the launch, and a second round costs more than any tile saves (1.3 to 1.7 times the time of the 64x64 tile).
 // Measured over 489 problems of 16 to 1280 x 64 to 8192 x 128 to 8192, against the kernels that ran them before:
@@ -348,17 +392,11 @@ static bool multiple16(const void *x) { return ((uintptr_t)x & 15) == 0; }
 kwave_tile kwave_pays(const gemm_params &g, int c_type, int d_type, bool in_place, int cus)
 {
     constexpr kwave_tile none = {0, 0};
-    const long I = g.d_row ? g.N : g.M, J = g.d_row ? g.M : g.N;
-    const bool xk = g.d_row ? g.b_row == 0 : g.a_row != 0, yk = g.d_row ? g.a_row != 0 : g.b_row == 0;
-    // What the 16-byte loads and the 8- and 16-byte stores assume, and 32-bit offsets inside a slot.
-    const long cper = c_type == 0 ? 8 : 4, dper = d_type == 0 ? 8 : 4;
-    if (g.K < 2 * KGRAN || g.K > (1l << 30) || I > (1l << 30) || J > (1l << 30)) return none;
-    if (!multiple16(g.A) || !multiple16(g.B) || !multiple16(g.D) || g.lda % 8 || g.ldb % 8 || g.sa % 8 || g.sb % 8) return none;
-    if (g.ldd % dper || g.sd % dper || (g.use_c && (!multiple16(g.C) || g.ldc % cper || g.sc % cper))) return none;
-    if (g.lda * 256 >= (1l << 31) || g.ldb * 256 >= (1l << 31)) return none;
-
+    if (!kwave_runs(g, c_type, d_type)) return none;
+    bool xk, yk;
+    layouts(g, &xk, &yk);
     const bool both = xk && yk;
-    const long wide = std::max(I, J), thin = std::min(I, J);
+    const long wide = std::max(g.M, g.N), thin = std::min(g.M, g.N);
     if (thin < 64) {
         if (both && (g.lda % 64 || g.ldb % 64)) return none;
         const bool rounds = wide / 16 * g.batch > cus;
@@ -366,12 +404,9 @@ kwave_tile kwave_pays(const gemm_params &g, int c_type, int d_type, bool in_plac
     } else if (skinny_beats_tiles(g, d_type, false) && g.K < 768) {
         return none;
     }
-    constexpr kwave_tile tiles[] = {{32, 16}, {16, 32}, {32, 32}, {64, 32}, {32, 64}};
-    for (const kwave_tile t : tiles) {
-        int lds;
-        if (I < t.bi || J < t.bj || !kwave_kernel(t.bi, t.bj, xk, yk, &lds)) continue;
-        if (in_place && (I % t.bi || J % t.bj)) continue;  // (edge tiles overlap their neighbours)
-        if ((I + t.bi - 1) / t.bi * ((J + t.bj - 1) / t.bj) * g.batch > cus) continue;
+    for (const kwave_tile t : kwave_tiles) {
+        const long groups = kwave_groups(g, t, in_place);
+        if (groups == 0 || groups > cus) continue;
         if (t.bi * t.bj > 32 * 32 && (g.K < (both ? 512 : 768) || (thin >= 64 && skinny_beats_tiles(g, d_type, false)))) continue;
         return t;
     }

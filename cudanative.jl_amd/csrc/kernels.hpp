@@ -54,6 +54,8 @@ inline bool fragops_run_skinny(const gemm_params &p, int d_type, bool f16acc)
 struct kwave_tile {
     int bi, bj;  // along D's contiguous dimension and the other; 0: the kernel does not run the problem, or not faster
 };
+// The smallest tile on which the kernel runs the problem in one round over the CUs, else the largest on which it runs it.
+kwave_tile kwave_fits(const gemm_params &p, int c_type, int d_type, bool in_place, int cus);
 // The tile with which the kernel is the fastest one for the problem.  in_place: C and D share memory.
 kwave_tile kwave_pays(const gemm_params &p, int c_type, int d_type, bool in_place, int cus);
 double kwave_estimate_us(const gemm_params &p, int c_type, int d_type, kwave_tile t);

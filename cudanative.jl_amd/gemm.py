@@ -120,13 +120,13 @@ def pick_variant(desc):
 
 
 def plan(desc, in_place=False):
-    """The launches gemm() makes for this descriptor: a list of dicts (variant id, first row, column and
-    k-value, sizes).  One entry unless the sizes are ragged and cutting the problem up is estimated faster."""
+    """The launches gemm() makes for this descriptor: a list of dicts (variant id as pick_variant answers, id of the
+    kernel that runs, first row, column and k-value, sizes).  One entry unless the sizes are ragged and cutting the problem up is estimated faster."""
     lib = _lib.load()
     n = ctypes.c_int()
     parts = (_lib.GemmPart * 64)()
     _lib.check(lib.miw_gemm_plan(ctypes.byref(desc), int(bool(in_place)), parts, 64, ctypes.byref(n)))
-    return [{"variant": q.variant, "m0": q.m0, "n0": q.n0, "k0": q.k0, "m": q.m, "n": q.n, "k": q.k}
+    return [{"variant": q.variant, "kernel": q.kernel, "m0": q.m0, "n0": q.n0, "k0": q.k0, "m": q.m, "n": q.n, "k": q.k}
             for q in parts[:min(n.value, 64)]]
 
 
@@ -137,9 +137,9 @@ def acc_chunk(desc):
 
 
 def resolve(A, B, C, D, desc):
-    """(variant, acc_chunk) of the launch gemm(A, B, C, D, desc) makes first: the same checks and plan on
-    the real operand addresses (alignment, C sharing memory with D), without a launch.  acc_chunk is 0
-    with Float32 accumulation."""
+    """(variant, acc_chunk) of the launch gemm(A, B, C, D, desc) makes first, the variant being the id whose
+    kernel runs: the same checks and plan on the real operand addresses (alignment, C sharing memory with
+    D), without a launch.  acc_chunk is 0 with Float32 accumulation."""
     v, chunk = ctypes.c_int(), ctypes.c_int()
     _lib.check(_lib.load().miw_gemm_resolve(ctypes.byref(desc), _ptr(A), _ptr(B), _ptr(C), _ptr(D), ctypes.byref(v),
                                             ctypes.byref(chunk)))

@@ -645,7 +645,7 @@ end
 
 struct GemmPart
     variant::Cint
-    reserved::Cint
+    kernel::Cint
     m0::Int64; n0::Int64; k0::Int64
     m::Int64; n::Int64; k::Int64
 end

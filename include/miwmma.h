@@ -200,13 +200,16 @@ typedef struct miw_gemm_variant_info {
     int waves_m, waves_n;
     int stages;
     int lds_bytes;
-    int fragment_ops;   /* 1: operands go from global memory to registers, not through LDS tiles; runs every
+    int fragment_ops;   /* 1: operands go to registers without LDS tiles that the workgroup shares; runs every
                            problem.  "fragment_ops": one wavefront per 16x16 tile built from load_a/load_b/mma, or
                            the kernel that serves the problem faster (K of at most 64; few tiles and a long K; less
                            than 64 rows or columns with k contiguous in both operands).  "narrow_k_contiguous":
                            at most 128 rows or columns, k contiguous in both operands, 16-byte aligned; what it
-                           cannot run goes to fragment_ops' kernels.  stages and lds_bytes are the operand ring's:
-                           0 here, although partial sums of wavefronts that share K go through up to 64 KiB of LDS */
+                           cannot run goes to fragment_ops' kernels.  "shared_k": tiles of at most 64 x 32 (the
+                           smallest that the CUs take in one round; the block is the middle one), K shared by four
+                           wavefronts, each with a ring of its own, K of at least 128, 16-byte aligned, Float32
+                           accumulation; what it cannot run goes to fragment_ops' kernels.  stages and lds_bytes are
+                           the operand ring's: 0 for the other two, although partial sums of wavefronts that share K go through up to 64 KiB of LDS */
     int f16_accumulate; /* 1: has a Float16-accumulate form (accumulators fit in ordinary VGPRs) */
     int pingpong;       /* 1: the two wavefronts of a SIMD alternate between matrix-core and memory phases;
                            2: one wavefront per SIMD with a 128x128 sub-tile issues its memory instructions
@@ -221,12 +224,12 @@ int miw_gemm_variant_supports(const miw_gemm_desc *desc, int variant, int *suppo
 /* Variant of a single launch of this descriptor (what miw_gemm runs unless miw_gemm_plan
    cuts the problem up): the one with the shortest estimated duration
    (rounds of workgroups over the CUs, C and D traffic, and the K loop at each kernel's measured
-   pace per 64 k-values) among those that can run it.  With batch 1, Float32 accumulation and
-   desc.variant 0, a problem that tiles of at most 64 x 32 cover in one round over the CUs may run
-   on a kernel without an id, whose wavefronts share K: tile64x64_w2x2's stands for it, where the
-   pitches are no whole cache lines narrow_k_contiguous', and fragment_ops' below 64 rows or
-   columns.  An id asked for in desc.variant runs its own kernel, which differs from that one by
-   the order of the Float32 additions. */
+   pace per 64 k-values) among those that can run it.  Where "shared_k" then takes its place (with
+   batch 1, Float32 accumulation and desc.variant 0, for problems that its tiles cover in one round
+   over the CUs), miw_gemm_part.kernel and miw_gemm_resolve say so, this query does not: it answers
+   tile64x64_w2x2, narrow_k_contiguous where the pitches are no whole cache lines, or fragment_ops
+   below 64 rows or columns.  An id asked for in desc.variant runs its own kernel; those three
+   differ from shared_k by the order of the Float32 additions. */
 int miw_gemm_pick_variant(const miw_gemm_desc *desc, int *variant);
 /* The launches miw_gemm makes for this descriptor (no counterpart in the reference, whose GEMM
    would be the caller's own kernel over docs/src/device/wmma.md:51-52).  The LDS-tiled kernels take any M and N of
@@ -245,8 +248,8 @@ int miw_gemm_pick_variant(const miw_gemm_desc *desc, int *variant);
        large tiles, which would take two rounds over the CUs).
    Writes min(*count, capacity) parts; *count is the number of launches. */
 typedef struct miw_gemm_part {
-    int variant;          /* as in miw_gemm_desc.variant */
-    int reserved;
+    int variant;          /* as miw_gemm_pick_variant answers for the part */
+    int kernel;           /* the id whose kernel runs it: asked for in desc.variant, a single part runs the same again */
     int64_t m0, n0, k0;   /* first row, column and k-value of the part in the caller's problem */
     int64_t m, n, k;      /* its sizes */
 } miw_gemm_part;
@@ -257,7 +260,8 @@ int miw_gemm_plan(const miw_gemm_desc *desc, int in_place, miw_gemm_part *parts,
    miw_gemm to another kernel with another acc_chunk: miw_gemm_resolve answers for the real ones. */
 int miw_gemm_acc_chunk(const miw_gemm_desc *desc, int *acc_chunk);
 /* What miw_gemm(desc, A, B, C, D, ...) will run, from the same checks and plan but without a
-   launch: *variant = the variant of its first launch, *acc_chunk = the k-values between two
+   launch: *variant = the id whose kernel its first launch runs (asked for in desc.variant, a call of one
+   launch runs the same again, bit for bit), *acc_chunk = the k-values between two
    roundings of the Float16 running sum (0 with Float32 accumulation).  Either output may be null.
    No counterpart in the reference (its mma chain always rounds once per 16 x 16 x 16 tile). */
 int miw_gemm_resolve(const miw_gemm_desc *desc, const void *A, const void *B, const void *C, const void *D,

@@ -831,6 +831,37 @@ def test_kernel_whose_wavefronts_share_k(gpu, orc, shared_k_tile, tile, al, bl, 
         assert np.array_equal(D, orc.gemm(g, A, B, C)), (tile, al, bl, dl, K, form)
 
 
+@pytest.mark.parametrize("al,bl,dl", itertools.product((0, 1), repeat=3))
+def test_shared_k_kernel_by_its_id(gpu, orc, shared_k_tile, al, bl, dl):
+    """What resolve answers, asked for, runs the same bits; so do the members of a batch and problems of several rounds over
+    the CUs, whose tiles are larger; C in D's place; and what the kernel cannot run (K of one slot, operands off 16 bytes)
+    runs as the fragment-op id does."""
+    vid, frag = _vid(gpu, "shared_k"), _vid(gpu, "fragment_ops")
+    for M, N, K, batch in ((80, 112, 784, 1), (80, 112, 784, 3), (1040, 1072, 272, 2), (2064, 2064, 144, 1)):
+        g = orc.GemmDesc(M=M, N=N, K=K, a_layout=al, b_layout=bl, c_layout=dl, d_layout=dl, batch=batch, alpha=0.5, beta=-2.0)
+        A, B, C = _inputs(orc, g, 50 + M)
+        D = _run(gpu, orc, g, A, B, C, variant=vid)
+        assert orc.normalized_error(g, D, orc.gemm_f64(g, A, B, C)) <= TIGHT_F32, (M, N, K, batch)
+        if M > 80:
+            continue
+        r, g1 = g.resolved(), orc.GemmDesc(**{**g.__dict__, "batch": 1})
+        for bt in range(batch):
+            own = [x[bt * s:(bt + 1) * s] for x, s in ((A, r.stride_a), (B, r.stride_b), (C, r.stride_c))]
+            assert shared_k_tile(M, N, K, a_row=int(al == orc.ROW), b_row=int(bl == orc.ROW), c_row=int(dl == orc.ROW), d_row=int(dl == orc.ROW), use_c=1, d_type=1)
+            assert np.array_equal(D[bt * r.stride_d:(bt + 1) * r.stride_d].view(np.uint32), _run(gpu, orc, g1, *own).view(np.uint32)), bt
+    g = orc.GemmDesc(M=96, N=128, K=256, a_layout=al, b_layout=bl, c_layout=dl, d_layout=dl, beta=0.5)
+    A, B, C = _inputs(orc, g, 51)
+    desc = gpu.GEMM.make_desc(96, 128, 256, a_layout=_W(gpu, al), b_layout=_W(gpu, bl), c_layout=_W(gpu, dl), d_layout=_W(gpu, dl), beta=0.5, variant=vid)
+    dA, dB, dD = gpu.DeviceArray(A), gpu.DeviceArray(B), gpu.DeviceArray(C)
+    gpu.GEMM.gemm(dA, dB, dD, dD, desc)
+    gpu.synchronize()
+    assert np.array_equal(dD.to_host().view(np.uint32), _run(gpu, orc, g, A, B, C, variant=vid).view(np.uint32))
+    for K, pad in ((96, 0), (256, 4)):
+        g = orc.GemmDesc(M=96, N=112, K=K, a_layout=al, b_layout=bl, c_layout=dl, d_layout=dl, lda=256 + pad, ldb=256 + pad)
+        A, B, C = _inputs(orc, g, 52 + K)
+        assert np.array_equal(_run(gpu, orc, g, A, B, C, variant=vid).view(np.uint32), _run(gpu, orc, g, A, B, C, variant=frag).view(np.uint32)), (K, pad)
+
+
 def test_tiles_of_a_batch_in_one_run(gpu, orc):
     """Several tiles per batch member: the XCDs' runs go over the whole batch; counts that 8 does not divide, partial raster groups."""
     for v, (M, N, batch) in itertools.product(("tile64x64_w2x2", "tile128x128_w2x2", "tile128x128_pingpong"), ((192, 320, 5), (400, 208, 3), (144, 1040, 2))):

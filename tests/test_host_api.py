@@ -352,12 +352,39 @@ def test_shared_k_kernel_runs_where_it_was_measured_ahead(miw, shared_k_tile):
             # slices of K, and fewer CUs
             ((32, 32), 128, 128, 1024, dict(a_row=0, b_row=1, batch=16)), (None, 128, 128, 1024, dict(a_row=0, b_row=1, batch=33)), ((32, 32), 512, 256, 128, dict(cus=128))):
         assert shared_k_tile(M, N, K, **kw) == want, (M, N, K, kw)
-    # it has no id: the smallest tile's stands for it, the fragment-op one below 64 rows or columns, and a batch never takes it
+    # pick_variant answers for what it takes the place of: the smallest tile, or the fragment-op kernels below 64 rows or columns
     G, W = miw.GEMM, miw.WMMA
     rc = dict(a_layout=W.RowMajor, b_layout=W.ColMajor, d_layout=W.RowMajor, d_type=np.float16, use_c=False)
     by = {v["name"]: v["id"] for v in G.variants()}
     assert G.pick_variant(G.make_desc(128, 4096, 4096, **rc)) == by["tile64x64_w2x2"]
     assert G.pick_variant(G.make_desc(48, 4096, 4096, **rc)) == by["fragment_ops"]
+
+
+def test_plan_and_resolve_name_the_kernel_that_runs(miw):
+    """The id of the kernel whose wavefronts share K: in plan's `kernel` and resolve's answer wherever the rule takes it, alone
+    or as a strip; a forced id resolves to itself, and a batch never takes this one unasked."""
+    G, W = miw.GEMM, miw.WMMA
+    vs = G.variants()
+    by = {v["name"]: v["id"] for v in vs}
+    at = tuple((1 << 32) + (i << 40) for i in range(4))
+    rc = dict(a_layout=W.RowMajor, b_layout=W.ColMajor, d_layout=W.RowMajor, d_type=np.float16, use_c=False)
+    assert vs[by["shared_k"] - 1]["fragment_ops"] and vs[by["shared_k"] - 1]["lds_bytes"] == 160 * 1024
+    for m, n, k, stands_for in ((128, 4096, 4096, "tile64x64_w2x2"), (48, 4096, 4096, "fragment_ops"), (64, 4096, 3088, "narrow_k_contiguous")):
+        d = G.make_desc(m, n, k, **rc)
+        (part,) = G.plan(d)
+        assert part["variant"] == G.pick_variant(d) == by[stands_for]
+        assert part["kernel"] == G.resolve(at[0], at[1], None, at[3], d)[0] == by["shared_k"]
+        for v in vs:
+            d = G.make_desc(m, n, k, variant=v["id"], **rc)
+            if G.variant_supports(d, v["id"]):
+                assert [(q["variant"], q["kernel"]) for q in G.plan(d)] == [(v["id"], v["id"])] and G.resolve(at[0], at[1], None, at[3], d)[0] == v["id"]
+        d = G.make_desc(m, n, k, batch=2, **rc)
+        assert all(q["kernel"] == q["variant"] != by["shared_k"] for q in G.plan(d))
+    body, strip = G.plan(G.make_desc(4144, 4096, 4096, **dict(rc, b_layout=W.RowMajor)))
+    assert body["kernel"] == body["variant"] and strip["kernel"] == by["shared_k"] != strip["variant"]
+    # Float16 accumulation is not its: the fragment-op kernels run the forced id, rounding every 16 k-values
+    d = G.make_desc(256, 256, 256, c_type=np.float16, d_type=np.float16, acc_type=np.float16, variant=by["shared_k"])
+    assert G.resolve(*at, d) == (by["shared_k"], 16) and G.acc_chunk(d) == 16
 
 
 def test_fragment_signature_tables_agree_with_the_checks(miw):
