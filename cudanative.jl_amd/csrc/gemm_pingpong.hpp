@@ -626,7 +626,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
     MIW_PP_STAMP(6)
     ts[7] = wall_clock64();
     if (p.ts && lane == 0)
-        for (int i = 0; i < 10; i++) p.ts[((long)(tile + (long)blockIdx.y * gridDim.x) * 8 + wave) * 10 + i] = ts[i];
+        for (int i = 0; i < 10; i++) p.ts[(launch_tile(tile, p.span, blockIdx.y, gridDim.x) * 8 + wave) * 10 + i] = ts[i];
     ts[0] = clock64();
     ts[8] = wall_clock64();
 #endif

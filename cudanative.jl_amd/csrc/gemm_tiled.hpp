@@ -191,6 +191,13 @@ __device__ inline tile_place workgroup_tile(const tiled_params &p, int bi, int b
     return tile_at(p, (int)(blockIdx.x + blockIdx.y * (unsigned)p.span), (int)blockIdx.y, bi, bj);
 }
 
+// Number of a tile over the whole launch, from its number as tile_at takes it (which counts on over the members where there is
+// a span): measurement builds write their records there.
+__host__ __device__ inline long launch_tile(int id, int span, unsigned member, unsigned member_tiles)
+{
+    return span ? id : id + (long)member * member_tiles;
+}
+
 // Arguments into scalar registers, at the start of the kernel or behind the first requests.  Left to itself the compiler
 // puts the loads of some off to where they are first used, behind the K loop or right in front of the first operand load,
 // where each waits for memory (0.15 us of a launch); waiting at the start for C's and D's too costs 0.05.
