@@ -490,7 +490,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
     constexpr std::true_type any{};     // the cluster's requests may reach the last pair
     constexpr std::false_type plain{};
 
-    for (bool later = false;; later = true) {  // tiles of this workgroup
+    for (bool later = false;;) {  // tiles of this workgroup
     // Does another tile follow (then NP >= 4, see tiled_params::work), and how do the operands get there?
     auto first_args = arguments();
     has_next = tile + (int)gridDim.x < first_args->work;
@@ -573,8 +573,10 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
         if constexpr (__is_same(DT, float)) __builtin_nontemporal_store(v, (float4_t *)to);
         else *(half4_t *)to = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
     };
-    // C_AT 0: no C, 1: laid out as D, 2: the other way round
-    auto epilogue = [&]<int C_AT, bool STREAM>(std::integral_constant<int, C_AT>, std::bool_constant<STREAM>) MIW_INLINE {
+    // C_AT 0: no C, 1: laid out as D, 2: the other way round; EDGE: see own_from
+    auto epilogue = [&]<int C_AT, bool STREAM, bool EDGE = false>(std::integral_constant<int, C_AT>, std::bool_constant<STREAM>,
+                                                                  std::bool_constant<EDGE> = {}) MIW_INLINE {
+        const int row = i0 + wi * WTI + 16 * odd, first_row = own_from<BI>(i0), col = j0 + wj * WTJ, first_col = own_from<BJ>(j0);
         const CT *C = nullptr;
         if constexpr (C_AT == 1) C = (const CT *)args->C + bt * args->sc + (long)(j0 + wj * WTJ) * ldc + (i0 + wi * WTI) + pair_place(lane, ldc);
         // (columns r - odd and the next, rows 16 odd + 4 q ..)
@@ -589,7 +591,8 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
 #pragma unroll
                     for (int e = 0; e < 4; e++) v[t][e] *= alpha;
                 if constexpr (C_AT == 0) {
-                    store_pair_at<STREAM>(D + 16 * b * ldd + 16 * a, ldd, odd, v[0], v[1]);
+                    store_pair_at<STREAM>(D + 16 * b * ldd + 16 * a, ldd, odd, v[0], v[1],
+                                          !EDGE || (row + 16 * a >= first_row && col + 16 * b >= first_col));
                 } else {
                     pair_exchange(odd, v[0], v[1]);
 #pragma unroll
@@ -615,7 +618,9 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
     // A Float32 D is written past the L2 where C or the operands of more tiles come through it at the same time
     // (4096x4096x512 with C from HBM: 34 us, 42 through the L2; 8192x8192x1024 without C 126 and 134), and through it
     // where nothing follows in the launch (4096x4096x512 without C: 26 us, 28 past it).
-    if (FOLD) epilogue(std::integral_constant<int, 0>{}, std::true_type{});
+    const bool edge = FOLD && (i0 % BI || j0 % BJ);
+    if (edge) epilogue(std::integral_constant<int, 0>{}, std::true_type{}, std::true_type{});
+    else if (FOLD) epilogue(std::integral_constant<int, 0>{}, std::true_type{});
     else if (args->use_c && args->c_trans) epilogue(std::integral_constant<int, 2>{}, std::true_type{});
     else if (args->use_c) epilogue(std::integral_constant<int, 1>{}, std::true_type{});
     else if (args->work) epilogue(std::integral_constant<int, 0>{}, std::true_type{});
@@ -631,6 +636,7 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
     ts[8] = wall_clock64();
 #endif
     if (!has_next) break;
+    later = !edge;  // (a tile at the edge may have stored less)
     tile += (int)gridDim.x;
     at = tile_at(*arguments(), tile, 0, BI, BJ);
     }
@@ -1180,7 +1186,7 @@ void k_gemm_pp64(tiled_params p)
 
     // Epilogue: each lane owns 4 consecutive i of one column j per MFMA tile.
     static_assert(TI % 2 == 0, "the epilogue stores pairs of tiles");
-    auto epilogue = [&](bool with_c, bool trans) {
+    auto epilogue = [&]<bool EDGE = false>(bool with_c, bool trans, std::bool_constant<EDGE> = {}) {
         auto value = [&](int a, int b) {
             float4_t v = separate_sum ? cinit[a][b] : acc[a][b];
             if constexpr (!F16ACC) {
@@ -1198,9 +1204,11 @@ void k_gemm_pp64(tiled_params p)
         for (int b = 0; b < TJ; b++)
 #pragma unroll
             for (int a = 0; a < TI; a += 2)
-                store_tile_pair<DT>(D, p.ldd, i0 + wi * WTI + 16 * a, j0 + wj * WTJ + 16 * b, lane, value(a, b), value(a + 1, b));
+                store_tile_pair<DT>(D, p.ldd, i0 + wi * WTI + 16 * a, j0 + wj * WTJ + 16 * b, lane, value(a, b), value(a + 1, b),
+                                    !EDGE || (i0 + wi * WTI + 16 * a + 16 * (lane & 1) >= own_from<BI>(i0) && j0 + wj * WTJ + 16 * b >= own_from<BJ>(j0)));
     };
-    if (F16ACC || !p.use_c || fold_c) epilogue(false, false);
+    if (CAN_FOLD && fold_c && (i0 % BI || j0 % BJ)) epilogue(false, false, std::true_type{});
+    else if (F16ACC || !p.use_c || fold_c) epilogue(false, false);
     else if (p.c_trans) epilogue(true, true);
     else epilogue(true, false);
 #ifdef MIW_PP_TS

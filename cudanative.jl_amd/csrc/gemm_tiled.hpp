@@ -75,8 +75,9 @@ struct tiled_params {
     const half_t *Y;
     // tiles_i = ceil(I / BI), tiles_j = ceil(J / BJ).  Where the tile does not divide an extent the
     // last tile starts at I - BI (J - BJ) and overlaps its neighbour: both workgroups compute the
-    // overlap from the same operands in the same order and store equal values.  The host allows
-    // this only when C and D do not share memory.
+    // overlap from the same operands in the same order and store equal values, or, where C is folded
+    // into the K loop, only the neighbour stores it (own_from).  The host allows this only when C and
+    // D do not share memory.
     int tiles_i, tiles_j, group_i;
     // What workgroup_tile divides by, as multipliers (see quotient); shifts: one byte for each.
     int span;                                  // tiles of a batch member where the XCDs' runs go over the whole batch, else 0
@@ -353,12 +354,14 @@ __device__ inline void pair_exchange(bool odd, float4_t &v0, float4_t &v1)
     v0 = __builtin_bit_cast(float4_t, s0);
     v1 = __builtin_bit_cast(float4_t, s1);
 }
-// STREAM: write past the L2 (Float32 only: half lines, as Float16 pairs write them, are better gathered there).
+// STREAM: write past the L2 (Float32 only: half lines, as Float16 pairs write them, are better gathered there).  mine: this
+// lane's rows are written.
 template <bool STREAM = false, class DT>
-__device__ inline void store_pair_at(DT *even, long ldd, bool odd, float4_t v0, float4_t v1)
+__device__ inline void store_pair_at(DT *even, long ldd, bool odd, float4_t v0, float4_t v1, bool mine = true)
 {
     if constexpr (__is_same(DT, float)) {
         pair_exchange(odd, v0, v1);
+        if (!mine) return;
         if constexpr (STREAM) {
             __builtin_nontemporal_store(v0, (float4_t *)even);
             __builtin_nontemporal_store(v1, (float4_t *)(even + ldd));
@@ -377,6 +380,7 @@ __device__ inline void store_pair_at(DT *even, long ldd, bool odd, float4_t v0, 
             s0[e] = odd ? ts : p[e];
             s1[e] = odd ? t[e] : ps;
         }
+        if (!mine) return;
         *(uint2_t *)even = s0;
         *(uint2_t *)(even + ldd) = s1;
     }
@@ -388,12 +392,21 @@ __device__ inline long pair_place(int lane, long ldd)
     const int r = lane & 15, q = lane >> 4, odd = r & 1;
     return (long)(r - odd) * ldd + 16 * odd + 4 * q;
 }
+// A tile that folds C and is shifted back to end at the edge writes only what its neighbour does not: C joins the sums of
+// what they share at another k-step in each, and the last bits differ.  First row (column) that the tile at x0 writes.
+template <int B>
+__device__ inline int own_from(int x0)
+{
+    static_assert((B & (B - 1)) == 0, "tile extents are powers of two");
+    return (x0 + B - 1) & ~(B - 1);
+}
+
 template <class DT>
-__device__ inline void store_tile_pair(DT *D, long ldd, int row, int col0, int lane, float4_t v0, float4_t v1)
+__device__ inline void store_tile_pair(DT *D, long ldd, int row, int col0, int lane, float4_t v0, float4_t v1, bool mine = true)
 {
     const int r = lane & 15, q = lane >> 4;
     const bool odd = r & 1;
-    store_pair_at(D + (long)(col0 + r - (odd ? 1 : 0)) * ldd + (row + (odd ? 16 : 0) + 4 * q), ldd, odd, v0, v1);
+    store_pair_at(D + (long)(col0 + r - (odd ? 1 : 0)) * ldd + (row + (odd ? 16 : 0) + 4 * q), ldd, odd, v0, v1, mine);
 }
 
 // Ordinal of the direct-to-LDS load issued after MFMA m of a step of nmfma
@@ -766,7 +779,7 @@ void k_gemm_tiled(tiled_params p)
 
     // Epilogue: each lane owns 4 consecutive i of one column j per MFMA tile.
     static_assert(TI % 2 == 0, "the epilogue stores pairs of tiles");
-    auto epilogue = [&](bool with_c, bool trans) {
+    auto epilogue = [&]<bool EDGE = false>(bool with_c, bool trans, std::bool_constant<EDGE> = {}) {
         auto value = [&](int a, int b) {
             float4_t v = acc[a][b];
             if constexpr (!F16ACC) {
@@ -784,9 +797,11 @@ void k_gemm_tiled(tiled_params p)
         for (int b = 0; b < TJ; b++)
 #pragma unroll
             for (int a = 0; a < TI; a += 2)
-                store_tile_pair<DT>(D, p.ldd, i0 + wi * WTI + 16 * a, j0 + wj * WTJ + 16 * b, lane, value(a, b), value(a + 1, b));
+                store_tile_pair<DT>(D, p.ldd, i0 + wi * WTI + 16 * a, j0 + wj * WTJ + 16 * b, lane, value(a, b), value(a + 1, b),
+                                    !EDGE || (i0 + wi * WTI + 16 * a + 16 * (lane & 1) >= own_from<BI>(i0) && j0 + wj * WTJ + 16 * b >= own_from<BJ>(j0)));
     };
-    if (F16ACC || !p.use_c || fold_c) epilogue(false, false);
+    if (CAN_FOLD && fold_c && (i0 % BI || j0 % BJ)) epilogue(false, false, std::true_type{});
+    else if (F16ACC || !p.use_c || fold_c) epilogue(false, false);
     else if (p.c_trans) epilogue(true, true);
     else epilogue(true, false);
 }

@@ -236,7 +236,7 @@ int miw_gemm_pick_variant(const miw_gemm_desc *desc, int *variant);
    at least one tile and any K of at least 64 (multiples of 16, as everywhere).  Where the tile does
    not divide an extent the last tile is shifted back so that it ends at the edge and overlaps its
    neighbour; both workgroups compute the overlap from the same operands in the same order and
-   store equal values.  When C and D share memory (in_place != 0 here; miw_gemm looks at the
+   store equal values, or only one of them stores it: a launch gives the same bits every time.  When C and D share memory (in_place != 0 here; miw_gemm looks at the
    pointers) that is not allowed and only whole tiles are used.  Where 64 does not divide K the
    last slot of 64 k-values is shifted back so that it ends at K, and the k-values it repeats are
    zeroed in the fragments: K is never cut, and with Float16 accumulation the last rounding follows

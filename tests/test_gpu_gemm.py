@@ -253,6 +253,33 @@ def test_c_folded_into_the_loop_matches_the_epilogue_path(gpu, orc):
     assert orc.normalized_error(g4, _run(gpu, orc, g4, A, B, C, variant=fold), orc.gemm_f64(g4, A, B, C)) <= TIGHT_F32
 
 
+@pytest.mark.parametrize("al,bl,dl", itertools.product((0, 1), repeat=3))
+def test_folded_c_where_edge_tiles_overlap(gpu, orc, al, bl, dl):
+    """C folded into the loop and extents that the tile does not divide: exact on integers with D's padding untouched, and on
+    random inputs the same bits every time (what two tiles share is stored by one of them).  More tiles than CUs for the
+    256x256 ping-pong tile: workgroups walk from edge tiles to whole ones and back."""
+    folding = [v for v in _variants(gpu) if v["waves"][0] * v["waves"][1] == 8 and (v["stages"] <= 3 or v["pingpong"])]
+    for v in folding:
+        bm, bn = v["block"][:2]
+        bi, bj = (bm + 16, 2 * bn + 48) if dl == orc.COL else (2 * bn + 48, bm + 16)      # (bm tiles D's contiguous dimension)
+        walks = v["name"] == "tile256x256_pingpong"
+        kw = dict(M=bi, N=bj, K=1104, a_layout=al, b_layout=bl, c_layout=dl, d_layout=dl, beta=-2.0)
+        g = orc.GemmDesc(ldd=(bj if dl == orc.ROW else bi) + 8, batch=50 if walks else 1, **kw)
+        A, B, C = _inputs(orc, g, 1800 + v["id"], ints=True)
+        D = _run(gpu, orc, g, A, B, C, variant=v["id"], prefill=7.0)
+        if D is None:
+            continue
+        want = orc.gemm(g, A, B, C)
+        inner = bj if dl == orc.ROW else bi
+        got, want = (x.reshape(-1, inner + 8) for x in (D, want))
+        assert np.array_equal(got[:, :inner], want[:, :inner]) and np.all(got[:, inner:] == 7.0), (v["name"], al, bl, dl)
+        g = orc.GemmDesc(batch=150 if walks else 20, **kw)
+        A, B, C = _inputs(orc, g, 1900 + v["id"])
+        first = _run(gpu, orc, g, A, B, C, variant=v["id"])
+        for _ in range(3):
+            assert np.array_equal(_run(gpu, orc, g, A, B, C, variant=v["id"]).view(np.uint32), first.view(np.uint32)), (v["name"], al, bl, dl)
+
+
 def test_c_and_d_may_be_one_buffer(gpu, orc):
     """In place: D = A*B + beta*D.  Every workgroup reads its tile of C before it stores that tile."""
     for variant, (M, N, K) in ((1, (512, 256, 1600)), (1, (256, 256, 256)), (7, (256, 128, 192)), (0, (48, 80, 64))):
