@@ -179,24 +179,50 @@ def test_c_folded_into_the_loop_exact_on_integers(gpu, orc, al, bl, dl, K):
         assert np.array_equal(D, orc.gemm(g, A, B, C)), (v["name"], al, bl, dl, K)
 
 
+# forms of C and D, and K: from four slots, the shortest that workgroups walk on, over sixteen (C behind the loop) to more than
+# sixteen (alpha 1, C laid out as D: folded behind one, two, three and four plain pairs); whole and ragged last slots
+WALKS = [(256, dict(use_c=0)), (272, dict(use_c=0, d_type=0)), (320, dict(c_type=0, d_type=0)), (976, dict(alpha=-1.0, beta=2.0)),
+         (960, dict(c_type=0)), (1024, dict(alpha=0.5, beta=0.5)), (1040, dict(other_layout=True)), (1024, dict(alpha=-1.0)),
+         (1088, dict(beta=-2.0)), (1104, dict(beta=2.0)), (1168, dict(d_type=0)), (1280, dict(beta=0.5))]
+
+
+@pytest.mark.parametrize("K,form", WALKS)
 @pytest.mark.parametrize("al,bl", itertools.product((0, 1), repeat=2))
-@pytest.mark.parametrize("K", [256, 272, 960, 976, 1024, 1040])
-def test_workgroups_that_walk_several_tiles(gpu, orc, al, bl, K):
-    """More 256x256 tiles than CUs: a workgroup's operand requests run on from one tile into the next.  Four slots
-    of K (the shortest that do), ragged last slots, fifteen (C added behind the loop) and sixteen (added from the
-    first step on); tiles of several batch members and shifted edge tiles; every form of C; bit-exact on integers."""
-    v = _vid(gpu, "tile256x256_pingpong")
-    rng = np.random.default_rng(K + 2 * al + bl)
-    forms = [dict(c_type=orc.F32, alpha=-1.0, beta=2.0), dict(c_type=orc.F32, use_c=0), dict(c_type=orc.F16, alpha=1.0),
-             dict(c_type=orc.F32, alpha=0.5, beta=0.5), dict(c_type=orc.F32, other_layout=True)]
-    for i in rng.permutation(len(forms))[:2]:
-        form = dict(forms[i])
-        dl = int(rng.integers(0, 2))
-        cl = 1 - dl if form.pop("other_layout", False) else dl
-        g = orc.GemmDesc(M=272 if dl else 256, N=256 if dl else 272, K=K, a_layout=al, b_layout=bl, c_layout=cl, d_layout=dl, batch=131, **form)
-        A, B, C = _inputs(orc, g, K + int(i), ints=True)
-        D = _run(gpu, orc, g, A, B, C if g.use_c else None, variant=v)
-        assert np.array_equal(D, orc.gemm(g, A, B, C)), (al, bl, cl, dl, K, form)
+def test_workgroups_that_walk_several_tiles(gpu, orc, al, bl, K, form):
+    """More 256x256 tiles than CUs: a workgroup's operand requests run on from one tile into the next.  Tiles of several
+    batch members and shifted edge tiles; every form of C and D in every canonical layout; bit-exact on integers."""
+    v, form = _vid(gpu, "tile256x256_pingpong"), dict(form)
+    dl = (K // 16 + al) % 2
+    cl = 1 - dl if form.pop("other_layout", False) else dl
+    g = orc.GemmDesc(M=272 if dl else 256, N=256 if dl else 272, K=K, a_layout=al, b_layout=bl, c_layout=cl, d_layout=dl, batch=131, **form)
+    A, B, C = _inputs(orc, g, K, ints=True)
+    D = _run(gpu, orc, g, A, B, C if g.use_c else None, variant=v)
+    assert np.array_equal(D, orc.gemm(g, A, B, C)), (al, bl, cl, dl, K, form)
+
+
+@pytest.mark.parametrize("al,bl,dl", itertools.product((0, 1), repeat=3))
+def test_workgroups_that_walk_three_tiles_and_in_place(gpu, orc, al, bl, dl):
+    """524 tiles of 256x256, so that twelve workgroups take a third one: the bits of launches that give every workgroup one
+    tile, with C behind the loop, folded, and in D's place."""
+    v, batch, part = _vid(gpu, "tile256x256_pingpong"), 262, 128
+    for K, in_place, form in ((272, False, dict(alpha=-1.0)), (1168, False, dict(d_type=0)), (272, True, dict(alpha=-1.0)), (1104, True, dict(beta=0.5))):
+        M, N = (256, 512) if in_place else (272, 256) if dl == orc.COL else (256, 272)
+        g = orc.GemmDesc(M=M, N=N, K=K, a_layout=al, b_layout=bl, c_layout=dl, d_layout=dl, batch=batch, **form)
+        r, lay = g.resolved(), [_W(gpu, x) for x in (al, bl, dl)]
+        A, B, C = (np.resize(x, n * batch) for x, n in zip(_inputs(orc, orc.GemmDesc(M=1040, N=1040, K=1040), 60 + K), (r.stride_a, r.stride_b, r.stride_c)))
+        dA, dB = gpu.DeviceArray(A), gpu.DeviceArray(B)
+        outs = []
+        for count in (batch, part):
+            dC = gpu.DeviceArray(C)
+            dD = dC if in_place else gpu.DeviceArray(np.full(r.stride_d * batch, np.nan, dtype=orc.np_dtype(g.d_type)))
+            for first in range(0, batch, count):
+                desc = gpu.GEMM.make_desc(M, N, K, a_layout=lay[0], b_layout=lay[1], c_layout=lay[2], d_layout=lay[2], c_type=F32, d_type=orc.np_dtype(g.d_type),
+                                          alpha=g.alpha, beta=g.beta, use_c=bool(g.use_c), batch=min(count, batch - first), variant=v)
+                gpu.GEMM.gemm(dA.ptr + 2 * first * r.stride_a, dB.ptr + 2 * first * r.stride_b, dC.ptr + 4 * first * r.stride_c if g.use_c else None,
+                              dD.ptr + dD.dtype.itemsize * first * r.stride_d, desc)
+            gpu.synchronize()
+            outs.append(dD.to_host())
+        assert not np.isnan(outs[0].max()) and np.array_equal(*(x.view(np.uint8 if x.nbytes % 8 else np.uint64) for x in outs)), (al, bl, dl, K, in_place, form)
 
 
 @pytest.mark.parametrize("alpha,K", [(-1.0, 976), (-1.0, 1024), (-1.0, 1168), (1.0, 976), (1.0, 1024)])

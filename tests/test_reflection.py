@@ -35,18 +35,19 @@ def test_fragment_mma_uses_the_16x16x16_matrix_instruction(miw):
 
 
 def test_default_gemm_kernel_codegen_and_resources(miw):
-    name = "k_gemm_pp<256, 256, 2, 4, false, true, float, float>"    # column-major A and B: the benchmark's kernel
-    isa = miw.reflection.code_gcn(name)
-    assert len(isa) == 1
-    ops = _ops(next(iter(isa.values())))
-    assert ops["v_mfma_f32_16x16x32_f16"] >= 64                  # two unrolled clusters of 8 x 4 tiles
-    assert ops["global_load_lds_dwordx4"] >= 8                   # direct-to-LDS operand loads
-    assert ops["ds_read_b64_tr_b16"] >= 16 and ops["ds_read_b128"] >= 4   # transpose reads for A, b128 for B
-    assert not any(o.startswith(("scratch_", "flat_", "ds_write", "v_accvgpr")) for o in ops)
-    res = {k: v for k, v in miw.reflection.kernel_resources().items() if name in k}
-    (r,) = res.values()
-    assert r["spills"] == 0 and r["scratch"] == 0 and r["max_threads"] == 512
-    assert r["vgpr"] + r["agpr"] <= 256                          # two wavefronts per SIMD
+    # column-major A and B: the benchmark's kernel, which folds C, and the one that adds it behind the loop
+    for name in ("k_gemm_pp_fold<256, 256, 2, 4, false, true, float>", "k_gemm_pp<256, 256, 2, 4, false, true, float, float>"):
+        isa = miw.reflection.code_gcn(name)
+        assert len(isa) == 1
+        ops = _ops(next(iter(isa.values())))
+        assert ops["v_mfma_f32_16x16x32_f16"] >= 64                  # two unrolled clusters of 8 x 4 tiles
+        assert ops["global_load_lds_dwordx4"] >= 8                   # direct-to-LDS operand loads
+        assert ops["ds_read_b64_tr_b16"] >= 16 and ops["ds_read_b128"] >= 4   # transpose reads for A, b128 for B
+        assert not any(o.startswith(("scratch_", "flat_", "ds_write", "v_accvgpr")) for o in ops)
+        res = {k: v for k, v in miw.reflection.kernel_resources().items() if name in k}
+        (r,) = res.values()
+        assert r["spills"] == 0 and r["scratch"] == 0 and r["max_threads"] == 512
+        assert r["vgpr"] + r["agpr"] <= 256                          # two wavefronts per SIMD
     # both operands K-major: no transpose read at all
     kk = miw.reflection.code_gcn("k_gemm_pp<256, 256, 2, 4, true, true, float, float>")
     assert "ds_read_b64_tr_b16" not in _ops(next(iter(kk.values())))
@@ -54,9 +55,11 @@ def test_default_gemm_kernel_codegen_and_resources(miw):
 
 def test_auto_picked_4096_kernels_have_no_spills(miw):
     """The kernels miw_gemm picks by itself for a 4096^3 problem, one per operand layout: the 256 x 256
-    ping-pong kernel.  None of them may touch scratch memory, and all fit two wavefronts per SIMD."""
+    ping-pong kernel that folds C, and the one that does not.  None of them may touch scratch memory, and all fit two
+    wavefronts per SIMD."""
     res = miw.reflection.kernel_resources()
-    picked = ["k_gemm_pp<256, 256, 2, 4, %s, float, float>" % l for l in ("true, false", "false, true", "false, false", "true, true")]
+    picked = [k % l for l in ("true, false", "false, true", "false, false", "true, true")
+              for k in ("k_gemm_pp_fold<256, 256, 2, 4, %s, float>", "k_gemm_pp<256, 256, 2, 4, %s, float, float>")]
     for name in picked:
         (r,) = [v for k, v in res.items() if name in k]
         assert r["spills"] == 0 and r["scratch"] == 0 and r["vgpr"] + r["agpr"] <= 256 and r["max_threads"] == 512, name
@@ -66,9 +69,20 @@ def test_auto_picked_4096_kernels_have_no_spills(miw):
             assert r["spills"] == 0 and r["scratch"] == 0, k
 
 
+def test_walking_kernels_store_a_tile_in_32_instructions(miw):
+    """The waits behind a tile leave 32 stores in flight (NSTORE), so that many vector stores stand in every epilogue: of a whole
+    tile and of one at the edge where C is folded, and of four forms of C and D otherwise."""
+    for pattern, paths, count in (("k_gemm_pp_fold<", 2, 8), ("k_gemm_pp<", 4, 16)):
+        isa = miw.reflection.code_gcn(pattern)
+        assert len(isa) == count
+        for k, text in isa.items():
+            stores = {o: n for o, n in _ops(text).items() if "store" in o}
+            assert sum(stores.values()) == 32 * paths and set(stores) <= {"global_store_dwordx2", "global_store_dwordx4"}, (k, stores)
+
+
 def test_shared_k_kernels_stay_in_registers(miw):
-    """No scratch in any instance; the rings are counted in vmcnt, so nothing but the C ahead of them and the loads to LDS
-    may read global memory before the last wait."""
+    """No scratch in any instance; the rings are counted in vmcnt, so nothing but the loads to LDS may read global memory
+    from the first MFMA to the last (C goes ahead of the rings, or behind the loop)."""
     res = {k: v for k, v in miw.reflection.kernel_resources().items() if "k_gemm_kwave<" in k}
     assert len(res) == 10
     for k, r in res.items():
@@ -77,6 +91,9 @@ def test_shared_k_kernels_stay_in_registers(miw):
         ops = _ops(text)
         assert ops["v_mfma_f32_16x16x32_f16"] > 0 and ops["global_load_lds_dwordx4"] > 0, k
         assert not any(o.startswith(("scratch_", "flat_", "v_accvgpr")) for o in ops), k
+        order = [l.split()[0] for l in text.splitlines() if l.strip()]
+        mfma = [i for i, o in enumerate(order) if o.startswith("v_mfma")]
+        assert {o for o in order[mfma[0]:mfma[-1]] if o.startswith(("global_", "buffer_"))} == {"global_load_lds_dwordx4"}, k
 
 
 def test_narrow_kernel_codegen_and_resources(miw):
