@@ -378,15 +378,19 @@ kwave_tile kwave_fits(const gemm_params &g, int c_type, int d_type, bool in_plac
 
 // The smallest of the kernel's tiles that covers D in one round over the CUs: the fewer bytes a CU has to fetch the
 // shorter the launch, and a second round costs more than any tile saves (1.3 to 1.7 times the time of the 64x64 tile).
-// Measured over 489 problems of 16 to 1280 x 64 to 8192 x 128 to 8192, against the kernels that ran them before:
-//   32x16, 16x32, 32x32: 0.48 to 0.89 of the 64x64 tile's time from K = 128 on (256x256x2048 9.9 -> 6.3 us).
-//   64x32, 32x64: 0.70 to 1.0 from K = 512 on with k contiguous in both operands (128x4096x4096 15.3 -> 12.3 us; at K = 128
-//     1.05 to 1.1), 0.82 to 0.98 from 768 on otherwise (720x656x1280 8.5 -> 7.8; at 512 1.0).
+// Measured against the kernels that run them otherwise, on operands from the last-level cache and from HBM:
+//   32x16, 16x32, 32x32: 0.41 to 1.02 of the 64x64 tile's time from K = 128 on (256x256x2048 9.9 -> 6.3 us).
+//   64x32, 32x64 with a C operand, whose reading the K loop here hides: 0.74 to 1.0 from K = 512 on with k contiguous in
+//     both operands, 0.8 to 1.0 from 768 on otherwise.  Without C: 0.7 to 1.07 from K = 1024 on (128x4096x4096 15.3 ->
+//     12.3 us), below that 1.0 to 1.1 (720x656x832 6.5, 5.8 on the tile), but where whatever has k contiguous starts its
+//     rows off whole cache lines, which slows the tiles' loads: 0.92 to 1.06 from 512 (both operands) or 768 on.  Slices of
+//     K go by the lines for a C.
 //   Less than 64 rows or columns, against k_gemm_skinny and the fragment-op kernels: with k contiguous in both operands,
-//     and rows on whole cache lines, which these loads need and those do not (16x4096x2064: 1.28), 0.34 to 0.96 where
-//     those take a second round, and from K = 1024 (16 rows) or 512 on where they take one (16x4096x4096 10.1 -> 8.7,
-//     48x4096x4096 17.4 -> 9.9; 16x4096x512 1.03).  In other layouts 0.52 to 0.98 from K = 1024 on, or 512 with 2048 of
-//     the long extent (48x4096x4096 27.7 -> 15.0; 48x256x512 1.1).
+//     and rows on whole cache lines, which these loads need and those do not (16x4096x2064: 1.2 to 1.4), 0.34 to 0.96 where
+//     those take a second round, and from K = 1024 (16 rows) or 512 on where they take one (48x4096x4096 17.4 -> 9.9;
+//     16x4096 0.77 to 1.03 from the cache, 1.05 to 1.13 from HBM).  In other layouts 0.4 to 1.0 with 1024 or more of the
+//     long extent, K from 1024 on, or 512 with 2048; shorter ones with k contiguous in one operand, the long one's up to
+//     1024, the other up to 512: 1.0 to 1.2 below K = 3072, 0.6 to 1.02 from there (48x64x1280 5.7, 4.9 on fragment ops).
 //   64 to 128 rows off whole cache lines, where k_gemm_skinny beats the 64x64 tile: up to 32x32 0.76 to 0.95 of its time
 //     from K = 768 on.
 kwave_tile kwave_pays(const gemm_params &g, int c_type, int d_type, bool in_place, int cus)
@@ -395,19 +399,27 @@ kwave_tile kwave_pays(const gemm_params &g, int c_type, int d_type, bool in_plac
     if (!kwave_runs(g, c_type, d_type)) return none;
     bool xk, yk;
     layouts(g, &xk, &yk);
-    const bool both = xk && yk;
+    const bool both = xk && yk, a_k = g.a_row != 0, b_k = g.b_row == 0;
     const long wide = std::max(g.M, g.N), thin = std::min(g.M, g.N);
+    const bool narrow_wins = skinny_beats_tiles(g, d_type, false);
     if (thin < 64) {
         if (both && (g.lda % 64 || g.ldb % 64)) return none;
-        const bool rounds = wide / 16 * g.batch > cus;
-        if (both ? !rounds && g.K < (thin == 16 ? 1024 : 512) : g.K < (wide >= 2048 ? 512 : 1024)) return none;
-    } else if (skinny_beats_tiles(g, d_type, false) && g.K < 768) {
+        const bool rounds = wide / 16 * g.batch > cus, wide_k = g.M >= g.N ? a_k : b_k;
+        const long least = both ? (rounds ? 0 : thin == 16 ? 1024 : 512)
+                           : wide >= 2048 ? 512
+                           : (a_k || b_k) && wide < (wide_k ? 1024 : 512) ? 3072
+                                                                          : 1024;
+        if (g.K < least) return none;
+    } else if (narrow_wins && g.K < 768) {
         return none;
     }
+    // rows of whatever has k contiguous start off whole cache lines
+    const bool off_lines = (a_k || b_k) && (!a_k || g.lda % 64) && (!b_k || g.ldb % 64);
+    const long least_64 = !g.use_c && g.batch == 1 && !off_lines ? 1024 : both ? 512 : 768;
     for (const kwave_tile t : kwave_tiles) {
         const long groups = kwave_groups(g, t, in_place);
         if (groups == 0 || groups > cus) continue;
-        if (t.bi * t.bj > 32 * 32 && (g.K < (both ? 512 : 768) || (thin >= 64 && skinny_beats_tiles(g, d_type, false)))) continue;
+        if (t.bi * t.bj > 32 * 32 && (g.K < least_64 || (thin >= 64 && narrow_wins))) continue;
         return t;
     }
     return none;

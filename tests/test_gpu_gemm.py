@@ -864,7 +864,7 @@ def test_narrow_problems_through_every_route(gpu, orc, narrow_kernel, cl, dl):
     ((32, 16), 0, 1, 144, 176, (128, 144, 336, 1104, 2064)), ((16, 32), 0, 1, 16, 48, (1024, 1600)), ((32, 32), 0, 1, 512, 304, (128, 400)),
     ((64, 32), 0, 1, 1008, 512, (512, 528)), ((32, 32), 1, 1, 80, 112, (128, 144, 336, 1104)), ((32, 32), 0, 0, 80, 112, (128, 144, 336, 1104)),
     ((32, 32), 1, 0, 80, 112, (128, 144, 336, 1104)), ((64, 32), 1, 1, 1008, 512, (768, 784)), ((32, 64), 0, 0, 512, 1008, (768, 784)),
-    ((64, 32), 1, 0, 1008, 512, (768, 784, 1360))])
+    ((64, 32), 1, 0, 1008, 512, (768, 1040, 1360))])
 @pytest.mark.parametrize("dl", (0, 1))
 def test_kernel_whose_wavefronts_share_k(gpu, orc, shared_k_tile, tile, al, bl, M, N, Ks, dl):
     """Every tile and operand layout, shifted edge tiles, whole and ragged K around the wavefronts' turns and rings, every

@@ -335,14 +335,21 @@ def test_shared_k_kernel_runs_where_it_was_measured_ahead(miw, shared_k_tile):
     for want, M, N, K, kw in (
             # k contiguous in both operands: the smallest tile whose count the CUs hold; K of two slots
             ((32, 16), 64, 64, 128, {}), (None, 64, 64, 112, {}), ((32, 16), 512, 256, 128, {}), ((32, 32), 512, 272, 128, {}),
-            ((32, 32), 512, 512, 128, {}), ((64, 32), 512, 528, 512, {}), (None, 512, 528, 496, {}), ((64, 32), 512, 1024, 512, {}), (None, 528, 1024, 512, {}),
-            # one operand or none: no 16-wide tiles, the 64-wide ones from K = 768 on
-            ((32, 32), 64, 64, 128, dict(a_row=0)), ((32, 32), 64, 64, 128, dict(a_row=0, b_row=1)), ((32, 64), 512, 1024, 768, dict(a_row=0)),
-            (None, 512, 1024, 752, dict(a_row=0)), ((64, 32), 512, 1024, 768, dict(b_row=1)), ((64, 32), 512, 1024, 768, dict(a_row=0, b_row=1)),
+            ((32, 32), 512, 512, 128, {}), ((64, 32), 512, 528, 512, dict(use_c=1)), (None, 512, 528, 496, dict(use_c=1)), ((64, 32), 512, 1024, 512, dict(use_c=1)), (None, 528, 1024, 512, dict(use_c=1)),
+            # ... without C from K = 1024 on, or 512 where both operands' rows start off whole lines
+            (None, 512, 528, 512, {}), (None, 512, 528, 960, {}), ((64, 32), 512, 528, 1024, {}), ((64, 32), 512, 1024, 528, {}), (None, 512, 1024, 528, dict(lda=576)),
+            # one operand or none: no 16-wide tiles, the 64-wide ones from K = 768 on, without C only off whole lines, else from 1024 on
+            ((32, 32), 64, 64, 128, dict(a_row=0)), ((32, 32), 64, 64, 128, dict(a_row=0, b_row=1)), ((32, 64), 512, 1024, 768, dict(a_row=0, use_c=1)),
+            (None, 512, 1024, 752, dict(a_row=0, use_c=1)), ((64, 32), 512, 1024, 768, dict(b_row=1, use_c=1)), ((64, 32), 512, 1024, 768, dict(a_row=0, b_row=1, use_c=1)),
+            ((32, 64), 512, 1024, 784, dict(a_row=0)), (None, 512, 1024, 752, dict(a_row=0)), (None, 512, 1024, 960, dict(a_row=0)), ((32, 64), 512, 1024, 1024, dict(a_row=0)),
+            ((64, 32), 512, 1024, 784, dict(b_row=1)), (None, 512, 1024, 960, dict(b_row=1)), (None, 512, 1024, 1008, dict(a_row=0, b_row=1)), ((64, 32), 512, 1024, 1024, dict(a_row=0, b_row=1)),
             # thinner than every other tile
             ((32, 16), 16, 4096, 1024, {}), (None, 16, 4096, 1008, {}), ((32, 16), 16, 4112, 128, {}), (None, 16, 8208, 4096, {}),
             ((32, 16), 32, 4096, 512, {}), (None, 32, 4096, 496, {}), ((32, 32), 48, 4096, 512, {}), (None, 16, 4096, 2064, {}), (None, 48, 4096, 4160, dict(lda=4168)),
             (None, 16, 4096, 4096, dict(a_row=0)), ((32, 32), 32, 2048, 512, dict(b_row=1)), (None, 32, 2032, 512, dict(b_row=1)), ((32, 32), 32, 2032, 1024, dict(b_row=1)),
+            # ... and short: k contiguous in one operand
+            (None, 32, 496, 3056, dict(b_row=1)), ((32, 32), 32, 496, 3072, dict(b_row=1)), ((32, 32), 32, 512, 1024, dict(b_row=1)), (None, 32, 1008, 3056, dict(a_row=0)),
+            ((32, 32), 32, 1008, 3072, dict(a_row=0)), ((32, 32), 32, 1024, 1024, dict(a_row=0)), ((32, 32), 32, 496, 1024, dict(a_row=0, b_row=1)),
             # rows off whole cache lines, where the narrow kernel beats the 64x64 tile
             ((32, 32), 64, 4096, 784, {}), (None, 64, 4096, 752, {}), (None, 64, 8192, 784, {}),
             # C in D's place: whole tiles
