@@ -396,7 +396,9 @@ def main():
               "k_gemm_fragops" if vinfo["fragment_ops"] else
               "k_gemm_w128" if vinfo["wave128"] else
               "k_gemm_tiled" if not vinfo["pingpong"] else
-              "k_gemm_pp" if vinfo["block"][:2] == (256, 256) else "k_gemm_pp64")
+              "k_gemm_pp64" if vinfo["block"][:2] != (256, 256) else
+              # (a Float32 C laid out as D, alpha 1 and more than sixteen slots of K: added in the K loop)
+              "k_gemm_pp_fold" if ct == np.float32 and not args.no_c and K > 1024 else "k_gemm_pp")
     roof["kernel"] = "%s<%s>" % (family, vinfo["name"])
     build_id = lib.miw_build_id().decode()
     roof["traffic"] = None
