@@ -93,7 +93,7 @@ class DeviceArray:
         self.dtype = np.dtype(dtype)
         self.dims = tuple(map(int, dims))
         count = math.prod(self.dims)
-        if not 0 <= count < 1 << 63:
+        if not 0 < count < 1 << 63:
             count = int(np.prod(self.dims, dtype=np.int64))  # refuses or wraps, as an Int does
         self.nbytes = count * self.dtype.itemsize
         p = ctypes.c_void_p()

@@ -414,6 +414,13 @@ def test_fragment_signature_tables_agree_with_the_checks(miw):
                                       for c in (f16, f32) for d in (f16, f32) for a in layouts for b in layouts)
 
 
+def test_extents_beyond_an_int_are_refused_in_empty_arrays_too(miw):
+    """2^70 x 0 elements: no Int holds the extents, whatever their product."""
+    for dims in ((1 << 70, 0), (0, 1 << 64), (1 << 70, 1 << 70)):
+        with pytest.raises(OverflowError):
+            miw.DeviceArray(dtype=np.float32, dims=dims)
+
+
 def test_variant_table_and_selection(miw):
     G = miw.GEMM
     vs = G.variants()
