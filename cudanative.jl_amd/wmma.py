@@ -319,13 +319,14 @@ def mma(a, b, c, config):
     if c.L is not Unspecified:
         raise TypeError("mma: the accumulator's layout must be Unspecified")
     found = _MMAS.get((a.T, b.T, c.T, config.d_type, a.L, b.L))
-    if found is None:  # one of these raises
+    if found is None:  # one of these raises, or a type goes by another of its names
         get_hl_frag_info("a", a.T)
         get_hl_frag_info("b", b.T)
         get_hl_frag_info("c", c.T)
-        get_hl_frag_info("d", config.d_type)
+        d_num, _ = get_hl_frag_info("d", config.d_type)
         get_hl_layout(a.L)
         get_hl_layout(b.L)
+        found = _layout_code(a.L), _layout_code(b.L), _dtype_code(c.T), _dtype_code(config.d_type), d_num
     get_hl_shape(M, N, K)
     a_order, b_order, c_ty, d_ty, d_num = found
     img = _new_image(config.d_type, d_num)

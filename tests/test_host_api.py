@@ -414,6 +414,33 @@ def test_fragment_signature_tables_agree_with_the_checks(miw):
                                       for c in (f16, f32) for d in (f16, f32) for a in layouts for b in layouts)
 
 
+@pytest.mark.parametrize("given", ["float32", np.dtype(np.float32), "f4"])
+def test_mma_takes_a_type_by_any_of_its_names(miw, monkeypatch, given):
+    """A Config or a fragment whose type was set by name passes mma's checks (up to the first use of the device here)."""
+    W = miw.WMMA
+
+    class Reached(Exception):
+        pass
+
+    def image(T, FS):
+        assert np.dtype(T) == np.float32 and FS == 4
+        raise Reached
+
+    monkeypatch.setattr(W, "_new_image", image)
+    config = W.Config(16, 16, 16, np.float32)
+    a, b, c = (W.Fragment(16, 16, 16, 4, t, L, U, image=object())
+               for t, L, U in ((np.float16, W.RowMajor, W.MatrixA), (np.float16, W.ColMajor, W.MatrixB), (np.float32, W.Unspecified, W.Accumulator)))
+    c.T = given
+    with pytest.raises(Reached):
+        W.mma(a, b, c, config)
+    config.d_type = given
+    with pytest.raises(Reached):
+        W.mma(a, b, c, config)
+    c.T = "int32"
+    with pytest.raises(W.WMMAError):
+        W.mma(a, b, c, config)
+
+
 def test_extents_beyond_an_int_are_refused_in_empty_arrays_too(miw):
     """2^70 x 0 elements: no Int holds the extents, whatever their product."""
     for dims in ((1 << 70, 0), (0, 1 << 64), (1 << 70, 1 << 70)):
