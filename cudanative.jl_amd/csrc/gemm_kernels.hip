@@ -166,6 +166,7 @@ static tiled_params canonical(const gemm_params &g, int bi, int bj, bool *xk, bo
     p.C = g.C; p.D = g.D;
     p.K = (int)g.K;
     p.work = 0;
+    p.c_spread = 0;
     p.ldc = g.ldc; p.ldd = g.ldd; p.sc = g.sc; p.sd = g.sd;
     p.use_c = g.use_c;
     p.alpha = g.alpha; p.beta = g.beta;
@@ -201,6 +202,12 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
     p.ts = nullptr;
     if (const char *e = getenv("MIW_TS")) p.ts = (long long *)strtoull(e, nullptr, 16);
 #endif
+    // A large C that all workgroups ask for at once is a burst that the first slots do not cover; a workgroup that asks for
+    // it in mid-loop waits too, for one latency.  256x128 tiles, at the start and spread: 32 MiB 74.0 and 71.4 us
+    // (8192x1024x4096), 22 MiB 21.2 and 19.7 (2304x2496x1152), 14 MiB 18.9 and 18.2 (7120x1024x720), 11 MiB 15.4 and 15.2
+    // (896x6528x544); on 128x128 tiles, which have less of it, spreading loses (4032x576x2368 19.5 and 21.1).
+    p.c_spread = v.kind == KIND_PINGPONG64 && v.bm * v.bn > 128 * 128 && g.use_c &&
+                 (long)p.I * p.J * g.batch * (c_type == 0 ? 2 : 4) >= (12l << 20);
     const bool fold = v.kind == KIND_PINGPONG32 && pp_folds(p, c_type);
     const void *fn = pick_kernel(i, xk, yk, c_type, d_type, f16acc, fold);
     if (!fn) return hipErrorInvalidValue;

@@ -682,7 +682,7 @@ void k_gemm_pp_fold(tiled_params p)
 // the accumulators start as half(beta * C) and the MFMAs accumulate onto the rounded sum in place,
 // otherwise the running sum is kept beside accumulators that restart from zero in every slot:
 // run = half(run + alpha * slot sum).  C is requested before anything else and converted once the
-// first pair's loads have landed.
+// first pair's loads have landed.  With Float32 accumulation C waits in registers for the end of the loop.
 template <int BI, int BJ, int WI, int WJ, int NSLOT, bool XK, bool YK, class CT, class DT, bool F16ACC>
 __global__ __launch_bounds__(WI *WJ * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void k_gemm_pp64(tiled_params p)
@@ -742,18 +742,10 @@ void k_gemm_pp64(tiled_params p)
 #pragma unroll
         for (int b = 0; b < TJ; b++) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-    auto read_c = [&](int a, int b, bool trans) -> float4_t {
+    auto read_c_across = [&](int a, int b) -> float4_t {
         float4_t c;
-        const int ii = row + 16 * a, jj = col + 16 * b;
-        if (trans) {
 #pragma unroll
-            for (int v = 0; v < 4; v++) c[v] = (float)C[(long)(ii + v) * p.ldc + jj];
-        } else if constexpr (__is_same(CT, float)) {
-            c = *(const float4_t *)(C + (long)jj * p.ldc + ii);
-        } else {
-            half4_t h = *(const half4_t *)(C + (long)jj * p.ldc + ii);
-            c = float4_t{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
-        }
+        for (int v = 0; v < 4; v++) c[v] = (float)C[(long)(row + 16 * a + v) * p.ldc + (col + 16 * b)];
         return c;
     };
 
@@ -863,8 +855,16 @@ void k_gemm_pp64(tiled_params p)
         end_request();
     }
     if constexpr (!F16ACC) fetch_result_arguments(p);
-    // The loop starts when pair 0 (and the C operand, requested before it) has landed: the wait at the
-    // end of memory cluster p leaves NSLOT - 2 pairs in flight, so pair p + 1 has landed by then, the
+    // Float32 accumulation: C laid out as D goes into registers while the loop runs (request_c), in the whole lines in which D
+    // is stored.  (Added to the sums in the loop's last pairs, as k_gemm_pp_fold does, it costs those pairs a quarter more each,
+    // and read behind the loop two loads at a time it waits for memory once per pair of tiles: 8192x1024x4096 from HBM
+    // 73.2 us -> 69.4, 7120x1024x720 with a Float16 C 19.4 -> 17.8, 2048x2048x128 11.1 -> 9.2.)
+    using cpieces = c_pieces<TI, TJ, CT>;
+    cpieces cp;
+    const bool early = !F16ACC && p.use_c && !p.c_trans;
+    auto request_c = [&]() MIW_INLINE { cp.request(C + (long)(j0 + wj * WTJ) * p.ldc + (i0 + wi * WTI) + pair_place(lane, p.ldc), p.ldc); };
+    // The loop starts when pair 0 (and, with Float16 accumulation, the C operand, requested before it) has landed: the
+    // wait at the end of memory cluster p leaves NSLOT - 2 pairs in flight, so pair p + 1 has landed by then, the
     // first time as every other.
     wait_loads_and_barrier<(NSLOT - 2) * LPAIR>();
     float4_t cinit[F16ACC ? TI : 1][F16ACC ? TJ : 1];
@@ -1008,39 +1008,6 @@ void k_gemm_pp64(tiled_params p)
         for (int m = NTILE - ROUND_DEFER; m < NTILE; m++) round_tile(tile_of_mfma(m), std::integral_constant<int, ZERO ? 3 : 1>{});
     };
 
-    // Folding C (Float32 C laid out as D, alpha == 1): CPT MFMA tiles per cluster over the last
-    // NFOLD clusters, requested at the end of a memory cluster with ordinary loads into registers
-    // (the lane fetches the 16 bytes it owns).  They are the youngest loads of their cluster; the
-    // wait LAG clusters later covers them and that cluster adds them in, so C has LAG clusters of
-    // both wavefront groups to arrive.  LAG + 1 register stages rotate.
-    constexpr int CPT = 1;
-    constexpr int NFOLD = NTILE / CPT;
-    constexpr int LAG = NSLOT - 1;
-    constexpr bool CAN_FOLD = !F16ACC && __is_same(CT, float) && TI % CPT == 0;
-    bool fold_c = false;
-    if constexpr (CAN_FOLD) fold_c = p.use_c && !p.c_trans && p.alpha == 1.0f && NP >= NFOLD + 1 && p.ldc < (1l << 22);
-    float4_t cst[LAG + 1][CPT];
-    const char *cnext = (const char *)(C + (long)j0 * p.ldc + i0);
-    const unsigned coff = 4u * (unsigned)((wj * WTJ + r) * (int)p.ldc + wi * WTI + 4 * q);
-    auto fold_request = [&]<int S>(std::integral_constant<int, S>) {
-        [&]<int... U>(std::integer_sequence<int, U...>) {
-            (([&] {
-                 constexpr int a = (S * CPT + U) % TI;
-                 asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(cst[S % (LAG + 1)][U]) : "v"(coff), "s"(cnext), "n"(64 * a) : "memory");
-                 if constexpr (a == TI - 1) cnext += 64 * p.ldc;
-             }()),
-             ...);
-        }(std::make_integer_sequence<int, CPT>{});
-    };
-    auto fold_add = [&]<int S>(std::integral_constant<int, S>) {
-#pragma unroll
-        for (int u = 0; u < CPT; u++) {
-            const int a = (S * CPT + u) % TI, b = (S * CPT + u) / TI;
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[a][b][e] = __builtin_fmaf(p.beta, cst[S % (LAG + 1)][u][e], acc[a][b][e]);
-        }
-    };
-    // One pair: memory cluster, barrier, compute cluster, barrier.  FS >= 0: fold cluster FS.
     // Zeroes the repeated k-values in the fragments of the shifted last pair.
     auto mask_tail = [&]() {
         const unsigned keep0 = tail_keep<0>(tail_skip), keep1 = tail_keep<1>(tail_skip);
@@ -1049,78 +1016,46 @@ void k_gemm_pp64(tiled_params p)
 #pragma unroll
         for (int b = 0; b < TJ; b++) { tail_apply(fy[0][b], keep0); tail_apply(fy[1][b], keep1); }
     };
-    // FS >= 0: fold pair FS (always folds).  FS == -1: a pair that does not fold.  FS == -2: the last
-    // pair: its fragments are masked, and it is fold pair NFOLD - 1 when the launch folds C, which is
-    // decided here at run time, so that the last pair is one piece of code for both cases (two
-    // alternative pieces that each update all accumulators cost spills where they join).
-    auto fold_wait = [&]<int FS>(std::integral_constant<int, FS>) {
-        // Allowed to stay in flight: the ring loads of the NSLOT - 2 youngest clusters with the fold
-        // loads issued after them, and the fold loads of the cluster before those (younger than
-        // that cluster's ring loads, which must have landed).
-        constexpr int YOUNGER = (NSLOT - 2) * LPAIR + CPT * (FS + 1 < NSLOT - 1 ? FS + 1 : NSLOT - 1);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt((YOUNGER & 15) | (7 << 4) | (0 << 8) | ((YOUNGER >> 4) << 14));
-        asm volatile("" ::: "memory");
-    };
-    // RMODE: how the compute cluster rounds its sums (0: fp32 accumulation; 1, 3: see round_tile).
-    auto pair = [&]<int FS, int RMODE, int SL = -2>(std::integral_constant<int, FS>, std::integral_constant<int, RMODE>, std::integral_constant<int, SL> sl = {}) {
+    // One pair: memory cluster, barrier, compute cluster, barrier.  LAST: its fragments are masked.  RMODE: how the
+    // compute cluster rounds its sums (0: fp32 accumulation; 1, 3: see round_tile).  fresh: C, requested behind the
+    // first NSLOT - 1 pairs, may still be in flight.
+    auto pair = [&]<bool LAST, int RMODE, int SL = -2>(std::bool_constant<LAST>, std::integral_constant<int, RMODE>, std::integral_constant<int, SL> sl = {}, bool fresh = false) {
         memory_cluster(sl);
         if constexpr (RMODE != 0) {
             round_deferred(std::bool_constant<RMODE == 3>{});
             __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (FS >= 0) {
-            fold_request(std::integral_constant<int, FS>{});
-            __builtin_amdgcn_sched_barrier(0);
-            fold_wait(std::integral_constant<int, FS>{});
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (FS >= LAG) fold_add(std::integral_constant<int, FS - LAG>{});
-            __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-        } else if constexpr (FS == -2 && CAN_FOLD) {
-            constexpr int LFS = NFOLD - 1;
-            if (fold_c) {
-                fold_request(std::integral_constant<int, LFS>{});
-                fold_wait(std::integral_constant<int, LFS>{});
-                fold_add(std::integral_constant<int, LFS - LAG>{});
-                __builtin_amdgcn_s_barrier();
-                asm volatile("" ::: "memory");
-            } else {
-                wait_loads_and_barrier<(NSLOT - 2) * LPAIR>();
-            }
-        } else {
-            wait_loads_and_barrier<(NSLOT - 2) * LPAIR>();
-        }
-        if constexpr (FS == -2) mask_tail();
+        if (fresh) wait_loads_and_barrier<(NSLOT - 2) * LPAIR + cpieces::LOADS>();
+        else wait_loads_and_barrier<(NSLOT - 2) * LPAIR>();
+        if constexpr (LAST) mask_tail();
         compute_cluster(std::bool_constant<RMODE == 3>{}, std::bool_constant<SL != -2>{});
         __builtin_amdgcn_s_barrier();
     };
-    constexpr std::integral_constant<int, -1> no_fold{};
+    constexpr std::false_type inner{};
+    constexpr std::true_type last_pair{};
     constexpr std::integral_constant<int, -1> fast_pair{};
     // NSLOT pairs that need no look at the end of K, the first of which reads slot 0
 #ifdef MIW_PP_TS
     bool stamp_pair = false;
 #endif
-    auto ring_of_pairs = [&]<int RMODE>(std::integral_constant<int, RMODE> rmode) {
+    // fresh: C has been asked for in front of them
+    auto ring_of_pairs = [&]<int RMODE>(std::integral_constant<int, RMODE> rmode, bool fresh = false) {
         [&]<int... S>(std::integer_sequence<int, S...>) {
             (([&] {
 #ifdef MIW_PP_TS
                  if constexpr (S == 1)
                      if (stamp_pair) MIW_PP_STAMP(3)
 #endif
-                 pair(std::integral_constant<int, -1>{}, rmode, std::integral_constant<int, S>{});
+                 pair(inner, rmode, std::integral_constant<int, S>{}, S < NSLOT - 2 && fresh);
              }()),
              ...);
         }(std::make_integer_sequence<int, NSLOT>{});
     };
-    constexpr std::integral_constant<int, -2> last_pair{};
     constexpr std::integral_constant<int, 0> plain{};
 
     MIW_PP_STAMP(1)
     if (late_group) __builtin_amdgcn_s_barrier();
-    // the loop runs the pairs that neither fold nor are the last one
-    const int NPM = fold_c ? NP - NFOLD : NP - 1;
+    const int NPM = NP - 1;  // pairs but the last
     // the request of pair pr is pair pr + NSLOT - 1; the pairs before NP - 1 lie a full step apart
     const int NFAST = min(NPM, max(0, NP - 1 - NSLOT));
     const bool separate_sum = F16ACC && p.alpha != 1.0f;
@@ -1132,9 +1067,9 @@ void k_gemm_pp64(tiled_params p)
         if (separate_sum) {
             int pr = 0;
             for (; pr + NSLOT <= NFAST; pr += NSLOT) ring_of_pairs(separate);
-            for (; pr < NFAST; pr++) pair(no_fold, separate, fast_pair);
+            for (; pr < NFAST; pr++) pair(inner, separate, fast_pair);
             next = NSLOT - 1 + pr;
-            for (; pr < NPM; pr++) pair(no_fold, separate);
+            for (; pr < NPM; pr++) pair(inner, separate);
             pair(last_pair, separate);
             round_deferred(std::true_type{});
         } else {
@@ -1147,70 +1082,70 @@ void k_gemm_pp64(tiled_params p)
                 MIW_PP_MIDDLE(pr)
                 ring_of_pairs(rolling);
             }
-            for (; pr < NFAST; pr++) pair(no_fold, rolling, fast_pair);
+            for (; pr < NFAST; pr++) pair(inner, rolling, fast_pair);
             next = NSLOT - 1 + pr;
-            for (; pr < NPM; pr++) pair(no_fold, rolling);
+            for (; pr < NPM; pr++) pair(inner, rolling);
             MIW_PP_STAMP(9)
             pair(last_pair, rolling);
             round_deferred(std::false_type{});
         }
     } else {
         int pr = 0;
+        // Which ring of pairs C is asked for in front of (see tiled_params::c_spread); without a ring, in front of the last
+        // pair: so few pairs end before C arrives, and C's loads would hold theirs up.
+        const int rings = max(0, NFAST / NSLOT);
+        const int c_at = BI * BJ > 128 * 128 && p.c_spread ? (rings * (int)((blockIdx.x >> 3) & 7) >> 3) * NSLOT : 0;
         for (; pr + NSLOT <= NFAST; pr += NSLOT) {
             MIW_PP_MIDDLE(pr)
-            ring_of_pairs(plain);
+            const bool now = early && pr == c_at;
+            if (now) request_c();
+            ring_of_pairs(plain, now);
         }
-        for (; pr < NFAST; pr++) pair(no_fold, plain, fast_pair);
+        for (; pr < NFAST; pr++) pair(inner, plain, fast_pair);
         next = NSLOT - 1 + pr;
-        for (; pr < NPM; pr++) pair(no_fold, plain);
+        for (; pr < NPM; pr++) pair(inner, plain);
+        if (early && rings == 0) request_c();
         MIW_PP_STAMP(9)
-        if constexpr (CAN_FOLD) {
-            if (fold_c) {
-                [&]<int... G>(std::integer_sequence<int, G...>) {
-                    (pair(std::integral_constant<int, G>{}, plain), ...);
-                }(std::make_integer_sequence<int, NFOLD - 1>{});
-            }
-        }
-        pair(last_pair, plain);
+        pair(last_pair, plain, std::integral_constant<int, -2>{}, early && rings == 0);  // (nothing that it reads is on the way any more)
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may outlive the workgroup's LDS
-    if constexpr (CAN_FOLD) {
-        if (fold_c) {
-            [&]<int... G>(std::integer_sequence<int, G...>) {
-                (fold_add(std::integral_constant<int, NFOLD - LAG + G>{}), ...);
-            }(std::make_integer_sequence<int, LAG>{});
-        }
-    }
     if (!late_group) __builtin_amdgcn_s_barrier();
     MIW_PP_STAMP(4)
 
-    // Epilogue: each lane owns 4 consecutive i of one column j per MFMA tile.
+    // Epilogue: each lane owns 4 consecutive i of one column j per MFMA tile; tiles go out in pairs.
     static_assert(TI % 2 == 0, "the epilogue stores pairs of tiles");
-    auto epilogue = [&]<bool EDGE = false>(bool with_c, bool trans, std::bool_constant<EDGE> = {}) {
-        auto value = [&](int a, int b) {
-            float4_t v = separate_sum ? cinit[a][b] : acc[a][b];
-            if constexpr (!F16ACC) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[e] *= p.alpha;
-                if (with_c) {
-                    float4_t c = read_c(a, b, trans);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = __builtin_fmaf(p.beta, c[e], v[e]);
-                }
-            }
-            return v;
-        };
+    const bool odd = lane & 1;
+    DT *to = D + (long)(j0 + wj * WTJ) * p.ldd + (i0 + wi * WTI) + pair_place(lane, p.ldd);
+    // C_AT 0: nothing to add, 1: C laid out as D, in registers, 2: C laid out the other way round
+    auto epilogue = [&]<int C_AT>(std::integral_constant<int, C_AT>) {
 #pragma unroll
         for (int b = 0; b < TJ; b++)
 #pragma unroll
-            for (int a = 0; a < TI; a += 2)
-                store_tile_pair<DT>(D, p.ldd, i0 + wi * WTI + 16 * a, j0 + wj * WTJ + 16 * b, lane, value(a, b), value(a + 1, b),
-                                    !EDGE || (i0 + wi * WTI + 16 * a + 16 * (lane & 1) >= own_from<BI>(i0) && j0 + wj * WTJ + 16 * b >= own_from<BJ>(j0)));
+            for (int a = 0; a < TI; a += 2) {
+                float4_t v[2];
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    v[t] = separate_sum ? cinit[a + t][b] : acc[a + t][b];
+                    if constexpr (!F16ACC) v[t] *= p.alpha;
+                    if constexpr (C_AT == 2) {
+                        const float4_t c = read_c_across(a + t, b);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) v[t][e] = __builtin_fmaf(p.beta, c[e], v[t][e]);
+                    }
+                }
+                DT *at = to + 16 * b * p.ldd + 16 * a;
+                if constexpr (C_AT == 1) {
+                    pair_exchange(odd, v[0], v[1]);
+                    cp.add(a, b, p.beta, v[0], v[1]);
+                    store_pieces_at<DT>(at, p.ldd, v[0], v[1]);
+                } else {
+                    store_pair_at(at, p.ldd, odd, v[0], v[1]);
+                }
+            }
     };
-    if (CAN_FOLD && fold_c && (i0 % BI || j0 % BJ)) epilogue(false, false, std::true_type{});
-    else if (F16ACC || !p.use_c || fold_c) epilogue(false, false);
-    else if (p.c_trans) epilogue(true, true);
-    else epilogue(true, false);
+    if (F16ACC || !p.use_c) epilogue(std::integral_constant<int, 0>{});
+    else if (p.c_trans) epilogue(std::integral_constant<int, 2>{});
+    else epilogue(std::integral_constant<int, 1>{});
 #ifdef MIW_PP_TS
     MIW_PP_STAMP(5)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -97,6 +97,7 @@ struct tiled_params {
     // Workgroups that walk several tiles (k_gemm_pp): number of tiles over the whole batch; a workgroup takes tile
     // blockIdx.x, then every gridDim.x-th.  0: one tile per workgroup.  Needs K of four slots or more.
     int work;
+    int c_spread;  // k_gemm_pp64: the workgroups ask for C at eight different times of their K loops, not all at its start
 #ifdef MIW_PP_TS
     long long *ts;  // measurement builds: 10 counters per wavefront (see k_gemm_pp64), or null
 #endif
@@ -385,6 +386,14 @@ __device__ inline void store_pair_at(DT *even, long ldd, bool odd, float4_t v0, 
         *(uint2_t *)(even + ldd) = s1;
     }
 }
+// The same for pieces that pair_exchange has made.
+template <class DT>
+__device__ inline void store_pieces_at(DT *even, long ldd, float4_t v0, float4_t v1)
+{
+    using piece = DT __attribute__((ext_vector_type(4)));
+    *(piece *)even = __builtin_convertvector(v0, piece);
+    *(piece *)(even + ldd) = __builtin_convertvector(v1, piece);
+}
 // Elements from the first value of a pair of tiles to where this lane writes in the even columns: rows
 // 16 * odd + 4 q .. + 3 of column r - odd.
 __device__ inline long pair_place(int lane, long ldd)
@@ -392,6 +401,31 @@ __device__ inline long pair_place(int lane, long ldd)
     const int r = lane & 15, q = lane >> 4, odd = r & 1;
     return (long)(r - odd) * ldd + 16 * odd + 4 * q;
 }
+// C of a wavefront's TI x TJ MFMA tiles, laid out as D, in the pieces that store_pair_at writes: requested in one go and
+// added behind pair_exchange.  `at`: this lane's place in the first pair of tiles, see pair_place.
+template <int TI, int TJ, class CT>
+struct c_pieces {
+    using piece = CT __attribute__((ext_vector_type(4)));
+    static constexpr int LOADS = TI * TJ;
+    piece v[TJ][TI];
+    __device__ inline void request(const CT *at, long ldc)
+    {
+#pragma unroll
+        for (int b = 0; b < TJ; b++)
+#pragma unroll
+            for (int a = 0; a < TI; a++) v[b][a] = *(const piece *)(at + (16 * b + (a & 1)) * ldc + 16 * (a & ~1));
+    }
+    // v0, v1: tiles (a, b) and (a + 1, b) times alpha, exchanged.
+    __device__ inline void add(int a, int b, float beta, float4_t &v0, float4_t &v1) const
+    {
+        const float4_t c0 = __builtin_convertvector(v[b][a], float4_t), c1 = __builtin_convertvector(v[b][a + 1], float4_t);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            v0[e] = __builtin_fmaf(beta, c0[e], v0[e]);
+            v1[e] = __builtin_fmaf(beta, c1[e], v1[e]);
+        }
+    }
+};
 // A tile that folds C and is shifted back to end at the edge writes only what its neighbour does not: C joins the sums of
 // what they share at another k-step in each, and the last bits differ.  First row (column) that the tile at x0 writes.
 template <int B>
@@ -657,7 +691,17 @@ void k_gemm_tiled(tiled_params p)
 #pragma unroll
     for (int s = 0; s < NSLOT; s++) request_pair();
     fetch_result_arguments(p);
-    wait_loads_and_barrier<(NSLOT - 1) * LPAIR>();
+    // C laid out as D goes into registers behind the first requests: read behind the loop, two loads at a time, it waits for
+    // memory once per pair of tiles (64x64 tiles: 768x1216x832 with a Float16 C 5.9 us -> 5.5, 672x864x512 5.1 -> 4.6;
+    // 128x128 tiles, two workgroups per CU: 512 problems of 128^3 19.4 -> 18.9, 192x128x256 397 times 33.8 -> 32.2).
+    constexpr bool EARLY_C = !F16ACC && fold_tiles(BI, BJ, NT, NSLOT) == 0 && TI * TJ <= 16;
+    using cpieces = c_pieces<TI, TJ, CT>;
+    cpieces cp;
+    const bool early = EARLY_C && p.use_c && !p.c_trans;
+    if constexpr (EARLY_C)
+        if (early) cp.request(C + (long)(j0 + wj * WTJ) * p.ldc + (i0 + wi * WTI) + pair_place(lane, p.ldc), p.ldc);
+    if (early) wait_loads_and_barrier<(NSLOT - 1) * LPAIR + cpieces::LOADS>();
+    else wait_loads_and_barrier<(NSLOT - 1) * LPAIR>();
     [&]<int... U>(std::integer_sequence<int, U...>) {
         (fetch_unit(f0, lds, std::integral_constant<int, U>{}, first_half), ...);
     }(std::make_integer_sequence<int, NUNIT>{});
@@ -727,12 +771,16 @@ void k_gemm_tiled(tiled_params p)
     // G >= 0: the trip folds group G of C.  RT: whether it does is decided at run time (fold_c): the two
     // trips that meet the last pair are one piece of code for launches that fold and launches that do
     // not (two alternative pieces that each update all accumulators cost spills where they join).
-    auto trip = [&]<int MASK, int G, bool RT>(std::integral_constant<int, MASK>, std::integral_constant<int, G>, std::bool_constant<RT>) {
+    // FRESH: C, requested behind the first NSLOT pairs, may still be in flight.
+    auto trip = [&]<int MASK, int G, bool RT, bool FRESH = false>(std::integral_constant<int, MASK>, std::integral_constant<int, G>, std::bool_constant<RT>,
+                                                                  std::bool_constant<FRESH> = {}) {
         step(f0, f1, rslot, second_half, dma_begin, dma_begin);
         if constexpr (MASK == 2) mask_tail(f1, second_half);
         if constexpr (G >= 0) {
             if (!RT || fold_c) wait_loads_and_barrier<(NSLOT - 2) * LPAIR + (G > 0 ? CPT : 0)>();
             else wait_loads_and_barrier<(NSLOT - 2) * LPAIR>();
+        } else if constexpr (FRESH) {
+            wait_loads_and_barrier<(NSLOT - 2) * LPAIR + cpieces::LOADS>();
         } else {
             wait_loads_and_barrier<(NSLOT - 2) * LPAIR>();
         }
@@ -754,7 +802,11 @@ void k_gemm_tiled(tiled_params p)
     constexpr std::integral_constant<int, -1> no_group{};
     // the loop runs the trips that neither fold nor meet the last pair
     const int NPM = fold_c ? NP - NCT : NP >= 2 ? NP - 2 : 0;
-    for (int pr = 0; pr < NPM; pr++) trip(std::integral_constant<int, 0>{}, no_group, std::false_type{});
+    int pr = 0;
+    if constexpr (EARLY_C)
+        if (early)
+            for (; pr < min(NPM, NSLOT - 1); pr++) trip(std::integral_constant<int, 0>{}, no_group, std::false_type{}, std::true_type{});
+    for (; pr < NPM; pr++) trip(std::integral_constant<int, 0>{}, no_group, std::false_type{});
     if constexpr (CAN_FOLD) {
         if (fold_c) {
             [&]<int... G>(std::integer_sequence<int, G...>) {
@@ -803,7 +855,21 @@ void k_gemm_tiled(tiled_params p)
     if (CAN_FOLD && fold_c && (i0 % BI || j0 % BJ)) epilogue(false, false, std::true_type{});
     else if (F16ACC || !p.use_c || fold_c) epilogue(false, false);
     else if (p.c_trans) epilogue(true, true);
-    else epilogue(true, false);
+    else if constexpr (EARLY_C) {
+        const bool odd = lane & 1;
+        DT *to = D + (long)(j0 + wj * WTJ) * p.ldd + (i0 + wi * WTI) + pair_place(lane, p.ldd);
+#pragma unroll
+        for (int b = 0; b < TJ; b++)
+#pragma unroll
+            for (int a = 0; a < TI; a += 2) {
+                float4_t v0 = acc[a][b] * p.alpha, v1 = acc[a + 1][b] * p.alpha;
+                pair_exchange(odd, v0, v1);
+                cp.add(a, b, p.beta, v0, v1);
+                store_pieces_at<DT>(to + 16 * b * p.ldd + 16 * a, p.ldd, v0, v1);
+            }
+    } else {
+        epilogue(true, false);
+    }
 }
 
 // ------------------------------------------------- kernel instance lookup --

@@ -24,7 +24,7 @@ CONFIGS = {  # M, N, K, batch, A layout, B layout, all-Float16 with fp16 accumul
     "c4": (8192, 1024, 4096, 1, "row", "col", False),
 }
 PHASES = [("entry -> prologue's loads landed", 0, 1), ("loop, first half", 1, 2), ("one pair of k-steps (64 k-values)", 2, 3),
-          ("loop, second half up to the pairs that fold C", 3, 9), ("pairs that fold C, last additions", 9, 4),
+          ("loop, second half up to the pairs that fold C (or the last pair)", 3, 9), ("pairs that fold C, last pair", 9, 4),
           ("epilogue until the last store is issued", 4, 5), ("stores drained", 5, 6)]
 
 

@@ -249,6 +249,40 @@ def test_c_is_added_once_behind_the_loop(gpu, orc, alpha, K, al, bl):
             assert np.array_equal(D.view(np.uint32), (F32(alpha) * S + C).view(np.uint32)), (v["name"], al, bl, dl, K, alpha)
 
 
+# slots of K around the 64-k ping-pong rings of three and four slots (none, one ring, several), the 64x64 tile's four
+@pytest.mark.parametrize("K", (64, 80, 256, 336, 448, 464, 576, 640, 1168))
+@pytest.mark.parametrize("al,bl,ct", itertools.product((0, 1), repeat=3))
+def test_c_waits_in_registers_for_the_end_of_the_loop(gpu, orc, al, bl, ct, K):
+    """The kernels that fetch C into registers while the K loop runs: D is the launch without C plus beta * C in one rounding,
+    on every tile, with padded leading dimensions, several tiles and shifted edge tiles, bit for bit."""
+    for v in _variants(gpu):
+        if v["fragment_ops"] or not (v["pingpong"] and max(v["block"][:2]) * min(v["block"][:2]) < 65536 or v["stages"] in (2, 4) and max(v["block"][:2]) < 256):
+            continue
+        bm, bn = v["block"][:2]
+        for dl in (0, 1):
+            M, N = (bm + 16, 2 * bn) if dl == orc.COL else (2 * bn, bm + 16)
+            kw = dict(M=M, N=N, K=K, a_layout=al, b_layout=bl, c_layout=dl, d_layout=dl, c_type=ct, beta=-0.5)
+            g = orc.GemmDesc(ldc=(N if dl == orc.ROW else M) + 8, **kw)
+            A, B, C = _inputs(orc, g, 2600 + K + v["id"], clo=-100.0, chi=100.0)
+            D = _run(gpu, orc, g, A, B, C, variant=v["id"])
+            S = _run(gpu, orc, orc.GemmDesc(use_c=0, **kw), A, B, None, variant=v["id"])
+            inner = N if dl == orc.ROW else M
+            C2 = C.reshape(-1, inner + 8)[:, :inner].astype(np.float64).reshape(-1)
+            assert np.array_equal(D.view(np.uint32), (S.astype(np.float64) - 0.5 * C2).astype(F32).view(np.uint32)), (v["name"], al, bl, dl, ct, K)
+
+
+@pytest.mark.parametrize("M,N,K,ct", [(2064, 1552, 592, 1), (1552, 2064, 1168, 1), (2576, 2512, 448, 0), (2560, 2560, 384, 0)])
+def test_workgroups_ask_for_a_large_c_at_different_times(gpu, orc, M, N, K, ct):
+    """From 12 MiB of C on: the workgroups of the 256x128 tiles ask for it in front of different rings of their loops (or, with no
+    ring, at the end).  The bits of the sum and one addition."""
+    for name in ("tile256x128_pingpong", "tile128x256_pingpong"):
+        kw = dict(M=M, N=N, K=K, a_layout=orc.ROW, c_type=ct)
+        A, B, C = _inputs(orc, orc.GemmDesc(**kw), 2700 + K, clo=-100.0, chi=100.0)
+        D = _run(gpu, orc, orc.GemmDesc(**kw), A, B, C, variant=_vid(gpu, name))
+        S = _run(gpu, orc, orc.GemmDesc(use_c=0, **kw), A, B, None, variant=_vid(gpu, name))
+        assert np.array_equal(D.view(np.uint32), (S + C.astype(F32)).view(np.uint32)), (name, M, N, K, ct)
+
+
 def test_c_folded_into_the_loop_matches_the_epilogue_path(gpu, orc):
     """Random inputs, padded leading dimensions, batches: the folded C (alpha == 1, C laid out as D)
     agrees with float64 as tightly as the kernels that add C after the loop (alpha != 1, the
