@@ -154,6 +154,7 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 bool tiled_fits(int i, const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place)
 {
     const miw::tiled_variant &v = miw::tiled_variant_at(i);
+    if (p.k_last && (v.kind == miw::KIND_PINGPONG32 || v.kind == miw::KIND_WAVE128)) return false;
     // In canonical terms bm tiles the contiguous dimension of D.
     const long I = p.d_row ? p.N : p.M, J = p.d_row ? p.M : p.N;
     if (I < v.bm || J < v.bn || p.K < v.bk) return false;  // (K is a multiple of 16: a last slot that 64 does not divide is shifted back and masked)
@@ -982,19 +983,23 @@ int splitk_scratch(void **out)
 
 struct splitk_plan {
     miw::gemm_params full;   // the caller's problem
-    miw::gemm_params slice;  // first pass: `splits` independent products of K / splits k-values each
+    miw::gemm_params slice;  // first pass: `splits` independent products of as many k-values each, the last one of no more
     int variant;             // tiled variant of the first pass (1-based)
     int splits;
     miw::kwave_tile kw;      // what runs in its place, see pick_variant
     size_t bytes;            // workspace the first pass fills
 };
 
+// Slots of 64 k-values in each of `splits` slices but the last, which may have fewer.
+long slice_slots(const miw::gemm_params &p, int splits) { return (p.K / 64 + splits - 1) / splits; }
+
 // The first pass of a split-K GEMM as a strided-batched problem over the K slices.
 miw::gemm_params splitk_slices(const miw::gemm_params &p, int splits, void *ws)
 {
     miw::gemm_params q = p;
-    const long klen = p.K / splits;
+    const long klen = slice_slots(p, splits) * 64, last = p.K - (splits - 1) * klen;
     q.K = klen;
+    q.k_last = last < klen ? last : 0;
     q.C = nullptr; q.use_c = 0; q.alpha = 1.0f; q.beta = 0.0f;
     q.D = ws;
     q.c_row = q.d_row = p.d_row;
@@ -1021,7 +1026,7 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     static char dummy alignas(128);
     // Variant and estimated duration of s slices (s = 1: the plain launch); false when no tiled kernel fits.
     auto try_splits = [&](const miw::gemm_params &o, bool in_place, int s, int *variant, miw::kwave_tile *kw, double *us) {
-        if (o.K % (64l * s)) return false;
+        if (o.K % 64) return false;
         if (s == 1) {
             if (!pick_tiled(o, d->c_type, d->d_type, false, 0, in_place, us)) return false;
             *variant = pick_variant(o, d->c_type, d->d_type, false, 0, in_place, kw);
@@ -1050,16 +1055,38 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     miw::kwave_tile kw = {0, 0};
     double us = 0.0;
     // The slice count with the shortest estimated duration, among 1 (no second pass) and the counts up to 64 that leave
-    // every slice two LDS slots' worth of K or more; 0 when none fits.
-    auto choose = [&](const miw::gemm_params &o, bool in_place) {
-        int best = 0, v;
+    // every slice two LDS slots' worth of K or more; 0 when none fits.  equal: slices of one length only.  Of the others, whose last slice is shorter, those
+    // that fill the CUs once or twice with tiles of some size, and no more (a search over all counts took 27 us per call, as
+    // long as the launches), and that add up no fewer sums over K, four per slice where wavefronts share it, than the
+    // best equal ones: fewer and longer sums are further from the exact result (448x384x18944: 3.1e-7 with eight, 3.6e-7 with six).
+    // Equal slices leave CUs without work where K / 64 has no fitting divisor: 160x208x29312 43.4 us in two, 14.5 in twelve;
+    // 704x336x12416 27.6 in two, 16.7 in fourteen; 192x768x28416 22.4 in twelve, 20.4 in fourteen.
+    auto choose = [&](const miw::gemm_params &o, bool in_place, bool equal) {
+        int best = 0, sums = 0;
         double best_us = 0.0;
-        miw::kwave_tile t;
-        for (int s = 1; s <= 64 && (s == 1 || o.K / s >= 128); s++) {
-            if (bytes(s) > cap) break;
-            if (!try_splits(o, in_place, s, &v, &t, &us)) continue;
-            if (best == 0 || us < 0.97 * best_us) { best = s; best_us = us; }
-        }
+        auto consider = [&](int s, int least) {
+            int v;
+            miw::kwave_tile t;
+            if ((s > 1 && o.K / s < 128) || bytes(s) > cap || !try_splits(o, in_place, s, &v, &t, &us)) return;
+            const int n = s * (t.bi ? 4 : 1);
+            if (n >= least && (best == 0 || us < 0.97 * best_us)) { best = s; best_us = us; sums = n; }
+        };
+        for (int s = 1; s <= 64; s++)
+            if (o.K % (64l * s) == 0) consider(s, 0);
+        if (equal || best == 0) return best;
+        unsigned long filling = 0;  // bit s - 1: count s
+        const long I = o.d_row ? o.N : o.M, J = o.d_row ? o.M : o.N;
+        for (const auto &[bi, bj] : {std::pair{256, 128}, {128, 256}, {128, 128}, {64, 64}, {64, 32}, {32, 64}, {32, 32}})
+            for (int rounds = 1; rounds <= 2; rounds++) {
+                const long most = std::min(64l, rounds * (long)cu_count() / (((I + bi - 1) / bi) * ((J + bj - 1) / bj)));
+                if (most < 1) continue;
+                // (as few slices as have no more than that many slots)
+                const long slots = slice_slots(o, (int)most), s = (o.K / 64 + slots - 1) / slots;
+                filling |= 1ul << (s - 1);
+            }
+        const int least = sums;
+        for (int s = 2; s <= 64; s++)
+            if ((filling >> (s - 1) & 1) && o.K % (64l * s)) consider(s, least);
         return best;
     };
     // The count is chosen from what the query for the workspace knows: operands on whole cache lines, C and D apart.
@@ -1068,12 +1095,31 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     lines.A = lines.B = (const _Float16 *)&dummy;
     lines.C = p.use_c ? &dummy : nullptr;
     lines.D = &dummy;
-    int count = splits ? splits : choose(lines, false);
+    // (a last slice shorter than the others: only with the count that is chosen here, and not for a workspace too small for it)
+    int count = splits;
+    if (splits == 0 || p.K % (64l * splits)) {
+        // (a program asks for the workspace and then calls: the thread's last choice is kept)
+        struct choice {
+            miw_gemm_desc desc;
+            size_t cap;
+            int cus, count = -1;
+        };
+        static thread_local choice last;
+        if (last.count < 0 || memcmp(&last.desc, d, sizeof *d) != 0 || last.cap != cap || last.cus != cu_count()) {
+            last.desc = *d;
+            last.cap = cap;
+            last.cus = cu_count();
+            last.count = choose(lines, false, false);
+        }
+        count = last.count;
+        if (splits && count != splits) count = 0;
+        if (!splits && bytes(count) > room) count = choose(lines, false, true);
+    }
     const bool runs = count && try_splits(p, shares, count, &variant, &kw, &us);
     if (!runs || bytes(count) > room) {
         // Addresses off 16 bytes, C in D's place with extents that no tile divides, or a workspace of another size than
         // the query's: what the real operands alone would choose.
-        const int other = splits ? 0 : choose(p, shares);
+        const int other = splits ? 0 : choose(p, shares, true);
         if (other && bytes(other) <= room) {
             count = other;
             try_splits(p, shares, count, &variant, &kw, &us);

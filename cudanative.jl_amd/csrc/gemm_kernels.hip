@@ -53,7 +53,7 @@ bool pp_folds(const tiled_params &p, int c_type);
 int pp_lds(int bm, int bn, bool xk, bool yk);
 const void *w128_kernel(bool xk, bool yk, int c_type, int d_type);
 const void *pp64_kernel(int bm, int bn, bool xk, bool yk, int c_type, int d_type, bool f16acc);
-const void *kwave_kernel(int bi, int bj, bool xk, bool yk, int *lds_bytes);
+const void *kwave_kernel(int bi, int bj, bool xk, bool yk, bool short_member, int *lds_bytes);
 hipError_t launch_kwave(const void *fn, const tiled_params &t, int c_type, int d_type, dim3 grid, int lds_bytes, hipStream_t s);
 
 
@@ -165,7 +165,9 @@ static tiled_params canonical(const gemm_params &g, int bi, int bj, bool *xk, bo
     }
     p.C = g.C; p.D = g.D;
     p.K = (int)g.K;
+    p.short_member = g.k_last ? (int)g.batch - 1 : -1;
     p.work = 0;
+    if (g.k_last) p.k_short = (int)g.k_last;
     p.c_spread = 0;
     p.ldc = g.ldc; p.ldd = g.ldd; p.sc = g.sc; p.sd = g.sd;
     p.use_c = g.use_c;
@@ -184,7 +186,7 @@ hipError_t launch_gemm_kwave(kwave_tile t, const gemm_params &g, int c_type, int
     bool xk, yk;
     const tiled_params p = canonical(g, t.bi, t.bj, &xk, &yk);
     int lds_bytes;
-    const void *fn = kwave_kernel(t.bi, t.bj, xk, yk, &lds_bytes);
+    const void *fn = kwave_kernel(t.bi, t.bj, xk, yk, g.k_last != 0, &lds_bytes);
     if (!fn || p.I < t.bi || p.J < t.bj || p.K < KGRAN) return hipErrorInvalidValue;
     hipError_t e = allow_dynamic_lds(fn, lds_bytes);
     if (e != hipSuccess) return e;
@@ -194,6 +196,7 @@ hipError_t launch_gemm_kwave(kwave_tile t, const gemm_params &g, int c_type, int
 hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type, bool f16acc, int cus, hipStream_t s)
 {
     const tiled_variant &v = g_variants[i];
+    if (g.k_last && (v.kind == KIND_PINGPONG32 || v.kind == KIND_WAVE128)) return hipErrorInvalidValue;
     bool xk, yk;
     tiled_params p = canonical(g, v.bm, v.bn, &xk, &yk);
 
@@ -237,58 +240,90 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
 // Second pass of the split-K GEMM.  The first pass left `splits` Float32 partial products in
 // `ws`, each I x J with I contiguous (canonical form: I runs along D's contiguous dimension);
 // this adds them in slice order and applies the scalars: D = alpha * sum_s P_s + beta * C.
-// One lane owns four consecutive i of one j.
+// One lane owns four consecutive i of one j.  Bound by the launch and the memory's latency: C and up to sixteen slices are
+// on the way at a time (four at a time, and C behind them: 512x512x16384 in sixteen slices 18.6 us, 17.8 like this;
+// 128x128x32768 12.5 and 10.9).
+struct reduce_params {
+    const float *ws;
+    const void *C;
+    void *D;
+    int splits;
+    unsigned quads_m, quads_s;  // quotient() by I / 4 where the lanes' numbers fit in 31 bits (quads_m 0: they do not)
+    long I, J, ldc, ldd;
+    int use_c, c_trans;
+    int whole;  // four elements of C and of D may be moved at once
+    float alpha, beta;
+};
 template <class CT, class DT>
-__global__ __launch_bounds__(256) void k_splitk_reduce(const float *ws, int splits, long I, long J, const CT *C, DT *D,
-                                                       long ldc, long ldd, int use_c, int c_trans, float alpha, float beta)
+__global__ __launch_bounds__(256) void k_splitk_reduce(reduce_params p)
 {
-    const long quads = I / 4;
-    const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= quads * J) return;
-    const long j = idx / quads, i = (idx - j * quads) * 4;
-    const float *src = ws + j * I + i;
-    // (four slices at a time are on the way; one at a time each addition waits for the memory's latency)
-    const long slice = I * J;
-    float4_t sum = *(const float4_t *)src;
-    int s = 1;
-    for (; s + 4 <= splits; s += 4) {
-        float4_t v[4];
+    using c4_t = CT __attribute__((ext_vector_type(4)));
+    using d4_t = DT __attribute__((ext_vector_type(4)));
+    const long quads = p.I / 4;
+    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= quads * p.J) return;
+    const long j = p.quads_m ? (long)quotient((int)idx, p.quads_m, p.quads_s) : idx / quads, i = (idx - j * quads) * 4;
+    const CT *C = (const CT *)p.C;
+    c4_t c;
+    if (p.use_c) {
+        if (p.whole && !p.c_trans) {
+            c = *(const c4_t *)(C + j * p.ldc + i);
+        } else {
 #pragma unroll
-        for (int u = 0; u < 4; u++) v[u] = *(const float4_t *)(src + (s + u) * slice);
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) sum[e] += v[u][e];
+            for (int e = 0; e < 4; e++) c[e] = p.c_trans ? C[(i + e) * p.ldc + j] : C[j * p.ldc + i + e];
+        }
     }
-    float4_t v[3];
+    const float *src = p.ws + j * p.I + i;
+    const long slice = p.I * p.J;
+    constexpr int FLIGHT = 16;
+    float4_t sum = {-0.f, -0.f, -0.f, -0.f};  // (adds nothing, whatever the sign of what it is added to)
+    for (int s = 0; s < p.splits; s += FLIGHT, src += FLIGHT * slice) {
+        float4_t v[FLIGHT];
 #pragma unroll
-    for (int u = 0; u < 3; u++)
-        if (s + u < splits) v[u] = *(const float4_t *)(src + (s + u) * slice);
+        for (int u = 0; u < FLIGHT; u++)
+            if (s + u < p.splits) v[u] = *(const float4_t *)(src + u * slice);
 #pragma unroll
-    for (int u = 0; u < 3; u++)
-        if (s + u < splits)
+        for (int u = 0; u < FLIGHT; u++)
+            if (s + u < p.splits)
 #pragma unroll
-            for (int e = 0; e < 4; e++) sum[e] += v[u][e];
+                for (int e = 0; e < 4; e++) sum[e] += v[u][e];
+    }
+    d4_t d;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-        float v = alpha * sum[e];
-        if (use_c) {
-            const float c = (float)(c_trans ? C[(i + e) * ldc + j] : C[j * ldc + i + e]);
-            v = __builtin_fmaf(beta, c, v);
-        }
-        D[j * ldd + i + e] = (DT)v;
+        float v = p.alpha * sum[e];
+        if (p.use_c) v = __builtin_fmaf(p.beta, (float)c[e], v);
+        d[e] = (DT)v;
+    }
+    DT *D = (DT *)p.D + j * p.ldd + i;
+    if (p.whole) {
+        *(d4_t *)D = d;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) D[e] = d[e];
     }
 }
 
 hipError_t launch_splitk_reduce(const gemm_params &g, int c_type, int d_type, int splits, const float *ws, hipStream_t s)
 {
-    const long I = g.d_row ? g.N : g.M, J = g.d_row ? g.M : g.N;
-    const int c_trans = g.d_row ? g.c_row == 0 : g.c_row != 0;
-    const long lanes = I / 4 * J;
-    const dim3 grid((unsigned)((lanes + 255) / 256)), block(256);
-#define MIW_REDUCE(CT, DT)                                                                                          \
-    hipLaunchKernelGGL((k_splitk_reduce<CT, DT>), grid, block, 0, s, ws, splits, I, J, (const CT *)g.C, (DT *)g.D, \
-                       g.ldc, g.ldd, g.use_c, c_trans, g.alpha, g.beta)
+    reduce_params p;
+    p.ws = ws; p.C = g.C; p.D = g.D;
+    p.splits = splits;
+    p.I = g.d_row ? g.N : g.M;
+    p.J = g.d_row ? g.M : g.N;
+    p.ldc = g.ldc; p.ldd = g.ldd;
+    p.use_c = g.use_c;
+    p.c_trans = g.d_row ? g.c_row == 0 : g.c_row != 0;
+    p.alpha = g.alpha; p.beta = g.beta;
+    const long lanes = p.I / 4 * p.J;
+    p.quads_s = 0;
+    p.quads_m = lanes + 256 < (1l << 31) ? multiplier(p.I / 4, &p.quads_s) : 0;
+    auto whole = [](const void *x, long ld, int type) { return (uintptr_t)x % (type == 0 ? 8 : 16) == 0 && ld % 4 == 0; };
+    p.whole = whole(g.D, g.ldd, d_type) && (!g.use_c || p.c_trans || whole(g.C, g.ldc, c_type));
+    // (one wavefront per workgroup where four each would leave CUs without one)
+    const unsigned threads = lanes < 256 * 256 ? 64 : 256;
+    const dim3 grid((unsigned)((lanes + threads - 1) / threads)), block(threads);
+#define MIW_REDUCE(CT, DT) hipLaunchKernelGGL((k_splitk_reduce<CT, DT>), grid, block, 0, s, p)
     if (c_type == 0 && d_type == 0) MIW_REDUCE(half_t, half_t);
     else if (c_type == 0) MIW_REDUCE(half_t, float);
     else if (d_type == 0) MIW_REDUCE(float, half_t);

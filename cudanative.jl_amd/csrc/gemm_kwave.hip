@@ -89,9 +89,8 @@ struct wave_operand {
 //   - The partial sums meet in LDS after the loop and are added in wavefront order.
 // With Float16 D and no C: 256x256x2048 9.9 us -> 6.3, 128x4096x4096 15.3 -> 12.3, 48x4096x4096 17.4 -> 9.9, against
 // the 64x64 tile and k_gemm_skinny.
-template <int BI, int BJ, bool XK, bool YK>
-__global__ __launch_bounds__(64 * KWAVES) __attribute__((amdgpu_waves_per_eu(2)))
-void k_gemm_kwave(kwave_params kp)
+template <int BI, int BJ, bool XK, bool YK, bool SHORT>
+__device__ __attribute__((always_inline)) inline void gemm_kwave(const kwave_params &kp)
 {
     using shape = kwave_shape<BI, BJ>;
     constexpr int TI = BI / 16, TJ = BJ / 16, NS = shape::SLOTS, XBYTES = BI * KGRAN * 2;
@@ -126,6 +125,7 @@ void k_gemm_kwave(kwave_params kp)
         }
     }
 
+    const int K = SHORT ? member_k(p, at.bt) : p.K;
     const half_t *X = p.X + bt * p.sx + (XK ? (long)i0 * p.ldx : (long)i0);
     const half_t *Y = p.Y + bt * p.sy + (YK ? (long)j0 * p.ldy : (long)j0);
     const long xk = XK ? 1 : p.ldx, yk = YK ? 1 : p.ldy;  // elements from one k to the next
@@ -136,7 +136,7 @@ void k_gemm_kwave(kwave_params kp)
 
     // Slots wave, wave + 4, ... of 64 k-values; the k-values that 64 leaves are the last slot, shifted back to
     // end at K, of the wavefront whose turn it is.
-    const int whole = p.K / KGRAN, tail_skip = whole * KGRAN == p.K ? 0 : (whole + 1) * KGRAN - p.K;
+    const int whole = K / KGRAN, tail_skip = whole * KGRAN == K ? 0 : (whole + 1) * KGRAN - K;
     const int own = (whole - wave + KWAVES - 1) / KWAVES;
     const bool has_tail = tail_skip && wave == whole % KWAVES;
     const int total = own + (has_tail ? 1 : 0);
@@ -144,7 +144,7 @@ void k_gemm_kwave(kwave_params kp)
     const half_t *xn, *yn;  // the slot being requested
     unsigned dst;
     auto begin_request = [&](int n, int slot) MIW_INLINE {
-        const long k = n < own ? (long)(wave + KWAVES * n) * KGRAN : (long)p.K - KGRAN;
+        const long k = n < own ? (long)(wave + KWAVES * n) * KGRAN : (long)K - KGRAN;
         xn = X + k * xk;
         yn = Y + k * yk;
         dst = ring + (unsigned)(slot * shape::SLOT);
@@ -307,14 +307,30 @@ void k_gemm_kwave(kwave_params kp)
     }
 }
 
+template <int BI, int BJ, bool XK, bool YK>
+__global__ __launch_bounds__(64 * KWAVES) __attribute__((amdgpu_waves_per_eu(2)))
+void k_gemm_kwave(kwave_params kp)
+{
+    gemm_kwave<BI, BJ, XK, YK, false>(kp);
+}
+
+// Slices of K of which the last one is shorter.  (A kernel of its own: the question alone, in front of the first request,
+// makes a launch of 8.14 us 8.19.)
+template <int BI, int BJ, bool XK, bool YK>
+__global__ __launch_bounds__(64 * KWAVES) __attribute__((amdgpu_waves_per_eu(2)))
+void k_gemm_kwave_slices(kwave_params kp)
+{
+    gemm_kwave<BI, BJ, XK, YK, true>(kp);
+}
+
 // Kernel for a tile and operand layouts, or null when there is none.
-const void *kwave_kernel(int bi, int bj, bool xk, bool yk, int *lds_bytes)
+const void *kwave_kernel(int bi, int bj, bool xk, bool yk, bool short_member, int *lds_bytes)
 {
     auto is = [&](int i, int j, bool x, bool y) { return bi == i && bj == j && xk == x && yk == y; };
 #define MIW_KWAVE(I, J, X, Y)                         \
-    if (is(I, J, X, Y)) {                             \
-        *lds_bytes = kwave_shape<I, J>::RING;         \
-        return (const void *)k_gemm_kwave<I, J, X, Y>; \
+    if (is(I, J, X, Y)) {                                                                                                       \
+        *lds_bytes = kwave_shape<I, J>::RING;                                                                                   \
+        return short_member ? (const void *)k_gemm_kwave_slices<I, J, X, Y> : (const void *)k_gemm_kwave<I, J, X, Y>; \
     }
     MIW_KWAVE(64, 32, true, true)
     MIW_KWAVE(64, 32, false, true)
@@ -358,7 +374,7 @@ static long kwave_groups(const gemm_params &g, kwave_tile t, bool in_place)
     bool xk, yk;
     layouts(g, &xk, &yk);
     int lds;
-    if (I < t.bi || J < t.bj || !kwave_kernel(t.bi, t.bj, xk, yk, &lds)) return 0;
+    if (I < t.bi || J < t.bj || !kwave_kernel(t.bi, t.bj, xk, yk, false, &lds)) return 0;
     if (in_place && (I % t.bi || J % t.bj)) return 0;  // (edge tiles overlap their neighbours)
     return (I + t.bi - 1) / t.bi * ((J + t.bj - 1) / t.bj) * g.batch;
 }

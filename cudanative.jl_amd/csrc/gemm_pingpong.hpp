@@ -749,9 +749,10 @@ void k_gemm_pp64(tiled_params p)
         return c;
     };
 
-    const int NP = (p.K + KGRAN - 1) / KGRAN;
+    const int K = has_slices<CT, DT, F16ACC> ? member_k(p, at.bt) : p.K;
+    const int NP = (K + KGRAN - 1) / KGRAN;
     // K tail: the last pair starts at K - 64; tail_skip of its k-values repeat the pair before
-    const int tail_skip = NP * KGRAN - p.K;
+    const int tail_skip = NP * KGRAN - K;
     const unsigned wave_dst = (unsigned)(uintptr_t)lds + (unsigned)wave * 1024u;
     int next = 0;          // next pair to request
     unsigned woff = 0;     // byte offset in the ring of the slot it goes to

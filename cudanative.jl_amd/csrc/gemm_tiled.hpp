@@ -87,6 +87,7 @@ struct tiled_params {
     // the last slot is shifted back to end at K, and the k-values it repeats from the slot before
     // (the first 64 * ceil(K / 64) - K of it) are zeroed in the fragments of both operands.
     int I, J, K;
+    int short_member;  // batch member with k_short k-values in place of K (a multiple of 64), or -1
     long ldx, ldy, sx, sy;
     const void *C;
     void *D;
@@ -96,7 +97,11 @@ struct tiled_params {
     float alpha, beta;
     // Workgroups that walk several tiles (k_gemm_pp): number of tiles over the whole batch; a workgroup takes tile
     // blockIdx.x, then every gridDim.x-th.  0: one tile per workgroup.  Needs K of four slots or more.
-    int work;
+    // (Its place is k_short's in the kernels that slices of K run on: 184 bytes of arguments in place of 176 cost launches of 6 us 0.05.)
+    union {
+        int work;
+        int k_short;  // see short_member
+    };
     int c_spread;  // k_gemm_pp64: the workgroups ask for C at eight different times of their K loops, not all at its start
 #ifdef MIW_PP_TS
     long long *ts;  // measurement builds: 10 counters per wavefront (see k_gemm_pp64), or null
@@ -193,6 +198,21 @@ __device__ inline tile_place workgroup_tile(const tiled_params &p, int bi, int b
     return tile_at(p, (int)(blockIdx.x + blockIdx.y * (unsigned)p.span), (int)blockIdx.y, bi, bj);
 }
 
+// Kernels on which slices of K run: their products are Float32.
+template <class CT, class DT, bool F16ACC>
+constexpr bool has_slices = !F16ACC && __is_same(CT, float) && __is_same(DT, float);
+// k-values of a batch member.  (A branch on an argument: where no member has fewer, nothing waits for the member's number.)
+__device__ inline int member_k(const tiled_params &p, int bt)
+{
+    int k = p.K;
+    if (p.short_member >= 0) {
+        int own = bt == p.short_member ? p.k_short : p.K;
+        asm volatile("" : "+s"(own));
+        k = own;
+    }
+    return k;
+}
+
 // Number of a tile over the whole launch, from its number as tile_at takes it (which counts on over the members where there is
 // a span): measurement builds write their records there.
 __host__ __device__ inline long launch_tile(int id, int span, unsigned member, unsigned member_tiles)
@@ -205,7 +225,7 @@ __host__ __device__ inline long launch_tile(int id, int span, unsigned member, u
 // where each waits for memory (0.15 us of a launch); waiting at the start for C's and D's too costs 0.05.
 __device__ inline void fetch_operand_arguments(const tiled_params &p)
 {
-    asm volatile("" ::"s"(p.X), "s"(p.Y), "s"(p.I), "s"(p.J), "s"(p.K), "s"(p.ldx), "s"(p.ldy), "s"(p.sx), "s"(p.sy));
+    asm volatile("" ::"s"(p.X), "s"(p.Y), "s"(p.I), "s"(p.J), "s"(p.K), "s"(p.short_member), "s"(p.ldx), "s"(p.ldy), "s"(p.sx), "s"(p.sy));
 }
 __device__ inline void fetch_result_arguments(const tiled_params &p)
 {
@@ -577,9 +597,10 @@ void k_gemm_tiled(tiled_params p)
         }
     }
 
-    const int NP = (p.K + KGRAN - 1) / KGRAN;  // slots' worth of K ("pairs" of steps)
+    const int K = has_slices<CT, DT, F16ACC> ? member_k(p, at.bt) : p.K;
+    const int NP = (K + KGRAN - 1) / KGRAN;  // slots' worth of K ("pairs" of steps)
     // K tail: the last pair starts at K - 64; tail_skip of its k-values repeat the pair before
-    const int tail_skip = NP * KGRAN - p.K;
+    const int tail_skip = NP * KGRAN - K;
     const unsigned wave_dst = (unsigned)(uintptr_t)lds + (unsigned)wave * 1024u;
     constexpr int NLX = xload::NLOAD, NLY = yload::NLOAD, LPAIR = NLX + NLY;  // loads per thread and pair
     int next = 0;          // next pair to request

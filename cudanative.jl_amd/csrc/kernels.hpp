@@ -20,6 +20,9 @@ struct gemm_params {
     int a_row, b_row, c_row, d_row;  // 1: row major, 0: column major
     int use_c;
     float alpha, beta;
+    // Slices of K as a batch (split-K): k-values of the last member where they are fewer than K, a multiple of 64; else 0.
+    // Not for the kernels with 256x256 tiles, which may walk from member to member.
+    long k_last;
 };
 
 // --- frag_kernels.hip

@@ -1240,6 +1240,42 @@ def test_splitk_random_types_scalars_and_padding(gpu, orc):
     assert orc.normalized_error(g, D, orc.gemm_f64(g, A, B, None)) <= TIGHT_F32
 
 
+@pytest.mark.parametrize("M,N,K", [(192, 64, 64 * 67), (160, 208, 64 * 229), (64, 64, 64 * 193), (704, 336, 64 * 97), (448, 320, 64 * 149), (640, 640, 64 * 181)])
+@pytest.mark.parametrize("al,bl,dl", itertools.product((0, 1), repeat=3))
+def test_splitk_slices_of_unequal_length(gpu, orc, M, N, K, al, bl, dl):
+    """K of a prime number of slots: a chosen count has a last slice that is shorter than the others, down to one slot, on tiles of
+    128, 64 and on the kernel whose wavefronts share K; sums of small integers are exact.  C is in D's place in one of two calls."""
+    G = gpu.GEMM
+    g = orc.GemmDesc(M=M, N=N, K=K, a_layout=al, b_layout=bl, c_layout=dl, d_layout=dl, alpha=0.5, beta=-2.0)
+    A, B, C = _inputs(orc, g, M + N + K + al + 2 * bl, ints=True)
+    desc = G.make_desc(M, N, K, a_layout=_W(gpu, al), b_layout=_W(gpu, bl), c_layout=_W(gpu, dl), d_layout=_W(gpu, dl), alpha=0.5, beta=-2.0)
+    n, nbytes = G.splitk_workspace(desc)
+    assert n > 1 and K // 64 % n and nbytes == 4 * n * M * N
+    assert G.splitk_workspace(desc, n) == (n, nbytes)
+    want = orc.gemm(g, A, B, C)
+    assert np.array_equal(_run_splitk(gpu, orc, g, A, B, C), want)
+    dA, dB, dD = (gpu.DeviceArray(x) for x in (A, B, C))
+    G.gemm_splitk(dA, dB, dD, dD, desc)
+    gpu.synchronize()
+    assert np.array_equal(dD.to_host(), want)
+
+
+@pytest.mark.parametrize("splits", [2, 15, 16, 17, 33])
+@pytest.mark.parametrize("ct,dt,offset", [(0, 0, 0), (0, 1, 0), (1, 0, 0), (1, 1, 0), (0, 0, 1), (1, 1, 1)])
+def test_splitk_second_kernel_adds_any_number_of_slices(gpu, orc, splits, ct, dt, offset):
+    """Counts around the sixteen slices that are on the way together, C and D of each type and off the addresses of four-element
+    accesses; a D small enough for workgroups of one wavefront and one that is not."""
+    for M, N in ((80, 64), (512, 528)):
+        g = orc.GemmDesc(M=M, N=N, K=64 * splits, c_type=ct, d_type=dt, beta=2.0, ldc=M + 2 * offset, ldd=M + 2 * offset)
+        A, B, C = _inputs(orc, g, 700 + splits + offset, ints=True)
+        A, B = np.sign(A).astype(A.dtype), np.sign(B).astype(B.dtype)  # sums of at most 64 * splits, whole in Float16 too
+        want = orc.gemm(g, A, B, C)
+        assert np.array_equal(_run_splitk(gpu, orc, g, A, B, C, splits, prefill=3.0)[:M], want[:M]), (M, N)
+        got = _run_splitk(gpu, orc, g, A, B, C, splits, prefill=0.0)
+        cols = np.arange(N)[:, None] * (M + 2 * offset) + np.arange(M)
+        assert np.array_equal(got[cols], want[cols]), (M, N)
+
+
 def test_splitk_in_place_on_extents_that_no_tile_divides(gpu, orc):
     """One slice by the query, and no tile for it when C is D: the plain launch; with room for slices, slices."""
     G = gpu.GEMM

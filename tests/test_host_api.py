@@ -576,6 +576,37 @@ def test_splitk_takes_the_workspace_its_query_reports(miw):
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stderr
 
 
+def test_splitk_slices_of_unequal_length_are_only_chosen(miw):
+    """A count that leaves the last slice shorter is taken where the library chooses it, and asked for by that number; any other such
+    count is refused, and a workspace that only slices of one length fit gets those, as one that is too small for them is refused."""
+    import subprocess, sys
+    code = ("import sys, ctypes, random; sys.path.insert(0, %r); from tests.conftest import load_package; m = load_package();\n"
+            "L, G, W = m._lib, m.GEMM, m.WMMA; lib = L.load(); rng = random.Random(11); p = lambda i: ctypes.c_void_p((1 << 32) + (i << 40))\n"
+            "unequal = 0\n"
+            "for _ in range(400):\n"
+            "    M, N, K = 16 * rng.randint(4, 64), 16 * rng.randint(4, 64), 64 * rng.randint(32, 512)\n"
+            "    d = G.make_desc(M, N, K, a_layout=rng.choice((W.RowMajor, W.ColMajor)), b_layout=rng.choice((W.RowMajor, W.ColMajor)))\n"
+            "    n, nbytes = G.splitk_workspace(d)\n"
+            "    assert nbytes == (0 if n == 1 else 4 * n * M * N)\n"
+            "    call = lambda splits, room: lib.miw_gemm_splitk(ctypes.byref(d), p(0), p(1), p(2), p(3), splits, p(4), room, None)\n"
+            "    for s in range(2, 24):\n"
+            "        splits, size = ctypes.c_int(), ctypes.c_size_t()\n"
+            "        rc = lib.miw_gemm_splitk_workspace(ctypes.byref(d), s, ctypes.byref(splits), ctypes.byref(size))\n"
+            "        assert rc == (0 if s == n or K // 64 %% s == 0 else L.ERR_UNSUPPORTED), (M, N, K, s, n, rc)\n"
+            "    if K // 64 %% n == 0: continue\n"
+            "    unequal += 1\n"
+            "    assert call(n, nbytes) == call(0, nbytes) == L.ERR_NOT_INITIALIZED\n"
+            "    assert call(n, nbytes - 4) == L.ERR_INVALID_VALUE\n"
+            "    equal = [s for s in range(1, 65) if K // 64 %% s == 0 and K // s >= 128]\n"
+            "    fits = [call(0, 4 * s * M * N if s > 1 else 0) == L.ERR_NOT_INITIALIZED for s in equal if s < n]\n"
+            "    assert fits == sorted(fits), (M, N, K, n, fits)\n"
+            "    if all(s < n for s in equal): assert fits[-1]\n"
+            "assert unequal > 100, unequal\n"
+            "print('ok')\n") % ROOT
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0 and out.stdout.strip() == "ok", out.stderr
+
+
 def test_tiled_gemm_kernels_are_not_launchable_by_name(miw):
     """The LDS-tiled kernels take a private argument block, a fixed workgroup and dynamic LDS: they can be
     looked up (attribute queries) but miw_launch refuses them and points to miw_gemm."""
