@@ -53,8 +53,7 @@ bool pp_folds(const tiled_params &p, int c_type);
 int pp_lds(int bm, int bn, bool xk, bool yk);
 const void *w128_kernel(bool xk, bool yk, int c_type, int d_type);
 const void *pp64_kernel(int bm, int bn, bool xk, bool yk, int c_type, int d_type, bool f16acc);
-const void *kwave_kernel(int bi, int bj, bool xk, bool yk, bool short_member, int *lds_bytes);
-hipError_t launch_kwave(const void *fn, const tiled_params &t, int c_type, int d_type, dim3 grid, int lds_bytes, hipStream_t s);
+const void *kwave_kernel(int bi, int bj, bool xk, bool yk, int c_type, int d_type, bool slices, int *lds_bytes);
 
 
 // Tile shape in canonical (I, J) terms: bm applies to I, bn to J.
@@ -184,13 +183,14 @@ static tiled_params canonical(const gemm_params &g, int bi, int bj, bool *xk, bo
 hipError_t launch_gemm_kwave(kwave_tile t, const gemm_params &g, int c_type, int d_type, hipStream_t s)
 {
     bool xk, yk;
-    const tiled_params p = canonical(g, t.bi, t.bj, &xk, &yk);
+    tiled_params p = canonical(g, t.bi, t.bj, &xk, &yk);
     int lds_bytes;
-    const void *fn = kwave_kernel(t.bi, t.bj, xk, yk, g.k_last != 0, &lds_bytes);
+    const void *fn = kwave_kernel(t.bi, t.bj, xk, yk, g.use_c ? c_type : NO_C, d_type, g.k_last != 0, &lds_bytes);
     if (!fn || p.I < t.bi || p.J < t.bj || p.K < KGRAN) return hipErrorInvalidValue;
     hipError_t e = allow_dynamic_lds(fn, lds_bytes);
     if (e != hipSuccess) return e;
-    return launch_kwave(fn, p, c_type, d_type, dim3((unsigned)(p.tiles_i * p.tiles_j), (unsigned)g.batch), lds_bytes, s);
+    void *args[] = {&p};
+    return hipLaunchKernel(fn, dim3((unsigned)(p.tiles_i * p.tiles_j), (unsigned)g.batch), dim3(256), args, (size_t)lds_bytes, s);
 }
 
 hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type, bool f16acc, int cus, hipStream_t s)
@@ -212,7 +212,9 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
     p.c_spread = v.kind == KIND_PINGPONG64 && v.bm * v.bn > 128 * 128 && g.use_c &&
                  (long)p.I * p.J * g.batch * (c_type == 0 ? 2 : 4) >= (12l << 20);
     const bool fold = v.kind == KIND_PINGPONG32 && pp_folds(p, c_type);
-    const void *fn = pick_kernel(i, xk, yk, c_type, d_type, f16acc, fold);
+    // (slices of K run on the instances with a Float32 C, see has_slices)
+    const bool without_c = v.kind == KIND_PIPELINED && !g.use_c && !g.k_last;
+    const void *fn = pick_kernel(i, xk, yk, without_c ? NO_C : c_type, d_type, f16acc, fold);
     if (!fn) return hipErrorInvalidValue;
     // (the 64-k ping-pong kernels stage a Float16 C tile beside the ring where both fit)
     const int c_stage = v.kind == KIND_PINGPONG64 && f16acc && v.lds_bytes + v.bm * v.bn * 2 <= 160 * 1024 ? v.bm * v.bn * 2 : 0;

@@ -5,11 +5,6 @@
 
 namespace miw {
 
-struct kwave_params {
-    tiled_params t;
-    int c_f32, d_f32;
-};
-
 constexpr int KWAVES = 4;
 
 template <int BI, int BJ>
@@ -89,15 +84,15 @@ struct wave_operand {
 //   - The partial sums meet in LDS after the loop and are added in wavefront order.
 // With Float16 D and no C: 256x256x2048 9.9 us -> 6.3, 128x4096x4096 15.3 -> 12.3, 48x4096x4096 17.4 -> 9.9, against
 // the 64x64 tile and k_gemm_skinny.
-template <int BI, int BJ, bool XK, bool YK, bool SHORT>
-__device__ __attribute__((always_inline)) inline void gemm_kwave(const kwave_params &kp)
+template <int BI, int BJ, bool XK, bool YK, class CT, class DT, bool SHORT>
+__device__ __attribute__((always_inline)) inline void gemm_kwave(const tiled_params &p)
 {
+    constexpr bool HAS_C = !__is_same(CT, no_c_t);
     using shape = kwave_shape<BI, BJ>;
     constexpr int TI = BI / 16, TJ = BJ / 16, NS = shape::SLOTS, XBYTES = BI * KGRAN * 2;
     using xoperand = wave_operand<BI, XK>;
     using yoperand = wave_operand<BJ, YK>;
     constexpr int LOADS = xoperand::NLOAD + yoperand::NLOAD;
-    const tiled_params &p = kp.t;
 
     extern __shared__ __attribute__((aligned(128))) char smem[];
     MIW_LDS char *lds = (MIW_LDS char *)smem;
@@ -114,15 +109,13 @@ __device__ __attribute__((always_inline)) inline void gemm_kwave(const kwave_par
     constexpr int UNITS = BI * BJ / 4 <= 64 * KWAVES ? 1 : BI * BJ / 4 / (64 * KWAVES), STEP = 64 * KWAVES / (BI / 4);
     const bool takes = BI * BJ / 4 >= 64 * KWAVES || tid < BI * BJ / 4;
     const long oi = i0 + 4 * (tid % (BI / 4)), oj = j0 + tid / (BI / 4);
-    float4_t cf[UNITS];
-    half4_t ch[UNITS];
-    if (takes && p.use_c && !p.c_trans) {
-        const long at = bt * p.sc + oj * p.ldc + oi;
+    using c4_t = CT __attribute__((ext_vector_type(4)));
+    using d4_t = DT __attribute__((ext_vector_type(4)));
+    c4_t cv[UNITS];
+    if (HAS_C && takes && !p.c_trans) {
+        const CT *at = (const CT *)p.C + bt * p.sc + oj * p.ldc + oi;
 #pragma unroll
-        for (int u = 0; u < UNITS; u++) {
-            if (kp.c_f32) cf[u] = *(const float4_t *)((const float *)p.C + at + (long)u * STEP * p.ldc);
-            else ch[u] = *(const half4_t *)((const half_t *)p.C + at + (long)u * STEP * p.ldc);
-        }
+        for (int u = 0; u < UNITS; u++) cv[u] = *(const c4_t *)(at + (long)u * STEP * p.ldc);
     }
 
     const int K = SHORT ? member_k(p, at.bt) : p.K;
@@ -285,52 +278,72 @@ __device__ __attribute__((always_inline)) inline void gemm_kwave(const kwave_par
         const long j = oj + (long)u * STEP;
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] *= p.alpha;
-        if (p.use_c) {
+        if constexpr (HAS_C) {
             float4_t c;
             if (p.c_trans) {
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    const long at = bt * p.sc + (oi + e) * p.ldc + j;
-                    c[e] = kp.c_f32 ? ((const float *)p.C)[at] : (float)((const half_t *)p.C)[at];
+                    c[e] = (float)((const CT *)p.C)[bt * p.sc + (oi + e) * p.ldc + j];
                 }
-            } else if (kp.c_f32) {
-                c = cf[u];
             } else {
-                c = float4_t{(float)ch[u][0], (float)ch[u][1], (float)ch[u][2], (float)ch[u][3]};
+                c = __builtin_convertvector(cv[u], float4_t);
             }
 #pragma unroll
             for (int e = 0; e < 4; e++) v[e] = __builtin_fmaf(p.beta, c[e], v[e]);
         }
         const long at = bt * p.sd + j * p.ldd + oi;
-        if (kp.d_f32) *(float4_t *)((float *)p.D + at) = v;
-        else *(half4_t *)((half_t *)p.D + at) = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+        *(d4_t *)((DT *)p.D + at) = __builtin_convertvector(v, d4_t);
     }
 }
 
+// A launch pays for the instructions it passes by, which it fetches from a cold cache: so the types, and whether there is a C,
+// are the instance's.  With both asked for at run time decode 16x4096x4096 takes 8.17 us, 8.02 like this, 128x4096x4096
+// 11.5 and 11.1, 640x576x1840 8.3 and 8.0, 720x656x784 with a Float32 C 6.40 and 6.25.
+// Float32 C and D.
 template <int BI, int BJ, bool XK, bool YK>
 __global__ __launch_bounds__(64 * KWAVES) __attribute__((amdgpu_waves_per_eu(2)))
-void k_gemm_kwave(kwave_params kp)
+void k_gemm_kwave(tiled_params p)
 {
-    gemm_kwave<BI, BJ, XK, YK, false>(kp);
+    gemm_kwave<BI, BJ, XK, YK, float, float, false>(p);
 }
 
-// Slices of K of which the last one is shorter.  (A kernel of its own: the question alone, in front of the first request,
-// makes a launch of 8.14 us 8.19.)
+// Other types of C and D, or no C.
+template <int BI, int BJ, bool XK, bool YK, class CT, class DT>
+__global__ __launch_bounds__(64 * KWAVES) __attribute__((amdgpu_waves_per_eu(2)))
+void k_gemm_kwave_types(tiled_params p)
+{
+    gemm_kwave<BI, BJ, XK, YK, CT, DT, false>(p);
+}
+
+// Slices of K of which the last one is shorter.  (The question alone, in front of the first request, makes a launch of 8.14 us 8.19.)
 template <int BI, int BJ, bool XK, bool YK>
 __global__ __launch_bounds__(64 * KWAVES) __attribute__((amdgpu_waves_per_eu(2)))
-void k_gemm_kwave_slices(kwave_params kp)
+void k_gemm_kwave_slices(tiled_params p)
 {
-    gemm_kwave<BI, BJ, XK, YK, true>(kp);
+    gemm_kwave<BI, BJ, XK, YK, no_c_t, float, true>(p);
 }
 
-// Kernel for a tile and operand layouts, or null when there is none.
-const void *kwave_kernel(int bi, int bj, bool xk, bool yk, bool short_member, int *lds_bytes)
+template <int BI, int BJ, bool XK, bool YK>
+static const void *kwave_types(int c_type, int d_type, bool slices)
+{
+    if (slices) return (const void *)k_gemm_kwave_slices<BI, BJ, XK, YK>;
+    if (c_type == NO_C && d_type == 0) return (const void *)k_gemm_kwave_types<BI, BJ, XK, YK, no_c_t, half_t>;
+    if (c_type == NO_C) return (const void *)k_gemm_kwave_types<BI, BJ, XK, YK, no_c_t, float>;
+    if (c_type == 0 && d_type == 0) return (const void *)k_gemm_kwave_types<BI, BJ, XK, YK, half_t, half_t>;
+    if (c_type == 0) return (const void *)k_gemm_kwave_types<BI, BJ, XK, YK, half_t, float>;
+    if (d_type == 0) return (const void *)k_gemm_kwave_types<BI, BJ, XK, YK, float, half_t>;
+    return (const void *)k_gemm_kwave<BI, BJ, XK, YK>;
+}
+
+// Kernel for a tile, operand layouts and types (c_type NO_C: no C), or null when there is none; slices: of K, the last one
+// shorter (no C, Float32).
+const void *kwave_kernel(int bi, int bj, bool xk, bool yk, int c_type, int d_type, bool slices, int *lds_bytes)
 {
     auto is = [&](int i, int j, bool x, bool y) { return bi == i && bj == j && xk == x && yk == y; };
-#define MIW_KWAVE(I, J, X, Y)                         \
-    if (is(I, J, X, Y)) {                                                                                                       \
-        *lds_bytes = kwave_shape<I, J>::RING;                                                                                   \
-        return short_member ? (const void *)k_gemm_kwave_slices<I, J, X, Y> : (const void *)k_gemm_kwave<I, J, X, Y>; \
+#define MIW_KWAVE(I, J, X, Y)                                        \
+    if (is(I, J, X, Y)) {                                            \
+        *lds_bytes = kwave_shape<I, J>::RING;                        \
+        return kwave_types<I, J, X, Y>(c_type, d_type, slices);      \
     }
     MIW_KWAVE(64, 32, true, true)
     MIW_KWAVE(64, 32, false, true)
@@ -374,7 +387,7 @@ static long kwave_groups(const gemm_params &g, kwave_tile t, bool in_place)
     bool xk, yk;
     layouts(g, &xk, &yk);
     int lds;
-    if (I < t.bi || J < t.bj || !kwave_kernel(t.bi, t.bj, xk, yk, false, &lds)) return 0;
+    if (I < t.bi || J < t.bj || !kwave_kernel(t.bi, t.bj, xk, yk, 1, 1, false, &lds)) return 0;
     if (in_place && (I % t.bi || J % t.bj)) return 0;  // (edge tiles overlap their neighbours)
     return (I + t.bi - 1) / t.bi * ((J + t.bj - 1) / t.bj) * g.batch;
 }
@@ -449,13 +462,6 @@ double kwave_estimate_us(const gemm_params &g, int c_type, int d_type, kwave_til
     const double mn = (double)g.M * (double)g.N * (double)g.batch;
     const double cd_bytes = mn * ((d_type == 0 ? 2 : 4) + (g.use_c ? (c_type == 0 ? 2 : 4) : 0));
     return 3.5 + cd_bytes / 5.5e6 + 2.0 * (double)(t.bi + t.bj) * (double)g.K / (both ? 90e3 : 70e3);
-}
-
-hipError_t launch_kwave(const void *fn, const tiled_params &t, int c_type, int d_type, dim3 grid, int lds_bytes, hipStream_t s)
-{
-    kwave_params p{t, c_type, d_type};
-    void *args[] = {&p};
-    return hipLaunchKernel(fn, grid, dim3(64 * KWAVES), args, (size_t)lds_bytes, s);
 }
 
 }  // namespace miw

@@ -509,6 +509,10 @@ constexpr int fold_tiles(int bi, int bj, int nt, int nslot)
 }
 constexpr int fold_stage_bytes(int bi, int bj, int nt, int nslot) { return (nt / 64) * 2 * fold_tiles(bi, bj, nt, nslot) * 1024; }
 
+// C's type in the instances for problems without C, and its number.
+typedef signed char no_c_t;
+constexpr int NO_C = 2;
+
 template <int BI, int BJ, int WI, int WJ, int NSLOT, bool XK, bool YK, class CT, class DT, bool F16ACC>
 __global__ __launch_bounds__(WI *WJ * 64) __attribute__((amdgpu_waves_per_eu(waves_per_simd(BI, BJ, WI *WJ * 64))))
 void k_gemm_tiled(tiled_params p)
@@ -715,7 +719,10 @@ void k_gemm_tiled(tiled_params p)
     // C laid out as D goes into registers behind the first requests: read behind the loop, two loads at a time, it waits for
     // memory once per pair of tiles (64x64 tiles: 768x1216x832 with a Float16 C 5.9 us -> 5.5, 672x864x512 5.1 -> 4.6;
     // 128x128 tiles, two workgroups per CU: 512 problems of 128^3 19.4 -> 18.9, 192x128x256 397 times 33.8 -> 32.2).
-    constexpr bool EARLY_C = !F16ACC && fold_tiles(BI, BJ, NT, NSLOT) == 0 && TI * TJ <= 16;
+    // Problems without C have instances of their own: a short launch pays for the instructions it passes by, which it fetches
+    // from a cold cache (640x640x496 4.52 us -> 4.40, 400 products of 64x128x96 7.72 -> 7.43).
+    constexpr bool HAS_C = !__is_same(CT, no_c_t);
+    constexpr bool EARLY_C = HAS_C && !F16ACC && fold_tiles(BI, BJ, NT, NSLOT) == 0 && TI * TJ <= 16;
     using cpieces = c_pieces<TI, TJ, CT>;
     cpieces cp;
     const bool early = EARLY_C && p.use_c && !p.c_trans;
@@ -874,7 +881,7 @@ void k_gemm_tiled(tiled_params p)
                                     !EDGE || (i0 + wi * WTI + 16 * a + 16 * (lane & 1) >= own_from<BI>(i0) && j0 + wj * WTJ + 16 * b >= own_from<BJ>(j0)));
     };
     if (CAN_FOLD && fold_c && (i0 % BI || j0 % BJ)) epilogue(false, false, std::true_type{});
-    else if (F16ACC || !p.use_c || fold_c) epilogue(false, false);
+    else if (F16ACC || !HAS_C || !p.use_c || fold_c) epilogue(false, false);
     else if (p.c_trans) epilogue(true, true);
     else if constexpr (EARLY_C) {
         const bool odd = lane & 1;
@@ -912,6 +919,12 @@ inline const void *pick_types(bool xk, bool yk, int c_type, int d_type, bool f16
         if constexpr (waves_per_simd(BI, BJ, WI * WJ * 64) < 2) return nullptr;
         else return pick_layout<BI, BJ, WI, WJ, NS, half_t, half_t, true>(xk, yk);
     }
+    // (the small tiles, whose launches are short enough to show it)
+    if constexpr (BI * BJ <= 128 * 128) {
+        if (c_type == NO_C && d_type == 0) return pick_layout<BI, BJ, WI, WJ, NS, no_c_t, half_t, false>(xk, yk);
+        if (c_type == NO_C) return pick_layout<BI, BJ, WI, WJ, NS, no_c_t, float, false>(xk, yk);
+    }
+    if (c_type == NO_C) c_type = 1;
     if (c_type == 0 && d_type == 0) return pick_layout<BI, BJ, WI, WJ, NS, half_t, half_t, false>(xk, yk);
     if (c_type == 0 && d_type == 1) return pick_layout<BI, BJ, WI, WJ, NS, half_t, float, false>(xk, yk);
     if (c_type == 1 && d_type == 0) return pick_layout<BI, BJ, WI, WJ, NS, float, half_t, false>(xk, yk);

@@ -4,6 +4,8 @@ string matches, test/device/wmma.jl:254-291 (store_d on a Global / Shared pointe
 import collections
 import re
 
+import pytest
+
 
 def _ops(text):
     return collections.Counter(l.split()[0] for l in text.splitlines()
@@ -130,6 +132,23 @@ def test_tiled_kernels_keep_spills_out_of_the_steady_state(miw):
         if "256, 256, 2, 2, 2" in name:
             continue    # 256 accumulators per lane: the 4-wavefront tile spills around its loop
         assert sum(1 for l in lines[mfma[0]:mfma[-1]] if re.match(r"\s*scratch_", l)) <= 48, name
+
+
+@pytest.mark.parametrize("kernel,count,c_loads", [("k_gemm_kwave_types<", 50, None), ("k_gemm_kwave_slices<", 10, 0)])
+def test_shared_k_kernels_of_other_types_stay_in_registers(miw, kernel, count, c_loads):
+    """What test_shared_k_kernels_stay_in_registers asks, of the instances for other types, no C and slices of K; an instance
+    without C reads nothing but its operands."""
+    res = {k: v for k, v in miw.reflection.kernel_resources().items() if kernel in k}
+    assert len(res) == count
+    for k, r in res.items():
+        assert r["spills"] == 0 and r["scratch"] == 0 and r["max_threads"] == 256, k
+    for k, text in miw.reflection.code_gcn(kernel).items():
+        order = [l.split()[0] for l in text.splitlines() if l.strip()]
+        assert not any(o.startswith(("scratch_", "flat_", "v_accvgpr")) for o in order), k
+        mfma = [i for i, o in enumerate(order) if o.startswith("v_mfma")]
+        assert {o for o in order[mfma[0]:mfma[-1]] if o.startswith(("global_", "buffer_"))} == {"global_load_lds_dwordx4"}, k
+        if c_loads == 0 or "signed char" in k:
+            assert not any(o.startswith("global_load_") and "lds" not in o for o in order), k
 
 
 def _regs(tok):
