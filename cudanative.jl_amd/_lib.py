@@ -128,6 +128,8 @@ SIGNATURES = {
     "miw_event_elapsed_ms": (_i, [ctypes.POINTER(_f), _vp, _vp]),
     "miw_frag_elems_per_lane": (_i, [_i, _i]),
     "miw_frag_image_bytes": (_sz, [_i, _i]),
+    "miw_frag_image_new": (_i, [_sz, _i, _vpp]),
+    "miw_frag_image_release": (_i, [_vp, _i]),
     "miw_frag_load": (_i, [_i, _i, _i, _i, _i, _i, _i, _vp, _i64, _vp, _vp]),
     "miw_frag_store": (_i, [_i, _i, _i, _i, _i, _i, _vp, _vp, _i64, _vp]),
     "miw_frag_fill": (_i, [_i, _f, _vp, _vp]),

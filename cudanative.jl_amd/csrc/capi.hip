@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <map>
 #include <mutex>
 #include <unordered_map>
 #include <cstdarg>
@@ -233,6 +234,44 @@ bool image_fits(const void *image, size_t bytes)
         if (size >= 4 && memcmp(img + off, "\177ELF", 4) == 0 && !elf_fits(img + off, size)) return false;
     }
     return true;
+}
+
+// Images of fragments (miw_frag_image_new).  A program made of fragment operations takes and drops one per operation:
+// with hipMalloc and hipFree, which waits for the device, load_a took 15 us where its launch takes 3.4, 6.5 now; load, load,
+// load, mma, store 39.4 us, 31.5 now.  Idle ones are only
+// handed to operations on the default stream, which alone has used them: the stream's order is what keeps two owners apart.
+constexpr size_t IMAGE_BYTES[2] = {512, 1024};
+constexpr size_t IDLE_IMAGES = 128;
+struct image_pool {
+    std::mutex mu;
+    std::map<std::pair<int, int>, std::vector<void *>> idle;      // by device and size
+    std::unordered_map<void *, std::pair<int, int>> all;         // idle or not
+};
+image_pool &images()
+{
+    static image_pool *pool = new image_pool;  // (images may be dropped while the process ends)
+    return *pool;
+}
+
+// hipMalloc that gives the idle images back where it finds no memory.
+hipError_t device_malloc(void **out, size_t bytes)
+{
+    hipError_t e = hipMalloc(out, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    std::vector<void *> idle;
+    {
+        image_pool &pool = images();
+        std::lock_guard<std::mutex> lock(pool.mu);
+        for (auto &[key, list] : pool.idle) {
+            idle.insert(idle.end(), list.begin(), list.end());
+            list.clear();
+        }
+        for (void *p : idle) pool.all.erase(p);
+    }
+    if (idle.empty()) return e;
+    for (void *p : idle) (void)hipFree(p);
+    (void)hipGetLastError();
+    return hipMalloc(out, bytes);
 }
 
 bool is_module_kernel(void *kernel)
@@ -606,7 +645,7 @@ int miw_malloc(void **out, size_t bytes)
     *out = nullptr;
     if (bytes == 0) return 0;
     REQUIRE_INIT("malloc");
-    HIP_TRY(hipMalloc(out, bytes));
+    HIP_TRY(device_malloc(out, bytes));
     return 0;
 }
 
@@ -733,6 +772,51 @@ size_t miw_frag_image_bytes(int use, int dtype)
 {
     int n = miw_frag_elems_per_lane(use, dtype);
     return n > 0 ? (size_t)n * 64 * dtype_size(dtype) : 0;
+}
+
+int miw_frag_image_new(size_t bytes, int reuse, void **image)
+{
+    if (!image) return fail(MIW_ERR_NULL_POINTER, "frag_image_new: null output");
+    *image = nullptr;
+    if (bytes == 0 || bytes > IMAGE_BYTES[1]) return fail(MIW_ERR_INVALID_VALUE, "frag_image_new: %zu bytes, an image has 1 to %zu", bytes, IMAGE_BYTES[1]);
+    REQUIRE_INIT("frag_image_new");
+    int device;
+    HIP_TRY(hipGetDevice(&device));
+    const int size = bytes > IMAGE_BYTES[0];
+    image_pool &pool = images();
+    if (reuse) {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        auto &idle = pool.idle[{device, size}];
+        if (!idle.empty()) {
+            *image = idle.back();
+            idle.pop_back();
+            return 0;
+        }
+    }
+    HIP_TRY(device_malloc(image, IMAGE_BYTES[size]));
+    std::lock_guard<std::mutex> lock(pool.mu);
+    pool.all[*image] = {device, size};
+    return 0;
+}
+
+int miw_frag_image_release(void *image, int reuse)
+{
+    if (!image) return 0;
+    REQUIRE_INIT("frag_image_release");
+    image_pool &pool = images();
+    {
+        std::lock_guard<std::mutex> lock(pool.mu);
+        auto it = pool.all.find(image);
+        if (it == pool.all.end()) return fail(MIW_ERR_INVALID_VALUE, "frag_image_release: not an image of miw_frag_image_new");
+        auto &idle = pool.idle[it->second];
+        if (reuse && idle.size() < IDLE_IMAGES) {
+            idle.push_back(image);
+            return 0;
+        }
+        pool.all.erase(it);
+    }
+    HIP_TRY(hipFree(image));
+    return 0;
 }
 
 int miw_frag_load(int use, int dtype, int layout, int addr_space, int m, int n, int k, const void *addr,

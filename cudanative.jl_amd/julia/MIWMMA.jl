@@ -281,6 +281,14 @@ elems_per_lane(::Type{U}, ::Type{T}) where {U, T} =
 image_bytes(::Type{U}, ::Type{T}) where {U, T} =
     Int(ccall((:miw_frag_image_bytes, libmiwmma), Csize_t, (Cint, Cint), use_code(U), dtype_code(T)))
 
+"Device memory for one image; `reuse`: of the default stream's operations only (see miwmma.h)."
+function image_new(bytes::Integer, reuse::Bool)
+    p = Ref{Ptr{Cvoid}}(C_NULL)
+    check(ccall((:miw_frag_image_new, libmiwmma), Cint, (Csize_t, Cint, Ptr{Ptr{Cvoid}}), bytes, reuse, p))
+    return p[]
+end
+image_release(p::Ptr{Cvoid}, reuse::Bool) = check(ccall((:miw_frag_image_release, libmiwmma), Cint, (Ptr{Cvoid}, Cint), p, reuse))
+
 # One launch that reads a tile into a fresh fragment image.
 function load_image(::Type{U}, ::Type{T}, ::Type{L}, ::Type{A}, addr::UInt, stride::Integer) where {U, T, L, A}
     img = DeviceBuffer{T,2}(undef, (FS, WAVEFRONT))

@@ -17,6 +17,7 @@ host from a tuple (test/device/wmma.jl:180-184) are computed on the host.
 """
 import contextlib
 import ctypes
+import gc
 import threading
 
 import numpy as np
@@ -171,7 +172,7 @@ class Fragment:
 
     def __init__(self, M, N, K, FS, T, L, U, x=None, image=None):
         self.M, self.N, self.K, self.FS = M, N, K, FS
-        self.T = np.dtype(T).type
+        self.T = T if T is Float16 or T is Float32 else np.dtype(T).type
         self.L, self.U = L, U
         self._image = image
         self._x = None
@@ -225,9 +226,11 @@ class Fragment:
             s = self.T(scalar)
             vals = tuple(self.T(s * v) if op == _lib.OP_MUL else self.T(s + v) for v in self._x)
             return Fragment(*self.type_params(), x=vals)
-        out = self._image.similar()
+        stream = _stream()
+        _used_on(stream, self)
+        out = _new_image(self.T, self.FS)
         _lib.check(_lib.load().miw_frag_map(_dtype_code(self.T), op, float(scalar), self._image.ptr, out.ptr,
-                                            WAVEFRONT * self.FS, _stream()))
+                                            WAVEFRONT * self.FS, stream))
         return Fragment(*self.type_params(), image=out)
 
     def __mul__(self, s):
@@ -241,8 +244,40 @@ class Fragment:
     __radd__ = __add__
 
 
+class _Image(DeviceArray):
+    """A fragment's registers in device memory.  One that only the default stream has used goes to the next fragment, in
+    that stream's order; any other is freed."""
+
+    def __init__(self, T, FS):
+        lib = _lib.load()
+        self.dtype = dtype = np.dtype(T)
+        self.dims = (FS, WAVEFRONT)
+        self.nbytes = nbytes = FS * WAVEFRONT * dtype.itemsize
+        self.reuse = reuse = _stream() is None
+        p = ctypes.c_void_p()
+        if lib.miw_frag_image_new(nbytes, reuse, ctypes.byref(p)) != 0:
+            gc.collect()  # (unreachable buffers first, as DeviceArray does)
+            _lib.check(lib.miw_frag_image_new(nbytes, reuse, ctypes.byref(p)))
+        self.ptr = p.value
+
+    def __del__(self):
+        ptr, self.ptr = getattr(self, "ptr", 0), 0
+        if ptr:
+            try:
+                _lib.load().miw_frag_image_release(ptr, self.reuse)
+            except Exception:
+                pass
+
+
 def _new_image(T, FS):
-    return DeviceArray(dtype=T, dims=(FS, WAVEFRONT))
+    return _Image(T, FS)
+
+
+def _used_on(stream, *fragments):
+    """Notes that an operation on `stream` reads these fragments."""
+    if stream is not None:
+        for f in fragments:
+            f._image.reuse = False
 
 
 # ------------------------------------------------------------ load ----------
@@ -329,8 +364,10 @@ def mma(a, b, c, config):
         found = _layout_code(a.L), _layout_code(b.L), _dtype_code(c.T), _dtype_code(config.d_type), d_num
     get_hl_shape(M, N, K)
     a_order, b_order, c_ty, d_ty, d_num = found
+    stream = _stream()
+    _used_on(stream, a, b, c)
     img = _new_image(config.d_type, d_num)
-    _lib.check(_lib.load().miw_frag_mma(a_order, b_order, c_ty, d_ty, a._image.ptr, b._image.ptr, c._image.ptr, img.ptr, _stream()))
+    _lib.check(_lib.load().miw_frag_mma(a_order, b_order, c_ty, d_ty, a._image.ptr, b._image.ptr, c._image.ptr, img.ptr, stream))
     return Fragment(M, N, K, d_num, config.d_type, Unspecified, Accumulator, image=img)
 
 
@@ -351,8 +388,10 @@ def store_d(addr, d, stride, layout, config):
     get_hl_layout(layout)
     get_hl_shape(config.M, config.N, config.K)
     get_hl_frag_info("d", d.T)
+    stream = _stream()
+    _used_on(stream, d)
     _lib.check(_lib.load().miw_frag_store(_dtype_code(d.T), _layout_code(layout), addr.addrspace, config.M, config.N,
-                                          config.K, addr.addr, d._image.ptr, int(stride), _stream()))
+                                          config.K, addr.addr, d._image.ptr, int(stride), stream))
     return None
 
 

@@ -125,6 +125,13 @@ int miw_event_elapsed_ms(float *ms, void *start, void *stop);
 int miw_frag_elems_per_lane(int use, int dtype);
 /* Bytes of a fragment image (64 lanes). */
 size_t miw_frag_image_bytes(int use, int dtype);
+/* Device memory for one fragment image of at most 1024 bytes on the current device.  reuse != 0 may return memory that
+   work queued on the default stream still uses: only operations on the default stream may touch the image then.  reuse == 0
+   returns memory that nothing uses.  miw_frag_image_release gives it back: with reuse != 0, which asserts that only the
+   default stream has touched it, without waiting for the device and for the next image (at most 128 idle images per device and
+   size, 192 KiB, are kept; an allocation that finds no memory gives them back first); with reuse == 0 as miw_free does. */
+int miw_frag_image_new(size_t bytes, int reuse, void **image);
+int miw_frag_image_release(void *image, int reuse);
 
 /* load_a / load_b / load_c (src/device/cuda/wmma.jl:507-530;
    llvm_wmma_load_* :104-137).  use selects a/b/c; A and B must be MIW_F16.

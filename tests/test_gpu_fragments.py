@@ -423,6 +423,66 @@ def test_launches_from_host_threads(gpu):
     assert not errors
 
 
+def test_images_go_from_fragment_to_fragment_in_stream_order(gpu):
+    """Four hundred chains of operations queued without a wait, each chain's images dropped as it ends and taken by the next, on
+    the default stream, from two threads at once and with chains on a stream of their own between them: every D is its own."""
+    W = gpu.WMMA
+    cfg = W.Config(16, 16, 16, np.float32)
+    rng = np.random.default_rng(5)
+    A = [gpu.DeviceArray(rng.integers(-4, 5, (16, 16)).astype(np.float16)) for _ in range(8)]
+    C = gpu.DeviceArray(rng.integers(-9, 9, (16, 16)).astype(np.float32))
+    host = [x.to_host().astype(np.float64) for x in A]
+    D = [gpu.DeviceArray(np.zeros((16, 16), np.float32)) for _ in range(400)]
+    stream = gpu.Stream()
+
+    def chain(i):
+        a = W.load_a(A[i % 8].pointer(), 16, W.ColMajor, cfg)
+        b = W.load_b(A[i * 5 % 8].pointer(), 16, W.ColMajor, cfg)
+        c = W.load_c(C.pointer(), 16, W.ColMajor, cfg)
+        W.store_d(D[i].pointer(), W.mma(a, b, c * np.float32(i % 3), cfg), 16, W.ColMajor, cfg)
+        return a, c
+
+    def run(first):
+        for i in range(first, 400, 2):
+            if i % 5 == 4:
+                with W.on_stream(stream.handle):
+                    assert not any(f._image.reuse for f in chain(i))
+            else:
+                assert all(f._image.reuse for f in chain(i))
+
+    threads = [threading.Thread(target=run, args=(t,)) for t in (0, 1)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    stream.synchronize()
+    gpu.synchronize()
+    for i in range(400):
+        assert np.array_equal(D[i].to_host(), host[i % 8] @ host[i * 5 % 8] + (i % 3) * C.to_host()), i
+    # one that another stream has read does not go to the default stream's next fragment; more than are kept are freed
+    f = W.load_c(C.pointer(), 16, W.ColMajor, cfg)
+    gpu.synchronize()
+    with W.on_stream(stream.handle):
+        W.store_d(D[0].pointer(), f, 16, W.ColMajor, cfg)
+    assert not f._image.reuse
+    many = [W.fill_c(np.float32(i), cfg) for i in range(300)]
+    assert len({g._image.ptr for g in many}) == 300
+    assert all((g.x == i).all() for i, g in enumerate(many))
+    del many
+    assert (W.fill_c(np.float32(7), cfg).x == 7).all()
+
+
+def test_image_entries_check_their_arguments(gpu):
+    L = gpu._lib
+    lib, p = L.load(), ctypes.c_void_p()
+    for bytes_, code in ((0, L.ERR_INVALID_VALUE), (1025, L.ERR_INVALID_VALUE), (1, 0), (1024, 0)):
+        assert lib.miw_frag_image_new(bytes_, 1, ctypes.byref(p)) == code and bool(p.value) == (code == 0)
+        if p.value:
+            assert lib.miw_frag_image_release(p, 0) == 0
+            assert lib.miw_frag_image_release(p, 1) == L.ERR_INVALID_VALUE  # (gone)
+    assert lib.miw_frag_image_new(512, 0, None) == L.ERR_NULL_POINTER
+    other = gpu.DeviceArray(np.zeros(4, np.float32))
+    assert lib.miw_frag_image_release(other.ptr, 1) == L.ERR_INVALID_VALUE and lib.miw_frag_image_release(None, 1) == 0
+
+
 def test_device_array_semantics(gpu):
     # src/array.jl:45-60: similar keeps type and dims; round trip; column-major first index contiguous
     a = np.arange(12, dtype=F32).reshape(3, 4)
