@@ -231,6 +231,9 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
     // Below four slots of K there is too little of it to request across two tiles, and the launch is bound by C and D.
     if (v.kind == KIND_PINGPONG32 && tiles > cus && tiles < (1l << 30) && p.K > 3 * KGRAN) {
         p.work = (int)tiles;
+        // A Float32 C and D take longer than a loop over up to sixteen slots of K.  With both in Float16 the loop is the longer part
+        // and the spread start costs more than it gives (8192x8192x1024 150.5 us and 154.2, 8192x6144x2048 182 and 185).
+        p.c_spread = g.use_c && !p.c_trans && !fold && c_type == 1 && d_type == 1 && p.K <= 16 * KGRAN && tiles >= 2l * cus;
         set_raster(&p, g.batch, true);
         grid = dim3((unsigned)cus, 1);
     }

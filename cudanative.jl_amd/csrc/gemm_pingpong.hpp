@@ -59,6 +59,7 @@ namespace miw {
 
 constexpr int PP_KMAJOR_SLOTS = 3;
 constexpr int PP_IMAJOR_ENTRIES = 4;
+constexpr int PP_SPREAD_SLEEP = 64;  // units of 64 cycles between the starts of workgroups, see tiled_params::c_spread
 constexpr int PP_FOLD_STEPS = 32;  // k-steps of 32 over which k_gemm_pp_fold adds C: one MFMA tile of the wavefront's 8 x 4 each
 
 // Slots of a K-major Y: two when X is K-major as well (see above), else three.
@@ -332,6 +333,15 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
             y_advance(std::true_type{});
         }
     };
+    // Workgroups that all end their loops at once leave HBM idle during the loops and share it in the epilogues.  Where C and D
+    // take longer than the loop (tiled_params::c_spread) they start at eight different times over 29000 cycles, so that
+    // some loop while others read C and store D; every start waits a fixed time and nobody waits for another workgroup.
+    // 8192x8192x1024, alpha = -1: 181.5 us at once and 176.2 like this, 8192x8192x512 138.8 and 126.1, 8192x8192x256 116.7 and
+    // 110.5, 6144x8192x1024 145.3 and 134.2, two tiles each (4096x8192x1024) 95.7 and 90.9.
+    if constexpr (!FOLD && __is_same(CT, float) && __is_same(DT, float)) {
+        if (p.c_spread)
+            for (int phase = (blockIdx.x >> 3) & 7; phase > 0; phase--) __builtin_amdgcn_s_sleep(PP_SPREAD_SLEEP);
+    }
     constexpr std::integral_constant<int, 0> unit0{};
     constexpr std::integral_constant<int, 1> unit1{};
     constexpr std::integral_constant<int, 2> unit2{};

@@ -102,7 +102,9 @@ struct tiled_params {
         int work;
         int k_short;  // see short_member
     };
-    int c_spread;  // k_gemm_pp64: the workgroups ask for C at eight different times of their K loops, not all at its start
+    // k_gemm_pp64: the workgroups ask for C at eight different times of their K loops, not all at its start.  k_gemm_pp: they
+    // start at eight different times.
+    int c_spread;
 #ifdef MIW_PP_TS
     long long *ts;  // measurement builds: 10 counters per wavefront (see k_gemm_pp64), or null
 #endif

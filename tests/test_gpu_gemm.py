@@ -225,6 +225,27 @@ def test_workgroups_that_walk_three_tiles_and_in_place(gpu, orc, al, bl, dl):
         assert not np.isnan(outs[0].max()) and np.array_equal(*(x.view(np.uint8 if x.nbytes % 8 else np.uint64) for x in outs)), (al, bl, dl, K, in_place, form)
 
 
+@pytest.mark.parametrize("tiles,K,in_place", [(511, 208, False), (512, 208, False), (771, 272, True), (512, 1024, False), (512, 1040, False)])
+def test_workgroups_that_start_at_different_times(gpu, orc, tiles, K, in_place):
+    """Float32 C and D, from two tiles per workgroup to sixteen slots of K (and one past each line): the bits of launches that
+    give every workgroup one tile."""
+    v, alpha = _vid(gpu, "tile256x256_pingpong"), -1.0
+    M, col = 256, _W(gpu, orc.COL)
+    A, B, C = (np.resize(x, tiles * n) for x, n in zip(_inputs(orc, orc.GemmDesc(M=1040, N=1040, K=K), 7 + K), (M * K, K * M, M * M)))
+    dA, dB = gpu.DeviceArray(A), gpu.DeviceArray(B)
+    outs = []
+    for count in (tiles, 128):
+        dC = gpu.DeviceArray(C)
+        dD = dC if in_place else gpu.DeviceArray(np.full(C.size, np.nan, dtype=np.float32))
+        for first in range(0, tiles, count):
+            desc = gpu.GEMM.make_desc(M, M, K, a_layout=col, b_layout=col, c_layout=col, d_layout=col, c_type=F32, d_type=F32, alpha=alpha,
+                                      batch=min(count, tiles - first), variant=v)
+            gpu.GEMM.gemm(dA.ptr + 2 * first * M * K, dB.ptr + 2 * first * M * K, dC.ptr + 4 * first * M * M, dD.ptr + 4 * first * M * M, desc)
+        gpu.synchronize()
+        outs.append(dD.to_host())
+    assert not np.isnan(outs[0].max()) and np.array_equal(*(x.view(np.uint64) for x in outs)), (tiles, K, in_place)
+
+
 @pytest.mark.parametrize("alpha,K", [(-1.0, 976), (-1.0, 1024), (-1.0, 1168), (1.0, 976), (1.0, 1024)])
 @pytest.mark.parametrize("al,bl", itertools.product((0, 1), repeat=2))
 def test_c_is_added_once_behind_the_loop(gpu, orc, alpha, K, al, bl):
