@@ -213,7 +213,7 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
                  (long)p.I * p.J * g.batch * (c_type == 0 ? 2 : 4) >= (12l << 20);
     const bool fold = v.kind == KIND_PINGPONG32 && pp_folds(p, c_type);
     // (slices of K run on the instances with a Float32 C, see has_slices)
-    const bool without_c = v.kind == KIND_PIPELINED && !g.use_c && !g.k_last;
+    const bool without_c = (v.kind == KIND_PIPELINED || (v.kind == KIND_PINGPONG64 && !f16acc)) && !g.use_c && !g.k_last;
     const void *fn = pick_kernel(i, xk, yk, without_c ? NO_C : c_type, d_type, f16acc, fold);
     if (!fn) return hipErrorInvalidValue;
     // (the 64-k ping-pong kernels stage a Float16 C tile beside the ring where both fit)

@@ -872,7 +872,10 @@ void k_gemm_pp64(tiled_params p)
     // 73.2 us -> 69.4, 7120x1024x720 with a Float16 C 19.4 -> 17.8, 2048x2048x128 11.1 -> 9.2.)
     using cpieces = c_pieces<TI, TJ, CT>;
     cpieces cp;
-    const bool early = !F16ACC && p.use_c && !p.c_trans;
+    // Problems without C have instances of their own, without C's registers: 1280x5168x1408 23.0 us -> 22.6, 8192x768x1024
+    // 17.8 -> 17.2, 1024x3072x1024 11.3 -> 11.1 (2048^3 22.1 -> 22.7, as before C waited in registers).
+    constexpr bool HAS_C = !__is_same(CT, no_c_t);
+    const bool early = HAS_C && !F16ACC && p.use_c && !p.c_trans;
     auto request_c = [&]() MIW_INLINE { cp.request(C + (long)(j0 + wj * WTJ) * p.ldc + (i0 + wi * WTI) + pair_place(lane, p.ldc), p.ldc); };
     // The loop starts when pair 0 (and, with Float16 accumulation, the C operand, requested before it) has landed: the
     // wait at the end of memory cluster p leaves NSLOT - 2 pairs in flight, so pair p + 1 has landed by then, the
@@ -1154,7 +1157,7 @@ void k_gemm_pp64(tiled_params p)
                 }
             }
     };
-    if (F16ACC || !p.use_c) epilogue(std::integral_constant<int, 0>{});
+    if (F16ACC || !HAS_C || !p.use_c) epilogue(std::integral_constant<int, 0>{});
     else if (p.c_trans) epilogue(std::integral_constant<int, 2>{});
     else epilogue(std::integral_constant<int, 1>{});
 #ifdef MIW_PP_TS

@@ -16,6 +16,8 @@ template <int BI, int BJ, int WI, int WJ, int NS>
 static const void *pp64_types(bool xk, bool yk, int c_type, int d_type, bool f16acc)
 {
     if (f16acc) return pp64_layout<BI, BJ, WI, WJ, NS, half_t, half_t, true>(xk, yk);
+    if (c_type == NO_C && d_type == 0) return pp64_layout<BI, BJ, WI, WJ, NS, no_c_t, half_t, false>(xk, yk);
+    if (c_type == NO_C) return pp64_layout<BI, BJ, WI, WJ, NS, no_c_t, float, false>(xk, yk);
     if (c_type == 0 && d_type == 0) return pp64_layout<BI, BJ, WI, WJ, NS, half_t, half_t, false>(xk, yk);
     if (c_type == 0 && d_type == 1) return pp64_layout<BI, BJ, WI, WJ, NS, half_t, float, false>(xk, yk);
     if (c_type == 1 && d_type == 0) return pp64_layout<BI, BJ, WI, WJ, NS, float, half_t, false>(xk, yk);
