@@ -59,10 +59,13 @@ def splitk_workspace(desc, splits=0):
 
 def gemm_splitk(A, B, C, D, desc, splits=0, workspace=None, stream=None):
     """Split-K launch of D = alpha*A*B + beta*C: K cut into slices whose Float32 products go through
-    `workspace` (a DeviceArray; allocated here when None) and are added in order by a second kernel."""
+    `workspace` (a DeviceArray; allocated here when None) and are added in order by a second kernel.  splits = 0 with a
+    workspace of the caller's that holds fewer slices than the library would choose: as many of one length as pay in it."""
     n, nbytes = splitk_workspace(desc, splits)
     if workspace is None:
         workspace = DeviceArray.undef(np.float32, max(nbytes // 4, 4))
+    elif workspace.nbytes < nbytes:
+        n = splits
     _lib.check(_lib.load().miw_gemm_splitk(ctypes.byref(desc), _ptr(A), _ptr(B), _ptr(C), _ptr(D), n, _ptr(workspace),
                                            workspace.nbytes, _stream(stream)))
     return workspace

@@ -576,6 +576,31 @@ def test_splitk_takes_the_workspace_its_query_reports(miw):
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stderr
 
 
+def test_gemm_splitk_takes_a_workspace_smaller_than_the_query_asks_for(miw):
+    """A caller's workspace that holds the best count of equal slices, but not the unequal slices that the library would choose,
+    gets the equal ones; one slice less, or the larger count by name, is refused."""
+    import subprocess, sys
+    code = ("import sys; sys.path.insert(0, %r); from tests.conftest import load_package; m = load_package(); L, G, W = m._lib, m.GEMM, m.WMMA\n"
+            "class Room:\n"
+            "    def __init__(self, nbytes): self.nbytes = nbytes\n"
+            "    def __int__(self): return 1 << 40\n"
+            "def code(d, nbytes, splits=0):\n"
+            "    try: G.gemm_splitk(1 << 32, 1 << 33, 1 << 34, 1 << 35, d, splits, workspace=Room(nbytes))\n"
+            "    except m.MIWError as e: return e.code\n"
+            "for M, N, K, equal in ((160, 208, 29312, 2), (704, 336, 12416, 2), (192, 768, 28416, 12), (448, 384, 18944, 8)):\n"
+            "    d = G.make_desc(M, N, K, a_layout=W.ColMajor, b_layout=W.RowMajor, c_layout=W.RowMajor, d_layout=W.RowMajor)\n"
+            "    n, nbytes = G.splitk_workspace(d)\n"
+            "    assert n > equal and K // 64 %% n and nbytes == 4 * n * M * N\n"
+            "    for held in range(equal, n + 1):\n"
+            "        assert code(d, 4 * held * M * N) == L.ERR_NOT_INITIALIZED, (M, N, K, held)\n"
+            "    assert code(d, 4 * equal * M * N - 4) == L.ERR_INVALID_VALUE\n"
+            "    assert code(d, 4 * equal * M * N, n) == L.ERR_INVALID_VALUE\n"
+            "    assert code(d, 4 * equal * M * N, equal) == L.ERR_NOT_INITIALIZED\n"
+            "print('ok')\n") % ROOT
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0 and out.stdout.strip() == "ok", out.stderr
+
+
 def test_splitk_slices_of_unequal_length_are_only_chosen(miw):
     """A count that leaves the last slice shorter is taken where the library chooses it, and asked for by that number; any other such
     count is refused, and a workspace that only slices of one length fit gets those, as one that is too small for them is refused."""
