@@ -243,9 +243,13 @@ bool image_fits(const void *image, size_t bytes)
 constexpr size_t IMAGE_BYTES[2] = {512, 1024};
 constexpr size_t IDLE_IMAGES = 128;
 struct image_pool {
+    struct image {
+        std::pair<int, int> key;  // device and size
+        bool idle;
+    };
     std::mutex mu;
-    std::map<std::pair<int, int>, std::vector<void *>> idle;      // by device and size
-    std::unordered_map<void *, std::pair<int, int>> all;         // idle or not
+    std::map<std::pair<int, int>, std::vector<void *>> idle;
+    std::unordered_map<void *, image> all;  // idle or in a caller's hands
 };
 image_pool &images()
 {
@@ -653,6 +657,15 @@ int miw_free(void *p)
 {
     if (!p) return 0;
     REQUIRE_INIT("free");
+    {
+        image_pool &pool = images();
+        std::lock_guard<std::mutex> lock(pool.mu);
+        auto it = pool.all.find(p);
+        if (it != pool.all.end()) {
+            if (it->second.idle) return fail(MIW_ERR_INVALID_VALUE, "free: a fragment image that has been released");
+            pool.all.erase(it);
+        }
+    }
     HIP_TRY(hipFree(p));
     return 0;
 }
@@ -790,12 +803,13 @@ int miw_frag_image_new(size_t bytes, int reuse, void **image)
         if (!idle.empty()) {
             *image = idle.back();
             idle.pop_back();
+            pool.all.at(*image).idle = false;
             return 0;
         }
     }
     HIP_TRY(device_malloc(image, IMAGE_BYTES[size]));
     std::lock_guard<std::mutex> lock(pool.mu);
-    pool.all[*image] = {device, size};
+    pool.all[*image] = {{device, size}, false};
     return 0;
 }
 
@@ -807,10 +821,12 @@ int miw_frag_image_release(void *image, int reuse)
     {
         std::lock_guard<std::mutex> lock(pool.mu);
         auto it = pool.all.find(image);
-        if (it == pool.all.end()) return fail(MIW_ERR_INVALID_VALUE, "frag_image_release: not an image of miw_frag_image_new");
-        auto &idle = pool.idle[it->second];
+        if (it == pool.all.end() || it->second.idle)
+            return fail(MIW_ERR_INVALID_VALUE, "frag_image_release: not an image of miw_frag_image_new, or released before");
+        auto &idle = pool.idle[it->second.key];
         if (reuse && idle.size() < IDLE_IMAGES) {
             idle.push_back(image);
+            it->second.idle = true;
             return 0;
         }
         pool.all.erase(it);

@@ -129,7 +129,8 @@ size_t miw_frag_image_bytes(int use, int dtype);
    work queued on the default stream still uses: only operations on the default stream may touch the image then.  reuse == 0
    returns memory that nothing uses.  miw_frag_image_release gives it back: with reuse != 0, which asserts that only the
    default stream has touched it, without waiting for the device and for the next image (at most 128 idle images per device and
-   size, 192 KiB, are kept; an allocation that finds no memory gives them back first); with reuse == 0 as miw_free does. */
+   size, 192 KiB, are kept; an allocation that finds no memory gives them back first); with reuse == 0 as miw_free does.  miw_free frees an image
+   as well; one that has been released is refused by both (MIW_ERR_INVALID_VALUE). */
 int miw_frag_image_new(size_t bytes, int reuse, void **image);
 int miw_frag_image_release(void *image, int reuse);
 

@@ -479,6 +479,15 @@ def test_image_entries_check_their_arguments(gpu):
             assert lib.miw_frag_image_release(p, 0) == 0
             assert lib.miw_frag_image_release(p, 1) == L.ERR_INVALID_VALUE  # (gone)
     assert lib.miw_frag_image_new(512, 0, None) == L.ERR_NULL_POINTER
+    # an idle image has no owner who could give it back again, or free it; the next owner can
+    for again in (lambda x: lib.miw_frag_image_release(x, 1), lambda x: lib.miw_frag_image_release(x, 0), lib.miw_free):
+        q, r = ctypes.c_void_p(), ctypes.c_void_p()
+        assert lib.miw_frag_image_new(512, 1, ctypes.byref(p)) == 0 and lib.miw_frag_image_release(p, 1) == 0
+        assert again(p) == L.ERR_INVALID_VALUE
+        assert lib.miw_frag_image_new(512, 1, ctypes.byref(q)) == lib.miw_frag_image_new(512, 1, ctypes.byref(r)) == 0
+        assert q.value != r.value
+        # freed by miw_free: no image any more
+        assert again(q) == 0 and lib.miw_free(r) == 0 and lib.miw_frag_image_release(r, 1) == L.ERR_INVALID_VALUE
     other = gpu.DeviceArray(np.zeros(4, np.float32))
     assert lib.miw_frag_image_release(other.ptr, 1) == L.ERR_INVALID_VALUE and lib.miw_frag_image_release(None, 1) == 0
 
