@@ -233,7 +233,11 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
         p.work = (int)tiles;
         // A Float32 C and D take longer than a loop over up to sixteen slots of K.  With both in Float16 the loop is the longer part
         // and the spread start costs more than it gives (8192x8192x1024 150.5 us and 154.2, 8192x6144x2048 182 and 185).
-        p.c_spread = g.use_c && !p.c_trans && !fold && c_type == 1 && d_type == 1 && p.K <= 16 * KGRAN && tiles >= 2l * cus;
+        // Beyond six rounds of tiles the workgroups' times drift apart by themselves, and only loops of up to eight slots gain
+        // (at once and spread: 12288x8192x1024 in six rounds 268.5 us and 257.1; 16384x8192 in eight, K = 496 250.4 and 246.7,
+        // K = 1008 333.7 and 336.4; 16384x16384x1024 644.6 and 651.7).
+        p.c_spread = g.use_c && !p.c_trans && !fold && c_type == 1 && d_type == 1 && p.K <= 16 * KGRAN && tiles >= 2l * cus &&
+                     (tiles <= 6l * cus || p.K <= 8 * KGRAN);
         set_raster(&p, g.batch, true);
         grid = dim3((unsigned)cus, 1);
     }

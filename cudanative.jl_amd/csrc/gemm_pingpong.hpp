@@ -334,13 +334,14 @@ __device__ __attribute__((always_inline)) inline void gemm_pp(const tiled_params
         }
     };
     // Workgroups that all end their loops at once leave HBM idle during the loops and share it in the epilogues.  Where C and D
-    // take longer than the loop (tiled_params::c_spread) they start at eight different times over 29000 cycles, so that
-    // some loop while others read C and store D; every start waits a fixed time and nobody waits for another workgroup.
-    // 8192x8192x1024, alpha = -1: 181.5 us at once and 176.2 like this, 8192x8192x512 138.8 and 126.1, 8192x8192x256 116.7 and
-    // 110.5, 6144x8192x1024 145.3 and 134.2, two tiles each (4096x8192x1024) 95.7 and 90.9.
+    // take longer than the loop (tiled_params::c_spread) they start at four different times over 25000 cycles, eight tiles of one
+    // column together (see spread_phase), so that some loop while others read C and store D; every start waits a fixed time and
+    // nobody waits for another workgroup.  alpha = -1, all at once, by rows of tiles and by columns: 8192x8192x1024 180.2 us,
+    // 168.8 and 165.8; 8192x8192x208 115.4, 113.1 and 104.1; two tiles each: 8192x4096x512 75.9, 86.0 and 69.6, 4096x8192x512
+    // 73.9, 71.5 and 67.1; 8000x4400x208 81.7, 84.3 and 71.6.
     if constexpr (!FOLD && __is_same(CT, float) && __is_same(DT, float)) {
         if (p.c_spread)
-            for (int phase = (blockIdx.x >> 3) & 7; phase > 0; phase--) __builtin_amdgcn_s_sleep(PP_SPREAD_SLEEP);
+            for (int phase = spread_phase() & 6; phase > 0; phase--) __builtin_amdgcn_s_sleep(PP_SPREAD_SLEEP);
     }
     constexpr std::integral_constant<int, 0> unit0{};
     constexpr std::integral_constant<int, 1> unit1{};

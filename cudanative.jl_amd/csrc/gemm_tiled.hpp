@@ -103,7 +103,7 @@ struct tiled_params {
         int k_short;  // see short_member
     };
     // k_gemm_pp64: the workgroups ask for C at eight different times of their K loops, not all at its start.  k_gemm_pp: they
-    // start at eight different times.
+    // start at four different times.
     int c_spread;
 #ifdef MIW_PP_TS
     long long *ts;  // measurement builds: 10 counters per wavefront (see k_gemm_pp64), or null
@@ -199,6 +199,10 @@ __device__ inline tile_place workgroup_tile(const tiled_params &p, int bi, int b
 {
     return tile_at(p, (int)(blockIdx.x + blockIdx.y * (unsigned)p.span), (int)blockIdx.y, bi, bj);
 }
+
+// 0 to 7, for workgroups that are to do something at different times: the same for four of an XCD's, whose tiles lie in one column.
+// Along i neighbours touch neighbouring lines of C and D, and the memory serves those better together.
+__device__ inline int spread_phase() { return (int)(blockIdx.x >> 5) & 7; }
 
 // Kernels on which slices of K run: their products are Float32.
 template <class CT, class DT, bool F16ACC>
