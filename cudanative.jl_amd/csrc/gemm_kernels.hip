@@ -206,11 +206,13 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
     if (const char *e = getenv("MIW_TS")) p.ts = (long long *)strtoull(e, nullptr, 16);
 #endif
     // A large C that all workgroups ask for at once is a burst that the first slots do not cover; a workgroup that asks for
-    // it in mid-loop waits too, for one latency.  256x128 tiles, at the start and spread: 32 MiB 74.0 and 71.4 us
-    // (8192x1024x4096), 22 MiB 21.2 and 19.7 (2304x2496x1152), 14 MiB 18.9 and 18.2 (7120x1024x720), 11 MiB 15.4 and 15.2
-    // (896x6528x544); on 128x128 tiles, which have less of it, spreading loses (4032x576x2368 19.5 and 21.1).
+    // it in mid-loop waits too, for one latency.  256x128 tiles, one time and eight, by rows of tiles and by columns: 32 MiB
+    // 71.1 us, 70.2 and 68.0 (8192x1024x4096); one time and two: 35 MiB 30.0 and 27.7 (7552x1216x512), 24 MiB 15.4 and 14.4
+    // (5632x1104x448, Float16 D), 11.9 MiB 17.7 and 17.1 (5632x1104x832, Float16); from 4 to 10 MiB it is 0.5 to 1 % behind.
+    // 128x128 tiles keep one time: to choose costs their loops 1 to 3 %, what it gives (2048x2048x2048 21.5 and 20.6) and
+    // more where C is small (1024x1536x2048 16.2 and 16.5).
     p.c_spread = v.kind == KIND_PINGPONG64 && v.bm * v.bn > 128 * 128 && g.use_c &&
-                 (long)p.I * p.J * g.batch * (c_type == 0 ? 2 : 4) >= (12l << 20);
+                 (long)p.I * p.J * g.batch * (c_type == 0 ? 2 : 4) >= (11l << 20);
     const bool fold = v.kind == KIND_PINGPONG32 && pp_folds(p, c_type);
     // (slices of K run on the instances with a Float32 C, see has_slices)
     const bool without_c = (v.kind == KIND_PIPELINED || (v.kind == KIND_PINGPONG64 && !f16acc)) && !g.use_c && !g.k_last;

@@ -1106,10 +1106,11 @@ void k_gemm_pp64(tiled_params p)
         }
     } else {
         int pr = 0;
-        // Which ring of pairs C is asked for in front of (see tiled_params::c_spread); without a ring, in front of the last
-        // pair: so few pairs end before C arrives, and C's loads would hold theirs up.
+        // The ring of pairs that C is asked for in front of (see tiled_params::c_spread); behind all rings, in front of the last
+        // pair.  Without a ring it is there in any case: so few pairs end before C arrives, and C's loads would hold theirs up.
         const int rings = max(0, NFAST / NSLOT);
-        const int c_at = BI * BJ > 128 * 128 && p.c_spread ? (rings * (int)((blockIdx.x >> 3) & 7) >> 3) * NSLOT : 0;
+        const int c_ring = BI * BJ > 128 * 128 && p.c_spread ? max(2, rings) * spread_phase() >> 3 : 0, c_at = c_ring * NSLOT;
+        const bool late = c_ring >= rings;
         for (; pr + NSLOT <= NFAST; pr += NSLOT) {
             MIW_PP_MIDDLE(pr)
             const bool now = early && pr == c_at;
@@ -1119,9 +1120,9 @@ void k_gemm_pp64(tiled_params p)
         for (; pr < NFAST; pr++) pair(inner, plain, fast_pair);
         next = NSLOT - 1 + pr;
         for (; pr < NPM; pr++) pair(inner, plain);
-        if (early && rings == 0) request_c();
+        if (early && late) request_c();
         MIW_PP_STAMP(9)
-        pair(last_pair, plain, std::integral_constant<int, -2>{}, early && rings == 0);  // (nothing that it reads is on the way any more)
+        pair(last_pair, plain, std::integral_constant<int, -2>{}, early && late);  // (nothing that it reads is on the way any more)
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may outlive the workgroup's LDS
     if (!late_group) __builtin_amdgcn_s_barrier();

@@ -294,7 +294,7 @@ def test_c_waits_in_registers_for_the_end_of_the_loop(gpu, orc, al, bl, ct, K):
 
 @pytest.mark.parametrize("M,N,K,ct", [(2064, 1552, 592, 1), (1552, 2064, 1168, 1), (2576, 2512, 448, 0), (2560, 2560, 384, 0)])
 def test_workgroups_ask_for_a_large_c_at_different_times(gpu, orc, M, N, K, ct):
-    """From 12 MiB of C on: the workgroups of the 256x128 tiles ask for it in front of different rings of their loops (or, with no
+    """From 11 MiB of C on: the workgroups of the 256x128 tiles ask for it in front of different rings of their loops (or, with no
     ring, at the end).  The bits of the sum and one addition."""
     for name in ("tile256x128_pingpong", "tile128x256_pingpong"):
         kw = dict(M=M, N=N, K=K, a_layout=orc.ROW, c_type=ct)
@@ -302,6 +302,30 @@ def test_workgroups_ask_for_a_large_c_at_different_times(gpu, orc, M, N, K, ct):
         D = _run(gpu, orc, orc.GemmDesc(**kw), A, B, C, variant=_vid(gpu, name))
         S = _run(gpu, orc, orc.GemmDesc(use_c=0, **kw), A, B, None, variant=_vid(gpu, name))
         assert np.array_equal(D.view(np.uint32), (S + C.astype(F32)).view(np.uint32)), (name, M, N, K, ct)
+
+
+@pytest.mark.parametrize("K", (368, 384, 448, 576, 592, 640, 784, 832, 1040, 1600))
+def test_rings_of_pairs_that_a_large_c_is_asked_for_in_front_of(gpu, orc, K):
+    """None, one, two, three and more rings of three pairs, 11 MiB of Float32 and of Float16 C and just below, Float16 D: the bits of
+    the sum and one addition, and those of a call with C in D's place."""
+    for M, N, ct, name in ((1808, 1600, 1, "tile256x128_pingpong"), (2576, 2256, 0, "tile128x256_pingpong"), (1792, 1600, 1, "tile128x256_pingpong")):
+        kw = dict(M=M, N=N, K=K, a_layout=orc.ROW, c_type=ct, d_type=1)
+        A, B, C = _inputs(orc, orc.GemmDesc(**kw), 2750 + K, clo=-100.0, chi=100.0)
+        S = _run(gpu, orc, orc.GemmDesc(use_c=0, **kw), A, B, None, variant=_vid(gpu, name))
+        want = S + C.astype(F32)
+        assert np.array_equal(_run(gpu, orc, orc.GemmDesc(**kw), A, B, C, variant=_vid(gpu, name)).view(np.uint32), want.view(np.uint32)), (name, K)
+        kw["d_type"] = 0
+        assert np.array_equal(_run(gpu, orc, orc.GemmDesc(**kw), A, B, C, variant=_vid(gpu, name)).view(np.uint16),
+                              want.astype(F16).view(np.uint16)), (name, K)
+    M, N = 2048, 1536  # whole tiles
+    kw = dict(M=M, N=N, K=K, a_layout=orc.ROW)
+    A, B, C = _inputs(orc, orc.GemmDesc(**kw), 2760 + K, clo=-100.0, chi=100.0)
+    desc = gpu.GEMM.make_desc(M, N, K, a_layout=_W(gpu, orc.ROW), variant=_vid(gpu, "tile256x128_pingpong"))
+    dA, dB, dD = (gpu.DeviceArray(x) for x in (A, B, C))
+    gpu.GEMM.gemm(dA, dB, dD, dD, desc)
+    gpu.synchronize()
+    want = _run(gpu, orc, orc.GemmDesc(**kw), A, B, C, variant=_vid(gpu, "tile256x128_pingpong"))
+    assert np.array_equal(dD.to_host().view(np.uint32), want.view(np.uint32)), K
 
 
 def test_c_folded_into_the_loop_matches_the_epilogue_path(gpu, orc):
