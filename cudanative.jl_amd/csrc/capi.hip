@@ -160,7 +160,7 @@ bool tiled_fits(int i, const miw::gemm_params &p, int c_type, int d_type, bool f
     const long I = p.d_row ? p.N : p.M, J = p.d_row ? p.M : p.N;
     if (I < v.bm || J < v.bn || p.K < v.bk) return false;  // (K is a multiple of 16: a last slot that 64 does not divide is shifted back and masked)
     if (v.kind == miw::KIND_WAVE128 && p.K < 2 * v.bk) return false;  // (its loop is peeled over the last two slots)
-    if ((I % v.bm || J % v.bn) && in_place) return false;
+    if (in_place && (I % v.bm || J % v.bn)) return false;
     if (!miw::tiled_supports_layout(i, p) || !miw::tiled_grid_fits(i, p)) return false;
     if (!aligned16(p.A) || !aligned16(p.B) || !aligned16(p.D) || (p.use_c && !aligned16(p.C))) return false;
     if (p.lda % 8 || p.ldb % 8 || p.sa % 8 || p.sb % 8) return false;
@@ -346,7 +346,7 @@ int small_id()
     return id;
 }
 
-// 1-based id of the LDS-tiled variant for this problem and its estimated duration, 0 when none fits.
+// 1-based id of the LDS-tiled variant for this problem and its estimated duration, both 0 when none fits.
 int pick_tiled(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place, double *us_out = nullptr)
 {
     // Candidates in the order of variant_order(); a later candidate replaces an earlier one only when it is estimated 3 % faster.
@@ -364,12 +364,13 @@ int pick_tiled(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, i
 }
 
 // *kw: the tile of k_gemm_kwave where that runs in the picked variant's place, which is the smallest tile's, below 64 rows
-// or columns fragment_ops', or narrow_k_contiguous'.  The launch's own id is then shared_k_id().
-int pick_variant(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place, miw::kwave_tile *kw_out = nullptr)
+// or columns fragment_ops', or narrow_k_contiguous'.  The launch's own id is then shared_k_id().  *tiled_us: as pick_tiled's.
+int pick_variant(const miw::gemm_params &p, int c_type, int d_type, bool f16acc, int acc_chunk, bool in_place, miw::kwave_tile *kw_out = nullptr,
+                 double *tiled_us = nullptr)
 {
     // (a batch keeps the bits that each of its members has under the picked id)
     miw::kwave_tile kw = f16acc || p.batch > 1 ? miw::kwave_tile{0, 0} : miw::kwave_pays(p, c_type, d_type, in_place, cu_count());
-    int v = pick_tiled(p, c_type, d_type, f16acc, acc_chunk, in_place);
+    int v = pick_tiled(p, c_type, d_type, f16acc, acc_chunk, in_place, tiled_us);
     if (v) {
         if (miw::skinny_beats_tiles(p, d_type, f16acc)) v = narrow_id();
         else if (kw.bi) v = small_id();
@@ -1128,8 +1129,8 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     auto try_splits = [&](const miw::gemm_params &o, bool in_place, int s, int *variant, miw::kwave_tile *kw, double *us) {
         if (o.K % 64) return false;
         if (s == 1) {
-            if (!pick_tiled(o, d->c_type, d->d_type, false, 0, in_place, us)) return false;
-            *variant = pick_variant(o, d->c_type, d->d_type, false, 0, in_place, kw);
+            *variant = pick_variant(o, d->c_type, d->d_type, false, 0, in_place, kw, us);
+            if (*us == 0.0) return false;
             // (ragged extents are priced as a tile's launch, which is what C in D's place may get)
             if (kw->bi && o.M % 64 == 0 && o.N % 64 == 0) *us = miw::kwave_estimate_us(o, d->c_type, d->d_type, *kw);
             return true;
@@ -1155,19 +1156,24 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     miw::kwave_tile kw = {0, 0};
     double us = 0.0;
     // The slice count with the shortest estimated duration, among 1 (no second pass) and the counts up to 64 that leave
-    // every slice two LDS slots' worth of K or more; 0 when none fits.  equal: slices of one length only.  Of the others, whose last slice is shorter, those
-    // that fill the CUs once or twice with tiles of some size, and no more (a search over all counts took 27 us per call, as
-    // long as the launches), and that add up no fewer sums over K, four per slice where wavefronts share it, than the
-    // best equal ones: fewer and longer sums are further from the exact result (448x384x18944: 3.1e-7 with eight, 3.6e-7 with six).
+    // every slice two LDS slots' worth of K or more on average (the last one may have a single slot); 0 when none fits.
+    // equal: slices of one length only.  Of the others, whose last slice is shorter, those that fill the CUs once or twice
+    // with tiles of some size, and no more (a search over all counts took 27 us per call, as long as the launches), and that
+    // add up no fewer sums over K, four per slice where wavefronts share it, than the best equal ones: fewer and longer sums
+    // are further from the exact result (448x384x18944: 3.1e-7 with eight, 3.6e-7 with six).
     // Equal slices leave CUs without work where K / 64 has no fitting divisor: 160x208x29312 43.4 us in two, 14.5 in twelve;
     // 704x336x12416 27.6 in two, 16.7 in fourteen; 192x768x28416 22.4 in twelve, 20.4 in fourteen.
-    auto choose = [&](const miw::gemm_params &o, bool in_place, bool equal) {
+    auto choose = [&](const miw::gemm_params &o, bool in_place, bool equal, size_t most_bytes) {
         int best = 0, sums = 0;
         double best_us = 0.0;
+        const double mn = (double)o.M * (double)o.N;
         auto consider = [&](int s, int least) {
             int v;
             miw::kwave_tile t;
-            if ((s > 1 && o.K / s < 128) || bytes(s) > cap || !try_splits(o, in_place, s, &v, &t, &us)) return;
+            if ((s > 1 && o.K / s < 128) || bytes(s) > most_bytes || 4 * s < least) return;
+            // (below what try_splits will say, whatever it picks)
+            if (s > 1 && best && 6.0 + 0.03 * s + 8.0 * mn * s / 5.5e6 + 0.06 * (double)slice_slots(o, s) >= 0.97 * best_us) return;
+            if (!try_splits(o, in_place, s, &v, &t, &us)) return;
             const int n = s * (t.bi ? 4 : 1);
             if (n >= least && (best == 0 || us < 0.97 * best_us)) { best = s; best_us = us; sums = n; }
         };
@@ -1195,31 +1201,35 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     lines.A = lines.B = (const _Float16 *)&dummy;
     lines.C = p.use_c ? &dummy : nullptr;
     lines.D = &dummy;
-    // (a last slice shorter than the others: only with the count that is chosen here, and not for a workspace too small for it)
-    int count = splits;
-    if (splits == 0 || p.K % (64l * splits)) {
-        // (a program asks for the workspace and then calls: the thread's last choice is kept)
-        struct choice {
+    // A program asks for the workspace and then calls, for layer after layer: each thread keeps the counts of its last eight
+    // questions, which hang on the descriptor alone (one kept 1.0 us, chosen 2.3 to 4.3, on the host).
+    auto chosen = [&](bool equal, size_t most_bytes) {
+        struct question {
             miw_gemm_desc desc;
-            size_t cap;
-            int cus, count = -1;
+            size_t most_bytes;
+            int cus, equal, count;  // cus 0: none yet
         };
-        static thread_local choice last;
-        if (last.count < 0 || memcmp(&last.desc, d, sizeof *d) != 0 || last.cap != cap || last.cus != cu_count()) {
-            last.desc = *d;
-            last.cap = cap;
-            last.cus = cu_count();
-            last.count = choose(lines, false, false);
-        }
-        count = last.count;
-        if (splits && count != splits) count = 0;
-        if (!splits && bytes(count) > room) count = choose(lines, false, true);
+        static thread_local question kept[8];
+        static thread_local unsigned next;
+        for (const question &q : kept)
+            if (q.cus == cu_count() && q.equal == equal && q.most_bytes == most_bytes && memcmp(&q.desc, d, sizeof *d) == 0) return q.count;
+        question &q = kept[next++ % 8];
+        q = {*d, most_bytes, cu_count(), equal, choose(lines, false, equal, most_bytes)};
+        return q.count;
+    };
+    // A last slice shorter than the others: only with the count that is chosen here, and not for a workspace too small for it.
+    int count = splits;
+    if (splits == 0) {
+        count = chosen(false, cap);
+        if (bytes(count) > room) count = chosen(true, cap);
+    } else if (p.K % (64l * splits) && count != chosen(false, cap)) {
+        count = 0;
     }
     const bool runs = count && try_splits(p, shares, count, &variant, &kw, &us);
     if (!runs || bytes(count) > room) {
         // Addresses off 16 bytes, C in D's place with extents that no tile divides, or a workspace of another size than
         // the query's: what the real operands alone would choose.
-        const int other = splits ? 0 : choose(p, shares, true);
+        const int other = splits ? 0 : choose(p, shares, true, cap);
         if (other && bytes(other) <= room) {
             count = other;
             try_splits(p, shares, count, &variant, &kw, &us);

@@ -632,6 +632,31 @@ def test_splitk_slices_of_unequal_length_are_only_chosen(miw):
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stderr
 
 
+def test_splitk_counts_do_not_hang_on_earlier_questions(miw):
+    """More descriptors in turn than a thread keeps answers for, asked of both queries and from several threads: the answers of a
+    thread that asks one question only."""
+    import threading
+    G = miw.GEMM
+    descs = [G.make_desc(64 * m, 64 * n, 64 * k) for m, n, k in ((2, 3, 67), (4, 4, 256), (11, 5, 97), (7, 6, 296), (3, 12, 444), (21, 23, 374), (1, 1, 193), (8, 8, 128), (5, 5, 211), (16, 2, 60))]
+    ask = lambda i: (G.splitk_workspace(descs[i]), G.splitk_static_plan(descs[i]))  # noqa: E731
+    alone, turns = [None] * len(descs), [[] for _ in range(4)]
+
+    def first(i):
+        alone[i] = ask(i)
+
+    def many(t):
+        for step in (1, 3, 7):
+            turns[t].extend((i * step % len(descs), ask(i * step % len(descs))) for i in range(3 * len(descs)))
+
+    for run, count in ((first, len(descs)), (many, len(turns))):
+        threads = [threading.Thread(target=run, args=(i,)) for i in range(count)]
+        [t.start() for t in threads]
+        [t.join() for t in threads]
+    assert len({a for a in alone}) > 5
+    for got in turns:
+        assert len(got) == 9 * len(descs) and all(answer == alone[i] for i, answer in got)
+
+
 def test_tiled_gemm_kernels_are_not_launchable_by_name(miw):
     """The LDS-tiled kernels take a private argument block, a fixed workgroup and dynamic LDS: they can be
     looked up (attribute queries) but miw_launch refuses them and points to miw_gemm."""
