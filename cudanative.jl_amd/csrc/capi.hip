@@ -1217,12 +1217,13 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
         q = {*d, most_bytes, cu_count(), equal, choose(lines, false, equal, most_bytes)};
         return q.count;
     };
-    // A last slice shorter than the others: only with the count that is chosen here, and not for a workspace too small for it.
+    // A last slice shorter than the others: only with a count that is chosen here, by this entry or by the one with the other
+    // limit, and not for a workspace too small for it.
     int count = splits;
     if (splits == 0) {
         count = chosen(false, cap);
         if (bytes(count) > room) count = chosen(true, cap);
-    } else if (p.K % (64l * splits) && count != chosen(false, cap)) {
+    } else if (p.K % (64l * splits) && count != chosen(false, SIZE_MAX) && count != chosen(false, SPLITK_STATIC_BYTES)) {
         count = 0;
     }
     const bool runs = count && try_splits(p, shares, count, &variant, &kw, &us);
@@ -1244,8 +1245,8 @@ int plan_splitk(const miw_gemm_desc *d, const void *A, const void *B, const void
     }
     if (count == 0)
         return fail(MIW_ERR_UNSUPPORTED,
-                    "gemm_splitk: needs K divisible by 64 * splits, M and N of at least one LDS tile (64), "
-                    "16-byte aligned operands and leading dimensions");
+                    "gemm_splitk: needs K divisible by 64 * splits (by 64, with the count that the library chooses), M and N of at "
+                    "least one LDS tile (64), 16-byte aligned operands and leading dimensions");
     out->full = p;
     out->splits = count;
     out->variant = variant;

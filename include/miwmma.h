@@ -276,9 +276,12 @@ int miw_gemm_resolve(const miw_gemm_desc *desc, const void *A, const void *B, co
                      int *variant, int *acc_chunk);
 
 /* Split-K form of miw_gemm for problems with few output tiles and a long K: the chain of mma
-   calls over K (docs/src/device/wmma.md:51-52) is cut into `splits` slices (each a multiple
-   of 64 k-values; of one length where the count is asked for, the last one shorter where the library
-   chooses a count that needs it: that count may then be asked for too), the LDS-tiled kernels write every slice's product as Float32 into `workspace`
+   calls over K (docs/src/device/wmma.md:51-52) is cut into `splits` slices, each a multiple of 64
+   k-values: of one length, or the last one shorter where the library's own count needs that (a count
+   that miw_gemm_splitk_workspace or miw_gemm_splitk_static_plan chose on this machine may be asked for
+   by number; any other that does not divide K / 64 is refused).  With splits = 0 and a workspace too
+   small for that count the library chooses among slices of one length.  The LDS-tiled kernels write
+   every slice's product as Float32 into `workspace`
    (splits * m * n * 4 bytes, 16-byte aligned, contents on entry irrelevant), and a second kernel
    adds the slices in order: D = alpha * sum_s A_s*B_s + beta*C.  The result does not depend on
    timing; it differs from miw_gemm's by the rounding of one Float32 sum per slice.  Float32

@@ -632,6 +632,22 @@ def test_splitk_slices_of_unequal_length_are_only_chosen(miw):
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stderr
 
 
+def test_splitk_takes_the_counts_that_either_query_answers(miw):
+    """The static workspace's limit makes its query answer with other counts, of unequal slices too: asked for by number they are
+    taken by both entries, and one that does not fit is refused for its size."""
+    G, L = miw.GEMM, miw._lib
+    for M, N, K in ((1376, 1504, 23936), (592, 1696, 32000), (2048, 864, 32704), (1776, 1632, 12352)):
+        d = G.make_desc(M, N, K)
+        n, nbytes = G.splitk_static_plan(d)
+        more, more_bytes = G.splitk_workspace(d)
+        assert 1 < n < more and K // 64 % n and more_bytes > G.splitk_static_capacity() >= nbytes
+        assert G.splitk_workspace(d, n) == G.splitk_static_plan(d, n) == (n, nbytes)
+        assert G.splitk_workspace(d, more) == (more, more_bytes)
+        with pytest.raises(miw.MIWError, match="the static workspace holds") as e:
+            G.splitk_static_plan(d, more)
+        assert e.value.code == L.ERR_UNSUPPORTED
+
+
 def test_splitk_counts_do_not_hang_on_earlier_questions(miw):
     """More descriptors in turn than a thread keeps answers for, asked of both queries and from several threads: the answers of a
     thread that asks one question only."""
