@@ -281,7 +281,10 @@ elems_per_lane(::Type{U}, ::Type{T}) where {U, T} =
 image_bytes(::Type{U}, ::Type{T}) where {U, T} =
     Int(ccall((:miw_frag_image_bytes, libmiwmma), Csize_t, (Cint, Cint), use_code(U), dtype_code(T)))
 
-"Device memory for one image; `reuse`: of the default stream's operations only (see miwmma.h)."
+"""
+Device memory for one image; `reuse`: of the default stream's operations only (see miwmma.h).  For programs that keep
+images of their own: a fragment's image here is a DeviceBuffer, which any stream may be given and a finalizer frees.
+"""
 function image_new(bytes::Integer, reuse::Bool)
     p = Ref{Ptr{Cvoid}}(C_NULL)
     check(ccall((:miw_frag_image_new, libmiwmma), Cint, (Csize_t, Cint, Ptr{Ptr{Cvoid}}), bytes, reuse, p))
