@@ -247,9 +247,10 @@ struct image_pool {
         std::pair<int, int> key;  // device and size
         bool idle;
     };
+    using table = std::unordered_map<void *, image>;
     std::mutex mu;
-    std::map<std::pair<int, int>, std::vector<void *>> idle;
-    std::unordered_map<void *, image> all;  // idle or in a caller's hands
+    table all;  // idle or in a caller's hands
+    std::map<std::pair<int, int>, std::vector<table::value_type *>> idle;
 };
 image_pool &images()
 {
@@ -267,7 +268,7 @@ hipError_t device_malloc(void **out, size_t bytes)
         image_pool &pool = images();
         std::lock_guard<std::mutex> lock(pool.mu);
         for (auto &[key, list] : pool.idle) {
-            idle.insert(idle.end(), list.begin(), list.end());
+            for (auto *entry : list) idle.push_back(entry->first);
             list.clear();
         }
         for (void *p : idle) pool.all.erase(p);
@@ -802,9 +803,9 @@ int miw_frag_image_new(size_t bytes, int reuse, void **image)
         std::lock_guard<std::mutex> lock(pool.mu);
         auto &idle = pool.idle[{device, size}];
         if (!idle.empty()) {
-            *image = idle.back();
+            *image = idle.back()->first;
+            idle.back()->second.idle = false;
             idle.pop_back();
-            pool.all.at(*image).idle = false;
             return 0;
         }
     }
@@ -826,7 +827,7 @@ int miw_frag_image_release(void *image, int reuse)
             return fail(MIW_ERR_INVALID_VALUE, "frag_image_release: not an image of miw_frag_image_new, or released before");
         auto &idle = pool.idle[it->second.key];
         if (reuse && idle.size() < IDLE_IMAGES) {
-            idle.push_back(image);
+            idle.push_back(&*it);
             it->second.idle = true;
             return 0;
         }
