@@ -207,7 +207,7 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
 #endif
     // A large C that all workgroups ask for at once is a burst that the first slots do not cover; a workgroup that asks for
     // it in mid-loop waits too, for one latency.  256x128 tiles, one time and eight, by rows of tiles and by columns: 32 MiB
-    // 71.1 us, 70.2 and 68.0 (8192x1024x4096); one time and two: 35 MiB 30.0 and 27.7 (7552x1216x512), 24 MiB 15.4 and 14.4
+    // 72.6 us, 69.5 and 68.3 (8192x1024x4096); one time and two: 35 MiB 30.0 and 27.7 (7552x1216x512), 24 MiB 15.4 and 14.4
     // (5632x1104x448, Float16 D), 11.9 MiB 17.7 and 17.1 (5632x1104x832, Float16); from 4 to 10 MiB it is 0.5 to 1 % behind.
     // 128x128 tiles keep one time: to choose costs their loops 1 to 3 %, what it gives (2048x2048x2048 21.5 and 20.6) and
     // more where C is small (1024x1536x2048 16.2 and 16.5).
@@ -252,8 +252,10 @@ hipError_t launch_gemm_tiled(int i, const gemm_params &g, int c_type, int d_type
 // `ws`, each I x J with I contiguous (canonical form: I runs along D's contiguous dimension);
 // this adds them in slice order and applies the scalars: D = alpha * sum_s P_s + beta * C.
 // One lane owns four consecutive i of one j.  Bound by the launch and the memory's latency: C and up to sixteen slices are
-// on the way at a time (four at a time, and C behind them: 512x512x16384 in sixteen slices 18.6 us, 17.8 like this;
-// 128x128x32768 12.5 and 10.9).
+// on the way at a time, four elements in an access, one wavefront per workgroup where D is small.  In two kernel traces of
+// whole calls: 512x512 in sixteen slices, element by element and C behind four slices at a time, 5.5 and 5.6 us, like this
+// 4.7 and 5.0, with four slices on the way 4.5 and 4.7 (the calls: 20.9 us, 20.0 and 19.9); 128x128 in sixteen 4.0 and 4.1,
+// 3.5 and 3.8, 3.8 and 3.9 (the calls: 12.8 us, 11.0 and 11.6).
 struct reduce_params {
     const float *ws;
     const void *C;

@@ -298,7 +298,7 @@ __device__ __attribute__((always_inline)) inline void gemm_kwave(const tiled_par
 
 // A launch pays for the instructions it passes by, which it fetches from a cold cache: so the types, and whether there is a C,
 // are the instance's.  With both asked for at run time decode 16x4096x4096 takes 8.17 us, 8.02 like this, 128x4096x4096
-// 11.5 and 11.1, 640x576x1840 8.3 and 8.0, 720x656x784 with a Float32 C 6.40 and 6.25.
+// 11.5 and 11.1, 640x576x1840 8.3 and 8.0, 720x656x784 with a Float32 C 6.24 and 5.99.
 // Float32 C and D.
 template <int BI, int BJ, bool XK, bool YK>
 __global__ __launch_bounds__(64 * KWAVES) __attribute__((amdgpu_waves_per_eu(2)))

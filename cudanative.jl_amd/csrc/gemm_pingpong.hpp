@@ -870,11 +870,13 @@ void k_gemm_pp64(tiled_params p)
     // Float32 accumulation: C laid out as D goes into registers while the loop runs (request_c), in the whole lines in which D
     // is stored.  (Added to the sums in the loop's last pairs, as k_gemm_pp_fold does, it costs those pairs a quarter more each,
     // and read behind the loop two loads at a time it waits for memory once per pair of tiles: 8192x1024x4096 from HBM
-    // 73.2 us -> 69.4, 7120x1024x720 with a Float16 C 19.4 -> 17.8, 2048x2048x128 11.1 -> 9.2.)
+    // 73.1 us -> 68.0, with the times of tiled_params::c_spread, 7120x1024x720 with a Float16 C 18.9 -> 17.9, 2048x2048x128
+    // 11.1 -> 8.9.  128x128 tiles in one round with a Float32 C, alpha of 1 and K above 1024 are 1 to 2.5 % behind the
+    // folded form, whose sums are further from the exact result: 2048x2048x2048 20.4 -> 20.9, 1600x2064x2048 18.6 -> 19.0.)
     using cpieces = c_pieces<TI, TJ, CT>;
     cpieces cp;
     // Problems without C have instances of their own, without C's registers: 1280x5168x1408 23.0 us -> 22.6, 8192x768x1024
-    // 17.8 -> 17.2, 1024x3072x1024 11.3 -> 11.1 (2048^3 22.1 -> 22.7, as before C waited in registers).
+    // 17.9 -> 17.7, 1024x3072x1024 11.5 -> 11.0 (2048^3 level).
     constexpr bool HAS_C = !__is_same(CT, no_c_t);
     const bool early = HAS_C && !F16ACC && p.use_c && !p.c_trans;
     auto request_c = [&]() MIW_INLINE { cp.request(C + (long)(j0 + wj * WTJ) * p.ldc + (i0 + wi * WTI) + pair_place(lane, p.ldc), p.ldc); };

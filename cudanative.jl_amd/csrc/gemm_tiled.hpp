@@ -102,8 +102,8 @@ struct tiled_params {
         int work;
         int k_short;  // see short_member
     };
-    // k_gemm_pp64: the workgroups ask for C at eight different times of their K loops, not all at its start.  k_gemm_pp: they
-    // start at four different times.
+    // k_gemm_pp64: the workgroups ask for C at up to eight different times of their K loops, not all at its start.  k_gemm_pp:
+    // they start at four different times.
     int c_spread;
 #ifdef MIW_PP_TS
     long long *ts;  // measurement builds: 10 counters per wavefront (see k_gemm_pp64), or null
@@ -724,7 +724,7 @@ void k_gemm_tiled(tiled_params p)
     fetch_result_arguments(p);
     // C laid out as D goes into registers behind the first requests: read behind the loop, two loads at a time, it waits for
     // memory once per pair of tiles (64x64 tiles: 768x1216x832 with a Float16 C 5.9 us -> 5.5, 672x864x512 5.1 -> 4.6;
-    // 128x128 tiles, two workgroups per CU: 512 problems of 128^3 19.4 -> 18.9, 192x128x256 397 times 33.8 -> 32.2).
+    // 128x128 tiles, two workgroups per CU: 192x128x256 397 times 33.8 -> 32.2; 512 problems of 128^3, at a copy's rate, 19.5 both).
     // Problems without C have instances of their own: a short launch pays for the instructions it passes by, which it fetches
     // from a cold cache (640x640x496 4.52 us -> 4.40, 400 products of 64x128x96 7.72 -> 7.43).
     constexpr bool HAS_C = !__is_same(CT, no_c_t);

@@ -21,7 +21,7 @@ struct gemm_params {
     int use_c;
     float alpha, beta;
     // Slices of K as a batch (split-K): k-values of the last member where they are fewer than K, a multiple of 64; else 0.
-    // Not for the kernels with 256x256 tiles, which may walk from member to member.
+    // Not for the 32-k ping-pong kernel (KIND_PINGPONG32), which may walk from member to member, nor for KIND_WAVE128.
     long k_last;
 };
 
